@@ -521,6 +521,17 @@ int lq_rmsnorm_rope(void* out, const void* qkv, const void* context_qkv, const v
                     const void* rope, size_t rope_batch_stride, lq_dtype_t dtype, int batch, int seq, int context_seq,
                     int heads, int head_dim, float eps, lq_stream_t stream);
 
+/* Softmax attention without mask: out[b, i, h, :] = sum_j softmax_j(scale * q[b, i, h, :] . k[b, j, h, :]) v[b, j, h, :], fp32
+ * scores and accumulation (the flash attention the reference's attention processors call,
+ * layers/flux_attention_processor/FluxAttentionFP8Processor.cc:246-291,
+ * layers/basic_transformer/BasicTransformerInt8Block.cc:330-420).  q, k, v: heads of head_dim (64 or 128) elements side by side
+ * in a token, tokens *_row elements and batches *_batch elements apart (parts of a fused QKV tensor are strided tensors);
+ * out [batch, seq_q, heads, head_dim] dense.  dtype F16 or BF16; pointers 16-byte aligned, strides multiples of 8 elements;
+ * seq_k * k_row and seq_k * v_row below 2^31. */
+int lq_attention(void* out, const void* q, size_t q_row, size_t q_batch, const void* k, size_t k_row, size_t k_batch, const void* v,
+                 size_t v_row, size_t v_batch, lq_dtype_t dtype, int batch, int seq_q, int seq_k, int heads, int head_dim, float scale,
+                 lq_stream_t stream);
+
 /* dst[i] = T( dst[i] + T( src[i] * T(alpha) ) ): merges a full-rank LoRA delta into a 16-bit (or fp32) weight
  * (invokeLoadLora, kernels/lora/load_lora.h + load_lora.cu:6-14,92-96).  An FP8 weight is re-quantised after the
  * merge the way FP8LoraWeight::load_lora / clear_lora do (interface/IFLoraWeight.h:79-128): restore the 16-bit

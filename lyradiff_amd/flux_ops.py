@@ -7,8 +7,7 @@ th_op/flux_single_transformer_block/FluxSingleTransformerBlockOp.cc:6-98), so th
 (lyradiff/lyradiff_model/lyradiff_flux_transformer_model_v2.py:67-168) can hold one of these instead of a
 `torch.classes.lyradiff.*` object.  Every quantized linear, every adaLN / gate / residual step and every activation
 quantisation runs on this library's HIP kernels (flux_fp8.py), as do the per-head RMSNorm of q and k and the rotary
-embedding behind the QKV projection (lq_rmsnorm_rope); the softmax attention itself is not part of the quantized-linear
-path and is PyTorch's (`flux_attention_core`).
+embedding behind the QKV projection (lq_rmsnorm_rope) and the softmax attention (lq_attention).
 
 Supported quant levels: FP8_W8A8, FP8_W8A8_FULL, INT4_W4A4 and INT4_W4A4_FULL (W4A4 linears with their low-rank branch,
 th_op/flux_transformer_block/FluxTransformerBlockOp.h:165-182).  Any other level raises at construction.
@@ -48,17 +47,19 @@ def flux_attention_core(qkv: torch.Tensor, norm_q: torch.Tensor, norm_k: torch.T
     """The part of FluxAttentionFP8Processor::forward (FluxAttentionFP8Processor.cc:232-291) and
     FluxSingleAttentionFP8Processor::forward (FluxSingleAttentionFP8Processor.cc:183-213) between the QKV and the output
     projections: q/k RMSNorm per head, rotary embedding and the [text, image] concatenation in one HIP kernel
-    (ops.rmsnorm_rope = invokeFusedRmsNormCatAndRope), then softmax attention (PyTorch) on its [B, S, 3, H, Dh] output.
+    (ops.rmsnorm_rope = invokeFusedRmsNormCatAndRope), then softmax attention on its [B, S, 3, H, Dh] output.
     With `context_qkv` (image [B, S, D], text [B, Sc, D]) is returned; without it a single [B, S, D] tensor."""
-    b, s, d3 = qkv.shape
-    d = d3 // 3
-    sc = 0 if context_qkv is None else context_qkv.shape[1]
     added = None if context_qkv is None else torch.cat([norm_added_q, norm_added_k])
-    cat = ops.rmsnorm_rope(qkv.contiguous(), torch.cat([norm_q, norm_k]), rope_emb.contiguous(), heads,
-                           None if context_qkv is None else context_qkv.contiguous(), added)
-    q, k, v = (cat[:, :, i].transpose(1, 2) for i in range(3))  # [B, H, Sc + S, Dh] views
-    o = torch.nn.functional.scaled_dot_product_attention(q, k, v)
-    o = o.transpose(1, 2).reshape(b, sc + s, d)
+    return _attention_core(qkv, torch.cat([norm_q, norm_k]), rope_emb, heads, context_qkv, added)
+
+
+def _attention_core(qkv, norm_qk, rope_emb, heads, context_qkv=None, norm_added_qk=None):
+    """flux_attention_core with the norm weights as [2 * Dh] (q then k), as the block classes keep them."""
+    b, s, d3 = qkv.shape
+    sc = 0 if context_qkv is None else context_qkv.shape[1]
+    cat = ops.rmsnorm_rope(qkv.contiguous(), norm_qk, rope_emb.contiguous(), heads,
+                           None if context_qkv is None else context_qkv.contiguous(), norm_added_qk)
+    o = ops.softmax_attention(cat[:, :, 0], cat[:, :, 1], cat[:, :, 2]).reshape(b, sc + s, d3 // 3)
     if context_qkv is None:
         return o
     return o[:, sc:], o[:, :sc]
@@ -150,6 +151,7 @@ class FluxTransformerBlockOp(_BlockOpBase):
         get = W._source(src)
         self.norms = [get(prefix + f"attn.{n}.weight", (self.head_dim,), self.dtype).to(self.device)
                       for n in ("norm_q", "norm_k", "norm_added_q", "norm_added_k")]
+        self.norm_qk, self.norm_added_qk = torch.cat(self.norms[:2]), torch.cat(self.norms[2:])
 
     def _fp8_linears(self):
         w = self._loaded()
@@ -165,8 +167,7 @@ class FluxTransformerBlockOp(_BlockOpBase):
         for n, t in (("hidden_states", hidden_states), ("encoder_hidden_states", encoder_hidden_states),
                      ("rope_emb", rope_emb), ("temb_emb", temb_emb)):
             self._check(n, t)
-        nq, nk, naq, nak = self.norms
-        core = lambda qkv, cqkv: flux_attention_core(qkv, nq, nk, rope_emb, self.heads, cqkv, naq, nak)
+        core = lambda qkv, cqkv: _attention_core(qkv, self.norm_qk, rope_emb, self.heads, cqkv, self.norm_added_qk)
         block = I4.flux_double_block_int4 if self.int4 else F.flux_double_block_fp8
         out, ctx = block(hidden_states, encoder_hidden_states, temb_emb, w, core)
         return [out, ctx]
@@ -191,6 +192,7 @@ class FluxSingleTransformerBlockOp(_BlockOpBase):
                                                         keep_master=True, full=self.quant_level is LyraQuantLevel.FP8_W8A8_FULL)
         get = W._source(src)
         self.norms = [get(prefix + f"attn.{n}.weight", (self.head_dim,), self.dtype).to(self.device) for n in ("norm_q", "norm_k")]
+        self.norm_qk = torch.cat(self.norms)
 
     def _fp8_linears(self):
         w = self._loaded()
@@ -200,6 +202,5 @@ class FluxSingleTransformerBlockOp(_BlockOpBase):
         w = self._loaded()
         for n, t in (("hidden_states", hidden_states), ("rope_emb", rope_emb), ("temb_emb", temb_emb)):
             self._check(n, t)
-        nq, nk = self.norms
         block = I4.flux_single_block_int4 if self.int4 else F.flux_single_block_fp8
-        return block(hidden_states, temb_emb, w, lambda qkv: flux_attention_core(qkv, nq, nk, rope_emb, self.heads))
+        return block(hidden_states, temb_emb, w, lambda qkv: _attention_core(qkv, self.norm_qk, rope_emb, self.heads))

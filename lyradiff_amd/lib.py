@@ -110,6 +110,7 @@ SYMBOLS = {
     "lq_lora_down": (_I, [_P, _I, _P, _P, _I, _I, _I, _I, _P]),
     "lq_w4a4_quantize_lora_down": (_I, [_P, _P, _I, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _P]),
     "lq_rmsnorm_rope": (_I, [_P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _F, _P]),
+    "lq_attention": (_I, [_P, _P, _Z, _Z, _P, _Z, _Z, _P, _Z, _Z, _I, _I, _I, _I, _I, _I, _F, _P]),
     "lq_cast_f32": (_I, [_P, _I, _P, _Z, _P]),
     "lq_load_lora": (_I, [_P, _P, _I, _Z, _F, _P]),
     "lq_gemm_set_tactic": (_I, [_I, _I]),

@@ -953,6 +953,45 @@ def rmsnorm_rope(qkv, norm_qk, rope, heads: int, context_qkv=None, norm_added_qk
     return out
 
 
+def attention_supported(q, k, v) -> bool:
+    """True when `attention` runs q [B, Sq, H, Dh], k and v [B, Sk, H, Dh]: 16-bit tensors on the GPU, heads of 64 or 128
+    elements side by side in a token, 16-byte aligned tokens, no gradient recorded, keys within the kernel's 32-bit offsets."""
+    dh, width = q.shape[-1], q.shape[-2] * q.shape[-1]
+    if dh not in (64, 128) or q.dtype not in (torch.float16, torch.bfloat16) or q.numel() == 0 or k.numel() == 0:
+        return False
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+        return False
+    for t in (q, k, v):
+        if not t.is_cuda or t.dtype != q.dtype or t.stride(3) != 1 or (t.stride(2) != dh and t.shape[2] > 1) or t.data_ptr() % 16 or \
+                (t.stride(1) % 8 and t.shape[1] > 1) or (t.stride(0) % 8 and t.shape[0] > 1) or t.stride(1) < width:
+            return False
+    longest = max(k.stride(1), v.stride(1))
+    return longest < 1 << 23 and k.shape[1] * longest < 1 << 31 and q.stride(1) % 8 == 0 and longest % 8 == 0
+
+
+def attention(q, k, v, scale=None):
+    """Softmax attention without mask: q [B, Sq, H, Dh], k and v [B, Sk, H, Dh] (views into a fused QKV tensor are fine) ->
+    [B, Sq, H, Dh], contiguous.  `scale` defaults to Dh ** -0.5.  See attention_supported for what it takes."""
+    if k.shape != v.shape or k.shape[0] != q.shape[0] or k.shape[2:] != q.shape[2:]:
+        raise ValueError("attention: q must be [B, Sq, H, Dh], k and v [B, Sk, H, Dh]")
+    if not attention_supported(q, k, v):
+        raise ValueError("attention: needs fp16 / bf16 device tensors of 64- or 128-wide heads, dense within a token, 16-byte aligned")
+    b, sq, h, dh = q.shape
+    sk = k.shape[1]
+    batch = lambda t: t.stride(0) if b > 1 else 0
+    out = torch.empty((b, sq, h, dh), dtype=q.dtype, device=q.device)
+    _l.check(_l.load().lq_attention(_ptr(out), _ptr(q), q.stride(1), batch(q), _ptr(k), k.stride(1), batch(k), _ptr(v), v.stride(1), batch(v),
+                                    _DT[q.dtype], b, sq, sk, h, dh, float(dh ** -0.5 if scale is None else scale), _stream()), "lq_attention")
+    return out
+
+
+def softmax_attention(q, k, v):
+    """attention where it runs, PyTorch's elsewhere (other head sizes and types)."""
+    if attention_supported(q, k, v):
+        return attention(q, k, v)
+    return torch.nn.functional.scaled_dot_product_attention(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)).transpose(1, 2)
+
+
 _KINDS = {"int8": _l.LQ_W_INT8, "fp8": _l.LQ_W_FP8, "int4": _l.LQ_W_INT4}
 
 

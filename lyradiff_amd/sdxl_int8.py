@@ -19,7 +19,7 @@
       out       = (q8 . Wff^T + bff) + h2                          runGemmInt8, invokeFusedBiasResidualAdd
 
   The 16-bit linears of the lower levels and the text K/V projections are not quantized linears and run as plain PyTorch
-  matmuls; softmax attention is PyTorch's as well.  Weight keys follow BasicTransformerInt8BlockWeight::loadWeights
+  matmuls; softmax attention is ops.softmax_attention.  Weight keys follow BasicTransformerInt8BlockWeight::loadWeights
   (BasicTransformerInt8BlockWeight.cc:232-288): `<name>.weight_int8`, `.weight_quant_scale`, `.input_quant_scale`,
   `.pre_quant_scale` for an INT8 linear (MACROLoadLinearInt8WeightFromBin, utils/common_macro_def.h:51-59), `.weight` /
   `.bias` for 16-bit tensors, `norm{1,2,3}.weight` / `.bias`.
@@ -96,9 +96,8 @@ def _gemm_int8(q8: torch.Tensor, lin: Int8Linear, dtype, bias=None) -> torch.Ten
 
 def _attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int) -> torch.Tensor:
     b, s, d = q.shape
-    split = lambda t: t.view(b, t.shape[1], heads, d // heads).transpose(1, 2)
-    o = torch.nn.functional.scaled_dot_product_attention(split(q), split(k), split(v))
-    return o.transpose(1, 2).reshape(b, s, d)
+    split = lambda t: t.view(b, t.shape[1], heads, d // heads)
+    return ops.softmax_attention(split(q), split(k), split(v)).reshape(b, s, d)
 
 
 def _ln16(x, gb, eps):

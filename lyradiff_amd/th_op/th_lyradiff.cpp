@@ -9,14 +9,15 @@
 //
 // Quant levels 1, 2 (FP8_W8A8, FP8_W8A8_FULL) and 7, 8 (INT4_W4A4, INT4_W4A4_FULL) are built, the levels whose blocks
 // consist of quantized linears.  Every quantized linear, adaLN / gate / residual step, activation quantisation, the q/k
-// RMSNorm and the rotary embedding run on liblyraquant.so through its C ABI; PyTorch supplies device memory, the current
-// stream, the softmax attention between the projections and the 16-bit adaLN matmul of the non-FULL levels.
+// RMSNorm, the rotary embedding and the softmax attention run on liblyraquant.so through its C ABI; PyTorch supplies device
+// memory, the current stream and the 16-bit adaLN matmul of the non-FULL levels.
 // This file holds no device code and is compiled with the host compiler.
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/custom_class.h>
 #include <torch/script.h>
 
+#include <cmath>
 #include <cstdio>
 #include <map>
 #include <memory>
@@ -240,7 +241,7 @@ at::Tensor adaln_16(const at::Tensor& x, const at::Tensor& msa) {
 }
 
 // q/k RMSNorm + rotary embedding + [text, image] concatenation in one kernel (invokeFusedRmsNormCatAndRope,
-// kernels/rope/flux_apply_rope.cu:74-156), then softmax attention on its [B, Sc + S, 3, H, Dh] output.
+// kernels/rope/flux_apply_rope.cu:74-156), then softmax attention (lq_attention) on its [B, Sc + S, 3, H, Dh] output.
 // Returns [B, Sc + S, D] with the text tokens first.
 at::Tensor attention_core(const at::Tensor& qkv, const at::Tensor& ctx_qkv, const at::Tensor& norm_qk, const at::Tensor& norm_added_qk,
                           const at::Tensor& rope, int64_t heads) {
@@ -252,9 +253,14 @@ at::Tensor attention_core(const at::Tensor& qkv, const at::Tensor& ctx_qkv, cons
     ok(lq_rmsnorm_rope(P(cat), P(qkv), P(ctx_qkv), P(norm_qk), P(norm_added_qk), P(rope), rope.numel() != per_batch ? (size_t)per_batch : 0,
                        lq_dt(qkv.scalar_type()), (int)b, (int)s, (int)sc, (int)heads, (int)dh, 1e-6f, cur_stream()),
        "lq_rmsnorm_rope");
-    at::Tensor o = at::scaled_dot_product_attention(cat.select(2, 0).transpose(1, 2), cat.select(2, 1).transpose(1, 2),
-                                                    cat.select(2, 2).transpose(1, 2));
-    return o.transpose(1, 2).reshape({b, sc + s, d});
+    // q, k and v are strided parts of `cat`; dh is 64 or 128 here, lq_rmsnorm_rope takes no other
+    const char* parts = static_cast<const char*>(P(cat));
+    const size_t row = (size_t)(3 * d), batch = row * (size_t)(sc + s), part = (size_t)d * cat.element_size();
+    at::Tensor o = at::empty({b, sc + s, d}, qkv.options());
+    ok(lq_attention(P(o), parts, row, batch, parts + part, row, batch, parts + 2 * part, row, batch, lq_dt(qkv.scalar_type()), (int)b,
+                    (int)(sc + s), (int)(sc + s), (int)heads, (int)dh, 1.0f / std::sqrt((float)dh), cur_stream()),
+       "lq_attention");
+    return o;
 }
 
 // FluxAttnPostFP8Processor::forward (FluxAttnPostFP8Processor.cc:93-240) in three launches

@@ -1,0 +1,73 @@
+"""lq_attention against softmax attention evaluated in fp32 on the same 16-bit operands."""
+import ctypes as C
+
+import pytest
+import torch
+
+# (batch, queries, keys, heads, head_dim): one key, tiles of 64 keys less / exactly / more than full, 32-query wavefronts and the
+# blocks of 128 and 256 queries at their edges; with 24 heads 1408 queries are 264 blocks of 128, more than there are compute
+# units, which takes the form with two wavefront groups (head_dim 128), 1280 are 240
+SHAPES = [(1, 1, 1, 1, 128), (2, 33, 63, 3, 128), (1, 127, 64, 2, 64), (2, 128, 65, 3, 64), (1, 129, 77, 5, 64), (1, 257, 129, 2, 128),
+          (3, 96, 300, 4, 64), (1, 1280, 191, 24, 128), (1, 1408, 1, 24, 128), (1, 1409, 64, 24, 128), (1, 1471, 65, 24, 128),
+          (1, 1408, 128, 24, 128), (1, 1535, 260, 24, 128), (2, 1025, 1025, 16, 128)]
+
+
+def _reference(q, k, v, scale):
+    """(O, softmax(S) |V|) in fp32, head by head."""
+    o = torch.empty(q.shape, dtype=torch.float32, device=q.device)
+    mag = torch.empty_like(o)
+    for b in range(q.shape[0]):
+        for h in range(q.shape[2]):
+            p = ((q[b, :, h].float() @ k[b, :, h].float().t().contiguous()) * scale).softmax(-1)
+            vf = v[b, :, h].float().contiguous()
+            o[b, :, h], mag[b, :, h] = p @ vf, p @ vf.abs()
+    return o, mag
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_attention_matches_fp32(dev, shape, dt):
+    from lyradiff_amd import ops
+
+    b, sq, sk, h, dh = shape
+    g = torch.Generator(device=dev).manual_seed(sq * 1000 + sk)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    if sq == sk:  # parts of one fused tensor
+        q, k, v = (1.5 * rnd(b, sq, 3, h, dh)).to(dt).unbind(2)
+    else:
+        q, (k, v) = (1.5 * rnd(b, sq, h, dh)).to(dt), (1.5 * rnd(b, sk, 2, h, dh)).to(dt).unbind(2)
+    got = ops.attention(q, k, v)
+    assert got.shape == q.shape and got.is_contiguous()
+    want, mag = _reference(q, k, v, dh ** -0.5)
+    # u: rounding error of T.  Probabilities rounded to T, summed as rounded, the result rounded to T: 3 u of the sum of |terms|.
+    # Absolute part: scores in fp32 over dh products of size ~ 1.5^2 and the exponentials, a few 1e-6; fp16 probabilities under
+    # 2^-14 are rounded to a fixed step, 2^-25 for each of at most 1025 keys times |v| ~ 1.2: 4e-5
+    u = 2.0 ** -11 if dt is torch.float16 else 2.0 ** -8
+    assert ((got.float() - want).abs() <= 3 * u * mag + 5e-5).all()
+    assert torch.equal(got, ops.softmax_attention(q, k, v))
+
+
+@pytest.mark.gpu
+def test_attention_of_other_shapes_falls_back(dev):
+    from lyradiff_amd import ops
+
+    for dh, dt in ((40, torch.float16), (64, torch.float32), (160, torch.bfloat16)):
+        q, k, v = torch.randn(1, 20, 3, 2, dh, device=dev).to(dt).unbind(2)
+        assert not ops.attention_supported(q, k, v)
+        want, _ = _reference(q, k, v, dh ** -0.5)
+        assert (ops.softmax_attention(q, k, v).float() - want).abs().max() < 2e-2
+        with pytest.raises(ValueError):
+            ops.attention(q, k, v)
+
+
+def test_attention_argument_errors_do_not_reach_the_gpu():
+    from lyradiff_amd import lib as L
+
+    lib, one = L.load(), C.c_void_p(16)
+    call = lambda **kw: lib.lq_attention(*{**dict(out=one, q=one, qr=384, qb=0, k=one, kr=384, kb=0, v=one, vr=384, vb=0, dt=L.LQ_BF16, b=1, sq=8,
+                                                  sk=8, h=3, dh=128, s=1.0, st=None), **kw}.values())
+    assert call(dt=L.LQ_F32) == -4
+    assert call(dh=96) == -2 and call(sk=0) == -2 and call(kr=376) == -2 and call(sk=1 << 23) == -2
+    assert call(q=None) == -1 and call(q=C.c_void_p(8)) == -1 and call(qr=388) == -1
+    assert call(sq=0) == 0
