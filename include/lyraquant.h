@@ -502,6 +502,21 @@ int lq_w4a4_quantize_lora_down(uint32_t* q_words, void* scales, lq_dtype_t scale
                                lq_dtype_t act_dtype, const void* x, lq_dtype_t x_dtype, const float* smooth,
                                const void* lora_down, int m, int k, int rank, int group, lq_stream_t stream);
 
+/* W4A4 on codes: the same quantisation and the same GEMM (every result bit for bit that of the calls above with fp32 group
+ * scales) on operands that keep one e4m3 byte per 4-bit value -- every integer of [-8, 8] is an e4m3 number, so the fp8 matrix
+ * instruction forms the exact group sums -- and the group scales group-major, [k / 64][rows].
+ *   lq_w4a4_expand_rows32: packed weights in rows32 layout [n, k / 2] -> codes in rows32 layout [n, k]; n, k multiples of 32.
+ *   lq_w4a4_quantize_lora_down_codes: lq_w4a4_quantize_lora_down with codes [m, k] and scales [k / 64, m]; smooth required, rank 32,
+ *     k % 128 == 0, k <= 16384, lora_act in x's type (F16 or BF16).
+ *   lq_gemm_w4a4_codes: lq_gemm_w4a4_ex with sA [k / 64, m] and sB [k / 64, n] fp32; output F16 or BF16. */
+int lq_w4a4_expand_rows32(uint8_t* codes, const uint8_t* packed, size_t n, size_t k, lq_stream_t stream);
+int lq_w4a4_quantize_lora_down_codes(uint8_t* codes, float* scales, void* lora_act, lq_dtype_t act_dtype, const void* x,
+                                     lq_dtype_t x_dtype, const float* smooth, const void* lora_down, int m, int k, int rank,
+                                     lq_stream_t stream);
+int lq_gemm_w4a4_codes(void* C, lq_dtype_t out_dtype, const uint8_t* A_codes, const uint8_t* B_codes_rows32, const float* sA,
+                       const float* sB, const void* bias, const void* lora_act, const void* lora_up, lq_dtype_t lora_dtype,
+                       int lora_rank, int m, int n, int k, const lq_epilogue_t* epi, lq_stream_t stream);
+
 /* dst[i] = T(src[i]), the float -> T copy between the reference's two W4A4 kernels
  * (invokeCudaD2DcpyConvert<T, float>, utils/memory_utils.cu:398-402). */
 int lq_cast_f32(void* dst, lq_dtype_t dst_dtype, const float* src, size_t n, lq_stream_t stream);

@@ -236,9 +236,9 @@ __device__ __forceinline__ int cvt_i32_sat(float x) {
 // CLAMP false: the caller guarantees |t[i]| <= LIMIT * s * (1 + 2^-20) with LIMIT = HI (a scale derived from the maximum of
 // these very values), so rint(t/s) cannot leave [LO, HI] and the clamp is skipped.
 template <int HI> __device__ __forceinline__ constexpr float tie_margin() { return 2.0f * 2.4e-7f * (float)(HI + 1); }
-template <int LO, int HI, bool CLAMP = true>
-__device__ __forceinline__ void quant8(const float* t, float s, float r, bool slow, int* q) {
-    float rq[8], dev = 0.0f;
+// quant8_round: the quotients rounded, as floats; true when they come from the divisions.
+template <int HI> __device__ __forceinline__ bool quant8_round(const float* t, float s, float r, bool slow, float* rq) {
+    float dev = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         float qa = t[i] * r;
@@ -250,6 +250,12 @@ __device__ __forceinline__ void quant8(const float* t, float s, float r, bool sl
 #pragma unroll
         for (int i = 0; i < 8; ++i) rq[i] = __builtin_rintf(t[i] / s);
     }
+    return risky;
+}
+template <int LO, int HI, bool CLAMP = true>
+__device__ __forceinline__ void quant8(const float* t, float s, float r, bool slow, int* q) {
+    float rq[8];
+    quant8_round<HI>(t, s, r, slow, rq);
     // The hardware conversion saturates and turns NaN into 0, which is what the formula asks of a NaN
     // input; +-inf (t*r and t/s alike, r being a normal positive number here) saturates like any large value.
 #pragma unroll

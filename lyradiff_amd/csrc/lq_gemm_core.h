@@ -28,7 +28,10 @@ namespace lq {
 
 // K_W4A4H: W4A4 whose group scales are 16-bit floats; it converts the int32 group sums for free (see
 // compute_tile), which is exact only because three times such a scale is still an fp32 number.
-enum GemmKind { K_INT8 = 0, K_FP8 = 1, K_W4A4 = 2, K_W4A4H = 3 };
+// K_W4C: W4A4 on codes, both operands stored as one e4m3 byte per 4-bit value (every integer of [-8, 8] is an e4m3 number) and
+// the fp32 group scales stored group-major.  One fp8 matrix instruction forms the group sum as a float, exactly: products are
+// integers below 2^7, and the instruction keeps 13 bits under the largest of them.  No widening and no int->float conversion.
+enum GemmKind { K_INT8 = 0, K_FP8 = 1, K_W4A4 = 2, K_W4A4H = 3, K_W4C = 4 };
 
 struct GemmParams {
     void* C;
@@ -210,13 +213,14 @@ template <int NP, int G, int... I> __device__ __forceinline__ void sched_interle
 template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE>
 struct GemmKernel {
     static constexpr int NW = WM * WN;
-    static constexpr bool W4 = (KIND == K_W4A4 || KIND == K_W4A4H);
+    static constexpr bool W4C = KIND == K_W4C;
+    static constexpr bool W4 = (KIND == K_W4A4 || KIND == K_W4A4H || W4C);
     static constexpr int THREADS = NW * 64;
     static constexpr int TM = BM / WM, TN = BN / WN;  // wavefront tile
     static constexpr int MT = TM / 32, NT = TN / 32;  // 32x32 MFMA tiles per wavefront
     static constexpr int CH = BKB / 16;               // 16-byte chunks per tile row
     static constexpr int A_BYTES = BM * BKB, B_BYTES = BN * BKB;
-    static constexpr int NGS = BKB / 32;  // W4A4 groups per k-tile (one group of 64 int4 = 32 bytes)
+    static constexpr int NGS = BKB / (W4C ? 64 : 32);  // W4A4 groups per k-tile (one group of 64 int4 = 32 bytes, 64 as codes)
     static constexpr int NS = NGS * (BM + BN);
     static constexpr int S_DMA = W4 ? (NS + 64 * NW - 1) / (64 * NW) : 0;  // 4-byte scale transfers per wavefront per tile
     static constexpr int SCALE_BYTES = S_DMA * NW * 256;  // NS floats, padded to whole transfers
@@ -227,11 +231,11 @@ struct GemmKernel {
     static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0, "tile/wavefront mismatch");
     static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile must be a multiple of 32");
     static_assert(CH == 4 || CH == 8, "BKB must be 64 or 128");
-    static_assert(!W4 || ((NGS * BM) % 64 == 0 && NGS % 2 == 0), "scale transfer plan");
+    static_assert(!W4 || ((NGS * BM) % 64 == 0 && (W4C || NGS % 2 == 0)), "scale transfer plan");
     static_assert(PER_TILE * NSTAGE < 64, "vmcnt is a 6-bit counter");
-    using AccT = typename std::conditional<KIND == K_FP8, v16f, v16i>::type;
-    using FragT = typename std::conditional<KIND == K_FP8, v8i, v4i>::type;
-    static constexpr int KSTEP = (KIND == K_FP8) ? 64 : 32;  // operand bytes per MFMA k-step
+    using AccT = typename std::conditional<KIND == K_FP8 || W4C, v16f, v16i>::type;
+    using FragT = typename std::conditional<KIND == K_FP8 || W4C, v8i, v4i>::type;
+    static constexpr int KSTEP = (KIND == K_FP8 || W4C) ? 64 : 32;  // operand bytes per MFMA k-step
     static constexpr int KS = BKB / KSTEP;
 
     static __device__ __forceinline__ void run(const GemmParams& p, char* smem) {
@@ -285,19 +289,27 @@ struct GemmKernel {
                 if (!is_a && s >= NGS * BN) s = 0;  // padding slots of the last transfer: fetch something valid
                 const int g = is_a ? s / BM : s / BN, r = is_a ? s % BM : s % BN;
                 const int row = is_a ? min(r, row_last) : min(r, p.n - 1 - n0);
-                s_base[i] = static_cast<const char*>(is_a ? p.sA : p.sB) + (size_t)(is_a ? m0 : n0) * ng * sesz;
-                s_voff[i] = ((u32)(row * ng + g) * (u32)sesz) & ~3u;
+                if constexpr (W4C) {  // [k / 64][rows]: a transfer's 64 lanes read 64 neighbouring scales
+                    s_base[i] = static_cast<const char*>(is_a ? p.sA : p.sB) + (size_t)(is_a ? m0 : n0) * sesz;
+                    s_voff[i] = ((u32)g * (u32)(is_a ? p.m : p.n) + (u32)row) * (u32)sesz;
+                } else {
+                    s_base[i] = static_cast<const char*>(is_a ? p.sA : p.sB) + (size_t)(is_a ? m0 : n0) * ng * sesz;
+                    s_voff[i] = ((u32)(row * ng + g) * (u32)sesz) & ~3u;
+                }
             }
         }
         auto issue_scales = [&](int kt, int stage) {
             if constexpr (W4) {
                 const u32 ss = smem_base + stage * STAGE_BYTES + A_BYTES + B_BYTES + wave * (S_DMA * 256);
 #pragma unroll
-                for (int i = 0; i < S_DMA; ++i) dma4(s_base[i] + (size_t)kt * NGS * sesz, s_voff[i], ss + i * 256);
+                for (int i = 0; i < S_DMA; ++i) {
+                    const bool is_a = (wave * S_DMA + i) * 64 < NGS * BM;
+                    dma4(s_base[i] + (size_t)kt * NGS * sesz * (W4C ? (size_t)(is_a ? p.m : p.n) : 1), s_voff[i], ss + i * 256);
+                }
             }
         };
         auto convert_scales = [&](int stage) {
-            if constexpr (W4) {
+            if constexpr (W4 && !W4C) {
                 u32* ss = reinterpret_cast<u32*>(smem + stage * STAGE_BYTES + A_BYTES + B_BYTES) + wave * (S_DMA * 64) + lane;
 #pragma unroll
                 for (int i = 0; i < S_DMA; ++i) {
@@ -359,7 +371,7 @@ struct GemmKernel {
         const int w_off = wn * NT * (BKB * 32) + lane * 16;
         auto ldsv = [&](const char* ptr) -> v4i { return *reinterpret_cast<const v4i*>(ptr); };
         auto load_frags = [&](const char* sa, const char* sb, int ks, FragT* w, FragT* x) {
-            if constexpr (KIND == K_FP8) {
+            if constexpr (KIND == K_FP8 || W4C) {
 #pragma unroll
                 for (int j = 0; j < NT; ++j) {
                     v4i lo = ldsv(sb + w_off + j * (BKB * 32) + ks * 2048);
@@ -390,8 +402,51 @@ struct GemmKernel {
         // stage is a list of (group, n-tile, m-tile) items; the two MFMAs of item t+1 are issued before
         // the 48 scale operations of item t, so the matrix pipe works in the shadow of the VALU, which
         // is the bound of this kernel (cvt + mul + fma per output per group, see the header comment).
+        // On codes an item is one matrix instruction into a zero accumulator and two vector operations per output (the
+        // reference's multiply and fused multiply-add); per 64 x 32 wavefront tile and group that is 64 + 12 LDS reads and
+        // 2 matrix instructions where the nibbles took 64 + 32 conversions + 36 widening operations beside 4 of them.
         auto compute_tile = [&](int stage) {
-            if constexpr (W4) {
+            if constexpr (W4C) {
+                const char* sa = smem + stage * STAGE_BYTES;
+                const char* sb = sa + A_BYTES;
+                const float* ssa = reinterpret_cast<const float*>(sb + B_BYTES);  // [NGS][BM]
+                const float* ssb = ssa + NGS * BM;                                 // [NGS][BN]
+                constexpr int PER_GROUP = NT * MT;
+                FragT wq[2][NT], xq[2][MT];
+                v16f pz[2];
+                v16f zero;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) zero[v] = 0.0f;
+                auto issue_item = [&](int g, int t) {
+                    pz[(g * PER_GROUP + t) & 1] =
+                        __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wq[g & 1][t / MT], xq[g & 1][t % MT], zero, 0, 0, 0, 0, 0, 0);
+                };
+                load_frags(sa, sb, 0, wq[0], xq[0]);
+                issue_item(0, 0);
+#pragma unroll
+                for (int g = 0; g < NGS; ++g) {
+                    if (g + 1 < NGS) load_frags(sa, sb, g + 1, wq[(g + 1) & 1], xq[(g + 1) & 1]);
+                    float sbv[16];
+#pragma unroll
+                    for (int t = 0; t < PER_GROUP; ++t) {
+                        const int j = t / MT, i = t % MT;
+                        if (t + 1 < PER_GROUP) issue_item(g, t + 1);
+                        else if (g + 1 < NGS) issue_item(g + 1, 0);
+                        if (i == 0) {
+#pragma unroll
+                            for (int q4 = 0; q4 < 4; ++q4) {
+                                const float4 f = *reinterpret_cast<const float4*>(ssb + g * BN + wn * TN + j * 32 + q4 * 8 + lh * 4);
+                                sbv[q4 * 4] = f.x; sbv[q4 * 4 + 1] = f.y; sbv[q4 * 4 + 2] = f.z; sbv[q4 * 4 + 3] = f.w;
+                            }
+                        }
+                        const float sa_l = ssa[g * BM + xrow + i * 32];
+                        const v16f cur = pz[(g * PER_GROUP + t) & 1];
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) res[i][j][v] = __builtin_fmaf(cur[v] * sa_l, sbv[v], res[i][j][v]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else if constexpr (W4) {
                 const char* sa = smem + stage * STAGE_BYTES;
                 const char* sb = sa + A_BYTES;
                 const float* ssa = reinterpret_cast<const float*>(sb + B_BYTES);  // [NGS][BM]
@@ -874,6 +929,7 @@ struct GemmKernel {
 // small-tile configurations ask for more resident wavefronts instead.
 template <int KIND, int BM, int BN, int BKB, int WM, int WN> constexpr int min_workgroups_per_cu() {
     if ((BM / WM) * (BN / WN) >= 128 * 128) return 1;  // 256 accumulator registers: one wavefront per SIMD, the whole register file
+    if (KIND == K_W4C) return 4;
     if (KIND != K_W4A4 && KIND != K_W4A4H) return 2;
     if (WM * WN > 4) return 1;
     const int wave_tile = (BM / WM) * (BN / WN);

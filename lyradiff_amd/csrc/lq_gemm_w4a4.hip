@@ -28,15 +28,26 @@ template <int KIND, typename OutTag> static int run_w4a4(GemmParams p, hipStream
     }
 }
 
+// Tile configurations on codes, in the order of the size they are for (3072 outputs, K = 3072, us, tactic 0 / 1 / 2):
+//   2000 tokens  45.7 / 39.4 / 42.7     1000 tokens  28.9 / 24.3 / 23.9     333 tokens  25.1 / 18.4 / 16.0
+//   512 x 9216   41.2 / 34.4 / 39.2     4608 x 3072  77 / 88 / -
+// Larger problems are bound by the power the two scale multiplications, the matrix instruction and the operand traffic take
+// together (4096 x 4096 x 3072: 82 us with random operands, 73 with zeros, 42 for the scale multiplications alone), and six further
+// tile shapes measured within 4 % of tactic 0 there.
+template <typename OutTag> static int run_w4a4_codes(const GemmParams& p, hipStream_t st) {
+    const long big = (long)((p.m + 127) / 128) * ((p.n + 127) / 128), mid = (long)((p.m + 63) / 64) * ((p.n + 127) / 128);
+    if (big >= 512) return launch_gemm<K_W4C, OutTag, 128, 128, 128, 2, 4, 2>(p, st);  // two rounds of two workgroups per CU
+    if (mid >= 448) return launch_gemm<K_W4C, OutTag, 64, 128, 128, 2, 4, 2>(p, st);
+    return launch_gemm<K_W4C, OutTag, 64, 64, 128, 2, 2, 2>(p, st);  // few tiles: as many and as short as possible
+}
+
 }  // namespace lq
 
 using namespace lq;
 
-extern "C" int lq_gemm_w4a4_ex(void* C, lq_dtype_t out_dtype, const uint32_t* A_words, const uint8_t* B_rows32,
-                               const void* sA, const void* sB, lq_dtype_t scale_dtype, const void* bias,
-                               const void* lora_act, const void* lora_up, lq_dtype_t lora_dtype, int lora_rank, int m,
-                               int n, int k, int group, const lq_epilogue_t* epi, lq_stream_t stream) {
-    LQ_REQUIRE((C || (epi && epi->C_fp8)) && A_words && B_rows32 && sA && sB, LQ_ERR_ARG, "lq_gemm_w4a4: null pointer");
+// Checks and fills what the two forms of the operands have in common: the low-rank branch and the epilogue options.
+static int w4a4_options(GemmParams& p, const void* lora_act, const void* lora_up, lq_dtype_t lora_dtype, int lora_rank, int n,
+                        const lq_epilogue_t* epi) {
     if (epi != nullptr) {
         LQ_REQUIRE(epi->gelu >= 0 && epi->gelu <= 2, LQ_ERR_ARG, "lq_gemm_w4a4: gelu must be 0, 1 or 2");
         LQ_REQUIRE((epi->gate == nullptr) == (epi->residual == nullptr), LQ_ERR_ARG, "lq_gemm_w4a4: gate and residual go together");
@@ -49,6 +60,31 @@ extern "C" int lq_gemm_w4a4_ex(void* C, lq_dtype_t out_dtype, const uint32_t* A_
                        reinterpret_cast<uintptr_t>(epi->addend) % 16 == 0,
                    LQ_ERR_ARG, "lq_gemm_w4a4: gate, residual and addend must be 16-byte aligned");
     }
+    LQ_REQUIRE((lora_act == nullptr) == (lora_up == nullptr), LQ_ERR_ARG,
+               "lq_gemm_w4a4: the low-rank branch needs both lora_act and lora_up");
+    if (lora_act != nullptr) {
+        LQ_REQUIRE(lora_dtype == LQ_F16 || lora_dtype == LQ_BF16, LQ_ERR_UNSUPPORTED,
+                   "lq_gemm_w4a4: low-rank operands must be F16 or BF16");
+        LQ_REQUIRE(lora_rank > 0 && lora_rank % 16 == 0, LQ_ERR_SHAPE, "lq_gemm_w4a4: lora_rank=%d must be a multiple of 16", lora_rank);
+        LQ_REQUIRE(reinterpret_cast<uintptr_t>(lora_act) % 16 == 0 && reinterpret_cast<uintptr_t>(lora_up) % 16 == 0, LQ_ERR_ARG,
+                   "lq_gemm_w4a4: low-rank operands must be 16-byte aligned");
+    }
+    p.lora_act = lora_act; p.lora_up = lora_up; p.lora_rank = lora_rank; p.lora_f16 = lora_dtype == LQ_F16;
+    p.ldc8 = (size_t)n;
+    if (epi != nullptr) {
+        p.gelu = epi->gelu; p.addend = epi->addend; p.gate = epi->gate; p.gate_rows = epi->rows_per_gate;
+        p.residual = epi->residual; p.beta = 1.0f;
+        p.C8 = epi->C_fp8; p.c8_scale = epi->C_fp8_scale;
+        if (epi->C_fp8 != nullptr) p.ldc8 = epi->ldc_fp8;
+    }
+    return LQ_OK;
+}
+
+extern "C" int lq_gemm_w4a4_ex(void* C, lq_dtype_t out_dtype, const uint32_t* A_words, const uint8_t* B_rows32,
+                               const void* sA, const void* sB, lq_dtype_t scale_dtype, const void* bias,
+                               const void* lora_act, const void* lora_up, lq_dtype_t lora_dtype, int lora_rank, int m,
+                               int n, int k, int group, const lq_epilogue_t* epi, lq_stream_t stream) {
+    LQ_REQUIRE((C || (epi && epi->C_fp8)) && A_words && B_rows32 && sA && sB, LQ_ERR_ARG, "lq_gemm_w4a4: null pointer");
     LQ_REQUIRE(group == 64, LQ_ERR_SHAPE, "lq_gemm_w4a4: group=%d, only 64 is supported", group);
     LQ_REQUIRE(scale_dtype == LQ_F32 || scale_dtype == LQ_F16, LQ_ERR_UNSUPPORTED,
                "lq_gemm_w4a4: scale dtype must be F32 or F16");
@@ -59,27 +95,11 @@ extern "C" int lq_gemm_w4a4_ex(void* C, lq_dtype_t out_dtype, const uint32_t* A_
                LQ_ERR_ARG, "lq_gemm_w4a4: A, B, C must be 16-byte aligned and bias 8-byte aligned");
     LQ_REQUIRE(reinterpret_cast<uintptr_t>(sA) % 4 == 0 && reinterpret_cast<uintptr_t>(sB) % 4 == 0, LQ_ERR_ARG,
                "lq_gemm_w4a4: scale arrays must be 4-byte aligned");
-    LQ_REQUIRE((lora_act == nullptr) == (lora_up == nullptr), LQ_ERR_ARG,
-               "lq_gemm_w4a4: the low-rank branch needs both lora_act and lora_up");
-    if (lora_act != nullptr) {
-        LQ_REQUIRE(lora_dtype == LQ_F16 || lora_dtype == LQ_BF16, LQ_ERR_UNSUPPORTED,
-                   "lq_gemm_w4a4: low-rank operands must be F16 or BF16");
-        LQ_REQUIRE(lora_rank > 0 && lora_rank % 16 == 0, LQ_ERR_SHAPE, "lq_gemm_w4a4: lora_rank=%d must be a multiple of 16", lora_rank);
-        LQ_REQUIRE(reinterpret_cast<uintptr_t>(lora_act) % 16 == 0 && reinterpret_cast<uintptr_t>(lora_up) % 16 == 0, LQ_ERR_ARG,
-                   "lq_gemm_w4a4: low-rank operands must be 16-byte aligned");
-    }
-    if (m == 0) return LQ_OK;
     GemmParams p = {};
     p.C = C; p.A = reinterpret_cast<const uint8_t*>(A_words); p.B = B_rows32; p.bias = bias;
     p.sA = sA; p.sB = sB; p.scale_f16 = scale_dtype == LQ_F16;
-    p.lora_act = lora_act; p.lora_up = lora_up; p.lora_rank = lora_rank; p.lora_f16 = lora_dtype == LQ_F16;
-    p.ldc8 = (size_t)n;
-    if (epi != nullptr) {
-        p.gelu = epi->gelu; p.addend = epi->addend; p.gate = epi->gate; p.gate_rows = epi->rows_per_gate;
-        p.residual = epi->residual; p.beta = 1.0f;
-        p.C8 = epi->C_fp8; p.c8_scale = epi->C_fp8_scale;
-        if (epi->C_fp8 != nullptr) p.ldc8 = epi->ldc_fp8;
-    }
+    const int rc = w4a4_options(p, lora_act, lora_up, lora_dtype, lora_rank, n, epi);
+    if (rc != LQ_OK || m == 0) return rc;
     p.m = m; p.n = n; p.k = k; p.kb = k / 2;
     hipStream_t st = as_stream(stream);
     switch (out_dtype) {
@@ -87,6 +107,27 @@ extern "C" int lq_gemm_w4a4_ex(void* C, lq_dtype_t out_dtype, const uint32_t* A_
         case LQ_BF16: return p.scale_f16 ? run_w4a4<K_W4A4H, BF16Tag>(p, st) : run_w4a4<K_W4A4, BF16Tag>(p, st);
         case LQ_F32: return p.scale_f16 ? run_w4a4<K_W4A4H, F32Tag>(p, st) : run_w4a4<K_W4A4, F32Tag>(p, st);
         default: set_error("lq_gemm_w4a4: unsupported output dtype %d", (int)out_dtype); return LQ_ERR_UNSUPPORTED;
+    }
+}
+
+extern "C" int lq_gemm_w4a4_codes(void* C, lq_dtype_t out_dtype, const uint8_t* A_codes, const uint8_t* B_codes_rows32, const float* sA,
+                                  const float* sB, const void* bias, const void* lora_act, const void* lora_up, lq_dtype_t lora_dtype,
+                                  int lora_rank, int m, int n, int k, const lq_epilogue_t* epi, lq_stream_t stream) {
+    LQ_REQUIRE((C || (epi && epi->C_fp8)) && A_codes && B_codes_rows32 && sA && sB, LQ_ERR_ARG, "lq_gemm_w4a4_codes: null pointer");
+    LQ_REQUIRE(m >= 0 && n > 0 && k > 0 && n % 32 == 0 && k % 128 == 0, LQ_ERR_SHAPE,
+               "lq_gemm_w4a4_codes: need n %% 32 == 0 and k %% 128 == 0 (m=%d n=%d k=%d)", m, n, k);
+    LQ_REQUIRE((reinterpret_cast<uintptr_t>(A_codes) | reinterpret_cast<uintptr_t>(B_codes_rows32) | reinterpret_cast<uintptr_t>(C)) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(bias) % 8 == 0 && (reinterpret_cast<uintptr_t>(sA) | reinterpret_cast<uintptr_t>(sB)) % 4 == 0,
+               LQ_ERR_ARG, "lq_gemm_w4a4_codes: A, B, C must be 16-byte aligned, bias 8-byte, scales 4-byte aligned");
+    GemmParams p = {};
+    p.C = C; p.A = A_codes; p.B = B_codes_rows32; p.bias = bias; p.sA = sA; p.sB = sB;
+    const int rc = w4a4_options(p, lora_act, lora_up, lora_dtype, lora_rank, n, epi);
+    if (rc != LQ_OK || m == 0) return rc;
+    p.m = m; p.n = n; p.k = k; p.kb = k;
+    switch (out_dtype) {
+        case LQ_F16: return run_w4a4_codes<F16Tag>(p, as_stream(stream));
+        case LQ_BF16: return run_w4a4_codes<BF16Tag>(p, as_stream(stream));
+        default: set_error("lq_gemm_w4a4_codes: unsupported output dtype %d", (int)out_dtype); return LQ_ERR_UNSUPPORTED;
     }
 }
 

@@ -11,9 +11,10 @@ namespace lq {
 
 // One lane's eight consecutive elements of a group of 64 (eight adjacent lanes hold the group): divides by the smoothing
 // divisors (dv, with yv = fl(1/dv); both unused when !SMOOTHED), takes the group's absmax across the eight lanes, and returns
-// the packed word; `s` receives the group's scale (already an fp16 value when F16_SCALE).
-template <bool F16_SCALE, bool SMOOTHED>
-__device__ __forceinline__ u32 w4a4_quant_lane8(float (&v)[8], const float (&dv)[8], const float (&yv)[8], float& s) {
+// the packed word; `s` receives the group's scale (already an fp16 value when F16_SCALE).  CODES: the eight values as e4m3 bytes
+// instead (both words; otherwise the packed word is .x).
+template <bool F16_SCALE, bool SMOOTHED, bool CODES = false>
+__device__ __forceinline__ uint2 w4a4_quant_lane8(float (&v)[8], const float (&dv)[8], const float (&yv)[8], float& s) {
     float amax = 0.0f;
     if constexpr (SMOOTHED) {
         // v = fl(x/d) from the stored reciprocal: q0 = fl(x*y), rem = x - q0*d (exact in one
@@ -59,6 +60,19 @@ __device__ __forceinline__ u32 w4a4_quant_lane8(float (&v)[8], const float (&dv)
         if constexpr (F16_SCALE) s = round_through<F16Tag>(s);
     }
     const float r = fast_recip(s);
+    if constexpr (CODES) {  // every integer of [-8, 8] is an e4m3 number: the conversion is exact
+        float rq[8];
+        if (quant8_round<7>(v, s, r, slow, rq)) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) rq[i] = rq[i] != rq[i] ? 0.0f : fminf(fmaxf(rq[i], -8.0f), 7.0f);
+        }
+        uint2 o;
+        o.x = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(rq[0], rq[1], 0, false);
+        o.x = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(rq[2], rq[3], (int)o.x, true);
+        o.y = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(rq[4], rq[5], 0, false);
+        o.y = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(rq[6], rq[7], (int)o.y, true);
+        return o;
+    }
     int q[8];
     // fp32 scale: s = fl(absmax / 7) bounds every |v / s| by 7.000001, no clamp needed.  An fp16 scale may have been
     // rounded down by a large factor in the subnormal range, so those results are clamped.
@@ -68,7 +82,7 @@ __device__ __forceinline__ u32 w4a4_quant_lane8(float (&v)[8], const float (&dv)
     u32 word = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) word = __builtin_amdgcn_alignbit((u32)q[i], word, 4);
-    return word;
+    return make_uint2(word, 0u);
 }
 
 // SMOOTH 0: no smoothing vector; 1: the divisors d of the workgroup's column range and their correctly
@@ -148,7 +162,7 @@ __global__ __launch_bounds__(WAVES * 64) void w4a4_quant_kernel(u32* __restrict_
                 yv[0] = c.x; yv[1] = c.y; yv[2] = c.z; yv[3] = c.w; yv[4] = d.x; yv[5] = d.y; yv[6] = d.z; yv[7] = d.w;
             }
             float s;
-            const u32 word = w4a4_quant_lane8<F16_SCALE, SMOOTH == 1>(v, dv, yv, s);
+            const u32 word = w4a4_quant_lane8<F16_SCALE, SMOOTH == 1>(v, dv, yv, s).x;
             if (FULL || col < k) {
                 st4<STREAM>(q_words + (size_t)row * (k >> 3) + (col >> 3), word);
                 if ((lane & 7) == 0) {
@@ -196,7 +210,10 @@ constexpr int kFusedWaveStage = 2 * kFusedPark + 1024;        // x, lora_down, t
 constexpr int kFusedLds = kFusedWaves * kFusedWaveStage;
 
 // OUT: 0 fp32, 1 fp16, 2 bf16 (type of the low-rank result).
-template <bool F16, bool F16_SCALE, int OUT, bool STREAM>
+// CODES: the quantised values as e4m3 bytes [m, k] and fp32 scales group-major [k / 64, m], what the GEMM on codes reads: twice the
+// bytes written for 0.5 instead of 2 instructions per value to assemble them (4608 rows: 16.7 against 15.9 us at k = 3072, 50 against
+// 47 at 12288; the GEMM behind it gains 23 and 98).
+template <bool F16, bool F16_SCALE, int OUT, bool STREAM, bool CODES = false>
 __global__ __launch_bounds__(kFusedWaves * 64) void w4a4_quant_lora_kernel(u32* __restrict__ q_words, void* __restrict__ scales,
                                                                           void* __restrict__ act,
                                                                           const unsigned short* __restrict__ x,
@@ -217,9 +234,10 @@ __global__ __launch_bounds__(kFusedWaves * 64) void w4a4_quant_lora_kernel(u32* 
     // cover all banks
     const int gr = lane >> 4, gc = lane & 15;
     const int lr = lane & 31, lh = lane >> 5;
-    u32 xo[8];
+    const unsigned short* xb = x + (size_t)row0 * k;
+    u32 xo[8];  // inside this workgroup's rows
 #pragma unroll
-    for (int i = 0; i < 8; ++i) xo[i] = (u32)(row0 + min(4 * i + gr, rows - 1)) * (u32)k + gc * 8;
+    for (int i = 0; i < 8; ++i) xo[i] = (u32)min(4 * i + gr, rows - 1) * (u32)k + gc * 8;
     const u32 dofs = (u32)gr * (u32)k + gc * 8;
     const int nsl = k >> 7, ng = k >> 6;
     fv16f acc;
@@ -235,7 +253,7 @@ __global__ __launch_bounds__(kFusedWaves * 64) void w4a4_quant_lora_kernel(u32* 
         gs = *reinterpret_cast<const float2*>(smooth + k0 + 2 * lane);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-            if (i < ni) gx[i] = ld16<STREAM>(x + xo[i] + k0);
+            if (i < ni) gx[i] = ld16<STREAM>(xb + xo[i] + k0);
 #pragma unroll
         for (int i = 0; i < 8; ++i) gd[i] = *reinterpret_cast<const v4i*>(down + dofs + (size_t)i * 4 * k + k0);
     };
@@ -284,12 +302,14 @@ __global__ __launch_bounds__(kFusedWaves * 64) void w4a4_quant_lora_kernel(u32* 
                 parked = *reinterpret_cast<const uint4*>(stage + rn * 256 + ((gc ^ (rn & 15)) << 4));
             }
             float s;
-            const u32 word = w4a4_quant_lane8<F16_SCALE, true>(v, dv, yv, s);
+            const uint2 word = w4a4_quant_lane8<F16_SCALE, true, CODES>(v, dv, yv, s);
             if (r < rows) {
                 const size_t row = (size_t)(row0 + r);
-                st4<STREAM>(q_words + row * (k >> 3) + (k0 >> 3) + gc, word);
+                if constexpr (CODES) st8<STREAM>(q_words + row * (k >> 2) + (k0 >> 2) + 2 * gc, word);
+                else st4<STREAM>(q_words + row * (k >> 3) + (k0 >> 3) + gc, word.x);
                 if ((lane & 7) == 0) {
-                    const size_t si = row * ng + (k0 >> 6) + (gc >> 3);
+                    const int grp = (k0 >> 6) + (gc >> 3);
+                    const size_t si = CODES ? (size_t)grp * m + row : row * ng + grp;
                     if constexpr (F16_SCALE) static_cast<unsigned short*>(scales)[si] = (unsigned short)f32_to_f16_bits(s);  // s is already an fp16 value
                     else static_cast<float*>(scales)[si] = s;
                 }
@@ -325,6 +345,28 @@ __global__ __launch_bounds__(kFusedWaves * 64) void w4a4_quant_lora_kernel(u32* 
                 *reinterpret_cast<uint2*>(static_cast<unsigned short*>(act) + idx) = o;
             }
         }
+    }
+}
+
+// ---- packed 4-bit weights in rows32 layout -> e4m3 codes in rows32 layout: a 16-byte chunk (32 values of a row) becomes two
+__global__ __launch_bounds__(256) void w4a4_expand_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src, size_t chunks) {
+    for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < chunks; t += (size_t)gridDim.x * blockDim.x) {
+        const uint4 w = src[t];
+        const u32 in[4] = {w.x, w.y, w.z, w.w};
+        u32 out[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float f[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[e] = (float)((int)(in[i] << (28 - 4 * (4 * h + e))) >> 28);  // nibble, sign extended
+                const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+                out[2 * i + h] = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
+            }
+        const size_t r = t & 31, kc = t >> 5;  // chunk columns counted through all 32-row blocks
+        dst[(2 * kc) * 32 + r] = make_uint4(out[0], out[1], out[2], out[3]);
+        dst[(2 * kc + 1) * 32 + r] = make_uint4(out[4], out[5], out[6], out[7]);
     }
 }
 
@@ -416,7 +458,7 @@ extern "C" int lq_w4a4_quantize(uint32_t* q_words, void* scales, lq_dtype_t scal
     return check_launch("w4a4_quantize");
 }
 
-template <bool F16, bool F16_SCALE, int OUT, bool STREAM>
+template <bool F16, bool F16_SCALE, int OUT, bool STREAM, bool CODES = false>
 static int launch_quant_lora(u32* q_words, void* scales, void* act, const void* x, const float* smooth, const void* down, int m, int k,
                              hipStream_t st) {
     static const int num_cu = [] {
@@ -424,7 +466,7 @@ static int launch_quant_lora(u32* q_words, void* scales, void* act, const void* 
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
         return n;
     }();
-    auto kern = w4a4_quant_lora_kernel<F16, F16_SCALE, OUT, STREAM>;
+    auto kern = w4a4_quant_lora_kernel<F16, F16_SCALE, OUT, STREAM, CODES>;
     static bool raised = false;  // idempotent, a race only repeats it
     if (!raised) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kFusedLds);
@@ -468,6 +510,40 @@ extern "C" int lq_w4a4_quantize_lora_down(uint32_t* q_words, void* scales, lq_dt
     return f16s ? LQ_QL_OUT(false, true) : LQ_QL_OUT(false, false);
 #undef LQ_QL_OUT
 #undef LQ_QL_GO
+}
+
+extern "C" int lq_w4a4_quantize_lora_down_codes(uint8_t* codes, float* scales, void* lora_act, lq_dtype_t act_dtype, const void* x,
+                                                lq_dtype_t x_dtype, const float* smooth, const void* lora_down, int m, int k, int rank,
+                                                lq_stream_t stream) {
+    LQ_REQUIRE(m >= 0 && k > 0 && k % 128 == 0 && k <= 16384 && rank == 32, LQ_ERR_SHAPE,
+               "lq_w4a4_quantize_lora_down_codes: need k %% 128 == 0, k <= 16384 and rank 32 (m=%d k=%d rank=%d)", m, k, rank);
+    LQ_REQUIRE((x_dtype == LQ_F16 || x_dtype == LQ_BF16) && act_dtype == x_dtype, LQ_ERR_UNSUPPORTED,
+               "lq_w4a4_quantize_lora_down_codes: x and the low-rank result must be F16 or both BF16");
+    if (m == 0) return LQ_OK;
+    LQ_REQUIRE(codes && scales && lora_act && x && smooth && lora_down, LQ_ERR_ARG, "lq_w4a4_quantize_lora_down_codes: null pointer");
+    LQ_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(smooth) | reinterpret_cast<uintptr_t>(lora_down) |
+                reinterpret_cast<uintptr_t>(lora_act) | reinterpret_cast<uintptr_t>(codes)) % 16 == 0 && reinterpret_cast<uintptr_t>(scales) % 4 == 0,
+               LQ_ERR_ARG, "lq_w4a4_quantize_lora_down_codes: buffers must be 16-byte aligned, scales 4-byte aligned");
+    hipStream_t st = as_stream(stream);
+    u32* out = reinterpret_cast<u32*>(codes);
+    const bool stream_io = (size_t)m * k * 2 >= kStreamQuantBytes;  // read-once input, write-once codes
+    if (x_dtype == LQ_F16)
+        return stream_io ? launch_quant_lora<true, false, 1, true, true>(out, scales, lora_act, x, smooth, lora_down, m, k, st)
+                         : launch_quant_lora<true, false, 1, false, true>(out, scales, lora_act, x, smooth, lora_down, m, k, st);
+    return stream_io ? launch_quant_lora<false, false, 2, true, true>(out, scales, lora_act, x, smooth, lora_down, m, k, st)
+                     : launch_quant_lora<false, false, 2, false, true>(out, scales, lora_act, x, smooth, lora_down, m, k, st);
+}
+
+extern "C" int lq_w4a4_expand_rows32(uint8_t* codes, const uint8_t* packed, size_t n, size_t k, lq_stream_t stream) {
+    LQ_REQUIRE(codes && packed && codes != packed, LQ_ERR_ARG, "lq_w4a4_expand_rows32: null pointer or in-place call");
+    LQ_REQUIRE(n % 32 == 0 && k % 32 == 0, LQ_ERR_SHAPE, "lq_w4a4_expand_rows32: n=%zu and k=%zu must be multiples of 32", n, k);
+    LQ_REQUIRE((reinterpret_cast<uintptr_t>(codes) | reinterpret_cast<uintptr_t>(packed)) % 16 == 0, LQ_ERR_ARG,
+               "lq_w4a4_expand_rows32: buffers must be 16-byte aligned");
+    const size_t chunks = n * (k / 32);
+    if (chunks == 0) return LQ_OK;
+    hipLaunchKernelGGL(w4a4_expand_kernel, dim3((unsigned)std::min<size_t>((chunks + 255) / 256, 65535)), dim3(256), 0, as_stream(stream),
+                       reinterpret_cast<uint4*>(codes), reinterpret_cast<const uint4*>(packed), chunks);
+    return check_launch("w4a4_expand_rows32");
 }
 
 extern "C" size_t lq_weight_row_bytes(lq_weight_kind_t kind, size_t k) { return kind == LQ_W_INT4 ? k / 2 : k; }

@@ -59,16 +59,6 @@ def load_flux_single_mlp_int4(src, prefix: str, dim: int, mlp_scale: int = 4, dt
         load_w4a4_linear(src, prefix + "proj_out.linears.1.linear.", dim, mlp_scale * dim, lora_rank, False, dtype, device))
 
 
-def _w4a4(lin: W4A4Linear, x2: torch.Tensor, **epilogue):
-    """W4A4Gemm::forward (W4A4Gemm.cc:113-169) with epilogue options: quantise, low-rank down, GEMM."""
-    if lin.lora_down is not None:
-        q, s, act = ops.w4a4_quant_lora_down(x2, lin.smooth, lin.lora_down, torch.float32)
-    else:
-        (q, s), act = ops.w4a4_quant(x2, lin.smooth, torch.float32), None
-    return ops.w4a4_linear(q, lin.weight_rows32, s, lin.weight_scale, lin.bias, x2.dtype, 64, act,
-                           lin.lora_up if act is not None else None, **epilogue)
-
-
 def flux_attn_post_int4(x: torch.Tensor, attn_output: torch.Tensor, msa: torch.Tensor, w: FluxAttnPostInt4Weights,
                         eps: float = 1e-6) -> torch.Tensor:
     """x, attn_output [B, S, D]; msa [6, B, D] -> output [B, S, D]."""
@@ -76,7 +66,7 @@ def flux_attn_post_int4(x: torch.Tensor, attn_output: torch.Tensor, msa: torch.T
     if tuple(msa.shape) != (6, b, d):
         raise ValueError("msa must be [6, B, D]")
     norm, hidden = ops.gate_residual_layernorm_mod(x, msa[4], msa[3], attn_output, msa[2], eps)
-    q2 = _w4a4(w.gelu_proj, norm.view(b * s, d), gelu=2, out_fp8_scale=w.ff_linear.input_scale, want_output=False)
+    q2 = w.gelu_proj.run(norm.view(b * s, d), gelu=2, out_fp8_scale=w.ff_linear.input_scale, want_output=False)
     out = ops.fp8_linear_gated(q2, w.ff_linear.weight_rows32, w.ff_linear.input_scale, w.ff_linear.weight_scale,
                                w.ff_linear.bias, msa[5], hidden.view(b * s, d), rows_per_gate=s)
     return out.view(b, s, d)
@@ -87,9 +77,9 @@ def flux_single_mlp_int4(x: torch.Tensor, norm_hidden: torch.Tensor, attn_output
     """x, norm_hidden, attn_output [B, S, D]; gate [B, D] -> output [B, S, D]."""
     b, s, d = x.shape
     m = b * s
-    mlp = _w4a4(w.proj_mlp, norm_hidden.view(m, d), gelu=2)
-    h1 = _w4a4(w.proj_out_1, attn_output.view(m, d))
-    out = _w4a4(w.proj_out_2, mlp, addend=h1, gate=gate, residual=x.view(m, d), rows_per_gate=s)
+    mlp = w.proj_mlp.run(norm_hidden.view(m, d), gelu=2)
+    h1 = w.proj_out_1.run(attn_output.view(m, d))
+    out = w.proj_out_2.run(mlp, addend=h1, gate=gate, residual=x.view(m, d), rows_per_gate=s)
     return out.view(b, s, d)
 
 
@@ -147,7 +137,7 @@ def load_flux_double_block_int4(src, prefix: str, dim: int, full: bool = True, d
 
 
 def _w4a4_3d(lin: W4A4Linear, x: torch.Tensor) -> torch.Tensor:
-    y = _w4a4(lin, x.reshape(-1, x.shape[-1]))
+    y = lin.run(x.reshape(-1, x.shape[-1]))
     return y.view(*x.shape[:-1], y.shape[-1])
 
 

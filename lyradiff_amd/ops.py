@@ -842,6 +842,38 @@ def w4a4_linear(a_words, w_rows32, sA, sB, bias=None, out_dtype=torch.bfloat16, 
     n = w_rows32.shape[0]
     if w_rows32.shape[1] * 2 != k:
         raise ValueError("K mismatch between activation and weight")
+    lib = _l.load()
+    return _w4a4_gemm(lambda c, lora, epi: lib.lq_gemm_w4a4_ex(c, _DT[out_dtype], _ptr(a_words), _ptr(w_rows32), _ptr(sA), _ptr(sB), _DT[sA.dtype],
+                                                               _ptr(bias), *lora, m, n, k, group, epi, _stream()),
+                      m, n, a_words.device, bias, out_dtype, lora_act, lora_up, gelu, addend, gate, residual, rows_per_gate, out_fp8_scale, out_fp8,
+                      col_offset, want_output, out)
+
+
+def w4a4_linear_codes(a_codes, w_codes_rows32, sA, sB, bias=None, out_dtype=torch.bfloat16, lora_act=None, lora_up=None, gelu: int = 0,
+                      addend=None, gate=None, residual=None, rows_per_gate: int = 1, out_fp8_scale=None, out_fp8=None, col_offset: int = 0,
+                      want_output: bool = True, out=None):
+    """w4a4_linear on operands with one e4m3 byte per 4-bit value: a_codes uint8 [M, K] and sA fp32 [K/64, M] from
+    w4a4_quant_lora_down_codes, w_codes_rows32 uint8 [N, K] from w4a4_expand_weight, sB fp32 [K/64, N].  Same bits as w4a4_linear with
+    fp32 scales; fp16 and bf16 outputs."""
+    _chk(a_codes, "a_codes", (torch.uint8,))
+    _chk(w_codes_rows32, "w_codes_rows32", (torch.uint8,))
+    _chk(sA, "sA", (torch.float32,))
+    _chk(sB, "sB", (torch.float32,))
+    m, k = a_codes.shape
+    n = w_codes_rows32.shape[0]
+    if w_codes_rows32.shape[1] != k or sA.numel() != m * (k // 64) or sB.numel() != n * (k // 64):
+        raise ValueError("w4a4_linear_codes: a_codes [M, K], w_codes_rows32 [N, K], sA [K/64, M] and sB [K/64, N] do not fit together")
+    lib = _l.load()
+    return _w4a4_gemm(lambda c, lora, epi: lib.lq_gemm_w4a4_codes(c, _DT[out_dtype], _ptr(a_codes), _ptr(w_codes_rows32), _ptr(sA), _ptr(sB), _ptr(bias),
+                                                                  *lora, m, n, k, epi, _stream()),
+                      m, n, a_codes.device, bias, out_dtype, lora_act, lora_up, gelu, addend, gate, residual, rows_per_gate, out_fp8_scale, out_fp8,
+                      col_offset, want_output, out)
+
+
+def _w4a4_gemm(launch, m, n, device, bias, out_dtype, lora_act, lora_up, gelu, addend, gate, residual, rows_per_gate, out_fp8_scale, out_fp8,
+               col_offset, want_output, out):
+    """What the two operand forms share: checks of the low-rank branch and the epilogue options, the outputs, the call
+    launch(output pointer, (lora_act, lora_up, their dtype, rank), epilogue pointer)."""
     if bias is not None:
         _chk(bias, "bias", (out_dtype,))
     rank, lora_dt = 0, _l.LQ_BF16
@@ -870,19 +902,17 @@ def w4a4_linear(a_words, w_rows32, sA, sB, bias=None, out_dtype=torch.bfloat16, 
         epi = _l.Epilogue(int(gelu), _ptr(addend), _ptr(gate), int(rows_per_gate), _ptr(residual), None, 0, None)
         if out_fp8_scale is not None:
             _chk(out_fp8_scale, "out_fp8_scale", (torch.float32,))
-            c8 = out_fp8 if out_fp8 is not None else torch.empty((m, n), dtype=torch.uint8, device=a_words.device)
+            c8 = out_fp8 if out_fp8 is not None else torch.empty((m, n), dtype=torch.uint8, device=device)
             _chk(c8, "out_fp8", (torch.uint8,))
             if c8.dim() != 2 or c8.shape[0] != m or col_offset < 0 or col_offset + n > c8.shape[1]:
                 raise ValueError("out_fp8 must be [M, W] with col_offset + N <= W")
             epi.C_fp8, epi.ldc_fp8, epi.C_fp8_scale = c8.data_ptr() + col_offset, c8.shape[1], _ptr(out_fp8_scale)
     if not want_output and c8 is None:
         raise ValueError("want_output=False needs out_fp8_scale")
-    c = (out if out is not None else torch.empty((m, n), dtype=out_dtype, device=a_words.device)) if want_output else None
+    c = (out if out is not None else torch.empty((m, n), dtype=out_dtype, device=device)) if want_output else None
     if c is not None:
         _chk(c, "out", (out_dtype,))
-    _l.check(_l.load().lq_gemm_w4a4_ex(_ptr(c), _DT[out_dtype], _ptr(a_words), _ptr(w_rows32), _ptr(sA), _ptr(sB),
-                                       _DT[sA.dtype], _ptr(bias), _ptr(lora_act), _ptr(lora_up), lora_dt, rank, m, n, k,
-                                       group, C.byref(epi) if epi is not None else None, _stream()), "lq_gemm_w4a4_ex")
+    _l.check(launch(_ptr(c), (_ptr(lora_act), _ptr(lora_up), lora_dt, rank), C.byref(epi) if epi is not None else None), "lq_gemm_w4a4")
     if c8 is None:
         return c
     return (c, c8) if want_output else c8
@@ -922,6 +952,31 @@ def w4a4_quant_lora_down(x, smooth, lora_down_w, scale_dtype=torch.float32, out_
                                                   _DT[x.dtype], _ptr(smooth), _ptr(lora_down_w), m, k, rank, group, _stream()),
              "lq_w4a4_quantize_lora_down")
     return q, s, act
+
+
+def w4a4_expand_weight(packed_rows32):
+    """Packed 4-bit weights in rows32 layout uint8 [N, K/2] -> e4m3 codes in rows32 layout uint8 [N, K], for w4a4_linear_codes."""
+    _chk(packed_rows32, "packed_rows32", (torch.uint8, torch.int8))
+    n, kb = packed_rows32.shape
+    out = torch.empty((n, 2 * kb), dtype=torch.uint8, device=packed_rows32.device)
+    _l.check(_l.load().lq_w4a4_expand_rows32(_ptr(out), _ptr(packed_rows32), n, 2 * kb, _stream()), "lq_w4a4_expand_rows32")
+    return out
+
+
+def w4a4_quant_lora_down_codes(x, smooth, lora_down_w):
+    """w4a4_quant_lora_down (fp32 scales) for w4a4_linear_codes: returns (codes uint8 [M, K], scales fp32 [K/64, M], lora_act [M, 32])."""
+    _chk(x, "x", (torch.float16, torch.bfloat16))
+    _chk(lora_down_w, "lora_down_w", (x.dtype,))
+    _chk(smooth, "smooth", (torch.float32,))
+    m, k = x.shape
+    if tuple(lora_down_w.shape) != (32, k) or smooth.numel() != k:
+        raise ValueError("lora_down_w must be [32, K] and smooth [K]")
+    codes = torch.empty((m, k), dtype=torch.uint8, device=x.device)
+    s = torch.empty((k // 64, m), dtype=torch.float32, device=x.device)
+    act = torch.empty((m, 32), dtype=x.dtype, device=x.device)
+    _l.check(_l.load().lq_w4a4_quantize_lora_down_codes(_ptr(codes), _ptr(s), _ptr(act), _DT[x.dtype], _ptr(x), _DT[x.dtype], _ptr(smooth),
+                                                        _ptr(lora_down_w), m, k, 32, _stream()), "lq_w4a4_quantize_lora_down_codes")
+    return codes, s, act
 
 
 def rmsnorm_rope(qkv, norm_qk, rope, heads: int, context_qkv=None, norm_added_qk=None, eps: float = 1e-6):

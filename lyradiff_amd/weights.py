@@ -159,16 +159,33 @@ class W4A4Linear:
     lora_up: Optional[torch.Tensor] = None    # T [N, R]
     lora_down: Optional[torch.Tensor] = None  # T [R, K]
     bias: Optional[torch.Tensor] = None
+    # the weight as one e4m3 byte per value (rows32) and its scales group-major, made by use_codes(); forward then runs on codes
+    weight_codes: Optional[torch.Tensor] = None    # uint8 [N, K], rows32
+    weight_scale_t: Optional[torch.Tensor] = None  # fp32 [K/64, N]
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        k = x.shape[-1]
-        x2 = x.reshape(-1, k)
+    def use_codes(self) -> "W4A4Linear":
+        """Lays the weight out for the GEMM on codes (1.5 bytes per value held instead of 0.5; same results, 4608x3072x3072 77 us against
+        100).  Call it again after writing into weight_rows32 or weight_scale."""
+        n, k = self.weight_rows32.shape[0], 2 * self.weight_rows32.shape[1]
+        if k % 128 == 0 and k <= 16384 and self.lora_down is not None and tuple(self.lora_down.shape) == (32, k):
+            self.weight_codes = ops.w4a4_expand_weight(self.weight_rows32)
+            self.weight_scale_t = self.weight_scale.t().contiguous()
+        return self
+
+    def run(self, x2: torch.Tensor, **epilogue):
+        """W4A4Gemm::forward (W4A4Gemm.cc:113-169) on x2 [M, K] with ops.w4a4_linear's epilogue options: quantise, low-rank down, GEMM."""
+        if self.weight_codes is not None and x2.dtype == self.lora_down.dtype:
+            q, s, act = ops.w4a4_quant_lora_down_codes(x2, self.smooth, self.lora_down)
+            return ops.w4a4_linear_codes(q, self.weight_codes, s, self.weight_scale_t, self.bias, x2.dtype, act, self.lora_up, **epilogue)
         if self.lora_down is not None:
             q, s, act = ops.w4a4_quant_lora_down(x2, self.smooth, self.lora_down, torch.float32)
         else:
             (q, s), act = ops.w4a4_quant(x2, self.smooth, torch.float32), None
-        y = ops.w4a4_linear(q, self.weight_rows32, s, self.weight_scale, self.bias, x.dtype, 64, act,
-                            self.lora_up if act is not None else None)
+        return ops.w4a4_linear(q, self.weight_rows32, s, self.weight_scale, self.bias, x2.dtype, 64, act,
+                               self.lora_up if act is not None else None, **epilogue)
+
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        y = self.run(x.reshape(-1, x.shape[-1]))
         return y.reshape(*x.shape[:-1], y.shape[-1])
 
 
@@ -212,7 +229,7 @@ def load_w4a4_linear(src, prefix: str, d_out: int, d_in: int, lora_rank: int = 3
         lin.lora_down = get(prefix + "lora_down", (lora_rank, d_in), dtype).to(device)
     if has_bias:
         lin.bias = get(prefix + "bias", (d_out,), dtype).to(device)
-    return lin
+    return lin.use_codes()
 
 
 # ---- int4 <-> int8 host helpers of the weight tooling (offline, CPU tensors, as in the reference) ------------------

@@ -1,0 +1,62 @@
+"""The W4A4 linear on codes (one e4m3 byte per 4-bit value) against the packed-nibble kernels, which tests/test_gpu_quant.py and
+tests/test_gpu_gemm.py hold against the oracle: the arithmetic is the same, so every bit has to be."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# rows, outputs, k: one row, tiles of 64 and 128 rows and columns less / exactly / more than full, one and several k-tiles; 1201 x
+# 3072 is 456 tiles of 64 x 128 and 2945 x 3072 is 552 of 128 x 128, where the next larger tile takes over
+SHAPES = [(1, 32, 128), (63, 96, 256), (64, 64, 384), (65, 160, 128), (129, 3072, 512), (1201, 3072, 256), (2945, 3072, 256), (4608, 9216, 128)]
+
+
+def _values(words):
+    """int32 words [R, K/8] -> signed values [R, K]."""
+    shifts = torch.arange(0, 32, 4, device=words.device, dtype=torch.int64)
+    v = (words.to(torch.int64)[..., None] >> shifts) & 15
+    return torch.where(v > 7, v - 16, v).reshape(words.shape[0], -1)
+
+
+def _make(dev, m, n, k, dt):
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    x = rnd(m, k)
+    x[0, :64] = 0.0         # a group of zeros
+    x[-1, 64:128] *= 1e-41  # subnormal scale: the exact-division path
+    return (x.to(dt), 0.5 + torch.rand(k, generator=g, device=dev), (0.05 * rnd(32, k)).to(dt), torch.randint(-128, 128, (n, k // 2), generator=g, device=dev, dtype=torch.int8),
+            0.01 * torch.rand(n, k // 64, generator=g, device=dev), (0.05 * rnd(n, 32)).to(dt), rnd(n).to(dt), rnd)
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_linear_on_codes_is_bit_identical(dev, m, n, k, dt):
+    from lyradiff_amd import ops
+
+    x, smooth, down, packed, sb, up, bias, rnd = _make(dev, m, n, k, dt)
+    words, sa, act = ops.w4a4_quant_lora_down(x, smooth, down)
+    codes, sa_t, act_c = ops.w4a4_quant_lora_down_codes(x, smooth, down)
+    assert torch.equal(codes.view(torch.float8_e4m3fn).float(), _values(words).float())
+    assert torch.equal(sa_t, sa.t()) and torch.equal(act_c, act)
+
+    w = ops.repack_weight(packed.view(torch.uint8))
+    wc = ops.w4a4_expand_weight(w)
+    assert torch.equal(ops.unpack_weight(wc).view(torch.float8_e4m3fn).float(), _values(packed.view(torch.int32)).float())
+    sb_t = sb.t().contiguous()
+    add, res, gate = rnd(m, n).to(dt), rnd(m, n).to(dt), rnd((m + 6) // 7, n).to(dt)
+    s8 = torch.tensor([0.05], device=dev)
+    for epi in ({}, {"gelu": 2}, {"addend": add, "gate": gate, "residual": res, "rows_per_gate": 7}, {"gelu": 1, "out_fp8_scale": s8, "want_output": False}):
+        want = ops.w4a4_linear(words, w, sa, sb, bias, dt, 64, act, up, **epi)
+        got = ops.w4a4_linear_codes(codes, wc, sa_t, sb_t, bias, dt, act, up, **epi)
+        assert torch.equal(got, want), (m, n, k, sorted(epi))
+    assert torch.equal(ops.w4a4_linear_codes(codes, wc, sa_t, sb_t, None, dt), ops.w4a4_linear(words, w, sa, sb, None, dt))
+
+
+def test_linear_module_takes_either_form(dev):
+    from lyradiff_amd import ops
+    from lyradiff_amd.weights import W4A4Linear
+
+    x, smooth, down, packed, sb, up, bias, _ = _make(dev, 200, 256, 384, torch.bfloat16)
+    lin = W4A4Linear(ops.repack_weight(packed.view(torch.uint8)), sb, smooth, up, down, bias)
+    want = lin.forward(x)  # as constructed: packed nibbles
+    assert lin.weight_codes is None and lin.use_codes().weight_codes is not None
+    assert torch.equal(lin.forward(x), want)
