@@ -352,8 +352,8 @@ int lq_fp8_scale_cast_2d(uint8_t* dst, size_t dst_ld, const void* src, size_t sr
  * Replaces CutlassFpAIntBGemmRunner<T, uint8_t | uint4b_t, PER_COLUMN_SCALE_ONLY>::gemm (A, B, weight_scales, [biases,]
  * C, m, n, k, ...) (kernels/cutlass_kernels/fpA_intB_gemm/fpA_intB_gemm.h:27-130).  The reference multiplies every
  * dequantised weight by the scale in T inside the main loop; here the scale is applied once per output.
- * Two tile configurations: 0 = 256x256 (eight wavefronts, three stages; chosen from 192 such tiles up), 1 = 256x128 (four
- * wavefronts, two stages); both walk k in the same order and give the same bits.  lq_gemm_set_thread_tactic(0 | 1) picks
+ * The tile form follows from m and n (see lq_gemm_wo.hip).  Two of them can be asked for: 0 = 256x256 outputs per workgroup,
+ * 1 = 128x256; both walk k in the same order and give the same bits.  lq_gemm_set_thread_tactic(0 | 1) picks
  * one for the calling thread's next calls (the gemm_config argument of CutlassFpAIntBGemmRunner::gemm), -1 the built-in rule. */
 int lq_gemm_weight_only(void* C, const void* A, lq_dtype_t dtype, const uint8_t* B_prepared, lq_weight_kind_t kind,
                         const void* scales, const void* bias, int m, int n, int k, lq_stream_t stream);

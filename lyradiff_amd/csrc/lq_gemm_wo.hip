@@ -24,9 +24,12 @@
 // (evaluated in fp32 and rounded once to bf16; q * s is exact in fp32).  The k-tile of 64 lies inside one group; the
 // scales (and zeros) of the tile's output channels travel to LDS with the operands (one 4-byte transfer per lane).
 //
-// Tiling: 256x128 outputs per workgroup of four wavefronts (2x2), 128x64 per wavefront (eight 32x32 MFMA tiles:
-// every converted weight fragment is used by four MFMAs), k-tile 64, two LDS stages filled from registers
-// (activations XOR-swizzled, weights copied as they lie), the next tile's global loads in flight during the MFMAs.
+// Tiling: 32 to 256 outputs each way per workgroup (wo_form), k-tile 64, two or three LDS stages filled by direct-to-LDS
+// transfers (activations XOR-swizzled, weights copied as they lie).  Large problems give a wavefront 128x64 outputs (eight 32x32
+// MFMA tiles: every converted weight fragment is used by four MFMAs) and are bound by the vector instructions of the conversion
+// next to the matrix ones: int4 with zeros in bf16, 4608x12288x3072, 419 -> 322 us (1.08 PFLOP/s; the library's plain bf16
+// product on this card 1.11) with 2.75 instead of 5 instructions per weight and two workgroups of four wavefronts per CU instead
+// of one of eight.  Small problems are bound by the latency of a k-tile and share k out between wavefronts.
 #include "lq_gemm_core.h"
 
 namespace lq {
@@ -49,10 +52,15 @@ template <int G> __device__ __forceinline__ int wo_apply_h2(h2_t q, u32 s2, u32 
     if constexpr (G == 2) q = q + __builtin_bit_cast(h2_t, z2);   // v_pk_add_f16: T(. + z)
     return __builtin_bit_cast(int, q);
 }
-template <int G> __device__ __forceinline__ float wo_apply_f32(float q, u32 s, u32 z) {
-    if constexpr (G == 1) return q * __uint_as_float(s);                                      // exact in fp32
-    if constexpr (G == 2) return __builtin_fmaf(q, __uint_as_float(s), __uint_as_float(z));
-    return q;
+// u: the unsigned code as a float; s, z: fp32 bit patterns, z = the addend that wo_addend made of the offset and the zero point
+template <int G> __device__ __forceinline__ u32 wo_addend(u32 s, u32 z, float offset) {
+    if constexpr (G == 1) return __float_as_uint(-offset * __uint_as_float(s));                                   // exact
+    if constexpr (G == 2) return __float_as_uint(__builtin_fmaf(-offset, __uint_as_float(s), __uint_as_float(z)));
+    return __float_as_uint(-offset);
+}
+template <int G> __device__ __forceinline__ float wo_apply_f32(u32 u, u32 s, u32 z) {
+    if constexpr (G == 0) return (float)u + __uint_as_float(z);
+    else return __builtin_fmaf((float)u, __uint_as_float(s), __uint_as_float(z));
 }
 template <int G> struct WoCvt<true, false, G> {  // fp16 <- uint8: d0 holds k0..k3, d1 holds k4..k7
     static __device__ __forceinline__ v4i run(u32 d0, u32 d1, u32 s2, u32 z2) {
@@ -77,62 +85,77 @@ template <int G> struct WoCvt<true, true, G> {  // fp16 <- uint4: d0 holds k0..k
         return o;
     }
 };
-template <int G> struct WoCvt<false, false, G> {  // bf16 <- uint8 (through fp32: bf16 cannot hold 1024 + u)
+// bf16 goes through fp32 (it cannot hold 1024 + u): v_cvt_f32_ubyte takes a code from any byte of a register, so a weight costs
+// that, one fused multiply-add and half a packed conversion (and a quarter of a mask where two nibbles share a byte)
+template <int G> struct WoCvt<false, false, G> {  // bf16 <- uint8
     static __device__ __forceinline__ v4i run(u32 d0, u32 d1, u32 s, u32 z) {
         v4i o;
         const u32 d[2] = {d0, d1};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const u32 w = d[i >> 1] >> (16 * (i & 1));
-            o[i] = (int)pack2_bf16(wo_apply_f32<G>((float)(w & 0xFFu) - 128.0f, s, z), wo_apply_f32<G>((float)((w >> 8) & 0xFFu) - 128.0f, s, z));
+            const u32 w = d[i >> 1];
+            const int sh = 16 * (i & 1);
+            o[i] = (int)pack2_bf16(wo_apply_f32<G>((w >> sh) & 0xFFu, s, z), wo_apply_f32<G>((w >> (sh + 8)) & 0xFFu, s, z));
         }
         return o;
     }
 };
-template <int G> struct WoCvt<false, true, G> {  // bf16 <- uint4
+template <int G> struct WoCvt<false, true, G> {  // bf16 <- uint4: bytes of the even nibbles are k0 k4 k1 k5, of the odd ones k2 k6 k3 k7
     static __device__ __forceinline__ v4i run(u32 d0, u32, u32 s, u32 z) {
         v4i o;
+        const u32 d[2] = {d0 & 0x0F0F0F0Fu, (d0 >> 4) & 0x0F0F0F0Fu};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const u32 w = d0 >> (4 * i);
-            o[i] = (int)pack2_bf16(wo_apply_f32<G>((float)(w & 0xFu) - 8.0f, s, z), wo_apply_f32<G>((float)((w >> 16) & 0xFu) - 8.0f, s, z));
+            const u32 w = d[i & 1];
+            const int sh = 8 * (i >> 1);
+            o[i] = (int)pack2_bf16(wo_apply_f32<G>((w >> sh) & 0xFFu, s, z), wo_apply_f32<G>((w >> (sh + 16)) & 0xFFu, s, z));
         }
         return o;
     }
 };
 
-// WN = 2: 256x128 outputs, four wavefronts, two workgroups per CU.  WN = 4: 256x256 outputs, eight wavefronts, one
-// workgroup per CU (more operand reuse per LDS byte; the choice for large problems).
+// A workgroup's tile is (32 MT WM) x (32 NT WN) outputs, a wavefront's (32 MT) x (32 NT); KW groups of WM x WN wavefronts take
+// every KW-th k-tile, each with LDS stages of its own, and their sums meet in LDS at the end, added in group order.
 // GROUPED 0: scales [n], applied to the sums; 1: scales [k / group, n] applied to every weight; 2: scales and zeros.
-template <typename Tag, bool W4, int WN, int NSTAGE, int GROUPED = 0>
-__global__ __launch_bounds__(128 * WN, (WN == 2 ? 2 : 1)) void wo_gemm_kernel(void* __restrict__ C, const void* __restrict__ A,
-                                                                              const uint8_t* __restrict__ B,
-                                                                              const void* __restrict__ scales,
-                                                                              const void* __restrict__ zeros,
-                                                                              const void* __restrict__ bias, int m, int n, int k,
-                                                                              int tiles_m, int tiles_n, int tiles_per_group) {
-    constexpr bool F16 = std::is_same<Tag, F16Tag>::value;
-    constexpr int NW = 2 * WN, BM = 256, BN = 64 * WN, BK = 64, TM = 128, TN = 64, MT = 4, NT = 2;
-    constexpr int A_BYTES = BM * BK * 2;                 // 32 KiB
-    constexpr int BCH = W4 ? 2 : 4;                      // 16-byte weight chunks per row per k-tile
-    constexpr int B_BYTES = BN * BCH * 16;
-    constexpr int SZ_BYTES = GROUPED ? 1024 : 0;          // scales of the tile's BN channels at +0, zeros at +512
-    constexpr int STAGE = A_BYTES + B_BYTES + SZ_BYTES;
-    constexpr int A_DMA = A_BYTES / 1024 / NW;           // 1 KiB transfers per wavefront per tile
-    constexpr int B_DMA = B_BYTES / 1024 / NW;
-    constexpr int PER_TILE = A_DMA + B_DMA + GROUPED;     // + one 4-byte-per-lane transfer for the scales, one for the zeros
-    static_assert(A_DMA * NW * 1024 == A_BYTES && B_DMA * NW * 1024 == B_BYTES && B_DMA >= 1, "stage / wavefront mismatch");
+template <bool W4, int MT, int NT, int WM, int WN, int KW, int NSTAGE, int GROUPED> struct WoTile {
+    static constexpr int GW = WM * WN, NW = GW * KW, BM = 32 * MT * WM, BN = 32 * NT * WN, BK = 64;
+    static constexpr int A_BYTES = BM * BK * 2;
+    static constexpr int BCH = W4 ? 2 : 4;                      // 16-byte weight chunks per row per k-tile
+    static constexpr int B_BYTES = BN * BCH * 16;
+    static constexpr int Z_OFF = BN > 128 ? 512 : 256;          // scales of the tile's channels, then the zeros
+    static constexpr int SZ_BYTES = GROUPED ? 2 * Z_OFF : 0;
+    static constexpr int STAGE = A_BYTES + B_BYTES + SZ_BYTES;
+    static constexpr int REDUCE = KW > 1 ? NW * MT * NT * 4096 : 0;
+    static constexpr int LDS = KW * NSTAGE * STAGE > REDUCE ? KW * NSTAGE * STAGE : REDUCE;
+    static constexpr int A_DMA = A_BYTES / 1024 / GW;           // 1 KiB transfers per wavefront per tile
+    static constexpr int B_DMA = B_BYTES / 1024 / GW;
+    static constexpr int PER_TILE = A_DMA + B_DMA + GROUPED;    // + one 4-byte-per-lane transfer for the scales, one for the zeros
+    static_assert(A_DMA * GW * 1024 == A_BYTES && B_DMA * GW * 1024 == B_BYTES && B_DMA >= 1, "stage / wavefront mismatch");
+    static_assert(BN <= 128 || (BN == 256 && GW > 1), "scale transfer plan");
     static_assert(PER_TILE * NSTAGE < 64, "vmcnt is a 6-bit counter");
-    extern __shared__ __attribute__((aligned(16))) char wo_smem[];
+    static_assert(LDS <= 160 * 1024, "LDS of a CU");
+};
+
+template <typename Tag, bool W4, int MT, int NT, int WM, int WN, int KW, int NSTAGE, int GROUPED>
+__global__ __launch_bounds__(64 * WM * WN * KW, 2) void wo_gemm_kernel(void* __restrict__ C, const void* __restrict__ A,
+                                                                       const uint8_t* __restrict__ B, const void* __restrict__ scales,
+                                                                       const void* __restrict__ zeros, const void* __restrict__ bias, int m,
+                                                                       int n, int k, int tiles_m, int tiles_n, int tiles_per_group) {
+    constexpr bool F16 = std::is_same<Tag, F16Tag>::value;
+    using T = WoTile<W4, MT, NT, WM, WN, KW, NSTAGE, GROUPED>;
+    constexpr int BM = T::BM, BN = T::BN, BK = T::BK, TM = 32 * MT, TN = 32 * NT;
+    constexpr int A_BYTES = T::A_BYTES, BCH = T::BCH, B_BYTES = T::B_BYTES, Z_OFF = T::Z_OFF, STAGE = T::STAGE;
+    constexpr int A_DMA = T::A_DMA, B_DMA = T::B_DMA, PER_TILE = T::PER_TILE;
+    extern __shared__ __attribute__((aligned(16))) char wo_smem_all[];
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kg = wave_all / T::GW, wave = wave_all % T::GW;
     const int wm = wave / WN, wn = wave % WN;
-    // consecutive workgroup ids of one XCD (ids congruent modulo 8) walk down a column of tiles, so that an XCD's
-    // L2 keeps one weight panel and streams activations
-    int bid = blockIdx.x;
-    const int total = tiles_m * tiles_n, per_xcd = total / 8;
-    if (bid < per_xcd * 8) bid = (bid & 7) * per_xcd + (bid >> 3);
-    const int tm = bid % tiles_m, tn = bid / tiles_m;
+    char* wo_smem = wo_smem_all + kg * (NSTAGE * STAGE);
+    // the workgroups an XCD runs at once cover a block of 8 tile rows: fewer activation rows than a column of tiles would
+    // take, and the weights are a quarter or half as wide
+    int tm, tn;
+    tile_coords<8>(blockIdx.x, tiles_m, tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     const int ktiles = k / BK;
     const size_t a_pitch = (size_t)k * 2;
@@ -161,7 +184,7 @@ __global__ __launch_bounds__(128 * WN, (WN == 2 ? 2 : 1)) void wo_gemm_kernel(vo
     // group scales / zeros: lane l of a transfer fetches the pair of channels (2l, 2l+1) of its half of the tile's
     // columns; BN / 128 wavefronts cover the tile, the others repeat them (same bytes to the same place)
     const int sz_part = BN == 256 ? (wave & 1) : 0;
-    const u32 sz_voff = (u32)min(n0 + sz_part * 128 + 2 * lane, n - 2) * 2u;
+    const u32 sz_voff = (u32)min(n0 + sz_part * 128 + 2 * min(lane, BN / 2 - 1), n - 2) * 2u;
     // transfers lo..hi-1 of tile kt (activations, weights, then the group scales and zeros); lo and hi are compile-time
     // values after unrolling
     auto issue_range = [&](int kt, int stage, int lo, int hi) {
@@ -178,7 +201,7 @@ __global__ __launch_bounds__(128 * WN, (WN == 2 ? 2 : 1)) void wo_gemm_kernel(vo
                 const size_t grow = (size_t)(kt / tiles_per_group) * (size_t)n * 2;
                 const u32 ss = smem_base + stage * STAGE + A_BYTES + B_BYTES + sz_part * 256;
                 if (d == A_DMA + B_DMA) dma4(static_cast<const char*>(scales) + grow, sz_voff, ss);
-                else dma4(static_cast<const char*>(zeros) + grow, sz_voff, ss + 512);
+                else dma4(static_cast<const char*>(zeros) + grow, sz_voff, ss + Z_OFF);
             }
         }
     };
@@ -195,17 +218,18 @@ __global__ __launch_bounds__(128 * WN, (WN == 2 ? 2 : 1)) void wo_gemm_kernel(vo
     const int lr = lane & 31, lh = lane >> 5;
     const int xrow = wm * TM + lr;
     const int xsw = wo_swizzle<8>(xrow);  // unchanged by +32*i
-    // One k-tile = 16 steps (half, s, i): one 16-byte activation fragment and NT MFMAs each.  Fragments are read two
+    // One k-tile = 4 MT steps (half, s, i): one 16-byte activation fragment and NT MFMAs each.  Fragments are read two
     // steps ahead of their use and the order "read, NT MFMAs" is pinned with scheduling barriers, so that the matrix
     // pipe does not wait for an LDS round trip at every step; the weights of the second half are converted while
     // the MFMAs of the first half run.
     // (with three stages the transfers of tile kt_next go out one or two at a time between the steps: a wavefront that
     // stalls on a full memory-instruction queue cannot issue its next MFMA)
+    constexpr int STEPS = 4 * MT;
     auto compute = [&](int stage, int kt_next, int stage_next) {
         const char* sa = wo_smem + stage * STAGE;
         const char* sb = sa + A_BYTES + (wn * NT) * (BCH * 512) + lr * 16;
         auto xptr = [&](int t) -> const v4i* {
-            const int half = t >> 3, s2 = (t >> 2) & 1, i = t & 3;
+            const int half = t / (2 * MT), s2 = t / MT & 1, i = t % MT;
             const int chunk = W4 ? lh * 4 + half * 2 + s2 : half * 4 + lh * 2 + s2;
             return reinterpret_cast<const v4i*>(sa + (xrow + i * 32) * 128 + ((chunk ^ xsw) << 4));
         };
@@ -228,10 +252,11 @@ __global__ __launch_bounds__(128 * WN, (WN == 2 ? 2 : 1)) void wo_gemm_kernel(vo
                 const u32 sv = *reinterpret_cast<const unsigned short*>(szp);
                 gs[j] = F16 ? (sv | (sv << 16)) : (sv << 16);
                 if constexpr (GROUPED == 2) {
-                    const u32 zv = *reinterpret_cast<const unsigned short*>(szp + 512);
+                    const u32 zv = *reinterpret_cast<const unsigned short*>(szp + Z_OFF);
                     gz[j] = F16 ? (zv | (zv << 16)) : (zv << 16);
                 }
             }
+            if constexpr (!F16) gz[j] = wo_addend<GROUPED>(gs[j], gz[j], W4 ? 8.0f : 128.0f);
         }
         v4i xb[3];
         xb[0] = *xptr(0);
@@ -251,10 +276,10 @@ __global__ __launch_bounds__(128 * WN, (WN == 2 ? 2 : 1)) void wo_gemm_kernel(vo
         };
         convert(0);
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            const int half = t >> 3, s2 = (t >> 2) & 1, i = t & 3;
-            if constexpr (NSTAGE >= 3) issue_range(kt_next, stage_next, t * PER_TILE / 16, (t + 1) * PER_TILE / 16);
-            if (t + 2 < 16) xb[(t + 2) % 3] = *xptr(t + 2);
+        for (int t = 0; t < STEPS; ++t) {
+            const int half = t / (2 * MT), s2 = t / MT & 1, i = t % MT;
+            if constexpr (NSTAGE >= 3) issue_range(kt_next, stage_next, t * PER_TILE / STEPS, (t + 1) * PER_TILE / STEPS);
+            if (t + 2 < STEPS) xb[(t + 2) % 3] = *xptr(t + 2);
             if (t == 2) convert(1);
             const v4i x = xb[t % 3];
 #pragma unroll
@@ -270,7 +295,7 @@ __global__ __launch_bounds__(128 * WN, (WN == 2 ? 2 : 1)) void wo_gemm_kernel(vo
         // MFMAs of the last two steps
         __builtin_amdgcn_sched_group_barrier(0x100, (W4 ? NT : 2 * NT) + 2 + GROUPED * NT, 0);  // DS reads
 #pragma unroll
-        for (int t = 0; t < 14; ++t) {
+        for (int t = 0; t < STEPS - 2; ++t) {
             __builtin_amdgcn_sched_group_barrier(0x008, NT, 0);  // MFMA
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);   // DS read
         }
@@ -281,55 +306,85 @@ __global__ __launch_bounds__(128 * WN, (WN == 2 ? 2 : 1)) void wo_gemm_kernel(vo
     // re-fetches the last tile into a stage nobody reads again), so the vmcnt threshold is a compile-time value:
     // when at most (NSTAGE-2) tiles of this wavefront's transfers are outstanding, its part of tile kt has landed;
     // after the barrier everybody's has, and everybody has finished reading the stage that is re-armed next.
+    // The tiles of a k-group are kg, kg + KW, ...; every group makes the same number of rounds.
+    const int rounds = (ktiles + KW - 1) / KW;
+    auto tile_of = [&](int i) { return min(kg + i * KW, ktiles - 1); };
 #pragma unroll
-    for (int t = 0; t < NSTAGE - 1; ++t) issue(min(t, ktiles - 1), t);
-    for (int kt = 0; kt < ktiles; ++kt) {
+    for (int t = 0; t < NSTAGE - 1; ++t) issue(tile_of(t), t);
+    for (int i = 0; i < rounds; ++i) {
         wait_vmcnt<PER_TILE*(NSTAGE - 2)>();
-        __syncthreads();
+        // a wavefront whose stages are its own only has to be done with its reads
+        if constexpr (T::GW > 1) __syncthreads();
+        else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         // two stages: the next tile must be on its way for the whole of this one, so its transfers go out at once
-        if constexpr (NSTAGE < 3) issue(min(kt + NSTAGE - 1, ktiles - 1), (kt + NSTAGE - 1) % NSTAGE);
-        compute(kt % NSTAGE, min(kt + NSTAGE - 1, ktiles - 1), (kt + NSTAGE - 1) % NSTAGE);
+        if constexpr (NSTAGE < 3) issue(tile_of(i + NSTAGE - 1), (i + NSTAGE - 1) % NSTAGE);
+        if (KW == 1 || kg + i * KW < ktiles) compute(i % NSTAGE, tile_of(i + NSTAGE - 1), (i + NSTAGE - 1) % NSTAGE);
+        else if constexpr (NSTAGE >= 3) issue(tile_of(i + NSTAGE - 1), (i + NSTAGE - 1) % NSTAGE);
     }
     wait_vmcnt<0>();  // nothing in flight towards LDS when the workgroup ends
 
     // ---- epilogue: weights were the first MFMA operand, so a lane holds one activation row (lr) and, per tile,
     // four runs of four consecutive output channels: 8-byte stores -------------------------------------------------
     const int mrow0 = m0 + wm * TM + lr;
+    struct Chan { float sc[4], bs[4]; };
+    auto channels = [&](int nn) {  // scale and bias of four consecutive channels
+        Chan c;
+        uint2 sv = make_uint2(0, 0), bv = make_uint2(0, 0);
+        if (nn < n && GROUPED == 0) sv = *reinterpret_cast<const uint2*>(static_cast<const unsigned short*>(scales) + nn);
+        if (nn < n && bias != nullptr) bv = *reinterpret_cast<const uint2*>(static_cast<const unsigned short*>(bias) + nn);
+        c.sc[0] = Elem<Tag>::load(sv.x & 0xFFFFu); c.sc[1] = Elem<Tag>::load(sv.x >> 16);
+        c.sc[2] = Elem<Tag>::load(sv.y & 0xFFFFu); c.sc[3] = Elem<Tag>::load(sv.y >> 16);
+        c.bs[0] = Elem<Tag>::load(bv.x & 0xFFFFu); c.bs[1] = Elem<Tag>::load(bv.x >> 16);
+        c.bs[2] = Elem<Tag>::load(bv.y & 0xFFFFu); c.bs[3] = Elem<Tag>::load(bv.y >> 16);
+        return c;
+    };
+    auto store4 = [&](const float* sum, const Chan& c, int mr, int nn) {
+        if (mr >= m || nn >= n) return;
+        float y[4];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        const int nb = n0 + wn * TN + j * 32;
-        float sc[16], bs[16];
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-            const int nn = nb + q4 * 8 + lh * 4;
-            const bool ok = nn < n;
-            uint2 sv = make_uint2(0, 0), bv = make_uint2(0, 0);
-            if (ok && GROUPED == 0) sv = *reinterpret_cast<const uint2*>(static_cast<const unsigned short*>(scales) + nn);
-            if (ok && bias != nullptr) bv = *reinterpret_cast<const uint2*>(static_cast<const unsigned short*>(bias) + nn);
-            sc[q4 * 4] = Elem<Tag>::load(sv.x & 0xFFFFu); sc[q4 * 4 + 1] = Elem<Tag>::load(sv.x >> 16);
-            sc[q4 * 4 + 2] = Elem<Tag>::load(sv.y & 0xFFFFu); sc[q4 * 4 + 3] = Elem<Tag>::load(sv.y >> 16);
-            bs[q4 * 4] = Elem<Tag>::load(bv.x & 0xFFFFu); bs[q4 * 4 + 1] = Elem<Tag>::load(bv.x >> 16);
-            bs[q4 * 4 + 2] = Elem<Tag>::load(bv.y & 0xFFFFu); bs[q4 * 4 + 3] = Elem<Tag>::load(bv.y >> 16);
+        for (int e = 0; e < 4; ++e) {
+            y[e] = GROUPED == 0 ? sum[e] * c.sc[e] : sum[e];
+            if (bias != nullptr) y[e] = y[e] + c.bs[e];
         }
+        uint2 o;
+        if constexpr (F16) { o.x = pack2_f16(y[0], y[1]); o.y = pack2_f16(y[2], y[3]); }
+        else { o.x = pack2_bf16(y[0], y[1]); o.y = pack2_bf16(y[2], y[3]); }
+        *reinterpret_cast<uint2*>(static_cast<unsigned short*>(C) + (size_t)mr * n + nn) = o;
+    };
+    if constexpr (KW == 1) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            const int mr = mrow0 + i * 32;
-            if (mr >= m) continue;
+        for (int j = 0; j < NT; ++j) {
+            Chan c[4];
 #pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const int nn = nb + q4 * 8 + lh * 4;
-                if (nn >= n) continue;
-                float y[4];
+            for (int q4 = 0; q4 < 4; ++q4) c[q4] = channels(n0 + wn * TN + j * 32 + q4 * 8 + lh * 4);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    y[e] = GROUPED == 0 ? acc[i][j][q4 * 4 + e] * sc[q4 * 4 + e] : acc[i][j][q4 * 4 + e];
-                    if (bias != nullptr) y[e] = y[e] + bs[q4 * 4 + e];
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    const float sum[4] = {acc[i][j][q4 * 4], acc[i][j][q4 * 4 + 1], acc[i][j][q4 * 4 + 2], acc[i][j][q4 * 4 + 3]};
+                    store4(sum, c[q4], mrow0 + i * 32, n0 + wn * TN + j * 32 + q4 * 8 + lh * 4);
                 }
-                uint2 o;
-                if constexpr (F16) { o.x = pack2_f16(y[0], y[1]); o.y = pack2_f16(y[2], y[3]); }
-                else { o.x = pack2_bf16(y[0], y[1]); o.y = pack2_bf16(y[2], y[3]); }
-                *reinterpret_cast<uint2*>(static_cast<unsigned short*>(C) + (size_t)mr * n + nn) = o;
+        }
+    } else {
+        constexpr int QUADS = MT * NT * 4;  // four channels per lane each; group g adds and stores the quads g, g + KW, ...
+        float4* part = reinterpret_cast<float4*>(wo_smem_all) + lane;
+        __syncthreads();  // everybody is done with the stages
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q) {
+            const v16f& a = acc[q / (4 * NT)][q / 4 % NT];
+            part[(wave_all * QUADS + q) * 64] = make_float4(a[q % 4 * 4], a[q % 4 * 4 + 1], a[q % 4 * 4 + 2], a[q % 4 * 4 + 3]);
+        }
+        __syncthreads();
+        for (int q = kg; q < QUADS; q += KW) {
+            const int nn = n0 + wn * TN + (q / 4 % NT) * 32 + q % 4 * 8 + lh * 4;
+            const Chan c = channels(nn);
+            float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int g = 0; g < KW; ++g) {
+                const float4 v = part[((g * T::GW + wave) * QUADS + q) * 64];
+                sum[0] += v.x; sum[1] += v.y; sum[2] += v.z; sum[3] += v.w;
             }
+            store4(sum, c, mrow0 + q / (4 * NT) * 32, nn);
         }
     }
 }
@@ -380,41 +435,67 @@ extern "C" int lq_repack_weight_only(uint8_t* dst, const int8_t* src_kn, lq_weig
     return check_launch("wo_repack");
 }
 
+// Tile forms: outputs of a workgroup and, after K, the number of its wavefront groups that share the k-tiles out.
+enum WoForm { WO_32x32_K8, WO_32x32_K4, WO_64x64_K4, WO_128x128_K2, WO_128x256, WO_256x256 };
+
+// The form whose rounds of workgroups on the chip take least.  `first` and `round`: time of a launch of at most 256 workgroups
+// and of one that fills the chip, measured at k = 3072 (us, int8 codes and fp16; int4 with zeros and bf16 gives 8, 10, 13, 35,
+// 51 / 88 and 80, nearly the same order); a longer k scales all of them.  A workgroup of a small tile that walks k alone takes 0.5 to
+// 0.8 us per k-tile however few there are (the 256x128 tiles that stood here: 28.7 us at 154x1280x2048, 51 us at 1x9216x3072,
+// 7.4 and 8.0 with k shared out), so the less the tiles fill the chip the more wavefronts share k.
+static WoForm wo_form(int m, int n) {
+    struct Cost { WoForm form; int bm, bn, slots; float first, round; };
+    static const Cost table[] = {{WO_256x256, 256, 256, 256, 75, 75}, {WO_128x256, 128, 256, 512, 42, 75}, {WO_128x128_K2, 128, 128, 256, 24, 28},
+                                 {WO_64x64_K4, 64, 64, 256, 10, 10}, {WO_32x32_K4, 32, 32, 512, 8, 8}, {WO_32x32_K8, 32, 32, 256, 7, 7}};
+    WoForm best = WO_256x256;
+    float least = 0.0f;
+    for (const Cost& c : table) {
+        const long tiles = ((long)m + c.bm - 1) / c.bm * (((long)n + c.bn - 1) / c.bn), left = tiles % c.slots;
+        const float cost = (float)(tiles / c.slots) * c.round + (left == 0 ? 0.0f : left <= 256 ? c.first : c.round);
+        if (least == 0.0f || cost < least) { best = c.form; least = cost; }
+    }
+    return best;
+}
+
 static int wo_launch(void* C, const void* A, lq_dtype_t dtype, const uint8_t* B_prepared, lq_weight_kind_t kind, const void* scales,
                      const void* zeros, const void* bias, int m, int n, int k, int group_size, lq_stream_t stream) {
     const bool w4 = kind == LQ_W_INT4;
     const int grouped = group_size == 0 ? 0 : (zeros == nullptr ? 1 : 2);
     const int tiles_per_group = group_size == 0 ? 1 : group_size / 64;
-    // 256x256 tiles (eight wavefronts, three stages) once they give every CU work; 256x128 tiles otherwise
-    // A tile configuration set with lq_gemm_set_thread_tactic wins: 0 = 256x256, 1 = 256x128.
-    const long big_tiles = (long)((m + 255) / 256) * ((n + 255) / 256);
+    // A tile configuration set with lq_gemm_set_thread_tactic wins: 0 = 256x256, 1 = 128x256.
     if (tl_forced_tactic > 1) {
-        set_error("gemm_weight_only: unknown tile configuration %d (0 = 256x256, 1 = 256x128)", tl_forced_tactic);
+        set_error("gemm_weight_only: unknown tile configuration %d (0 = 256x256, 1 = 128x256)", tl_forced_tactic);
         return LQ_ERR_ARG;
     }
-    const bool big = tl_forced_tactic >= 0 ? tl_forced_tactic == 0 : big_tiles >= 192;
+    const WoForm form = tl_forced_tactic >= 0 ? (tl_forced_tactic == 0 ? WO_256x256 : WO_128x256) : wo_form(m, n);
     hipStream_t st = as_stream(stream);
-#define LQ_WO_GO(TAG, W4V, WNV, NST, GRP)                                                                               \
+#define LQ_WO_GO(TAG, W4V, GRP, MT, NT, WM, WN, KW, NST)                                                                \
     do {                                                                                                                \
-        constexpr size_t lds = (size_t)(NST) * (256 * 64 * 2 + 64 * (WNV) * ((W4V) ? 2 : 4) * 16 + ((GRP) ? 1024 : 0)); \
+        using T = WoTile<W4V, MT, NT, WM, WN, KW, NST, GRP>;                                                            \
+        auto kern = &wo_gemm_kernel<TAG, W4V, MT, NT, WM, WN, KW, NST, GRP>;                                            \
         static bool attr_done = false;                                                                                  \
         if (!attr_done) {                                                                                               \
-            if (hipFuncSetAttribute(reinterpret_cast<const void*>(&wo_gemm_kernel<TAG, W4V, WNV, NST, GRP>),            \
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {              \
-                set_error("lq_gemm_weight_only: cannot raise the dynamic LDS limit to %zu bytes", lds);                 \
+            if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,    \
+                                    T::LDS) != hipSuccess) {                                                            \
+                set_error("lq_gemm_weight_only: cannot raise the dynamic LDS limit to %d bytes", T::LDS);               \
                 return LQ_ERR_HIP;                                                                                      \
             }                                                                                                           \
             attr_done = true;                                                                                           \
         }                                                                                                               \
-        const int tiles_m = (m + 255) / 256, tiles_n = (n + 64 * (WNV) - 1) / (64 * (WNV));                             \
-        hipLaunchKernelGGL((wo_gemm_kernel<TAG, W4V, WNV, NST, GRP>), dim3((unsigned)(tiles_m * tiles_n)),              \
-                           dim3(128 * (WNV)), lds, st, C, A, B_prepared, scales, zeros, bias, m, n, k, tiles_m, tiles_n, \
-                           tiles_per_group);                                                                            \
+        const int tiles_m = (m + T::BM - 1) / T::BM, tiles_n = (n + T::BN - 1) / T::BN;                                 \
+        hipLaunchKernelGGL(kern, dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * T::NW), T::LDS, st, C, A, B_prepared,   \
+                           scales, zeros, bias, m, n, k, tiles_m, tiles_n, tiles_per_group);                            \
     } while (0)
-#define LQ_WO_SIZE(TAG, W4V, GRP)                  \
-    do {                                           \
-        if (big) LQ_WO_GO(TAG, W4V, 4, 3, GRP);    \
-        else LQ_WO_GO(TAG, W4V, 2, 2, GRP);        \
+#define LQ_WO_SIZE(TAG, W4V, GRP)                                              \
+    do {                                                                       \
+        switch (form) {                                                        \
+            case WO_32x32_K8: LQ_WO_GO(TAG, W4V, GRP, 1, 1, 1, 1, 8, 3); break; \
+            case WO_32x32_K4: LQ_WO_GO(TAG, W4V, GRP, 1, 1, 1, 1, 4, 3); break; \
+            case WO_64x64_K4: LQ_WO_GO(TAG, W4V, GRP, 2, 2, 1, 1, 4, 3); break; \
+            case WO_128x128_K2: LQ_WO_GO(TAG, W4V, GRP, 2, 2, 2, 2, 2, 3); break; \
+            case WO_128x256: LQ_WO_GO(TAG, W4V, GRP, 4, 2, 1, 4, 1, (W4V ? 3 : 2)); break; \
+            case WO_256x256: LQ_WO_GO(TAG, W4V, GRP, 4, 2, 2, 4, 1, 3); break;  \
+        }                                                                      \
     } while (0)
 #define LQ_WO_KIND(TAG, GRP)                       \
     do {                                           \
