@@ -210,12 +210,15 @@ template <int NP, int G, int... I> __device__ __forceinline__ void sched_interle
     (sched_slot<NP, G, I>(), ...);
 }
 
-template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE>
+// KW > 1: KW groups of WM x WN wavefronts compute the same tile over every KW-th k-tile, each with LDS stages of its own, and
+// their accumulators meet in LDS, added in group order (kb % (KW * BKB) == 0).  For problems whose tiles leave most of the chip
+// idle: a workgroup alone on a CU takes about 0.3 us per k-tile whatever it computes (lq_gemm_small.h).
+template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE, int KW = 1>
 struct GemmKernel {
     static constexpr int NW = WM * WN;
     static constexpr bool W4C = KIND == K_W4C;
     static constexpr bool W4 = (KIND == K_W4A4 || KIND == K_W4A4H || W4C);
-    static constexpr int THREADS = NW * 64;
+    static constexpr int THREADS = NW * KW * 64;
     static constexpr int TM = BM / WM, TN = BN / WN;  // wavefront tile
     static constexpr int MT = TM / 32, NT = TN / 32;  // 32x32 MFMA tiles per wavefront
     static constexpr int CH = BKB / 16;               // 16-byte chunks per tile row
@@ -225,7 +228,11 @@ struct GemmKernel {
     static constexpr int S_DMA = W4 ? (NS + 64 * NW - 1) / (64 * NW) : 0;  // 4-byte scale transfers per wavefront per tile
     static constexpr int SCALE_BYTES = S_DMA * NW * 256;  // NS floats, padded to whole transfers
     static constexpr int STAGE_BYTES = A_BYTES + B_BYTES + SCALE_BYTES;
-    static constexpr int SMEM_BYTES = NSTAGE * STAGE_BYTES;
+    static constexpr int STAGES_B = KW * NSTAGE * STAGE_BYTES, REDUCE_B = KW > 1 ? KW * NW * MT * NT * 4096 : 0;
+    static constexpr int STRIPS_B = KW > 1 ? KW * NW * 32 * (TN * 4 + 16) : 0;
+    static constexpr int LARGER_B = STAGES_B > REDUCE_B ? STAGES_B : REDUCE_B;
+    static constexpr int SMEM_BYTES = LARGER_B > STRIPS_B ? LARGER_B : STRIPS_B;
+    static_assert(KW == 1 || !W4, "no k-groups for W4A4");
     static constexpr int A_DMA = A_BYTES / 1024 / NW, B_DMA = B_BYTES / 1024 / NW;  // transfers per wavefront per tile
     static constexpr int PER_TILE = A_DMA + B_DMA + S_DMA;
     static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0, "tile/wavefront mismatch");
@@ -238,24 +245,32 @@ struct GemmKernel {
     static constexpr int KSTEP = (KIND == K_FP8 || W4C) ? 64 : 32;  // operand bytes per MFMA k-step
     static constexpr int KS = BKB / KSTEP;
 
-    static __device__ __forceinline__ void run(const GemmParams& p, char* smem) {
+    // between the k-tiles of a group: a wavefront whose stages are its own only has to be done with its reads
+    static __device__ __forceinline__ void tile_barrier() {
+        if constexpr (NW > 1) __syncthreads();
+        else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+
+    static __device__ __forceinline__ void run(const GemmParams& p, char* smem_all) {
         const int tid = threadIdx.x, lane = tid & 63;
-        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int kg = KW > 1 ? wave_all / NW : 0, wave = KW > 1 ? wave_all % NW : wave_all;
+        char* smem = smem_all + kg * (NSTAGE * STAGE_BYTES);
         const int wm = wave / WN, wn = wave % WN;
         int tm, tn;
         // band height chosen so that the workgroups an XCD runs at once cover a roughly square block of C
         tile_coords<(BM >= 256 ? 4 : 8)>(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
         const int m0 = tm * BM, n0 = tn * BN;
         const int kb = p.kb;
-        const int ktiles = kb / BKB;
+        const int ktiles = kb / (BKB * KW);  // of this group
         const size_t b_block_stride = (size_t)(kb / 16) * 512;  // bytes per 32-row block in rows32 layout
         const u32 smem_base = (u32)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
 
         // ---- global -> LDS transfer plan (per lane offsets are fixed; the bases advance with k) ----
         const u32 a_pitch = p.a_panel ? (u32)BKB : (u32)kb;                      // bytes between two rows of A
-        const size_t a_kstep = p.a_panel ? (size_t)p.m * BKB : (size_t)BKB;  // bytes between two k-tiles of a row
-        const uint8_t* a_base = p.A + (size_t)m0 * a_pitch;
-        const uint8_t* b_base = p.B + (size_t)(n0 / 32) * b_block_stride;
+        const size_t a_kstep = (p.a_panel ? (size_t)p.m * BKB : (size_t)BKB) * KW;  // bytes between two k-tiles of a row
+        const uint8_t* a_base = p.A + (size_t)m0 * a_pitch + (size_t)kg * (a_kstep / KW);
+        const uint8_t* b_base = p.B + (size_t)(n0 / 32) * b_block_stride + (size_t)kg * (BKB * 32);
         u32 a_voff[A_DMA], b_voff[B_DMA];
         const int row_last = p.m - 1 - m0, blk_last = p.n / 32 - 1 - n0 / 32;
 #pragma unroll
@@ -328,7 +343,7 @@ struct GemmKernel {
 
         auto issue_tile = [&](int kt, int stage) {
             const uint8_t* ga = a_base + (size_t)kt * a_kstep;
-            const uint8_t* gb = b_base + (size_t)kt * (BKB * 32);
+            const uint8_t* gb = b_base + (size_t)kt * (BKB * 32 * KW);
             const u32 sa = smem_base + stage * STAGE_BYTES + wave * (A_DMA * 1024);
             const u32 sb = smem_base + stage * STAGE_BYTES + A_BYTES + wave * (B_DMA * 1024);
 #pragma unroll
@@ -341,7 +356,7 @@ struct GemmKernel {
         // between their MFMAs; lo and hi are compile-time values after unrolling.
         auto issue_range = [&](int kt, int stage, int lo, int hi) {
             const uint8_t* ga = a_base + (size_t)kt * a_kstep;
-            const uint8_t* gb = b_base + (size_t)kt * (BKB * 32);
+            const uint8_t* gb = b_base + (size_t)kt * (BKB * 32 * KW);
             const u32 sa = smem_base + stage * STAGE_BYTES + wave * (A_DMA * 1024);
             const u32 sb = smem_base + stage * STAGE_BYTES + A_BYTES + wave * (B_DMA * 1024);
 #pragma unroll
@@ -592,7 +607,7 @@ struct GemmKernel {
                         }
                         __builtin_amdgcn_sched_barrier(0);
                         wait_vmcnt<PER_TILE*(NSTAGE - 2)>();
-                        __syncthreads();
+                        tile_barrier();
                         const int t_next = min(kt + NSTAGE, ktiles - 1);
                         if constexpr (!SPREAD) issue_tile(t_next, kt % NSTAGE);
                         __builtin_amdgcn_sched_barrier(0);
@@ -620,7 +635,7 @@ struct GemmKernel {
                 for (int s = 0; s < NSTAGE; ++s) issue_tile(min(s, ktiles - 1), s);
                 wait_vmcnt<PER_TILE*(NSTAGE - 1)>();
             }
-            __syncthreads();
+            tile_barrier();
 #pragma unroll
             for (int pc = 0; pc < NPIECE; ++pc) load_piece(smem, 0, 0, pc);
             int kt = 0;
@@ -651,6 +666,36 @@ struct GemmKernel {
         }
         wait_vmcnt<0>();
         __syncthreads();  // every transfer has landed and nobody reads operands any more: LDS is reusable
+        // ---- k-groups: band i of a wavefront's tile is added up, scaled and stored by group i % KW ------------------------
+        if constexpr (KW > 1) {
+            v4i* part = reinterpret_cast<v4i*>(smem_all) + lane;
+            constexpr int QUADS = MT * NT * 4;
+#pragma unroll
+            for (int q = 0; q < QUADS; ++q) {
+                const v16i a = __builtin_bit_cast(v16i, acc[q / (4 * NT)][q / 4 % NT]);
+                const v4i w = {a[q % 4 * 4], a[q % 4 * 4 + 1], a[q % 4 * 4 + 2], a[q % 4 * 4 + 3]};
+                part[(wave_all * QUADS + q) * 64] = w;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                if (i % KW != kg) continue;
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; ++q4)
+#pragma unroll
+                        for (int g = 0; g < KW; ++g) {
+                            const v4i w = part[((g * NW + wave) * QUADS + (i * NT + j) * 4 + q4) * 64];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                if constexpr (KIND == K_INT8) acc[i][j][q4 * 4 + e] = g == 0 ? w[e] : acc[i][j][q4 * 4 + e] + w[e];
+                                else acc[i][j][q4 * 4 + e] = g == 0 ? __int_as_float(w[e]) : acc[i][j][q4 * 4 + e] + __int_as_float(w[e]);
+                            }
+                        }
+            }
+            __syncthreads();  // the strips below take the place of the parts
+        }
 
         // ---- W4A4 low-rank branch ---------------------------------------------------------------------------
         // res += act[m, 0:rank] . up[n, 0:rank]^T on the 16-bit float matrix instruction, straight onto the fp32
@@ -698,9 +743,9 @@ struct GemmKernel {
         constexpr int PITCH = TN * 4 + 16;  // strip row: TN raw values + one 16-byte pad slot
         constexpr int LPR = TN / 4;         // lanes per output row on the way out
         constexpr int RPI = 64 / LPR;       // rows per store instruction
-        static_assert(NW * 32 * PITCH <= SMEM_BYTES, "epilogue strip does not fit in the operand stages");
+        static_assert(KW * NW * 32 * PITCH <= SMEM_BYTES, "epilogue strip does not fit in the operand stages");
         static_assert(64 % LPR == 0 && 32 % RPI == 0, "wave tile width must be 32, 64, 128 or 256");
-        char* strip = smem + wave * (32 * PITCH);
+        char* strip = smem_all + wave_all * (32 * PITCH);
         const int out_row = lane / LPR, out_n = n0 + wn * TN + (lane % LPR) * 4;
         const bool n_ok = out_n < p.n;
         float alpha = 1.0f, bias4[4] = {0.f, 0.f, 0.f, 0.f}, acol4[4] = {0.f, 0.f, 0.f, 0.f}, arow_l[MT];
@@ -857,6 +902,7 @@ struct GemmKernel {
         auto all_bands = [&](auto mode_c, auto full_c) {
             auto one_band = [&](auto i_c) {
                 constexpr int i = decltype(i_c)::value;
+                if (KW > 1 && i % KW != kg) return;
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
 #pragma unroll
@@ -938,17 +984,17 @@ template <int KIND, int BM, int BN, int BKB, int WM, int WN> constexpr int min_w
     return BKB == 128 ? 1 : 2;
 }
 
-template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE>
-__global__ __launch_bounds__(WM* WN * 64, (min_workgroups_per_cu<KIND, BM, BN, BKB, WM, WN>())) void gemm_kernel(GemmParams p) {
+template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE, int KW = 1>
+__global__ __launch_bounds__(WM* WN * KW * 64, (min_workgroups_per_cu<KIND, BM, BN, BKB, WM, WN>())) void gemm_kernel(GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) char lq_smem[];
-    GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE>::run(p, lq_smem);
+    GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>::run(p, lq_smem);
 }
 
-template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE>
+template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE, int KW = 1>
 static int launch_gemm(GemmParams p, hipStream_t st) {
-    using GK = GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE>;
-    if (p.kb % BKB != 0) {
-        set_error("gemm: row length %d bytes is not a multiple of the %d-byte k-tile", p.kb, BKB);
+    using GK = GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>;
+    if (p.kb % (BKB * KW) != 0) {
+        set_error("gemm: row length %d bytes is not a multiple of the %d-byte k-tile", p.kb, BKB * KW);
         return LQ_ERR_SHAPE;
     }
     if (p.a_panel && BKB != 64) {
@@ -957,7 +1003,7 @@ static int launch_gemm(GemmParams p, hipStream_t st) {
     }
     p.tiles_m = (p.m + BM - 1) / BM;
     p.tiles_n = (p.n + BN - 1) / BN;
-    auto kern = gemm_kernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE>;
+    auto kern = gemm_kernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>;
     static bool attr_done = false;  // raising the dynamic LDS limit is idempotent; races are benign
     if (!attr_done && GK::SMEM_BYTES > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -978,6 +1024,15 @@ static int launch_gemm(GemmParams p, hipStream_t st) {
 // bias, an output type other than fp16 / bf16) -- the caller then runs the plain configuration -- negative on an error.
 int launch_persist_fp8(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st);
 int launch_persist_int8(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st);
+// Forms for problems of few tiles (lq_gemm_small.hip); numbered behind the tactics, which can be forced and cached: these cannot.
+enum SmallForm { SMALL_32x32_K4 = 64, SMALL_32x64_K4, SMALL_64x128_K2, SMALL_128x128_K2 };
+// the tactic or form for fewer than 192 tiles of 256x256, k > 1024 and 16-bit outputs
+int few_tiles_form(int m, int n, int k);
+int run_small(GemmKind kind, const GemmParams& p, lq_dtype_t out_dtype, int form, hipStream_t st);
+int run_small_fp8_bf16(const GemmParams& p, int form, hipStream_t st);  // lq_gemm_small_{bf16,f16}.hip
+int run_small_fp8_f16(const GemmParams& p, int form, hipStream_t st);
+int run_small_int8_bf16(const GemmParams& p, int form, hipStream_t st);
+int run_small_int8_f16(const GemmParams& p, int form, hipStream_t st);
 int device_cu_count();  // compute units of the current device (cached per device)
 
 }  // namespace lq
