@@ -541,7 +541,7 @@ int lq_rmsnorm_rope(void* out, const void* qkv, const void* context_qkv, const v
  * layers/flux_attention_processor/FluxAttentionFP8Processor.cc:246-291,
  * layers/basic_transformer/BasicTransformerInt8Block.cc:330-420).  q, k, v: heads of head_dim (64 or 128) elements side by side
  * in a token, tokens *_row elements and batches *_batch elements apart (parts of a fused QKV tensor are strided tensors);
- * out [batch, seq_q, heads, head_dim] dense.  dtype F16 or BF16; pointers 16-byte aligned, strides multiples of 8 elements;
+ * out [batch, seq_q, heads, head_dim] dense.  scale > 0; dtype F16 or BF16; pointers 16-byte aligned, strides multiples of 8 elements;
  * seq_k * k_row and seq_k * v_row below 2^31. */
 int lq_attention(void* out, const void* q, size_t q_row, size_t q_batch, const void* k, size_t k_row, size_t k_batch, const void* v,
                  size_t v_row, size_t v_batch, lq_dtype_t dtype, int batch, int seq_q, int seq_k, int heads, int head_dim, float scale,

@@ -161,7 +161,9 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
     for (int d = 0; d < DB; ++d)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[d][i] = 0.0f;
-    float m_run = -__builtin_inff(), l_run[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    // The maximum starts at the lowest finite float: a tile whose scores are all -inf then adds nothing, where a start at -inf
+    // would make (-inf) - (-inf) of it.
+    float m_run = -__FLT_MAX__, l_run[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const float c = p.scale_log2;
     u32 pw[16];  // probabilities of a tile, two keys per word: words 4 * kk .. 4 * kk + 3 are the operand of PV step kk
 
@@ -377,6 +379,7 @@ extern "C" int lq_attention(void* out, const void* q, size_t q_row, size_t q_bat
     LQ_REQUIRE(batch >= 0 && heads > 0 && seq_q >= 0 && seq_k > 0 && (head_dim == 64 || head_dim == 128), LQ_ERR_SHAPE,
                "lq_attention: need head_dim 64 or 128 and at least one key (batch=%d heads=%d seq_q=%d seq_k=%d head_dim=%d)", batch, heads,
                seq_q, seq_k, head_dim);
+    LQ_REQUIRE(scale > 0.0f, LQ_ERR_ARG, "lq_attention: the softmax scale must be positive");  // the largest score is taken before scaling
     if (batch == 0 || seq_q == 0) return LQ_OK;
     LQ_REQUIRE(out && q && k && v, LQ_ERR_ARG, "lq_attention: null pointer");
     const uintptr_t bits = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |

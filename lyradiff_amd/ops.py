@@ -1026,7 +1026,7 @@ def attention_supported(q, k, v) -> bool:
 
 def attention(q, k, v, scale=None):
     """Softmax attention without mask: q [B, Sq, H, Dh], k and v [B, Sk, H, Dh] (views into a fused QKV tensor are fine) ->
-    [B, Sq, H, Dh], contiguous.  `scale` defaults to Dh ** -0.5.  See attention_supported for what it takes."""
+    [B, Sq, H, Dh], contiguous.  `scale` (positive) defaults to Dh ** -0.5.  See attention_supported for what it takes."""
     if k.shape != v.shape or k.shape[0] != q.shape[0] or k.shape[2:] != q.shape[2:]:
         raise ValueError("attention: q must be [B, Sq, H, Dh], k and v [B, Sk, H, Dh]")
     if not attention_supported(q, k, v):

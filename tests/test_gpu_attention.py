@@ -49,6 +49,22 @@ def test_attention_matches_fp32(dev, shape, dt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("sq,h,dh", [(40, 2, 64), (40, 2, 128), (1408, 24, 128)])  # the three forms of the kernel
+def test_attention_leaves_out_keys_of_minus_infinity(dev, sq, h, dh):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(dh + sq)
+    q, k, v = (torch.rand(1, n, h, dh, generator=g, device=dev).bfloat16() for n in (sq, 200, 200))
+    k[:, :70] = -float("inf")  # the first tile of 64 keys and a part of the second: their scores are -inf for these positive queries
+    q.clamp_(min=0.01)
+    got = ops.attention(q, k, v)
+    assert torch.isfinite(got).all()
+    assert torch.allclose(got.float(), ops.attention(q, k[:, 70:].contiguous(), v[:, 70:].contiguous()).float(), rtol=2.0 ** -6, atol=0)
+    k[:] = -float("inf")
+    assert torch.isnan(ops.attention(q, k, v)).all()  # as softmax of a row of -inf
+
+
+@pytest.mark.gpu
 def test_attention_of_other_shapes_falls_back(dev):
     from lyradiff_amd import ops
 
@@ -69,5 +85,6 @@ def test_attention_argument_errors_do_not_reach_the_gpu():
                                                   sk=8, h=3, dh=128, s=1.0, st=None), **kw}.values())
     assert call(dt=L.LQ_F32) == -4
     assert call(dh=96) == -2 and call(sk=0) == -2 and call(kr=376) == -2 and call(sk=1 << 23) == -2
+    assert call(s=0.0) == -1 and call(s=-1.0) == -1
     assert call(q=None) == -1 and call(q=C.c_void_p(8)) == -1 and call(qr=388) == -1
     assert call(sq=0) == 0
