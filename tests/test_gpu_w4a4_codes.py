@@ -60,3 +60,34 @@ def test_linear_module_takes_either_form(dev):
     want = lin.forward(x)  # as constructed: packed nibbles
     assert lin.weight_codes is None and lin.use_codes().weight_codes is not None
     assert torch.equal(lin.forward(x), want)
+
+
+def test_linear_module_follows_its_weight_and_its_low_rank_branch(dev):
+    from lyradiff_amd import ops
+    from lyradiff_amd.weights import W4A4Linear
+
+    x, smooth, down, packed, sb, up, bias, rnd = _make(dev, 96, 256, 384, torch.bfloat16)
+    make = lambda: W4A4Linear(ops.repack_weight(packed.view(torch.uint8)), sb.clone(), smooth, up, down, bias)
+
+    def scale_in_place(lin):
+        lin.weight_scale.mul_(2.0)
+
+    def other_weight(lin):
+        lin.weight_rows32 = lin.weight_rows32.flip(0).contiguous()
+
+    def weight_in_place(lin):
+        lin.weight_rows32.copy_(lin.weight_rows32.flip(0))
+
+    def no_branch(lin):
+        lin.lora_up = lin.lora_down = None
+
+    def wider_branch(lin):
+        lin.lora_up, lin.lora_down = torch.cat([up, up], 1), torch.cat([down, down])
+
+    for change in (scale_in_place, other_weight, weight_in_place, no_branch, wider_branch):
+        lin, plain = make().use_codes(), make()
+        before = lin.forward(x)
+        change(lin), change(plain)
+        want = plain.forward(x)
+        assert not torch.equal(before, want) and torch.equal(lin.forward(x), want), change.__name__
+        assert torch.equal(lin.use_codes().forward(x), want), change.__name__
