@@ -380,8 +380,8 @@ def w4a4_quant(x, smooth=None, scale_dtype=torch.float32, group: int = 64):
     if smooth is not None:
         _chk(smooth, "smooth", (torch.float32,))
     m, k = x.shape
-    q = torch.empty((m, k // 8), dtype=torch.int32, device=x.device)
-    s = torch.empty((m, k // group), dtype=scale_dtype, device=x.device)
+    q = torch.empty(m, k // 8, dtype=torch.int32, device=x.device)
+    s = torch.empty(m, k // group, dtype=scale_dtype, device=x.device)
     _l.check(_l.load().lq_w4a4_quantize(_ptr(q), _ptr(s), _DT[scale_dtype], _ptr(x), _DT[x.dtype], _ptr(smooth),
                                         m, k, group, _stream()), "lq_w4a4_quantize")
     return q, s
@@ -432,7 +432,7 @@ def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.
         per_token = int(alpha_row.numel() == m and m != 1)
     if bias is not None:
         _chk(bias, "bias", (out_dtype,))
-    c = torch.empty((m, n), dtype=out_dtype, device=a_q.device)
+    c = torch.empty(m, n, dtype=out_dtype, device=a_q.device)
     _l.check(_l.load().lq_gemm_int8(_ptr(c), _DT[out_dtype], _ptr(a_q), _ptr(w_rows32), _ptr(alpha_col),
                                     _ptr(alpha_row), per_token, _ptr(bias), m, n, k, _stream()), "lq_gemm_int8")
     return c
@@ -461,8 +461,8 @@ def fp8_linear(a_q, w_rows32, a_scale, b_scale, bias=None, gelu: bool = False, r
             _chk(t, name, (torch.float32,))
     if not want_output and out_fp8_scale is None:
         raise ValueError("want_output=False needs out_fp8_scale")
-    c = torch.empty((m, n), dtype=out_dtype, device=a_q.device) if want_output else None
-    c8 = torch.empty((m, n), dtype=torch.uint8, device=a_q.device) if out_fp8_scale is not None else None
+    c = torch.empty(m, n, dtype=out_dtype, device=a_q.device) if want_output else None
+    c8 = torch.empty(m, n, dtype=torch.uint8, device=a_q.device) if out_fp8_scale is not None else None
     _l.check(_l.load().lq_gemm_fp8_ex(_ptr(c), _DT[out_dtype], _ptr(a_q), _ptr(w_rows32), _ptr(a_scale), _ptr(b_scale),
                                       _ptr(bias), int(gelu), _ptr(residual), float(beta), m, n, k, _ptr(out_scale), _ptr(c8),
                                       _ptr(out_fp8_scale), _stream()), "lq_gemm_fp8")
@@ -485,7 +485,7 @@ def fp8_linear_max(a_q, w_rows32, a_scale, b_scale, bias, out_max, out_dtype=tor
         raise ValueError("K mismatch between activation and weight")
     if bias is not None:
         _chk(bias, "bias", (out_dtype,))
-    c = torch.empty((m, n), dtype=out_dtype, device=a_q.device)
+    c = torch.empty(m, n, dtype=out_dtype, device=a_q.device)
     _l.check(_l.load().lq_gemm_fp8_max(_ptr(c), _DT[out_dtype], _ptr(a_q), _ptr(w_rows32), _ptr(a_scale), _ptr(b_scale),
                                        _ptr(bias), m, n, k, _ptr(out_max), _stream()), "lq_gemm_fp8_max")
     return c
@@ -538,7 +538,7 @@ def fp8_scale_cast_panels(x, scale, invert: bool = True, out=None, col_offset: i
         raise ValueError("fp8_scale_cast_panels: x must be [M, K] with K % 64 == 0")
     m, k = x.shape
     if out is None:
-        out = torch.empty((k // 64, m, 64), dtype=torch.uint8, device=x.device)
+        out = torch.empty(k // 64, m, 64, dtype=torch.uint8, device=x.device)
     _l.check(_l.load().lq_fp8_scale_cast_panels(_panel_block(out, m, k, col_offset), _ptr(x), _DT[x.dtype], _ptr(scale), int(invert), m, k,
                                                 _stream()), "lq_fp8_scale_cast_panels")
     return out
@@ -550,7 +550,7 @@ def fp8_quant_panels(x):
     if x.dim() != 2 or x.shape[1] % 64 != 0:
         raise ValueError("fp8_quant_panels: x must be [M, K] with K % 64 == 0")
     m, k = x.shape
-    q = torch.empty((k // 64, m, 64), dtype=torch.uint8, device=x.device)
+    q = torch.empty(k // 64, m, 64, dtype=torch.uint8, device=x.device)
     s = torch.empty(1, dtype=torch.float32, device=x.device)
     _l.check(_l.load().lq_fp8_amax_cast_panels(_ptr(q), _ptr(s), _ptr(x), _DT[x.dtype], m, k, _stream()), "lq_fp8_amax_cast_panels")
     return q, s
@@ -565,7 +565,7 @@ def fp8_gelu_quant_panels(y, y_max, clear_max=None):
     if y.dim() != 2 or y.shape[1] % 64 != 0:
         raise ValueError("fp8_gelu_quant_panels: y must be [M, K] with K % 64 == 0")
     m, k = y.shape
-    q = torch.empty((k // 64, m, 64), dtype=torch.uint8, device=y.device)
+    q = torch.empty(k // 64, m, 64, dtype=torch.uint8, device=y.device)
     s = torch.empty(1, dtype=torch.float32, device=y.device)
     _l.check(_l.load().lq_fp8_gelu_cast_panels(_ptr(q), _ptr(s), _ptr(y), _DT[y.dtype], m, k, _ptr(y_max), _ptr(clear_max), _stream()),
              "lq_fp8_gelu_cast_panels")
@@ -590,7 +590,7 @@ def fp8_linear_panels(a_panels, w_rows32, a_scale, b_scale, bias, out_max=None, 
         raise ValueError("K mismatch between activation and weight")
     if bias is not None:
         _chk(bias, "bias", (out_dtype,))
-    c = torch.empty((m, n), dtype=out_dtype, device=a_panels.device)
+    c = torch.empty(m, n, dtype=out_dtype, device=a_panels.device)
     _l.check(_l.load().lq_gemm_fp8_panels(_ptr(c), _DT[out_dtype], _ptr(a_panels), _ptr(w_rows32), _ptr(a_scale), _ptr(b_scale),
                                           _ptr(bias), m, n, k, _ptr(out_max), _stream()), "lq_gemm_fp8_panels")
     return c
@@ -606,7 +606,7 @@ def sq_quant_dynamic_panels(x, pre_quant_scale=None):
         _chk(pre_quant_scale, "pre_quant_scale", (torch.float32,))
         if pre_quant_scale.numel() != k:
             raise ValueError("pre_quant_scale must have K elements")
-    q = torch.empty((k // 64, m, 64), dtype=torch.int8, device=x.device)
+    q = torch.empty(k // 64, m, 64, dtype=torch.int8, device=x.device)
     s = torch.empty(m, dtype=torch.float32, device=x.device)
     _l.check(_l.load().lq_sq_dynamic_quant_panels(_ptr(q), _ptr(s), _ptr(x), _DT[x.dtype], _ptr(pre_quant_scale), m, k, _stream()),
              "lq_sq_dynamic_quant_panels")
@@ -635,7 +635,7 @@ def int8_linear_panels(a_panels, w_rows32, alpha_col, alpha_row, bias=None, out_
         per_token = int(alpha_row.numel() == m and m != 1)
     if bias is not None:
         _chk(bias, "bias", (out_dtype,))
-    c = torch.empty((m, n), dtype=out_dtype, device=a_panels.device)
+    c = torch.empty(m, n, dtype=out_dtype, device=a_panels.device)
     _l.check(_l.load().lq_gemm_int8_panels(_ptr(c), _DT[out_dtype], _ptr(a_panels), _ptr(w_rows32), _ptr(alpha_col),
                                            _ptr(alpha_row), per_token, _ptr(bias), m, n, k, _stream()), "lq_gemm_int8_panels")
     return c
@@ -659,7 +659,7 @@ def fp8_linear_gated(a_q, w_rows32, a_scale, b_scale, bias, gate, residual, rows
     if residual.numel() != m * n or rows_per_gate <= 0 or gate.numel() != ((m + rows_per_gate - 1) // rows_per_gate) * n:
         raise ValueError("residual must be [M,N] and gate [ceil(M/rows_per_gate), N]")
     if out is None:
-        out = torch.empty((m, n), dtype=residual.dtype, device=a_q.device)
+        out = torch.empty(m, n, dtype=residual.dtype, device=a_q.device)
     _chk(out, "out", (residual.dtype,))
     _l.check(_l.load().lq_gemm_fp8_gated(_ptr(out), _DT[residual.dtype], _ptr(a_q), _ptr(w_rows32), _ptr(a_scale), _ptr(b_scale),
                                          _ptr(bias), _ptr(gate), int(rows_per_gate), _ptr(residual), m, n, k, _stream()),
@@ -684,7 +684,7 @@ def fp8_linear_codes(a_q, w_rows32, a_scale, b_scale, bias, out_fp8_scale, gelu:
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
     if out is None:
-        out = torch.empty((m, n), dtype=torch.uint8, device=a_q.device)
+        out = torch.empty(m, n, dtype=torch.uint8, device=a_q.device)
     _chk(out, "out", (torch.uint8,))
     if out.dim() != 2 or out.shape[0] != m or col_offset < 0 or col_offset + n > out.shape[1]:
         raise ValueError("out must be [M, W] with col_offset + N <= W")
@@ -713,7 +713,7 @@ def fp8_linear_gated_panels(a_panels, w_rows32, a_scale, b_scale, bias, gate, re
     if residual.numel() != m * n or rows_per_gate <= 0 or gate.numel() != ((m + rows_per_gate - 1) // rows_per_gate) * n:
         raise ValueError("residual must be [M,N] and gate [ceil(M/rows_per_gate), N]")
     if out is None:
-        out = torch.empty((m, n), dtype=residual.dtype, device=a_panels.device)
+        out = torch.empty(m, n, dtype=residual.dtype, device=a_panels.device)
     _chk(out, "out", (residual.dtype,))
     _l.check(_l.load().lq_gemm_fp8_gated_panels(_ptr(out), _DT[residual.dtype], _ptr(a_panels), _ptr(w_rows32), _ptr(a_scale),
                                                 _ptr(b_scale), _ptr(bias), _ptr(gate), int(rows_per_gate), _ptr(residual), m, n, k,
@@ -784,7 +784,7 @@ def weight_only_linear(x, w_prepared, scales, bias=None, kind: str = "int8"):
     n = w_prepared.shape[0]
     if w_prepared.shape[1] != (k // 2 if kind == "int4" else k) or scales.numel() != n:
         raise ValueError("shape mismatch between x, w_prepared and scales")
-    c = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    c = torch.empty(m, n, dtype=x.dtype, device=x.device)
     _l.check(_l.load().lq_gemm_weight_only(_ptr(c), _ptr(x), _DT[x.dtype], _ptr(w_prepared), _KINDS[kind], _ptr(scales),
                                            _ptr(bias), m, n, k, _stream()), "lq_gemm_weight_only")
     return c
@@ -807,7 +807,7 @@ def weight_only_linear_grouped(x, w_prepared, scales, zeros=None, bias=None, kin
     if w_prepared.shape[1] != (k // 2 if kind == "int4" else k) or tuple(scales.shape) != (k // group_size, n) or \
             (zeros is not None and zeros.shape != scales.shape) or (bias is not None and bias.numel() != n):
         raise ValueError("shape mismatch between x, w_prepared, scales [K/group, N], zeros and bias")
-    c = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    c = torch.empty(m, n, dtype=x.dtype, device=x.device)
     _l.check(_l.load().lq_gemm_weight_only_grouped(_ptr(c), _ptr(x), _DT[x.dtype], _ptr(w_prepared), _KINDS[kind], _ptr(scales),
                                                    _ptr(zeros), _ptr(bias), m, n, k, int(group_size), _stream()),
              "lq_gemm_weight_only_grouped")
@@ -902,14 +902,14 @@ def _w4a4_gemm(launch, m, n, device, bias, out_dtype, lora_act, lora_up, gelu, a
         epi = _l.Epilogue(int(gelu), _ptr(addend), _ptr(gate), int(rows_per_gate), _ptr(residual), None, 0, None)
         if out_fp8_scale is not None:
             _chk(out_fp8_scale, "out_fp8_scale", (torch.float32,))
-            c8 = out_fp8 if out_fp8 is not None else torch.empty((m, n), dtype=torch.uint8, device=device)
+            c8 = out_fp8 if out_fp8 is not None else torch.empty(m, n, dtype=torch.uint8, device=device)
             _chk(c8, "out_fp8", (torch.uint8,))
             if c8.dim() != 2 or c8.shape[0] != m or col_offset < 0 or col_offset + n > c8.shape[1]:
                 raise ValueError("out_fp8 must be [M, W] with col_offset + N <= W")
             epi.C_fp8, epi.ldc_fp8, epi.C_fp8_scale = c8.data_ptr() + col_offset, c8.shape[1], _ptr(out_fp8_scale)
     if not want_output and c8 is None:
         raise ValueError("want_output=False needs out_fp8_scale")
-    c = (out if out is not None else torch.empty((m, n), dtype=out_dtype, device=device)) if want_output else None
+    c = (out if out is not None else torch.empty(m, n, dtype=out_dtype, device=device)) if want_output else None
     if c is not None:
         _chk(c, "out", (out_dtype,))
     _l.check(launch(_ptr(c), (_ptr(lora_act), _ptr(lora_up), lora_dt, rank), C.byref(epi) if epi is not None else None), "lq_gemm_w4a4")
@@ -927,7 +927,7 @@ def lora_down(x, lora_down_w, out_dtype=None):
     if lora_down_w.shape[1] != k:
         raise ValueError("K mismatch between x and lora_down_w")
     out_dtype = out_dtype or x.dtype
-    out = torch.empty((m, rank), dtype=out_dtype, device=x.device)
+    out = torch.empty(m, rank, dtype=out_dtype, device=x.device)
     _l.check(_l.load().lq_lora_down(_ptr(out), _DT[out_dtype], _ptr(x), _ptr(lora_down_w), _DT[x.dtype], m, k, rank, _stream()),
              "lq_lora_down")
     return out
@@ -945,9 +945,9 @@ def w4a4_quant_lora_down(x, smooth, lora_down_w, scale_dtype=torch.float32, out_
     if lora_down_w.shape[1] != k:
         raise ValueError("K mismatch between x and lora_down_w")
     out_dtype = out_dtype or x.dtype
-    q = torch.empty((m, k // 8), dtype=torch.int32, device=x.device)
-    s = torch.empty((m, k // group), dtype=scale_dtype, device=x.device)
-    act = torch.empty((m, rank), dtype=out_dtype, device=x.device)
+    q = torch.empty(m, k // 8, dtype=torch.int32, device=x.device)
+    s = torch.empty(m, k // group, dtype=scale_dtype, device=x.device)
+    act = torch.empty(m, rank, dtype=out_dtype, device=x.device)
     _l.check(_l.load().lq_w4a4_quantize_lora_down(_ptr(q), _ptr(s), _DT[scale_dtype], _ptr(act), _DT[out_dtype], _ptr(x),
                                                   _DT[x.dtype], _ptr(smooth), _ptr(lora_down_w), m, k, rank, group, _stream()),
              "lq_w4a4_quantize_lora_down")
@@ -971,9 +971,9 @@ def w4a4_quant_lora_down_codes(x, smooth, lora_down_w):
     m, k = x.shape
     if tuple(lora_down_w.shape) != (32, k) or smooth.numel() != k:
         raise ValueError("lora_down_w must be [32, K] and smooth [K]")
-    codes = torch.empty((m, k), dtype=torch.uint8, device=x.device)
-    s = torch.empty((k // 64, m), dtype=torch.float32, device=x.device)
-    act = torch.empty((m, 32), dtype=x.dtype, device=x.device)
+    codes = torch.empty(m, k, dtype=torch.uint8, device=x.device)
+    s = torch.empty(k // 64, m, dtype=torch.float32, device=x.device)
+    act = torch.empty(m, 32, dtype=x.dtype, device=x.device)
     _l.check(_l.load().lq_w4a4_quantize_lora_down_codes(_ptr(codes), _ptr(s), _ptr(act), _DT[x.dtype], _ptr(x), _DT[x.dtype], _ptr(smooth),
                                                         _ptr(lora_down_w), m, k, 32, _stream()), "lq_w4a4_quantize_lora_down_codes")
     return codes, s, act
