@@ -506,10 +506,14 @@ int lq_w4a4_quantize_lora_down(uint32_t* q_words, void* scales, lq_dtype_t scale
  * scales) on operands that keep one e4m3 byte per 4-bit value -- every integer of [-8, 8] is an e4m3 number, so the fp8 matrix
  * instruction forms the exact group sums -- and the group scales group-major, [k / 64][rows].
  *   lq_w4a4_expand_rows32: packed weights in rows32 layout [n, k / 2] -> codes in rows32 layout [n, k]; n, k multiples of 32.
+ *   lq_w4a4_weight_codes: that, and the weight's scales [n, k / 64] as [k / 64, n]; n a multiple of 32, k of 64.
+ *   lq_w4a4_prefers_codes: 1 where a linear whose weight is kept packed gains by lq_w4a4_weight_codes + these calls, else 0.
  *   lq_w4a4_quantize_lora_down_codes: lq_w4a4_quantize_lora_down with codes [m, k] and scales [k / 64, m]; smooth required, rank 32,
  *     k % 128 == 0, k <= 16384, lora_act in x's type (F16 or BF16).
  *   lq_gemm_w4a4_codes: lq_gemm_w4a4_ex with sA [k / 64, m] and sB [k / 64, n] fp32; output F16 or BF16. */
 int lq_w4a4_expand_rows32(uint8_t* codes, const uint8_t* packed, size_t n, size_t k, lq_stream_t stream);
+int lq_w4a4_weight_codes(uint8_t* codes, float* scales_t, const uint8_t* packed_rows32, const float* scales, int n, int k, lq_stream_t stream);
+int lq_w4a4_prefers_codes(int m, int n, int k);
 int lq_w4a4_quantize_lora_down_codes(uint8_t* codes, float* scales, void* lora_act, lq_dtype_t act_dtype, const void* x,
                                      lq_dtype_t x_dtype, const float* smooth, const void* lora_down, int m, int k, int rank,
                                      lq_stream_t stream);

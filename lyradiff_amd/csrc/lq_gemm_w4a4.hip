@@ -110,6 +110,14 @@ extern "C" int lq_gemm_w4a4_ex(void* C, lq_dtype_t out_dtype, const uint32_t* A_
     }
 }
 
+// Laying a packed weight out in the call costs 6-11 us whatever m is; the GEMM on codes saves about a fifth of its time behind it.
+// Measured, quantiser + layout + GEMM, packed / codes (us), m = 512, 1024, 2048, 4608:
+//   3072 x 3072   30 / 33, 36 / 40, 57 / 55, 118 / 98     12288 x 3072   55 / 58, 98 / 85, 177 / 145, 390 / 301
+//   9216 x 3072   55 / 53, 80 / 79, 139 / 117, 299 / 236  3072 x 12288   97 / 101, 121 / 109, 196 / 174, 425 / 340
+extern "C" int lq_w4a4_prefers_codes(int m, int n, int k) {
+    return n % 32 == 0 && k % 128 == 0 && k <= 16384 && (double)m * n * k >= 2e10;
+}
+
 extern "C" int lq_gemm_w4a4_codes(void* C, lq_dtype_t out_dtype, const uint8_t* A_codes, const uint8_t* B_codes_rows32, const float* sA,
                                   const float* sB, const void* bias, const void* lora_act, const void* lora_up, lq_dtype_t lora_dtype,
                                   int lora_rank, int m, int n, int k, const lq_epilogue_t* epi, lq_stream_t stream) {

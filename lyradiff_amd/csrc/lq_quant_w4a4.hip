@@ -349,25 +349,54 @@ __global__ __launch_bounds__(kFusedWaves * 64) void w4a4_quant_lora_kernel(u32* 
 }
 
 // ---- packed 4-bit weights in rows32 layout -> e4m3 codes in rows32 layout: a 16-byte chunk (32 values of a row) becomes two
+__device__ __forceinline__ void w4a4_expand_chunk(const uint4& w, uint4& lo, uint4& hi) {
+    const u32 in[4] = {w.x, w.y, w.z, w.w};
+    u32 out[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float f[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[e] = (float)((int)(in[i] << (28 - 4 * (4 * h + e))) >> 28);  // nibble, sign extended
+            const int half = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+            out[2 * i + h] = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], half, true);
+        }
+    lo = make_uint4(out[0], out[1], out[2], out[3]);
+    hi = make_uint4(out[4], out[5], out[6], out[7]);
+}
 __global__ __launch_bounds__(256) void w4a4_expand_kernel(uint4* __restrict__ dst, const uint4* __restrict__ src, size_t chunks) {
     for (size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x; t < chunks; t += (size_t)gridDim.x * blockDim.x) {
-        const uint4 w = src[t];
-        const u32 in[4] = {w.x, w.y, w.z, w.w};
-        u32 out[8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                float f[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) f[e] = (float)((int)(in[i] << (28 - 4 * (4 * h + e))) >> 28);  // nibble, sign extended
-                const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
-                out[2 * i + h] = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
-            }
+        uint4 lo, hi;
+        w4a4_expand_chunk(src[t], lo, hi);
         const size_t r = t & 31, kc = t >> 5;  // chunk columns counted through all 32-row blocks
-        dst[(2 * kc) * 32 + r] = make_uint4(out[0], out[1], out[2], out[3]);
-        dst[(2 * kc + 1) * 32 + r] = make_uint4(out[4], out[5], out[6], out[7]);
+        dst[(2 * kc) * 32 + r] = lo;
+        dst[(2 * kc + 1) * 32 + r] = hi;
     }
+}
+
+// What the GEMM on codes reads, from a packed weight and its scales [n, ng], in one launch ahead of each such GEMM: nothing derived
+// from a weight outlives a call, so that no write to the weight, however it is made, can be missed.  A workgroup takes 32 rows (a
+// block of the rows32 layout) by 512 of k: two chunks per lane, and eight groups of scales, read as 32 contiguous bytes of a row and
+// written as 128 of a group.  A pass over memory: 6 us of a
+// 98 us linear at 4608x3072x3072, 11 us at 12288x3072 (57 MB read and written).
+__global__ __launch_bounds__(256) void w4a4_weight_codes_kernel(uint4* __restrict__ codes, float* __restrict__ scales_t, const uint4* __restrict__ packed,
+                                                                const float* __restrict__ scales, int n, int kc, int parts) {
+    const int nb = blockIdx.x / parts, c0 = (int)(blockIdx.x % parts) * 16, tid = threadIdx.x;
+    const size_t block = (size_t)nb * kc * 32;  // first chunk of this row block
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int c = c0 + i * 8 + (tid >> 5);  // chunk column: 32 values of a row
+        if (c >= kc) continue;
+        const size_t t = block + (size_t)c * 32 + (tid & 31);
+        uint4 lo, hi;
+        w4a4_expand_chunk(packed[t], lo, hi);
+        const size_t d = 2 * block + (size_t)c * 64 + (tid & 31);
+        codes[d] = lo;
+        codes[d + 32] = hi;
+    }
+    const int ng = kc / 2, g = c0 / 2 + (tid >> 5), row = nb * 32 + (tid & 31);
+    if (g < ng) scales_t[(size_t)g * n + row] = scales[(size_t)row * ng + g];
 }
 
 // ---- rows32 repack: dst chunk ((nb*KC + kc)*32 + r) <- src chunk (row nb*32 + r, 16-byte column kc) ----
@@ -544,6 +573,21 @@ extern "C" int lq_w4a4_expand_rows32(uint8_t* codes, const uint8_t* packed, size
     hipLaunchKernelGGL(w4a4_expand_kernel, dim3((unsigned)std::min<size_t>((chunks + 255) / 256, 65535)), dim3(256), 0, as_stream(stream),
                        reinterpret_cast<uint4*>(codes), reinterpret_cast<const uint4*>(packed), chunks);
     return check_launch("w4a4_expand_rows32");
+}
+
+extern "C" int lq_w4a4_weight_codes(uint8_t* codes, float* scales_t, const uint8_t* packed, const float* scales, int n, int k, lq_stream_t stream) {
+    LQ_REQUIRE(n >= 0 && k >= 0 && n % 32 == 0 && k % 64 == 0, LQ_ERR_SHAPE, "lq_w4a4_weight_codes: need n %% 32 == 0 and k %% 64 == 0 (n=%d k=%d)", n, k);
+    if (n == 0 || k == 0) return LQ_OK;
+    LQ_REQUIRE(codes && scales_t && packed && scales && codes != packed && scales_t != scales, LQ_ERR_ARG,
+               "lq_w4a4_weight_codes: null pointer or in-place call");
+    LQ_REQUIRE((reinterpret_cast<uintptr_t>(codes) | reinterpret_cast<uintptr_t>(packed)) % 16 == 0 &&
+                   (reinterpret_cast<uintptr_t>(scales_t) | reinterpret_cast<uintptr_t>(scales)) % 4 == 0,
+               LQ_ERR_ARG, "lq_w4a4_weight_codes: weights must be 16-byte aligned, scales 4-byte aligned");
+    const int kc = k / 32, parts = (kc + 15) / 16;
+    LQ_REQUIRE((long long)(n / 32) * parts <= 0x7fffffffLL, LQ_ERR_SHAPE, "lq_w4a4_weight_codes: weight too large (n=%d k=%d)", n, k);
+    hipLaunchKernelGGL(w4a4_weight_codes_kernel, dim3((unsigned)(n / 32 * parts)), dim3(256), 0, as_stream(stream), reinterpret_cast<uint4*>(codes),
+                       scales_t, reinterpret_cast<const uint4*>(packed), scales, n, kc, parts);
+    return check_launch("w4a4_weight_codes");
 }
 
 extern "C" size_t lq_weight_row_bytes(lq_weight_kind_t kind, size_t k) { return kind == LQ_W_INT4 ? k / 2 : k; }

@@ -93,6 +93,8 @@ SYMBOLS = {
     "lq_gate_residual_layernorm_mod": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _Z, _Z, _Z, _F, _P]),
     "lq_gemm_w4a4_ex": (_I, [_P, _I, _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P, _P]),
     "lq_w4a4_expand_rows32": (_I, [_P, _P, _Z, _Z, _P]),
+    "lq_w4a4_weight_codes": (_I, [_P, _P, _P, _P, _I, _I, _P]),
+    "lq_w4a4_prefers_codes": (_I, [_I, _I, _I]),
     "lq_w4a4_quantize_lora_down_codes": (_I, [_P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _P]),
     "lq_gemm_w4a4_codes": (_I, [_P, _I, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P]),
     "lq_gemm_w4a4_lora": (_I, [_P, _I, _P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),

@@ -963,6 +963,24 @@ def w4a4_expand_weight(packed_rows32):
     return out
 
 
+def w4a4_weight_codes(packed_rows32, scale):
+    """w4a4_expand_weight and the weight's scales fp32 [N, K/64] group-major, in one launch: returns (codes uint8 [N, K], fp32 [K/64, N])."""
+    _chk(packed_rows32, "packed_rows32", (torch.uint8, torch.int8))
+    _chk(scale, "scale", (torch.float32,))
+    n, k = packed_rows32.shape[0], 2 * packed_rows32.shape[1]
+    if scale.numel() * 64 != n * k:
+        raise ValueError("scale must be [N, K/64]")
+    codes = torch.empty(n, k, dtype=torch.uint8, device=packed_rows32.device)
+    scale_t = torch.empty(k // 64, n, dtype=torch.float32, device=packed_rows32.device)
+    _l.check(_l.load().lq_w4a4_weight_codes(_ptr(codes), _ptr(scale_t), _ptr(packed_rows32), _ptr(scale), n, k, _stream()), "lq_w4a4_weight_codes")
+    return codes, scale_t
+
+
+def w4a4_prefers_codes(m: int, n: int, k: int) -> bool:
+    """Whether a linear on m rows whose weight is kept packed gains by w4a4_weight_codes and the kernels on codes."""
+    return bool(_l.load().lq_w4a4_prefers_codes(m, n, k))
+
+
 def w4a4_quant_lora_down_codes(x, smooth, lora_down_w):
     """w4a4_quant_lora_down (fp32 scales) for w4a4_linear_codes: returns (codes uint8 [M, K], scales fp32 [K/64, M], lora_act [M, 32])."""
     _chk(x, "x", (torch.float16, torch.bfloat16))

@@ -171,19 +171,18 @@ struct FP8Linear {
 };
 
 // W4A4 group-64 linear with its low-rank branch (W4A4GemmWeight.cc:65-83, W4A4Gemm.cc:113-169)
-// The weight is kept as one e4m3 byte per value with group-major scales (lq_gemm_w4a4_codes): same results, no widening in the GEMM.
+// Large problems run on one e4m3 byte per value, laid out from the packed weight in each call (lq_w4a4_weight_codes): same results, no
+// widening in the GEMM.
 struct W4A4Linear {
-    at::Tensor w_codes, w_scale_t, smooth, lora_up, lora_down, bias;
+    at::Tensor w_rows32, w_scale, smooth, lora_up, lora_down, bias;
     int64_t n = 0, k = 0, rank = 32;
 
     void load(const Source& src, const std::string& prefix, int64_t d_out, int64_t d_in, bool has_bias, at::ScalarType T) {
         n = d_out, k = d_in;
         at::Tensor packed = src.get(prefix + "packed_weight", {n, k / 2}, at::kChar).to(at::kCUDA);
-        at::Tensor w_rows32 = at::empty({n, k / 2}, on_gpu(at::kByte));
+        w_rows32 = at::empty({n, k / 2}, on_gpu(at::kByte));
         ok(lq_repack_rows32(P8(w_rows32), P8(packed), (size_t)n, (size_t)(k / 2), cur_stream()), "lq_repack_rows32");
-        w_codes = at::empty({n, k}, on_gpu(at::kByte));
-        ok(lq_w4a4_expand_rows32(P8(w_codes), P8(w_rows32), (size_t)n, (size_t)k, cur_stream()), "lq_w4a4_expand_rows32");
-        w_scale_t = src.get(prefix + "weight_scale", {n, k / 64}, at::kFloat).to(at::kCUDA).t().contiguous();
+        w_scale = src.get(prefix + "weight_scale", {n, k / 64}, at::kFloat).to(at::kCUDA);
         smooth = src.get(prefix + "smooth", {k}, at::kFloat).to(at::kCUDA);
         lora_up = src.get(prefix + "lora_up", {n, rank}, T).to(at::kCUDA);
         lora_down = src.get(prefix + "lora_down", {rank, k}, T).to(at::kCUDA);
@@ -194,16 +193,29 @@ struct W4A4Linear {
     at::Tensor run(const at::Tensor& x2, const lq_epilogue_t* epi, bool want_output) const {
         const int64_t m = x2.size(0);
         const at::ScalarType T = x2.scalar_type();
-        at::Tensor q = at::empty({m, k}, on_gpu(at::kByte)), s = at::empty({k / 64, m}, on_gpu(at::kFloat));
         at::Tensor act = at::empty({m, rank}, on_gpu(T));
-        ok(lq_w4a4_quantize_lora_down_codes(P8(q), static_cast<float*>(P(s)), P(act), lq_dt(T), P(x2), lq_dt(T), PF(smooth), P(lora_down),
-                                            (int)m, (int)k, (int)rank, cur_stream()),
-           "lq_w4a4_quantize_lora_down_codes");
         at::Tensor y;
         if (want_output) y = at::empty({m, n}, on_gpu(T));
-        ok(lq_gemm_w4a4_codes(P(y), lq_dt(T), P8(q), P8(w_codes), PF(s), PF(w_scale_t), P(bias), P(act), P(lora_up), lq_dt(T), (int)rank,
-                              (int)m, (int)n, (int)k, epi, cur_stream()),
-           "lq_gemm_w4a4_codes");
+        if (lq_w4a4_prefers_codes((int)m, (int)n, (int)k)) {
+            at::Tensor q = at::empty({m, k}, on_gpu(at::kByte)), s = at::empty({k / 64, m}, on_gpu(at::kFloat));
+            at::Tensor w = at::empty({n, k}, on_gpu(at::kByte)), ws = at::empty({k / 64, n}, on_gpu(at::kFloat));
+            ok(lq_w4a4_quantize_lora_down_codes(P8(q), static_cast<float*>(P(s)), P(act), lq_dt(T), P(x2), lq_dt(T), PF(smooth), P(lora_down),
+                                                (int)m, (int)k, (int)rank, cur_stream()),
+               "lq_w4a4_quantize_lora_down_codes");
+            ok(lq_w4a4_weight_codes(P8(w), static_cast<float*>(P(ws)), P8(w_rows32), PF(w_scale), (int)n, (int)k, cur_stream()),
+               "lq_w4a4_weight_codes");
+            ok(lq_gemm_w4a4_codes(P(y), lq_dt(T), P8(q), P8(w), PF(s), PF(ws), P(bias), P(act), P(lora_up), lq_dt(T), (int)rank, (int)m, (int)n,
+                                  (int)k, epi, cur_stream()),
+               "lq_gemm_w4a4_codes");
+            return y;
+        }
+        at::Tensor q = at::empty({m, k / 8}, on_gpu(at::kInt)), s = at::empty({m, k / 64}, on_gpu(at::kFloat));
+        ok(lq_w4a4_quantize_lora_down(static_cast<uint32_t*>(P(q)), P(s), LQ_F32, P(act), lq_dt(T), P(x2), lq_dt(T), PF(smooth),
+                                      P(lora_down), (int)m, (int)k, (int)rank, 64, cur_stream()),
+           "lq_w4a4_quantize_lora_down");
+        ok(lq_gemm_w4a4_ex(P(y), lq_dt(T), static_cast<const uint32_t*>(P(q)), P8(w_rows32), P(s), P(w_scale), LQ_F32, P(bias), P(act),
+                           P(lora_up), lq_dt(T), (int)rank, (int)m, (int)n, (int)k, 64, epi, cur_stream()),
+           "lq_gemm_w4a4_ex");
         return y;
     }
 };

@@ -167,38 +167,34 @@ class W4A4Linear:
     lora_up: Optional[torch.Tensor] = None    # T [N, R]
     lora_down: Optional[torch.Tensor] = None  # T [R, K]
     bias: Optional[torch.Tensor] = None
-    # the weight as one e4m3 byte per value (rows32) and its scales group-major, made by use_codes(); forward then runs on codes
-    weight_codes: Optional[torch.Tensor] = None    # uint8 [N, K], rows32
-    weight_scale_t: Optional[torch.Tensor] = None  # fp32 [K/64, N]
-    codes_source: Optional[tuple] = None           # the tensors they were made from and their versions
+    codes: bool = False  # large problems run on codes (same results, faster); use_codes()
 
     def use_codes(self) -> "W4A4Linear":
-        """Lays the weight out for the GEMM on codes (1.5 bytes per value held instead of 0.5; same results, 4608x3072x3072 77 us against
-        100).  Once weight_rows32 or weight_scale has been replaced or written into, forward takes the packed weight until the next call."""
+        """Lets large problems run on one e4m3 byte per value (ops.w4a4_linear_codes).  The codes are made from the packed weight in each
+        call and dropped behind it: 4608x3072x3072 98 us against 118, and every write to weight_rows32 or weight_scale counts."""
         n, k = self.weight_rows32.shape[0], 2 * self.weight_rows32.shape[1]
-        if k % 128 == 0 and k <= 16384 and self.lora_down is not None and tuple(self.lora_down.shape) == (32, k):
-            self.weight_codes = ops.w4a4_expand_weight(self.weight_rows32)
-            self.weight_scale_t = self.weight_scale.t().contiguous()
-            self.codes_source = self._source_state()
+        self.codes = k % 128 == 0 and k <= 16384 and self.lora_down is not None and tuple(self.lora_down.shape) == (32, k)
         return self
 
-    def _source_state(self):
-        version = lambda t: -1 if t.is_inference() else t._version
-        return (self.weight_rows32, version(self.weight_rows32), self.weight_scale, version(self.weight_scale))
+    @property
+    def weight_codes(self) -> Optional[torch.Tensor]:
+        """The packed weight as codes, uint8 [N, K] in rows32 layout, or None without use_codes()."""
+        return ops.w4a4_expand_weight(self.weight_rows32) if self.codes else None
 
-    def _codes_apply(self, x2: torch.Tensor) -> bool:
-        """The codes still are those of the packed weight, and x2 and the low-rank branch are what the kernels on codes take."""
-        if self.weight_codes is None or self.codes_source is None or self.lora_down is None or self.lora_up is None:
+    def _on_codes(self, x2: torch.Tensor) -> bool:
+        """The linear, its low-rank branch and x2 are what the kernels on codes take, and m is large enough to pay for the layout."""
+        if not self.codes or self.lora_down is None or self.lora_up is None or self.smooth is None:
             return False
-        made, now = self.codes_source, self._source_state()
-        return made[0] is now[0] and made[1] == now[1] and made[2] is now[2] and made[3] == now[3] and x2.dtype == self.lora_down.dtype and \
-            tuple(self.lora_down.shape) == (32, x2.shape[1])
+        n, k = self.weight_rows32.shape[0], x2.shape[1]
+        return tuple(self.lora_down.shape) == (32, k) and x2.dtype == self.lora_down.dtype and self.weight_scale.dtype == torch.float32 and \
+            2 * self.weight_rows32.shape[1] == k and self.smooth.numel() == k and ops.w4a4_prefers_codes(x2.shape[0], n, k)
 
     def run(self, x2: torch.Tensor, **epilogue):
         """W4A4Gemm::forward (W4A4Gemm.cc:113-169) on x2 [M, K] with ops.w4a4_linear's epilogue options: quantise, low-rank down, GEMM."""
-        if self._codes_apply(x2):
+        if self._on_codes(x2):
             q, s, act = ops.w4a4_quant_lora_down_codes(x2, self.smooth, self.lora_down)
-            return ops.w4a4_linear_codes(q, self.weight_codes, s, self.weight_scale_t, self.bias, x2.dtype, act, self.lora_up, **epilogue)
+            w, w_scale = ops.w4a4_weight_codes(self.weight_rows32, self.weight_scale)
+            return ops.w4a4_linear_codes(q, w, s, w_scale, self.bias, x2.dtype, act, self.lora_up, **epilogue)
         if self.lora_down is not None:
             q, s, act = ops.w4a4_quant_lora_down(x2, self.smooth, self.lora_down, torch.float32)
         else:

@@ -91,3 +91,50 @@ def test_linear_module_follows_its_weight_and_its_low_rank_branch(dev):
         want = plain.forward(x)
         assert not torch.equal(before, want) and torch.equal(lin.forward(x), want), change.__name__
         assert torch.equal(lin.use_codes().forward(x), want), change.__name__
+
+
+@pytest.mark.parametrize("inference", [False, True])  # the tensors of an inference_mode block count no versions
+@pytest.mark.parametrize("write", ["repack_out", "data", "in_place", "scale_data", "copy"])
+def test_linear_module_sees_writes_that_autograd_does_not(dev, write, inference):
+    from lyradiff_amd import ops
+    from lyradiff_amd.weights import W4A4Linear
+
+    with torch.inference_mode(inference):
+        x, smooth, down, packed, sb, up, bias, _ = _make(dev, 4608, 3072, 2048, torch.bfloat16)
+        make = lambda: W4A4Linear(ops.repack_weight(packed.view(torch.uint8)), sb.clone(), smooth, up, down, bias)
+        other = packed.flip(0).contiguous().view(torch.uint8)
+        change = {"repack_out": lambda lin: ops.repack_weight(other, out=lin.weight_rows32),  # the library's own writer
+                  "data": lambda lin: lin.weight_rows32.data.bitwise_xor_(0x11),
+                  "in_place": lambda lin: lin.weight_rows32.copy_(lin.weight_rows32.flip(0)),
+                  "scale_data": lambda lin: lin.weight_scale.data.mul_(2.0),
+                  "copy": lambda lin: lin.weight_scale.copy_(lin.weight_scale.flip(0))}[write]
+        lin, plain = make().use_codes(), make()
+        before = lin.forward(x)
+        assert torch.equal(before, plain.forward(x))
+        change(lin), change(plain)
+        want = plain.forward(x)
+        assert not torch.equal(before, want) and torch.equal(lin.forward(x), want)
+
+
+# edges of the kernel's 32-row, 512-wide pieces: the last one with two groups, with one (k % 128 == 64), with all eight
+@pytest.mark.parametrize("n,k", [(32, 64), (96, 448), (64, 512), (160, 640), (32, 1088), (3072, 3072)])
+def test_weight_laid_out_for_one_call(dev, n, k):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(n + k)
+    w = torch.randint(0, 256, (n, k // 2), generator=g, device=dev, dtype=torch.uint8)
+    sb = torch.rand(n, k // 64, generator=g, device=dev)
+    codes, sb_t = ops.w4a4_weight_codes(w, sb)
+    assert torch.equal(codes, ops.w4a4_expand_weight(w)) and torch.equal(sb_t, sb.t())
+
+
+def test_linear_module_without_smoothing_or_with_a_small_batch_takes_the_packed_weight(dev):
+    from lyradiff_amd import ops
+    from lyradiff_amd.weights import W4A4Linear
+
+    x, smooth, down, packed, sb, up, bias, _ = _make(dev, 4608, 3072, 2048, torch.bfloat16)
+    lin = W4A4Linear(ops.repack_weight(packed.view(torch.uint8)), sb, smooth, up, down, bias).use_codes()
+    assert lin._on_codes(x) and not lin._on_codes(x[:64])
+    lin.smooth = None  # the quantiser on codes needs divisors, the packed one does not
+    words, sa, act = ops.w4a4_quant_lora_down(x, None, down)
+    assert torch.equal(lin.forward(x), ops.w4a4_linear(words, lin.weight_rows32, sa, sb, bias, torch.bfloat16, 64, act, up))
