@@ -230,7 +230,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
         }
-        const float mc = m_run * c;
+        const float mc = fmaxf(m_run * c, -__FLT_MAX__);  // finite too: c > 1 would make -inf of the start, and NaN of a score of -inf
         float e[32];
 #pragma unroll
         for (int i = 0; i < 32; ++i) e[i] = __builtin_fmaf(s[i >> 4][i & 15], c, -mc);

@@ -65,6 +65,24 @@ def test_attention_leaves_out_keys_of_minus_infinity(dev, sq, h, dh):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1e-30, 0.5, 0.7, 1.0, 30.0])  # 0.693 * log2(e) = 1
+@pytest.mark.parametrize("sq,h,dh", [(40, 2, 64), (40, 2, 128), (1408, 24, 128)])  # the three forms of the kernel
+def test_attention_leaves_out_keys_of_minus_infinity_at_every_scale(dev, sq, h, dh, scale):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(dh + sq)
+    q, k, v = (torch.rand(1, n, h, dh, generator=g, device=dev).bfloat16() for n in (sq, 264, 264))
+    k[:, :136] = -float("inf")  # two tiles of 64 keys and a part of the third
+    q.clamp_(min=0.01)
+    got = ops.attention(q, k, v, scale)
+    assert torch.isfinite(got).all()
+    # the same 128 keys in other tiles: probabilities rounded to bf16 on both sides, positive v
+    assert torch.allclose(got.float(), ops.attention(q, k[:, 136:].contiguous(), v[:, 136:].contiguous(), scale).float(), rtol=2.0 ** -6, atol=0)
+    k[:] = -float("inf")
+    assert torch.isnan(ops.attention(q, k, v, scale)).all()
+
+
+@pytest.mark.gpu
 def test_attention_of_other_shapes_falls_back(dev):
     from lyradiff_amd import ops
 
