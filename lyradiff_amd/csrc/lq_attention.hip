@@ -123,6 +123,19 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
         attn_dma16(v_base, __umul24(src_row(t, i), v_pitch) + cv[i], smem_base + v_tile(t) + (wave * DMA + i) * 1024);
     };
 
+    // The rows of V past the last key, cleared by the wavefront that fetched them, after its wait and ahead of the barrier that hands
+    // the tile over: their probability is 0, which does not undo an infinity of the row they repeat.  (Of K they are masked.)
+    auto clear_v = [&](int t) {
+        if (t != ntiles - 1 || (t + 1) * KT <= p.sk) return;
+        int left = p.sk - t * KT;
+        asm volatile("" : "+s"(left));  // keeps the comparisons, of use in one tile, out of the registers of the loop
+#pragma unroll
+        for (int i = 0; i < DMA; ++i)
+            if ((wave * DMA + i) * RPD + d_row >= left)
+                *reinterpret_cast<uint4*>(lq_smem + v_tile(t) + (wave * DMA + i) * 1024 + lane * 16) = make_uint4(0, 0, 0, 0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    };
+
     // ---- operands: queries in registers for the whole kernel (lane: one row, chunks 2 * ks + lh)
     attn_s8 qf[KSTEPS];
     {
@@ -266,6 +279,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
     // taken again by tile t + 4, whose transfers start in phase 2t + 4 at the earliest; every wavefront has waited for its share
     // of tile t ahead of the barrier that opens phase 2t.
     attn_wait_vmcnt<2 * DMA>();
+    if constexpr (PHASES) clear_v(0);
     barrier();
     if constexpr (PHASES) {
         if (grp == 1) barrier();
@@ -278,17 +292,24 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
     // The QK part of the last iteration works on a repeated tile and is not used: one loop body keeps the accumulators in place.
     for (int t = 0; t < ntiles; ++t) {
         if constexpr (PHASES) {
-            if (grp == 1) attn_wait_vmcnt<2 * DMA>();  // this wavefront's share of tile t + 1
+            if (grp == 1) {
+                attn_wait_vmcnt<2 * DMA>();  // this wavefront's share of tile t + 1
+                clear_v(t + 1);
+            }
             barrier();
             softmax(t);
 #pragma unroll
             for (int n = 0; n < RING; ++n) fr[n] = load_step(t, n);
-            if (grp == 0) attn_wait_vmcnt<2 * DMA>();
+            if (grp == 0) {
+                attn_wait_vmcnt<2 * DMA>();
+                clear_v(t + 1);
+            }
             barrier();
             __builtin_amdgcn_s_setprio(1);
         } else {
             // K of tile t + 1 and V of tile t have landed, and everybody is done with K of tile t and V of tile t - 1
             attn_wait_vmcnt<0>();
+            clear_v(t);
             barrier();
 #pragma unroll
             for (int i = 0; i < DMA; ++i) { issue_k(t + 2, i); issue_v(t + 1, i); }

@@ -83,6 +83,21 @@ def test_attention_leaves_out_keys_of_minus_infinity_at_every_scale(dev, sq, h, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("sk", [13, 63, 77, 250])  # the last of one, two and four tiles; 64 keys fill one
+@pytest.mark.parametrize("sq,h,dh", [(40, 2, 64), (40, 2, 128), (1408, 24, 128)])  # the three forms of the kernel
+def test_attention_keeps_an_infinite_value_of_the_last_key(dev, sq, h, dh, sk):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(sk + sq)
+    q, k, v = (torch.randn(2, n, h, dh, generator=g, device=dev).bfloat16() for n in (sq, sk, sk))
+    want = ops.attention(q, k, v)
+    v[:, -1, :, 0], v[:, -1, :, dh - 1] = float("inf"), -float("inf")
+    got = ops.attention(q, k, v)
+    assert (got[..., 0] == float("inf")).all() and (got[..., dh - 1] == -float("inf")).all()
+    assert torch.equal(got[..., 1:dh - 1], want[..., 1:dh - 1])
+
+
+@pytest.mark.gpu
 def test_attention_of_other_shapes_falls_back(dev):
     from lyradiff_amd import ops
 
