@@ -1,6 +1,6 @@
 // Softmax attention of the transformer blocks (no mask, no dropout): O = softmax(scale * Q K^T) V per batch and head, 16-bit
-// operands, fp32 scores, maxima, sums and accumulators, probabilities rounded to T for the second product and summed as
-// rounded.  It stands where lyraDiff's attention processors call their flash attention
+// operands, fp32 scores, probabilities, maxima, sums and accumulators; for the second product alone the probabilities are rounded to
+// T.  It stands where lyraDiff's attention processors call their flash attention
 // (layers/flux_attention_processor/FluxAttentionFP8Processor.cc:246-291, layers/basic_transformer/BasicTransformerInt8Block.cc:
 // 330-420), between the q/k normalisation + rotary kernel and the output projection.
 //
@@ -20,8 +20,10 @@
 //     time.  NW == 4: two or more workgroups per CU run freely, one barrier per tile; a head dimension of 64 leaves registers
 //     for three wavefronts per SIMD, which cover for each other without phases.
 // Measured (settled, random operands, bf16; in parentheses the library attention that stood here before): 24 heads of 128,
-// 4608 tokens 261 us = 1.0 PFLOP/s (506), 6912 tokens 580 us (908), 1600 tokens 45 us (135); 2 x 10 heads of 64, 4096 tokens
-// 121 us (190).  NW == 4 at 24 x 4608 tokens of 128: 299 us; NW == 8 at 64: 147 us.
+// 4608 tokens 261 us = 1.0 PFLOP/s (506), 6912 tokens 583 us (908), 1600 tokens 45 us (135), 1000 tokens 24 us; 2 x 10 heads of 64,
+// 4096 tokens 120 us (190).  NW == 4 at 24 x 4608 tokens of 128: 299 us; NW == 8 at 64: 147 us.  The row sum of the fp32
+// probabilities takes as long as one of the rounded ones (262 / 583 / 24 / 120 us against 261 / 583 / 26 / 123), and makes the error
+// against 64 bits that of the library attention (bf16, 4608 tokens, 2-norm: 2.264e-3 both).
 #include "lq_common.h"
 
 namespace lq {
@@ -52,13 +54,6 @@ template <typename Tag> __device__ __forceinline__ v16f attn_mfma(attn_s8 a, att
 template <typename Tag> __device__ __forceinline__ u32 attn_pack(float a, float b) {
     if constexpr (std::is_same<Tag, BF16Tag>::value) return pack2_bf16(a, b);
     else return pack2_f16(a, b);
-}
-// sum + the two 16-bit values of w, in fp32
-template <typename Tag> __device__ __forceinline__ float attn_add2(u32 w, float sum) {
-    if constexpr (std::is_same<Tag, BF16Tag>::value)
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, w), __builtin_bit_cast(bf16x2_t, 0x3F803F80u), sum, false);
-    else
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2_t, w), __builtin_bit_cast(f16x2_t, 0x3C003C00u), sum, false);
 }
 // 16 bytes per lane from global memory to LDS byte address lds_addr + 16 * lane, awaited with attn_wait_vmcnt
 __device__ __forceinline__ void attn_dma16(const void* gbase, u32 voff, u32 lds_addr) {
@@ -178,7 +173,12 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
     // would make (-inf) - (-inf) of it.
     float m_run = -__FLT_MAX__, l_run[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const float c = p.scale_log2;
-    u32 pw[16];  // probabilities of a tile, two keys per word: words 4 * kk .. 4 * kk + 3 are the operand of PV step kk
+    // Probabilities of a tile, in fp32 and, two keys per word, in T: words 4 * kk .. 4 * kk + 3 are the operand of PV step kk.  The row
+    // sum takes the former, beside the matrix instructions (SUM_LATE); at a head dimension of 64 the 32 registers would cost the third
+    // wavefront per SIMD, and the sum is formed with the exponentials.
+    constexpr bool SUM_LATE = DH == 128;
+    float e[32];
+    u32 pw[16];
 
     // ---- the matrix instructions of one tile: PV (4 blocks of 16 keys x DB blocks of 32 columns), then QK of the next tile
     // (2 blocks of 32 keys x KSTEPS); the operand of step n is read RING steps ahead
@@ -244,7 +244,6 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
                 for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
         }
         const float mc = fmaxf(m_run * c, -__FLT_MAX__);  // finite too: c > 1 would make -inf of the start, and NaN of a score of -inf
-        float e[32];
 #pragma unroll
         for (int i = 0; i < 32; ++i) e[i] = __builtin_fmaf(s[i >> 4][i & 15], c, -mc);
         __builtin_amdgcn_sched_barrier(0);
@@ -259,6 +258,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
                     e[8 * g + 8 + 2 * i] = __builtin_amdgcn_exp2f(e[8 * g + 8 + 2 * i]);
                     e[8 * g + 9 + 2 * i] = __builtin_amdgcn_exp2f(e[8 * g + 9 + 2 * i]);
                 }
+                if constexpr (!SUM_LATE) { l_run[i] += e[8 * g + 2 * i]; l_run[i] += e[8 * g + 2 * i + 1]; }
                 pw[4 * g + i] = attn_pack<Tag>(e[8 * g + 2 * i], e[8 * g + 2 * i + 1]);
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -266,6 +266,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
         // all of it happens here: left alone, the compiler moves the exponentials next to the matrix instructions that use them
 #pragma unroll
         for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(pw[i]));
+#pragma unroll
+        for (int i = 0; i < (SUM_LATE ? 32 : 0); ++i) asm volatile("" : "+v"(e[i]));
         __builtin_amdgcn_sched_barrier(0);
     };
     auto barrier = [&] {
@@ -326,7 +328,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
 #pragma unroll
                 for (int u = 0; u < 16 / NQK; ++u) {
                     const int x = (n - NPV) * (16 / NQK) + u;
-                    l_run[x % 4] = attn_add2<Tag>(pw[x], l_run[x % 4]);
+                    if constexpr (SUM_LATE) { l_run[x % 4] += e[2 * x]; l_run[x % 4] += e[2 * x + 1]; }
                 }
             }
             if constexpr (PHASES) {  // tile t + 3, spread over the phase: a burst would stall the wavefront on the memory queue

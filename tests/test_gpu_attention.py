@@ -40,7 +40,7 @@ def test_attention_matches_fp32(dev, shape, dt):
     got = ops.attention(q, k, v)
     assert got.shape == q.shape and got.is_contiguous()
     want, mag = _reference(q, k, v, dh ** -0.5)
-    # u: rounding error of T.  Probabilities rounded to T, summed as rounded, the result rounded to T: 3 u of the sum of |terms|.
+    # u: rounding error of T.  Probabilities rounded to T, summed in fp32, the result rounded to T: 2 u of the sum of |terms|, 3 with room.
     # Absolute part: scores in fp32 over dh products of size ~ 1.5^2 and the exponentials, a few 1e-6; fp16 probabilities under
     # 2^-14 are rounded to a fixed step, 2^-25 for each of at most 1025 keys times |v| ~ 1.2: 4e-5
     u = 2.0 ** -11 if dt is torch.float16 else 2.0 ** -8
@@ -80,6 +80,25 @@ def test_attention_leaves_out_keys_of_minus_infinity_at_every_scale(dev, sq, h, 
     assert torch.allclose(got.float(), ops.attention(q, k[:, 136:].contiguous(), v[:, 136:].contiguous(), scale).float(), rtol=2.0 ** -6, atol=0)
     k[:] = -float("inf")
     assert torch.isnan(ops.attention(q, k, v, scale)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sk", [64, 200])  # one tile; three and a part
+@pytest.mark.parametrize("sq,h,dh", [(300, 2, 64), (300, 2, 128), (1408, 24, 128)])  # the three forms of the kernel
+def test_attention_sums_its_probabilities_in_32_bits(dev, sq, h, dh, sk, dt):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(sk + sq)
+    q, k, v = (torch.zeros(1, n, h, dh, dtype=dt, device=dev) for n in (sq, sk, sk))
+    q[..., 0] = (20 * torch.rand(1, sq, h, generator=g, device=dev)).to(dt)
+    k[:, 1:, :, 0] = -1  # scores 0, -x, -x, ..., so that the roundings of the probabilities to T all point the same way
+    v[:, 0] = 1
+    x = q[..., :1].double() * float(torch.tensor(dh ** -0.5))
+    want = (1 / (1 + (sk - 1) * torch.exp(-x))).to(dt).expand_as(q)
+    # fp32 scores, exponentials and sums: relative errors of about 2^-21, which move a result over a boundary between two numbers of T
+    # (2^-12 apart or more) for less than one row in 500; a sum of rounded probabilities moves every third one
+    assert (ops.attention(q, k, v) != want).float().mean() < 0.01
 
 
 @pytest.mark.gpu
