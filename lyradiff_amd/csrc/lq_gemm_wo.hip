@@ -27,8 +27,8 @@
 // Tiling: 32 to 256 outputs each way per workgroup (wo_form), k-tile 64, two or three LDS stages filled by direct-to-LDS
 // transfers (activations XOR-swizzled, weights copied as they lie).  Large problems give a wavefront 128x64 outputs (eight 32x32
 // MFMA tiles: every converted weight fragment is used by four MFMAs) and are bound by the vector instructions of the conversion
-// next to the matrix ones: int4 with zeros in bf16, 4608x12288x3072, 419 -> 322 us (1.08 PFLOP/s; the library's plain bf16
-// product on this card 1.11) with 2.75 instead of 5 instructions per weight and two workgroups of four wavefronts per CU instead
+// next to the matrix ones: int4 with zeros in bf16, 4608x12288x3072, 419 -> 326 us (1.07 PFLOP/s; the library's plain bf16
+// product on this card 1.11) with 3 instead of 5 instructions per weight and two workgroups of four wavefronts per CU instead
 // of one of eight.  Small problems are bound by the latency of a k-tile and share k out between wavefronts.
 #include "lq_gemm_core.h"
 
@@ -52,15 +52,11 @@ template <int G> __device__ __forceinline__ int wo_apply_h2(h2_t q, u32 s2, u32 
     if constexpr (G == 2) q = q + __builtin_bit_cast(h2_t, z2);   // v_pk_add_f16: T(. + z)
     return __builtin_bit_cast(int, q);
 }
-// u: the unsigned code as a float; s, z: fp32 bit patterns, z = the addend that wo_addend made of the offset and the zero point
-template <int G> __device__ __forceinline__ u32 wo_addend(u32 s, u32 z, float offset) {
-    if constexpr (G == 1) return __float_as_uint(-offset * __uint_as_float(s));                                   // exact
-    if constexpr (G == 2) return __float_as_uint(__builtin_fmaf(-offset, __uint_as_float(s), __uint_as_float(z)));
-    return __float_as_uint(-offset);
-}
-template <int G> __device__ __forceinline__ float wo_apply_f32(u32 u, u32 s, u32 z) {
-    if constexpr (G == 0) return (float)u + __uint_as_float(z);
-    else return __builtin_fmaf((float)u, __uint_as_float(s), __uint_as_float(z));
+// q: the signed code (int4: 16 times it, s a sixteenth of the scale) as a float; s, z: fp32 bit patterns
+template <int G> __device__ __forceinline__ float wo_apply_f32(float q, u32 s, u32 z) {
+    if constexpr (G == 1) return q * __uint_as_float(s);                                      // exact in fp32
+    if constexpr (G == 2) return __builtin_fmaf(q, __uint_as_float(s), __uint_as_float(z));
+    return q;
 }
 template <int G> struct WoCvt<true, false, G> {  // fp16 <- uint8: d0 holds k0..k3, d1 holds k4..k7
     static __device__ __forceinline__ v4i run(u32 d0, u32 d1, u32 s2, u32 z2) {
@@ -85,30 +81,40 @@ template <int G> struct WoCvt<true, true, G> {  // fp16 <- uint4: d0 holds k0..k
         return o;
     }
 };
-// bf16 goes through fp32 (it cannot hold 1024 + u): v_cvt_f32_ubyte takes a code from any byte of a register, so a weight costs
-// that, one fused multiply-add and half a packed conversion (and a quarter of a mask where two nibbles share a byte)
+// bf16 goes through fp32 (it cannot hold 1024 + u).  The conversion of an integer takes a signed byte from anywhere in a register, so
+// a weight costs that, one multiplication or fused multiply-add and half a packed conversion, and a part of what makes its code signed.
+// An int4 code is converted from the upper half of a byte, as 16 q: multiplied by a sixteenth of the scale, which is exact too.
 template <int G> struct WoCvt<false, false, G> {  // bf16 <- uint8
     static __device__ __forceinline__ v4i run(u32 d0, u32 d1, u32 s, u32 z) {
         v4i o;
-        const u32 d[2] = {d0, d1};
+        const u32 d[2] = {d0 ^ 0x80808080u, d1 ^ 0x80808080u};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const u32 w = d[i >> 1];
             const int sh = 16 * (i & 1);
-            o[i] = (int)pack2_bf16(wo_apply_f32<G>((w >> sh) & 0xFFu, s, z), wo_apply_f32<G>((w >> (sh + 8)) & 0xFFu, s, z));
+            o[i] = (int)pack2_bf16(wo_apply_f32<G>((float)(int8_t)(w >> sh), s, z), wo_apply_f32<G>((float)(int8_t)(w >> (sh + 8)), s, z));
         }
         return o;
     }
 };
 template <int G> struct WoCvt<false, true, G> {  // bf16 <- uint4: bytes of the even nibbles are k0 k4 k1 k5, of the odd ones k2 k6 k3 k7
+    static __device__ __forceinline__ float code(u32 byte) {
+        if constexpr (G == 0) return (float)(byte & 0xFFu) - 8.0f;
+        else return (float)(int8_t)byte;
+    }
     static __device__ __forceinline__ v4i run(u32 d0, u32, u32 s, u32 z) {
         v4i o;
-        const u32 d[2] = {d0 & 0x0F0F0F0Fu, (d0 >> 4) & 0x0F0F0F0Fu};
+        u32 d[2] = {d0 & 0x0F0F0F0Fu, (d0 >> 4) & 0x0F0F0F0Fu};
+        if constexpr (G != 0) {
+            const u32 t = d0 ^ 0x88888888u;
+            d[0] = (t << 4) & 0xF0F0F0F0u;
+            d[1] = t & 0xF0F0F0F0u;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const u32 w = d[i & 1];
             const int sh = 8 * (i >> 1);
-            o[i] = (int)pack2_bf16(wo_apply_f32<G>((w >> sh) & 0xFFu, s, z), wo_apply_f32<G>((w >> (sh + 16)) & 0xFFu, s, z));
+            o[i] = (int)pack2_bf16(wo_apply_f32<G>(code(w >> sh), s, z), wo_apply_f32<G>(code(w >> (sh + 16)), s, z));
         }
         return o;
     }
@@ -256,7 +262,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW, 2) void wo_gemm_kernel(void* __r
                     gz[j] = F16 ? (zv | (zv << 16)) : (zv << 16);
                 }
             }
-            if constexpr (!F16) gz[j] = wo_addend<GROUPED>(gs[j], gz[j], W4 ? 8.0f : 128.0f);
+            if constexpr (!F16 && W4) gs[j] = __float_as_uint(__uint_as_float(gs[j]) * 0.0625f);  // see WoCvt; exact, subnormal ones included
         }
         v4i xb[3];
         xb[0] = *xptr(0);

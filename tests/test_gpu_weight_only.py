@@ -103,6 +103,39 @@ def test_weight_only_grouped_dequantised_weights(ops, dev, dt, bits, with_zeros,
         assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("with_zeros", [False, True])
+def test_bf16_dequantised_weights_have_one_fp32_rounding(ops, dev, bits, with_zeros):
+    """w = T(fma(q, s, z)) bit for bit where z is far below the scale, where it cancels q * s, beside codes of 0, and with scales up
+    to 2^127 (q * s + z is exact in fp64; the identity as activation)."""
+    k, n, group = 256, 160, 64
+    rng = np.random.default_rng(bits)
+    half = 1 << (bits - 1)
+    q = rng.integers(-half, half, (k, n)).astype(np.int8)
+    q[:, ::5] = rng.integers(-1, 2, (k, n // 5))
+    scales = torch.from_numpy((0.002 + 0.02 * rng.random((k // group, n))).astype(np.float32))
+    scales[:, ::5] = torch.tensor([2.0 ** 127, 2.0 ** 126, 2.0 ** -120, 1.0])[:, None]
+    scales = scales.bfloat16()
+    zeros = -scales.float() * torch.from_numpy(q[::group].astype(np.float32))  # near -q s of each group's first row
+    zeros[:, 1::5] = torch.from_numpy((2.0 ** rng.uniform(-24, -6, (k // group, n // 5))).astype(np.float32)) * scales[:, 1::5].float()
+    zeros[:, ::5] = scales[:, ::5].float() * 2.0 ** -6
+    zeros = zeros.bfloat16()
+    kind = "int8" if bits == 8 else "int4"
+    wp = ops.repack_weight_only(torch.from_numpy(q if bits == 8 else _pack_n(q)).to(dev), kind)
+    wide = lambda v: v.double().repeat_interleave(group, 0)
+    want = torch.from_numpy(q).double() * wide(scales)
+    if with_zeros:
+        want = want + wide(zeros)
+    want = want.float().bfloat16()
+    got = ops.weight_only_linear_grouped(torch.eye(k, dtype=torch.bfloat16).to(dev), wp, scales.to(dev), zeros.to(dev) if with_zeros else None, None, kind, group)
+    assert torch.isfinite(want).all() and torch.equal(got.cpu(), want)
+    one = np.ones((k, n), dtype=np.int8)
+    scales[0, 0] = float("inf")
+    wp = ops.repack_weight_only(torch.from_numpy(one if bits == 8 else _pack_n(one)).to(dev), kind)
+    got = ops.weight_only_linear_grouped(torch.ones(3, k, dtype=torch.bfloat16).to(dev), wp, scales.to(dev), zeros.to(dev) if with_zeros else None, None, kind, group)
+    assert (got[:, 0] == float("inf")).all()
+
+
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
 @pytest.mark.parametrize("bits,with_zeros,group", [(8, False, 128), (8, True, 64), (4, True, 128), (4, False, 64)])
 @pytest.mark.parametrize("m,n,k,with_bias", [(256, 128, 128, True), (300, 160, 384, False), (1, 32, 128, True),
