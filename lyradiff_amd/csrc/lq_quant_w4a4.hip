@@ -16,6 +16,7 @@ namespace lq {
 template <bool F16_SCALE, bool SMOOTHED, bool CODES = false>
 __device__ __forceinline__ uint2 w4a4_quant_lane8(float (&v)[8], const float (&dv)[8], const float (&yv)[8], float& s) {
     float amax = 0.0f;
+    bool odd = false;
     if constexpr (SMOOTHED) {
         // v = fl(x/d) from the stored reciprocal: q0 = fl(x*y), rem = x - q0*d (exact in one
         // fma), v = fl(q0 + rem*y) is the correctly rounded quotient when y = fl(1/d) and no
@@ -36,7 +37,7 @@ __device__ __forceinline__ uint2 w4a4_quant_lane8(float (&v)[8], const float (&d
         }
         float mf = group8_max(__uint_as_float(mbits));  // non-negative patterns order like floats
         mbits = __float_as_uint(mf);
-        const bool odd = mbits != 0 && !(mbits >= 0x219392EFu /*1e-18f*/ && mbits <= 0x5D5E0B6Bu /*1e18f*/);
+        odd = mbits != 0 && !(mbits >= 0x219392EFu /*1e-18f*/ && mbits <= 0x5D5E0B6Bu /*1e18f*/);
         amax = mf;
         if (__builtin_expect(odd, 0)) {  // uniform over the 8 lanes of the group
             amax = 0.0f;
@@ -61,8 +62,10 @@ __device__ __forceinline__ uint2 w4a4_quant_lane8(float (&v)[8], const float (&d
     }
     const float r = fast_recip(s);
     if constexpr (CODES) {  // every integer of [-8, 8] is an e4m3 number: the conversion is exact
+        static_assert(SMOOTHED, "an unusual group has to be known: a NaN leaves both `slow` and the rounding's own test unmoved");
         float rq[8];
-        if (quant8_round<7>(v, s, r, slow, rq)) {
+        // the integer conversion of the packed form turns NaN into 0 by itself; this one has to be told
+        if (quant8_round<7>(v, s, r, slow | odd, rq)) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) rq[i] = rq[i] != rq[i] ? 0.0f : fminf(fmaxf(rq[i], -8.0f), 7.0f);
         }

@@ -51,6 +51,33 @@ def test_linear_on_codes_is_bit_identical(dev, m, n, k, dt):
     assert torch.equal(ops.w4a4_linear_codes(codes, wc, sa_t, sb_t, None, dt), ops.w4a4_linear(words, w, sa, sb, None, dt))
 
 
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_codes_of_nan_and_infinite_groups_are_those_of_the_packed_form(dev, dt):
+    """A NaN never enters a group's maximum and becomes 0, beside finite values as beside an infinity, whose group has an infinite scale."""
+    from lyradiff_amd import ops
+
+    m, n, k = 40, 64, 256
+    x, smooth, down, packed, sb, _, bias, _ = _make(dev, m, n, k, dt)
+    nan, inf = float("nan"), float("inf")
+    x[1, 3] = nan
+    x[2, 64:72] = nan                      # all of a lane
+    x[3, 128:192] = nan                    # all of a group
+    x[4, 10], x[4, 11] = inf, nan
+    x[5, 70] = -inf
+    x[6, 200], x[6, 207], x[6, 255] = nan, 3e4, -nan
+    words, sa, act = ops.w4a4_quant_lora_down(x, smooth, down)
+    codes, sa_t, act_c = ops.w4a4_quant_lora_down_codes(x, smooth, down)
+    assert torch.equal(codes.view(torch.float8_e4m3fn).float(), _values(words).float())
+    assert torch.equal(sa_t.view(torch.int32), sa.t().contiguous().view(torch.int32))
+    assert torch.equal(act_c.isnan(), act.isnan())
+
+    w = ops.repack_weight(packed.view(torch.uint8))
+    want = ops.w4a4_linear(words, w, sa, sb, bias, dt)
+    got = ops.w4a4_linear_codes(codes, ops.w4a4_expand_weight(w), sa_t, sb.t().contiguous(), bias, dt)
+    assert torch.isfinite(got[[1, 2, 3, 6]]).all()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 def test_linear_module_takes_either_form(dev):
     from lyradiff_amd import ops
     from lyradiff_amd.weights import W4A4Linear
