@@ -14,8 +14,8 @@ template <typename OutTag> static constexpr lq_dtype_t out_enum() {
 template <typename OutTag> static int run_fp8_as(GemmParams p, hipStream_t st) {
     constexpr bool out16 = out_enum<OutTag>() == LQ_F16 || out_enum<OutTag>() == LQ_BF16;
     const bool forced = tl_forced_tactic >= 0 || g_tactic_fp8 >= 0;
-    const int cached = requested_tactic(g_tactic_fp8, LQ_W_FP8, p.m, p.n, p.k);
-    int t = cached;
+    const int requested = requested_tactic(g_tactic_fp8, LQ_W_FP8, p.m, p.n, p.k);
+    int t = requested;
     // scales and bias, and at most the running maximum of the outputs (two instructions per four outputs)
     const bool plain_epilogue = p.gelu == 0 && p.out_scale == nullptr && p.C8 == nullptr && p.gate == nullptr &&
                                 p.residual == nullptr && p.addend == nullptr;
@@ -35,12 +35,10 @@ template <typename OutTag> static int run_fp8_as(GemmParams p, hipStream_t st) {
             out_enum<OutTag>() != LQ_F32)
             t = 7;
     }
-    // Too few 256x256 tiles: the form whose rounds of workgroups cost least.  One that shares k out also stands in for a cached
-    // tactic, which was measured among the tactics alone.  k <= 1024: a workgroup's ten or sixteen k-tiles leave nothing to share
-    // (1024x640x640: 4.7 us with 64x64 tiles, 4.9 with k shared).
-    if (!forced && out16 && p.k > 1024 && (long)((p.m + 255) / 256) * ((p.n + 255) / 256) < 192) {
-        const int form = few_tiles_form(p.m, p.n, p.k);
-        if (cached < 0 || form >= SMALL_32x32_K4) t = form;
+    // Too few 256x256 tiles: the form whose rounds of workgroups cost least.  A forced or cached tactic stands.  k <= 1024: a
+    // workgroup's ten or sixteen k-tiles leave nothing to share (1024x640x640: 4.7 us with 64x64 tiles, 4.9 with k shared).
+    if (requested < 0 && out16 && p.k > 1024 && (long)((p.m + 255) / 256) * ((p.n + 255) / 256) < 192) {
+        t = few_tiles_form(p.m, p.n, p.k);
         if (t >= SMALL_32x32_K4) return run_small(K_FP8, p, out_enum<OutTag>(), t, st);
     }
     if (t == 1 && (p.kb % 128 != 0 || p.a_panel)) t = 0;  // the 128-byte k-tile needs k % 128 == 0 and a row-major activation

@@ -62,3 +62,27 @@ def test_fp8_few_tiles(dev, dt):
         s8 = torch.full((1,), 0.05, device=dev)
         got8 = ops.fp8_linear_codes(codes, w32, sa, sw, bias, s8, 0, dt)
         assert torch.equal(got8, (y.float() * (1.0 / s8)).clamp(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8)), (m, n, k, "codes")
+
+
+def test_a_cached_tactic_stands(dev):
+    """The tactics add the k-tiles up in one sequence, where 2^-9 beside 448 * 448 is lost before that is taken off again; a form that
+    shares k keeps it, in a sum of another group."""
+    from lyradiff_amd import ops
+
+    m, n, k = 64, 64, 1280
+    a, w = (torch.zeros(r, k, device=dev) for r in (m, n))
+    a[:, [0, 64, 256]] = torch.tensor([448.0, 2.0 ** -6, 448.0], device=dev)
+    w[:, [0, 64, 256]] = torch.tensor([448.0, 2.0 ** -3, -448.0], device=dev)
+    a, w = (t.to(torch.float8_e4m3fn).view(torch.uint8) for t in (a, w))
+    one, w32 = torch.ones(1, device=dev), ops.repack_weight(w)
+    run = lambda: ops.fp8_linear(a, w32, one, one, None, out_dtype=torch.bfloat16)
+    shared = torch.full((m, n), 2.0 ** -9, dtype=torch.bfloat16, device=dev)
+    assert torch.equal(run(), shared)
+    for rows in (m, 128):  # the exact entry, and that of the next power of two for 65 to 128 rows
+        try:
+            ops.gemm_shape_tactic("fp8", rows, n, k, 3)
+            x = a if rows == m else torch.cat([a, a])[:100].contiguous()
+            assert not ops.fp8_linear(x, w32, one, one, None, out_dtype=torch.bfloat16).any()
+        finally:
+            ops.gemm_shape_tactic("fp8", rows, n, k, -1)
+    assert torch.equal(run(), shared)
