@@ -507,7 +507,8 @@ int lq_w4a4_quantize_lora_down(uint32_t* q_words, void* scales, lq_dtype_t scale
  * instruction forms the exact group sums -- and the group scales group-major, [k / 64][rows].
  *   lq_w4a4_expand_rows32: packed weights in rows32 layout [n, k / 2] -> codes in rows32 layout [n, k]; n, k multiples of 32.
  *   lq_w4a4_weight_codes: that, and the weight's scales [n, k / 64] as [k / 64, n]; n a multiple of 32, k of 64.
- *   lq_w4a4_prefers_codes: 1 where a linear whose weight is kept packed gains by lq_w4a4_weight_codes + these calls, else 0.
+ *   lq_w4a4_prefers_codes: 1 where a linear whose weight is kept packed gains by lq_w4a4_weight_codes + these calls, else 0; 0 too
+ *     where a tactic of kind INT4 is set for the thread, the process or the shape, since those configure the packed GEMM.
  *   lq_w4a4_quantize_lora_down_codes: lq_w4a4_quantize_lora_down with codes [m, k] and scales [k / 64, m]; smooth required, rank 32,
  *     k % 128 == 0, k <= 16384, lora_act in x's type (F16 or BF16).
  *   lq_gemm_w4a4_codes: lq_gemm_w4a4_ex with sA [k / 64, m] and sB [k / 64, n] fp32; output F16 or BF16. */

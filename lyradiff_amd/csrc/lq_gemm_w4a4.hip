@@ -114,8 +114,9 @@ extern "C" int lq_gemm_w4a4_ex(void* C, lq_dtype_t out_dtype, const uint32_t* A_
 // Measured, quantiser + layout + GEMM, packed / codes (us), m = 512, 1024, 2048, 4608:
 //   3072 x 3072   30 / 33, 36 / 40, 57 / 55, 118 / 98     12288 x 3072   55 / 58, 98 / 85, 177 / 145, 390 / 301
 //   9216 x 3072   55 / 53, 80 / 79, 139 / 117, 299 / 236  3072 x 12288   97 / 101, 121 / 109, 196 / 174, 425 / 340
+// Tactics of kind INT4 are configurations of the packed kernels: a shape with one keeps to those.
 extern "C" int lq_w4a4_prefers_codes(int m, int n, int k) {
-    return n % 32 == 0 && k % 128 == 0 && k <= 16384 && (double)m * n * k >= 2e10;
+    return n % 32 == 0 && k % 128 == 0 && k <= 16384 && (double)m * n * k >= 2e10 && requested_tactic(g_tactic_w4a4, LQ_W_INT4, m, n, k) < 0;
 }
 
 extern "C" int lq_gemm_w4a4_codes(void* C, lq_dtype_t out_dtype, const uint8_t* A_codes, const uint8_t* B_codes_rows32, const float* sA,

@@ -96,6 +96,27 @@ def test_shape_tactic_cache(lib):
     assert b"workspace" in lib.lq_last_error()
 
 
+def test_w4a4_linear_keeps_to_the_packed_kernels_under_a_tactic(lib):
+    """Tactics of kind INT4 name configurations of the packed GEMM: with one set for the shape, the thread or the process, a large linear
+    does not go over to codes, where it would not be obeyed."""
+    from lyradiff_amd import lib as L
+
+    shape = (4608, 3072, 3072)
+    prefers = lambda: lib.lq_w4a4_prefers_codes(*shape)
+    assert prefers() == 1 and lib.lq_w4a4_prefers_codes(64, 3072, 3072) == 0
+    for put in (lambda t: lib.lq_gemm_set_shape_tactic(L.LQ_W_INT4, *shape, t), lambda t: lib.lq_gemm_set_shape_tactic(L.LQ_W_INT4, 8192, 3072, 3072, t),
+                lambda t: lib.lq_gemm_set_thread_tactic(t), lambda t: lib.lq_gemm_set_tactic(L.LQ_W_INT4, t)):
+        try:
+            assert put(1) == 0 and prefers() == 0
+        finally:
+            put(-1)
+        assert prefers() == 1
+    try:
+        assert lib.lq_gemm_set_tactic(L.LQ_W_FP8, 1) == 0 and prefers() == 1  # another GEMM's
+    finally:
+        lib.lq_gemm_set_tactic(L.LQ_W_FP8, -1)
+
+
 def test_tactic_cache_round_trips_through_bytes(lib):
     """lq_gemm_tactics_serialize / deserialize (the reference's GemmPluginProfiler::serialize / deserialize,
     layers/gemm_utils/GemmProfiler.cc:26-65): the table survives a round trip, a damaged or foreign table is refused whole."""
