@@ -149,9 +149,14 @@ class FluxTransformerBlockOp(_BlockOpBase):
             self.weights = F.load_flux_double_block_fp8(src, prefix, self.dim, self.dtype, self.device, keep_master=True,
                                                         full=self.quant_level is LyraQuantLevel.FP8_W8A8_FULL)
         get = W._source(src)
-        self.norms = [get(prefix + f"attn.{n}.weight", (self.head_dim,), self.dtype).to(self.device)
-                      for n in ("norm_q", "norm_k", "norm_added_q", "norm_added_k")]
-        self.norm_qk, self.norm_added_qk = torch.cat(self.norms[:2]), torch.cat(self.norms[2:])
+        norms = [get(prefix + f"attn.{n}.weight", (self.head_dim,), self.dtype).to(self.device)
+                 for n in ("norm_q", "norm_k", "norm_added_q", "norm_added_k")]
+        self.norm_qk, self.norm_added_qk = torch.cat(norms[:2]), torch.cat(norms[2:])
+
+    @property
+    def norms(self):
+        """The q, k, added q and added k norm weights: parts of norm_qk and norm_added_qk, which forward reads, so that a write counts."""
+        return (*self.norm_qk.chunk(2), *self.norm_added_qk.chunk(2))
 
     def _fp8_linears(self):
         w = self._loaded()
@@ -191,8 +196,12 @@ class FluxSingleTransformerBlockOp(_BlockOpBase):
             self.weights = F.load_flux_single_block_fp8(src, prefix, self.dim, self.mlp_scale, self.dtype, self.device,
                                                         keep_master=True, full=self.quant_level is LyraQuantLevel.FP8_W8A8_FULL)
         get = W._source(src)
-        self.norms = [get(prefix + f"attn.{n}.weight", (self.head_dim,), self.dtype).to(self.device) for n in ("norm_q", "norm_k")]
-        self.norm_qk = torch.cat(self.norms)
+        self.norm_qk = torch.cat([get(prefix + f"attn.{n}.weight", (self.head_dim,), self.dtype).to(self.device) for n in ("norm_q", "norm_k")])
+
+    @property
+    def norms(self):
+        """The q and k norm weights: parts of norm_qk, which forward reads, so that a write counts."""
+        return self.norm_qk.chunk(2)
 
     def _fp8_linears(self):
         w = self._loaded()

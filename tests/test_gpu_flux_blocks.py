@@ -715,6 +715,32 @@ def _rel(a, b):
     return float((a.double() - b.double()).norm() / b.double().norm())
 
 
+def test_flux_block_ops_follow_their_norm_weights(ops, dev):
+    """A norm weight written in place after loading, seen by autograd or not, gives the output of a block loaded with it."""
+    from lyradiff_amd import flux_ops as FO
+
+    b, s, sc, heads, dh = 1, 64, 32, 2, 64
+    d = heads * dh
+    g = rng_t(431)
+    sd = _block_state(d, dh, 432, ("t.", "u."))
+    x, ctx, temb = (torch.randn(*shape, generator=g).bfloat16().to(dev) for shape in ((b, s, d), (b, sc, d), (b, d)))
+    rope = _rope_table(b, sc + s, dh, 433).bfloat16().to(dev)
+    xs = torch.cat([ctx, x], dim=1).contiguous()
+    level = FO.LyraQuantLevel.FP8_W8A8_FULL.value
+    for cls, pre, names in ((FO.FluxTransformerBlockOp, "t.", ("norm_q", "norm_k", "norm_added_q", "norm_added_k")),
+                            (FO.FluxSingleTransformerBlockOp, "u.", ("norm_q", "norm_k"))):
+        run = lambda op: torch.cat(op.forward(x, ctx, rope, temb), 1) if cls is FO.FluxTransformerBlockOp else op.forward(xs, rope, temb)
+        for i, n in enumerate(names):
+            op, other = cls("bf16", d, heads, dh, 4, level), cls("bf16", d, heads, dh, 4, level)
+            op.reload_model_from_state_dict(pre, sd, "cpu")
+            before = run(op)
+            assert len(op.norms) == len(names) and torch.equal(op.norms[i].cpu(), sd[f"{pre}attn.{n}.weight"])
+            op.norms[i].mul_(-1.0) if i % 2 else op.norms[i].data.mul_(-1.0)
+            other.reload_model_from_state_dict(pre, {**sd, f"{pre}attn.{n}.weight": -sd[f"{pre}attn.{n}.weight"]}, "cpu")
+            want = run(other)
+            assert not torch.equal(before, want) and torch.equal(run(op), want), n
+
+
 @pytest.mark.parametrize("level", ["FP8_W8A8_FULL", "FP8_W8A8"])
 def test_flux_block_ops_against_an_independent_fp64_restatement(ops, dev, level):
     """FluxTransformerBlockOp.forward and FluxSingleTransformerBlockOp.forward against oracle/flux_blocks_f64.py, an fp64
