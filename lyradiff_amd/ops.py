@@ -1036,10 +1036,10 @@ def attention_supported(q, k, v) -> bool:
         return False
     for t in (q, k, v):
         if not t.is_cuda or t.dtype != q.dtype or t.stride(3) != 1 or (t.stride(2) != dh and t.shape[2] > 1) or t.data_ptr() % 16 or \
-                (t.stride(1) % 8 and t.shape[1] > 1) or (t.stride(0) % 8 and t.shape[0] > 1) or t.stride(1) < width:
+                t.stride(1) % 8 or (t.stride(0) % 8 and t.shape[0] > 1) or t.stride(1) < width:
             return False
     longest = max(k.stride(1), v.stride(1))
-    return longest < 1 << 23 and k.shape[1] * longest < 1 << 31 and q.stride(1) % 8 == 0 and longest % 8 == 0
+    return longest < 1 << 23 and k.shape[1] < 1 << 24 and k.shape[1] * longest < 1 << 31
 
 
 def attention(q, k, v, scale=None):

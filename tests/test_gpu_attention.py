@@ -129,6 +129,39 @@ def test_attention_of_other_shapes_falls_back(dev):
             ops.attention(q, k, v)
 
 
+@pytest.mark.gpu
+def test_attention_follows_the_strides(dev):
+    """What the kernel reads in place (parts of wider tokens, a batch repeated by a stride of 0, heads from a wider tensor's start) and
+    what it leaves to PyTorch (strides off 16 bytes, also of a single token, heads apart or interleaved, tokens that overlap)."""
+    from lyradiff_amd import ops
+
+    h, dh = 3, 64
+    w = h * dh
+    buf = torch.randn(8 * 40 * 4 * w, generator=torch.Generator(device=dev).manual_seed(5), device=dev).bfloat16()
+    make = lambda b, s, row, batch, off=0, head=dh, elem=1: buf.as_strided((b, s, h, dh), (batch, row, head, elem), off)
+    dense = lambda b, s: make(b, s, w, s * w)
+    cases = [(dense(2, 9), make(2, 40, 4 * w, 160 * w), make(2, 40, 3 * w + 8, 160 * w, 64), True),
+             (make(3, 9, w, 0), make(3, 40, w, 0, 8), make(3, 40, 2 * w, 80 * w), True),
+             (make(1, 9, w, 3), make(1, 40, w, 5), make(1, 40, w, 7), True),                 # one batch: its stride is of no account
+             (dense(2, 9), make(2, 1, w + 3, 8 * w), make(2, 1, 2 * w, 8 * w), False),       # one key, at an odd stride
+             (make(2, 1, w + 3, 8 * w), dense(2, 40), dense(2, 40), False),
+             (dense(2, 9), make(2, 40, w + 4, 160 * w), dense(2, 40), False),
+             (dense(2, 9), dense(2, 40), make(2, 40, w, 40 * w + 2), False),
+             (dense(2, 9), dense(2, 40), make(2, 40, w, 40 * w, 4), False),
+             (dense(2, 9), make(2, 40, 2 * w, 80 * w, head=2 * dh), dense(2, 40), False),
+             (dense(2, 9), make(2, 40, w, 40 * w, head=1, elem=h), dense(2, 40), False),
+             (make(2, 9, 8, 9 * w), dense(2, 40), dense(2, 40), False)]
+    for i, (q, k, v, taken) in enumerate(cases):
+        assert ops.attention_supported(q, k, v) == taken, i
+        got = ops.softmax_attention(q, k, v)
+        if taken:
+            assert torch.equal(got, ops.attention(q.contiguous(), k.contiguous(), v.contiguous())), i
+        else:
+            assert (got.float() - _reference(q, k, v, dh ** -0.5)[0]).abs().max() < 2e-2, i  # of values up to 4, rounded to bf16
+            with pytest.raises(ValueError):
+                ops.attention(q, k, v)
+
+
 def test_attention_argument_errors_do_not_reach_the_gpu():
     from lyradiff_amd import lib as L
 
