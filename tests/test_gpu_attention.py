@@ -162,6 +162,37 @@ def test_attention_follows_the_strides(dev):
                 ops.attention(q, k, v)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("sq,h,dh", [(300, 2, 64), (300, 2, 128), (1408, 24, 128)])  # the three forms of the kernel
+def test_attention_on_a_side_stream_and_replayed_from_a_graph(dev, sq, h, dh):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(sq)
+    qkv = torch.randn(1, sq, 3, h, dh, generator=g, device=dev).bfloat16()
+    static = qkv.clone()
+    run = lambda t: ops.softmax_attention(*t.unbind(2))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    want = run(qkv)
+    with torch.cuda.stream(side):
+        got = run(static)
+    side.synchronize()
+    assert torch.equal(got, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        out = run(static)
+    for i in range(4):
+        new = (qkv * (1.0 + 0.25 * i)).bfloat16()
+        want = run(new)
+        static.copy_(new)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), i
+        run(qkv)  # eager work between the replays
+        torch.cuda.synchronize()
+
+
 def test_attention_argument_errors_do_not_reach_the_gpu():
     from lyradiff_amd import lib as L
 
