@@ -4,9 +4,12 @@
 // What bounds it: the weights' way from memory.  The tiled forms bring them to LDS through a few stages per wavefront group, each
 // with as many bytes of (repeated) activation rows, so that a workgroup has 16 KiB of weights on their way; here a wavefront
 // requests both operands straight into registers -- a 32-row by 64-byte piece of the rows32 layout is two lane-linear kilobytes,
-// already the matrix instruction's operand -- DEPTH k-tiles ahead, with neither a barrier nor an LDS round trip in the loop.
-// Measured (us, bf16, replayed back to back, the tiled form -> this one): 1x18432x3072 13.9 -> 10.3 (5.5 TB/s), 1x9216x3072 6.2 -> 4.7,
-// 1x3072x3072 4.8 -> 3.4, 1x3072x12288 12.8 -> 7.7, 8x12288x3072 9.4 -> 6.9, 32x18432x3072 15.1 -> 11.3, 32x9216x3072 6.6 -> 6.4.
+// already the matrix instruction's operand -- DEPTH k-tiles ahead, with neither a barrier nor an LDS round trip in the loop (it issues
+// in 8 % of its cycles and waits in the others).  Measured (us, bf16, activation in k-panels, the tiled form -> this one; first
+// weights from memory, 1.2 GB of them in turn, then one weight again and again, which the last-level cache keeps):
+//   1x18432x3072 15.6 -> 12.1 (4.7 TB/s), 13.1 -> 10.2     1x9216x3072 9.4 -> 8.3, 5.6 -> 4.8     1x3072x3072 7.1 -> 4.8, 4.2 -> 3.4
+//   1x3072x12288 17.7 -> 11.9, 12.2 -> 7.9     8x12288x3072 10.1 -> 8.8, 8.7 -> 6.7     24x9216x3072 9.7 -> 9.6, 5.8 -> 5.9
+//   32x18432x3072 17.4 -> 14.9, 13.7 -> 11.2     32x9216x3072 9.9 -> 10.2, 5.9 -> 6.3     32x3072x12288 18.5 -> 17.1, 12.5 -> 10.8
 // The order of the sums is that of the tiled forms with four k-groups (SMALL_32x32_K4, SMALL_32x64_K4): group g adds the k-tiles g,
 // g + 4, ... and the four sums are added in group order, so every result has the same bits whichever form computes it.
 #include "lq_gemm_core.h"
@@ -79,8 +82,12 @@ template <typename OutTag> __global__ __launch_bounds__(256, 2) void fp8_rows_ke
     if (lr < p.m) OutStore<OutTag>::store4(p.C, (size_t)lr * p.n + n0, y);
 }
 
+// Rows that are K bytes apart take a cache line each for the 64 bytes of a k-tile, which a workgroup of every 32 columns reads again;
+// k-panels put them side by side.  From 17 such rows up that costs more than the tiles' LDS (us from memory / cached, tiled -> this): 16x9216x3072 9.5 -> 9.7 / 5.6 -> 6.7,
+// 16x18432x3072 16.7 -> 13.8 / 13.4 -> 11.2, 16x3072x12288 17.9 -> 15.6 / 12.4 -> 11.7; 24x9216x3072 9.8 -> 10.8 / 5.9 -> 7.8,
+// 32x12288x3072 10.4 -> 12.5 / 9.3 -> 9.4, 32x3072x12288 19.8 -> 21.0 / 12.7 -> 15.7.
 bool fp8_rows_takes(const GemmParams& p) {
-    return p.m <= 32 && p.kb % 256 == 0 && p.C != nullptr && p.gelu == 0 && p.out_scale == nullptr && p.out_max == nullptr && p.C8 == nullptr &&
+    return p.m <= (p.a_panel ? 32 : 16) && p.kb % 256 == 0 && p.C != nullptr && p.gelu == 0 && p.out_scale == nullptr && p.out_max == nullptr && p.C8 == nullptr &&
            p.gate == nullptr && p.residual == nullptr && p.addend == nullptr;
 }
 

@@ -5,7 +5,7 @@
 // k shared between two or four groups of wavefronts the chain is that much shorter and the CU has as many more chains to switch
 // between; the partial sums meet in LDS (at most 128 KiB, about 1 us), not in memory.  Measured (us, FP8 to bf16, before -> now):
 // 154x9216x3072 14.8 -> 9.9, 512x3072x3072 11.6 -> 8.8, 512x3072x12288 42 -> 29; INT8 1024x1280x1280 8.4 -> 6.5, 333x1280x5120 16 ->
-// 10.  FP8 with at most 32 rows and no more than scales and bias goes to lq_gemm_rows.hip instead.
+// 10.  FP8 of few rows with no more than scales and bias goes to lq_gemm_rows.hip instead.
 #pragma once
 
 #include "lq_gemm_core.h"

@@ -30,9 +30,8 @@ bool fp8_rows_takes(const GemmParams& p);  // lq_gemm_rows.hip
 int run_fp8_rows(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st);
 
 int run_small(GemmKind kind, const GemmParams& p, lq_dtype_t out_dtype, int form, hipStream_t st) {
-    // Up to 32 rows: one pass over the weights (1x18432x3072 10.3 us against 13.9, 32x9216x3072 6.4 against 6.6; 33 rows would be
-    // a second pass).  Other epilogues take a form that sums in the same order, so that a linear with
-    // and without one agree to the bit.
+    // Few rows: one pass over the weights.  Up to 32 of them other epilogues, and rows of an activation that it does not take, have a
+    // form that sums in the same order, so that a linear with and without one agrees to the bit.
     if (kind == K_FP8 && fp8_rows_takes(p)) return run_fp8_rows(p, out_dtype, st);
     if (kind == K_FP8 && p.m <= 32 && p.kb % 256 == 0 && form != SMALL_32x32_K4) form = SMALL_32x64_K4;
     if (out_dtype == LQ_BF16) return kind == K_FP8 ? run_small_fp8_bf16(p, form, st) : run_small_int8_bf16(p, form, st);

@@ -22,3 +22,19 @@ def test_fp8_few_rows(dev, m, n, k, dt):
         want = ops.fp8_linear_panels(panels, w32, sa, sw, bias, torch.zeros(1, device=dev), dt)
         assert torch.equal(ops.fp8_linear_panels(panels, w32, sa, sw, bias, None, dt), want)
         assert torch.equal(ops.fp8_linear(a, w32, sa, sw, bias, out_dtype=dt), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [16, 17, 32, 33])  # rows of K bytes leave the form at 17, k-panels at 33
+def test_fp8_few_rows_leave_the_form_without_a_bit_changed(dev, m):
+    from lyradiff_amd import ops
+
+    n, k = 9216, 3072
+    g = torch.Generator(device=dev).manual_seed(m)
+    a, w = (torch.randn(r, k, generator=g, device=dev).to(torch.float8_e4m3fn).view(torch.uint8) for r in (33, n))
+    one, w32 = torch.ones(1, device=dev), ops.repack_weight(w)
+    a = a[:m].contiguous()
+    got = ops.fp8_linear(a, w32, one, one, None, out_dtype=torch.bfloat16)
+    assert torch.equal(got, ops.fp8_linear_panels(a.view(m, k // 64, 64).transpose(0, 1).contiguous(), w32, one, one, None, None, torch.bfloat16))
+    if m <= 32:  # the same sums, row by row
+        assert torch.equal(got[:1], ops.fp8_linear(a[:1].contiguous(), w32, one, one, None, out_dtype=torch.bfloat16))
