@@ -5,9 +5,10 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# (m, n, k): 32x32, 32x64 (k a multiple of 256), 64x128, 128x128 (a multiple of 128), and k that no form can share
+# (m, n, k): 32x32, 32x64 (k a multiple of 256), 64x128, 128x128 (a multiple of 128), and k that no form can share; 128x128 shared from
+# k = 2048 up, in 224 tiles, 256 and 264
 SIZES = [(1, 32, 1280), (33, 3072, 1280), (77, 3040, 1536), (65, 9216, 1152), (190, 9248, 1152), (333, 9216, 1152), (100, 12320, 2176),
-         (300, 1056, 1088)]
+         (300, 1056, 1088), (1000, 3552, 2048), (1024, 4096, 2176), (1000, 4128, 2048)]
 
 
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
