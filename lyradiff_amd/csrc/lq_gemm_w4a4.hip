@@ -31,12 +31,13 @@ template <int KIND, typename OutTag> static int run_w4a4(GemmParams p, hipStream
 // Tile configurations on codes, in the order of the size they are for (3072 outputs, K = 3072, us, tactic 0 / 1 / 2):
 //   2000 tokens  45.7 / 39.4 / 42.7     1000 tokens  28.9 / 24.3 / 23.9     333 tokens  25.1 / 18.4 / 16.0
 //   512 x 9216   41.2 / 34.4 / 39.2     4608 x 3072  77 / 88 / -
-// Larger problems are bound by the power the two scale multiplications, the matrix instruction and the operand traffic take
-// together (4096 x 4096 x 3072: 82 us with random operands, 73 with zeros, 42 for the scale multiplications alone), and six further
-// tile shapes measured within 4 % of tactic 0 there.
+// What bounds larger problems: no single pipe.  4608 x 3072 x 3072 takes 147 k cycles; on a SIMD the vector instructions take 97 k of
+// them (the two scale multiplications of every output and group 83 k), LDS 41 % and the matrix instructions 28 % beside them, and three
+// wavefronts wait for a third of their time.  The power limit makes 79 us of those cycles at 1.87 GHz; on operands of zeros, the same
+// cycles at 2.3, 64.  Six further tile shapes measured within 4 % of tactic 0.
 template <typename OutTag> static int run_w4a4_codes(const GemmParams& p, hipStream_t st) {
     const long big = (long)((p.m + 127) / 128) * ((p.n + 127) / 128), mid = (long)((p.m + 63) / 64) * ((p.n + 127) / 128);
-    if (big >= 512) return launch_gemm<K_W4C, OutTag, 128, 128, 128, 2, 4, 2>(p, st);  // two rounds of two workgroups per CU
+    if (big >= 512) return launch_gemm<K_W4C, OutTag, 128, 128, 128, 2, 4, 2>(p, st);  // a round of two workgroups per CU and more
     if (mid >= 448) return launch_gemm<K_W4C, OutTag, 64, 128, 128, 2, 4, 2>(p, st);
     return launch_gemm<K_W4C, OutTag, 64, 64, 128, 2, 2, 2>(p, st);  // few tiles: as many and as short as possible
 }
