@@ -328,6 +328,30 @@ int lq_gemm_fp8_gated(void* C, lq_dtype_t out_dtype, const uint8_t* A, const uin
                       const float* a_scale, const float* b_scale, const void* bias, const void* gate,
                       size_t rows_per_gate, const void* residual, int m, int n, int k, lq_stream_t stream);
 
+/* Two FP8 linears of one n and k (the image and the text half of a double-stream block, FluxTransformerFP8Block.cc:159-262), in one
+ * launch where that is faster.  Per half one of
+ *   C = scales and bias                                  (lq_gemm_fp8_panels)
+ *   C_fp8 = e4m3 codes of gelu(scales and bias)          (lq_gemm_fp8_codes_panels)
+ *   C = gate and residual behind scales and bias         (lq_gemm_fp8_gated_panels)
+ * the same for both; results as those calls give them, but for the order of the sums over k.  panels: A and C_fp8 are k-panels,
+ * otherwise row-major (C_fp8 dense).  T (bias, gate, residual, C) in {F16, BF16}; a half with m == 0 is skipped.  Neither half may
+ * read what the other writes. */
+typedef struct {
+    void* C;
+    const uint8_t* A;
+    const uint8_t* B_rows32;
+    const float* a_scale;
+    const float* b_scale;
+    const void* bias;
+    uint8_t* C_fp8;
+    const float* C_fp8_scale;
+    const void* gate;
+    size_t rows_per_gate;
+    const void* residual;
+    int m;
+} lq_fp8_half_t;
+int lq_gemm_fp8_pair(const lq_fp8_half_t* halves, lq_dtype_t dtype, int gelu, int panels, int n, int k, lq_stream_t stream);
+
 /* lq_gemm_fp8 that writes only e4m3 codes of its output, into a destination whose rows are `ldc` bytes apart:
  *   C_fp8[m*ldc + n] = e4m3( f32(T(act(y))) * (1 / C_fp8_scale[0]) ),  T = round_dtype (F16/BF16/F32)
  * gelu: 0 none; 1 tanh-GELU of the fp32 value (the GELU_BIAS epilogue, cublasMMWrapper.cc:1195-1199);

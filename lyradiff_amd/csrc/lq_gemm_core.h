@@ -251,7 +251,8 @@ struct GemmKernel {
         else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
 
-    static __device__ __forceinline__ void run(const GemmParams& p, char* smem_all) {
+    // bid: number of this workgroup's tile of C in the XCD-aware order of tile_coords
+    static __device__ __forceinline__ void run(const GemmParams& p, char* smem_all, const int bid) {
         const int tid = threadIdx.x, lane = tid & 63;
         const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6);
         const int kg = KW > 1 ? wave_all / NW : 0, wave = KW > 1 ? wave_all % NW : wave_all;
@@ -259,7 +260,7 @@ struct GemmKernel {
         const int wm = wave / WN, wn = wave % WN;
         int tm, tn;
         // band height chosen so that the workgroups an XCD runs at once cover a roughly square block of C
-        tile_coords<(BM >= 256 ? 4 : 8)>(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+        tile_coords<(BM >= 256 ? 4 : 8)>(bid, p.tiles_m, p.tiles_n, tm, tn);
         const int m0 = tm * BM, n0 = tn * BN;
         const int kb = p.kb;
         const int ktiles = kb / (BKB * KW);  // of this group
@@ -987,12 +988,24 @@ template <int KIND, int BM, int BN, int BKB, int WM, int WN> constexpr int min_w
 template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE, int KW = 1>
 __global__ __launch_bounds__(WM* WN * KW * 64, (min_workgroups_per_cu<KIND, BM, BN, BKB, WM, WN>())) void gemm_kernel(GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) char lq_smem[];
-    GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>::run(p, lq_smem);
+    GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>::run(p, lq_smem, (int)blockIdx.x);
 }
 
+// Two problems of one n and k in one launch (the image and the text half of a double-stream block: their own operands, scales and
+// outputs).  The second one has an eighth of the rows, and tiles that by themselves leave most of the chip idle for the length of
+// a whole walk over k; behind the first one's they fill its last round.  Figures: pair_form in lq_gemm_fp8.hip.
+struct GemmPair {
+    GemmParams p[2];
+};
 template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE, int KW = 1>
-static int launch_gemm(GemmParams p, hipStream_t st) {
-    using GK = GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>;
+__global__ __launch_bounds__(WM* WN * KW * 64, (min_workgroups_per_cu<KIND, BM, BN, BKB, WM, WN>())) void gemm_pair_kernel(GemmPair pair) {
+    extern __shared__ __attribute__((aligned(16))) char lq_smem[];
+    const int first = pair.p[0].tiles_m * pair.p[0].tiles_n, which = (int)blockIdx.x >= first ? 1 : 0;
+    GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>::run(pair.p[which], lq_smem, (int)blockIdx.x - which * first);
+}
+
+// Checks that a configuration takes the problem and fills in its tile counts.
+template <int BM, int BN, int BKB, int KW> static int plan_tiles(GemmParams& p) {
     if (p.kb % (BKB * KW) != 0) {
         set_error("gemm: row length %d bytes is not a multiple of the %d-byte k-tile", p.kb, BKB * KW);
         return LQ_ERR_SHAPE;
@@ -1003,20 +1016,45 @@ static int launch_gemm(GemmParams p, hipStream_t st) {
     }
     p.tiles_m = (p.m + BM - 1) / BM;
     p.tiles_n = (p.n + BN - 1) / BN;
-    auto kern = gemm_kernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>;
-    static bool attr_done = false;  // raising the dynamic LDS limit is idempotent; races are benign
-    if (!attr_done && GK::SMEM_BYTES > 48 * 1024) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           GK::SMEM_BYTES);
+    return LQ_OK;
+}
+
+// Launches with `lds` bytes of dynamic LDS; attr_done: the caller's per-kernel flag (raising the limit is idempotent, races are benign).
+template <typename Params>
+static int launch_with_lds(void (*kern)(Params), const Params& params, unsigned grid, unsigned block, int lds, bool& attr_done, hipStream_t st) {
+    if (!attr_done && lds > 48 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) {
-            set_error("gemm: cannot raise LDS limit to %d bytes: %s", GK::SMEM_BYTES, hipGetErrorString(e));
+            set_error("gemm: cannot raise LDS limit to %d bytes: %s", lds, hipGetErrorString(e));
             return LQ_ERR_HIP;
         }
         attr_done = true;
     }
-    dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(GK::THREADS);
-    hipLaunchKernelGGL(kern, grid, block, GK::SMEM_BYTES, st, p);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(block), lds, st, params);
     return check_launch("gemm");
+}
+
+template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE, int KW = 1>
+static int launch_gemm(GemmParams p, hipStream_t st) {
+    using GK = GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>;
+    const int rc = plan_tiles<BM, BN, BKB, KW>(p);
+    if (rc != LQ_OK) return rc;
+    static bool attr_done = false;
+    return launch_with_lds(gemm_kernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>, p, (unsigned)(p.tiles_m * p.tiles_n), GK::THREADS,
+                           GK::SMEM_BYTES, attr_done, st);
+}
+
+template <int KIND, typename OutTag, int BM, int BN, int BKB, int WM, int WN, int NSTAGE, int KW = 1>
+static int launch_gemm_pair(GemmPair pair, hipStream_t st) {
+    using GK = GemmKernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>;
+    for (GemmParams& p : pair.p) {
+        const int rc = plan_tiles<BM, BN, BKB, KW>(p);
+        if (rc != LQ_OK) return rc;
+    }
+    static bool attr_done = false;
+    const int tiles = pair.p[0].tiles_m * pair.p[0].tiles_n + pair.p[1].tiles_m * pair.p[1].tiles_n;
+    return launch_with_lds(gemm_pair_kernel<KIND, OutTag, BM, BN, BKB, WM, WN, NSTAGE, KW>, pair, (unsigned)tiles, GK::THREADS,
+                           GK::SMEM_BYTES, attr_done, st);
 }
 
 // Persistent one-wavefront-per-SIMD form (lq_gemm_persist.h, compiled in lq_gemm_persist.hip): LQ_OK when launched, 1 when
@@ -1026,8 +1064,9 @@ int launch_persist_fp8(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st
 int launch_persist_int8(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st);
 // Forms for problems of few tiles (lq_gemm_small.hip); numbered behind the tactics, which can be forced and cached: these cannot.
 enum SmallForm { SMALL_32x32_K4 = 64, SMALL_32x64_K4, SMALL_64x128_K2, SMALL_128x128_K2 };
-// the tactic or form for fewer than 192 tiles of 256x256, k > 1024 and 16-bit outputs
-int few_tiles_form(int m, int n, int k);
+// the tactic or form for fewer than 192 tiles of 256x256, k > 1024 and 16-bit outputs; m2: rows of a second problem in the same launch;
+// cost_out: its time by the table that it goes by
+int few_tiles_form(int m, int m2, int n, int k, float* cost_out = nullptr);
 int run_small(GemmKind kind, const GemmParams& p, lq_dtype_t out_dtype, int form, hipStream_t st);
 int run_small_fp8_bf16(const GemmParams& p, int form, hipStream_t st);  // lq_gemm_small_{bf16,f16}.hip
 int run_small_fp8_f16(const GemmParams& p, int form, hipStream_t st);

@@ -9,6 +9,8 @@ namespace lq {
 int run_fp8_f16(const GemmParams& p, hipStream_t st);   // lq_gemm_fp8_{f16,bf16,f32}.hip
 int run_fp8_bf16(const GemmParams& p, hipStream_t st);
 int run_fp8_f32(const GemmParams& p, hipStream_t st);
+int run_fp8_pair_f16(const GemmPair& pair, int form, hipStream_t st);  // lq_gemm_pair_{f16,bf16}.hip
+int run_fp8_pair_bf16(const GemmPair& pair, int form, hipStream_t st);
 
 }  // namespace lq
 
@@ -157,4 +159,69 @@ extern "C" int lq_gemm_fp8_codes_panels(uint8_t* C_fp8_panels, const float* C_fp
                                         const void* bias, int gelu, int m, int n, int k, lq_stream_t stream) {
     return gemm_fp8_codes(C_fp8_panels, (size_t)(n > 0 ? n : 0), C_fp8_scale, round_dtype, A_panels, B_rows32, a_scale, b_scale, bias, gelu,
                           m, n, k, 1, stream);
+}
+
+// The form for both problems in one launch, by the tiles of the two together and the lines of run_fp8_as; -1: one after the other.
+// The second problem's tiles by themselves leave most of the chip idle for a whole walk over k.  Measured (us, bf16, k-panels, two
+// launches / one), 4096 + 512 rows: 9216x3072 119 / 114, 3072x3072 48 / 39, 12288x3072 with GELU to codes 179 / 165, 3072x12288 with
+// gate 159 / 138; 1200 + 512 rows: 58 / 43, 27 / 23, 86 / 75, 80 / 79; 400 + 100 rows: 30 / 23, 16 / 10, 47 / 35, 47 / 31.
+static int pair_form(const GemmParams& a, const GemmParams& b) {
+    if (a.m <= 32 || b.m <= 32) return -1;  // few rows have a kernel of their own
+    for (const GemmParams* p : {&a, &b})
+        if (tl_forced_tactic >= 0 || requested_tactic(g_tactic_fp8, LQ_W_FP8, p->m, p->n, p->k) >= 0) return -1;  // tactics stand
+    auto tiles = [&](int rows, int cols) { return ((long)(a.m + rows - 1) / rows + (b.m + rows - 1) / rows) * ((a.n + cols - 1) / cols); };
+    const long t256 = tiles(256, 256), t128 = tiles(128, 128);
+    if (a.k <= 1024) return t128 >= 128 ? 2 : 3;
+    if (t256 < 192) {  // where the tiles of the second only open another round, two launches are ahead (2500 + 200 rows, 3072x12288: 115 against 126 us)
+        float both, first, second;
+        const int form = few_tiles_form(a.m, b.m, a.n, a.k, &both);
+        few_tiles_form(a.m, 0, a.n, a.k, &first);
+        few_tiles_form(b.m, 0, b.n, b.k, &second);
+        return both < first + second ? form : -1;
+    }
+    const bool plain = a.gelu == 0 && a.C8 == nullptr && a.gate == nullptr;
+    const long last256 = t256 % 256;
+    if (last256 != 0 && last256 < 128) return 4;
+    return plain ? 6 : (t256 > 256 ? 4 : 0);
+}
+
+extern "C" int lq_gemm_fp8_pair(const lq_fp8_half_t* halves, lq_dtype_t dtype, int gelu, int panels, int n, int k, lq_stream_t stream) {
+    LQ_REQUIRE(halves, LQ_ERR_ARG, "lq_gemm_fp8_pair: null pointer");
+    LQ_REQUIRE(dtype == LQ_F16 || dtype == LQ_BF16, LQ_ERR_UNSUPPORTED, "lq_gemm_fp8_pair: dtype must be F16 or BF16");
+    LQ_REQUIRE(gelu >= 0 && gelu <= 2, LQ_ERR_ARG, "lq_gemm_fp8_pair: gelu must be 0, 1 or 2");
+    GemmPair pair = {};
+    int problems = 0;
+    for (int i = 0; i < 2; ++i) {
+        const lq_fp8_half_t& h = halves[i];
+        const int rc = fp8_check("lq_gemm_fp8_pair", h.C, h.A, h.B_rows32, h.a_scale, h.b_scale, h.bias, h.residual, h.m, n, k);
+        if (rc < 0) return rc;
+        if (rc > 0) continue;
+        LQ_REQUIRE((h.C == nullptr) != (h.C_fp8 == nullptr), LQ_ERR_ARG, "lq_gemm_fp8_pair: one of C and C_fp8");
+        LQ_REQUIRE((h.C_fp8 == nullptr) == (h.C_fp8_scale == nullptr), LQ_ERR_ARG, "lq_gemm_fp8_pair: C_fp8 and C_fp8_scale go together");
+        LQ_REQUIRE(h.C_fp8 == nullptr || (reinterpret_cast<uintptr_t>(h.C_fp8) % 4 == 0 && (!panels || n % 64 == 0)), LQ_ERR_SHAPE,
+                   "lq_gemm_fp8_pair: need a 4-byte aligned C_fp8, and n %% 64 == 0 for k-panels (n=%d)", n);
+        LQ_REQUIRE((h.gate == nullptr) == (h.residual == nullptr) && (h.gate == nullptr || (h.C != nullptr && h.rows_per_gate > 0)), LQ_ERR_ARG,
+                   "lq_gemm_fp8_pair: gate and residual go together, with C and a positive rows_per_gate");
+        LQ_REQUIRE(reinterpret_cast<uintptr_t>(h.gate) % 16 == 0, LQ_ERR_ARG, "lq_gemm_fp8_pair: gate must be 16-byte aligned");
+        LQ_REQUIRE(gelu == 0 || h.C_fp8 != nullptr, LQ_ERR_ARG, "lq_gemm_fp8_pair: the activation comes with C_fp8");
+        GemmParams& p = pair.p[problems++];
+        p.C = h.C; p.A = h.A; p.B = h.B_rows32; p.bias = h.bias; p.a_scale = h.a_scale; p.b_scale = h.b_scale; p.gelu = gelu;
+        p.C8 = h.C_fp8; p.c8_scale = h.C_fp8_scale; p.ldc8 = (size_t)n;
+        p.gate = h.gate; p.gate_rows = h.rows_per_gate; p.residual = h.residual; p.beta = 1.0f;
+        p.m = h.m; p.n = n; p.k = k; p.kb = k;
+        p.a_panel = panels != 0;
+        p.c8_panel = panels != 0;
+    }
+    if (problems == 2) {
+        const GemmParams &a = pair.p[0], &b = pair.p[1];
+        LQ_REQUIRE((a.C8 == nullptr) == (b.C8 == nullptr) && (a.gate == nullptr) == (b.gate == nullptr), LQ_ERR_ARG,
+                   "lq_gemm_fp8_pair: both halves need the same outputs");
+        const int form = pair_form(a, b);
+        if (form >= 0) return dtype == LQ_BF16 ? run_fp8_pair_bf16(pair, form, as_stream(stream)) : run_fp8_pair_f16(pair, form, as_stream(stream));
+    }
+    for (int i = 0; i < problems; ++i) {
+        const int rc = fp8_dispatch("lq_gemm_fp8_pair", pair.p[i], dtype, stream);
+        if (rc != LQ_OK) return rc;
+    }
+    return LQ_OK;
 }

@@ -1,0 +1,8 @@
+// Two FP8 GEMMs in one launch with f16 outputs.
+#include "lq_gemm_pair.h"
+
+namespace lq {
+
+int run_fp8_pair_f16(const GemmPair& pair, int form, hipStream_t st) { return run_fp8_pair_as<F16Tag>(pair, form, st); }
+
+}  // namespace lq

@@ -3,7 +3,7 @@
 
 namespace lq {
 
-int few_tiles_form(int m, int n, int k) {
+int few_tiles_form(int m, int m2, int n, int k, float* cost_out) {
     // Time of a launch by the number of workgroups each CU of 256 has to hold (us at k = 3072): up to 256 of them, up to 512, ...; more
     // than fit make whole rounds.  128x128 tiles share k from k = 2048 up: below, adding up two halves costs what the shorter walk
     // saves (us, one walk / shared, 128 to 256 tiles -- FP8 k = 1152: 7.0-7.7 / 7.6-8.7, 1792: 8.5-11.4 / 8.9-10.8, 2048: 9.2-12.5 /
@@ -21,10 +21,11 @@ int few_tiles_form(int m, int n, int k) {
     float least = 0.0f;
     for (const Cost& c : table) {
         if (k % (64 * c.groups) != 0 || (c.form == SMALL_128x128_K2 && k < 2048)) continue;
-        const long tiles = ((long)m + c.bm - 1) / c.bm * (((long)n + c.bn - 1) / c.bn), left = tiles % c.per_round;
+        const long tiles = (((long)m + c.bm - 1) / c.bm + ((long)m2 + c.bm - 1) / c.bm) * (((long)n + c.bn - 1) / c.bn), left = tiles % c.per_round;
         const float cost = (float)(tiles / c.per_round) * c.us[(c.per_round + 255) / 256 - 1] + (left == 0 ? 0.0f : c.us[(left - 1) / 256]);
         if (least == 0.0f || cost < least) { best = c.form; least = cost; }
     }
+    if (cost_out != nullptr) *cost_out = least;
     return best;
 }
 

@@ -118,21 +118,42 @@ def ada_fp8_layernorm(x: torch.Tensor, temb: torch.Tensor, linear: Union[FP8Line
     return ops.layernorm_mod_fp8_dual(x, scale, shift, code_scales[0], code_scales[1], eps, panels=panels), msa
 
 
+def _gated_norm_codes(x, attn_output, msa, w: FluxAttnPostFP8Weights, eps: float):
+    """The first launch of flux_attn_post_fp8: (codes for gelu_proj as k-panels, hidden)."""
+    b, s, d = x.shape
+    if tuple(msa.shape) != (6, b, d):
+        raise ValueError("msa must be [6, B, D]")
+    gate_msa, shift_mlp, scale_mlp = msa[2], msa[3], msa[4]
+    # the two FP8 activations of the sequence travel as k-panels [K/64, B*S, 64] (whole cache lines for the GEMMs' transfers)
+    return ops.gate_residual_layernorm_mod_fp8(attn_output, gate_msa, x, scale_mlp, shift_mlp, w.gelu_proj.input_scale, eps, panels=True)
+
+
+def fp8_half(lin: FP8Linear, codes: torch.Tensor, **output) -> ops.FP8Half:
+    return ops.FP8Half(codes, lin.weight_rows32, lin.input_scale, lin.weight_scale, lin.bias, **output)
+
+
 def flux_attn_post_fp8(x: torch.Tensor, attn_output: torch.Tensor, msa: torch.Tensor, w: FluxAttnPostFP8Weights,
                        eps: float = 1e-6) -> torch.Tensor:
     """x, attn_output [B, S, D]; msa [6, B, D] -> output [B, S, D] in three launches."""
     b, s, d = x.shape
-    if tuple(msa.shape) != (6, b, d):
-        raise ValueError("msa must be [6, B, D]")
-    gate_msa, shift_mlp, scale_mlp, gate_mlp = msa[2], msa[3], msa[4], msa[5]
-    # the two FP8 activations of the sequence travel as k-panels [K/64, B*S, 64] (whole cache lines for the GEMMs' transfers)
-    q1, hidden = ops.gate_residual_layernorm_mod_fp8(attn_output, gate_msa, x, scale_mlp, shift_mlp, w.gelu_proj.input_scale, eps,
-                                                     panels=True)
+    q1, hidden = _gated_norm_codes(x, attn_output, msa, w, eps)
     q2 = ops.fp8_linear_codes_panels(q1, w.gelu_proj.weight_rows32, w.gelu_proj.input_scale, w.gelu_proj.weight_scale,
                                      w.gelu_proj.bias, w.ff_linear.input_scale, gelu=1, round_dtype=x.dtype)
     out = ops.fp8_linear_gated_panels(q2, w.ff_linear.weight_rows32, w.ff_linear.input_scale, w.ff_linear.weight_scale,
-                                      w.ff_linear.bias, gate_mlp, hidden.view(b * s, d), rows_per_gate=s)
+                                      w.ff_linear.bias, msa[5], hidden.view(b * s, d), rows_per_gate=s)
     return out.view(b, s, d)
+
+
+def flux_attn_post_fp8_pair(x, attn_output, msa, w: FluxAttnPostFP8Weights, context, context_attn, context_msa, wc: FluxAttnPostFP8Weights,
+                            eps: float = 1e-6):
+    """flux_attn_post_fp8 of the image and of the text half of a double-stream block, their linears two to a launch."""
+    q1, hidden = _gated_norm_codes(x, attn_output, msa, w, eps)
+    c1, chidden = _gated_norm_codes(context, context_attn, context_msa, wc, eps)
+    q2, c2 = ops.fp8_linear_pair(fp8_half(w.gelu_proj, q1, out_fp8_scale=w.ff_linear.input_scale),
+                                 fp8_half(wc.gelu_proj, c1, out_fp8_scale=wc.ff_linear.input_scale), x.dtype, gelu=1)
+    out, cout = ops.fp8_linear_pair(fp8_half(w.ff_linear, q2, gate=msa[5], residual=hidden, rows_per_gate=x.shape[1]),
+                                    fp8_half(wc.ff_linear, c2, gate=context_msa[5], residual=chidden, rows_per_gate=context.shape[1]), x.dtype)
+    return out.view(x.shape), cout.view(context.shape)
 
 
 def flux_single_mlp_fp8(x: torch.Tensor, norm_hidden, attn_output: torch.Tensor, gate: torch.Tensor,
@@ -230,8 +251,9 @@ def flux_double_block_fp8(x: torch.Tensor, context: torch.Tensor, temb: torch.Te
     context_attn [B, Sc, D]).  Returns (output, context_output)."""
     c, msa = ada_fp8_layernorm(x, temb, w.norm1, 6, (w.to_qkv.input_scale,), panels=True)
     cc, cmsa = ada_fp8_layernorm(context, temb, w.norm1_context, 6, (w.to_added_qkv.input_scale,), panels=True)
-    attn, cattn = attention(_linear_from_panels(w.to_qkv, c, x.shape[0], x.dtype),
-                            _linear_from_panels(w.to_added_qkv, cc, context.shape[0], x.dtype))
-    a_out = w.to_out.forward(attn.contiguous())
-    c_out = w.to_add_out.forward(cattn.contiguous())
-    return flux_attn_post_fp8(x, a_out, msa, w.ff), flux_attn_post_fp8(context, c_out, cmsa, w.ff_context)
+    qkv, cqkv = ops.fp8_linear_pair(fp8_half(w.to_qkv, c), fp8_half(w.to_added_qkv, cc), x.dtype)
+    attn, cattn = attention(qkv.view(*x.shape[:2], -1), cqkv.view(*context.shape[:2], -1))
+    rows = lambda t: t.contiguous().view(-1, t.shape[-1])
+    a_out, c_out = ops.fp8_linear_pair(fp8_half(w.to_out, ops.fp8_scale_cast_panels(rows(attn), w.to_out.input_scale)),
+                                       fp8_half(w.to_add_out, ops.fp8_scale_cast_panels(rows(cattn), w.to_add_out.input_scale)), x.dtype)
+    return flux_attn_post_fp8_pair(x, a_out.view(x.shape), msa, w.ff, context, c_out.view(context.shape), cmsa, w.ff_context)

@@ -27,7 +27,7 @@ from typing import Union
 import torch
 
 from . import ops
-from .flux_fp8 import AdaLinear16, ada_fp8_layernorm, load_ada_layernorm
+from .flux_fp8 import AdaLinear16, ada_fp8_layernorm, fp8_half, load_ada_layernorm
 from .weights import FP8Linear, W4A4Linear, load_fp8_linear, load_w4a4_linear
 
 
@@ -59,17 +59,34 @@ def load_flux_single_mlp_int4(src, prefix: str, dim: int, mlp_scale: int = 4, dt
         load_w4a4_linear(src, prefix + "proj_out.linears.1.linear.", dim, mlp_scale * dim, lora_rank, False, dtype, device))
 
 
-def flux_attn_post_int4(x: torch.Tensor, attn_output: torch.Tensor, msa: torch.Tensor, w: FluxAttnPostInt4Weights,
-                        eps: float = 1e-6) -> torch.Tensor:
-    """x, attn_output [B, S, D]; msa [6, B, D] -> output [B, S, D]."""
+def _post_activation(x, attn_output, msa, w: FluxAttnPostInt4Weights, eps: float):
+    """Everything of flux_attn_post_int4 up to ff_linear: (the codes of its input [B*S, 4D], hidden)."""
     b, s, d = x.shape
     if tuple(msa.shape) != (6, b, d):
         raise ValueError("msa must be [6, B, D]")
     norm, hidden = ops.gate_residual_layernorm_mod(x, msa[4], msa[3], attn_output, msa[2], eps)
-    q2 = w.gelu_proj.run(norm.view(b * s, d), gelu=2, out_fp8_scale=w.ff_linear.input_scale, want_output=False)
+    return w.gelu_proj.run(norm.view(b * s, d), gelu=2, out_fp8_scale=w.ff_linear.input_scale, want_output=False), hidden
+
+
+def flux_attn_post_int4(x: torch.Tensor, attn_output: torch.Tensor, msa: torch.Tensor, w: FluxAttnPostInt4Weights,
+                        eps: float = 1e-6) -> torch.Tensor:
+    """x, attn_output [B, S, D]; msa [6, B, D] -> output [B, S, D]."""
+    b, s, d = x.shape
+    q2, hidden = _post_activation(x, attn_output, msa, w, eps)
     out = ops.fp8_linear_gated(q2, w.ff_linear.weight_rows32, w.ff_linear.input_scale, w.ff_linear.weight_scale,
                                w.ff_linear.bias, msa[5], hidden.view(b * s, d), rows_per_gate=s)
     return out.view(b, s, d)
+
+
+def flux_attn_post_int4_pair(x, attn_output, msa, w: FluxAttnPostInt4Weights, context, context_attn, context_msa, wc: FluxAttnPostInt4Weights,
+                             eps: float = 1e-6):
+    """flux_attn_post_int4 of the image and of the text half of a double-stream block, their FP8 linears in one launch."""
+    q2, hidden = _post_activation(x, attn_output, msa, w, eps)
+    c2, chidden = _post_activation(context, context_attn, context_msa, wc, eps)
+    out, cout = ops.fp8_linear_pair(fp8_half(w.ff_linear, q2, gate=msa[5], residual=hidden, rows_per_gate=x.shape[1]),
+                                    fp8_half(wc.ff_linear, c2, gate=context_msa[5], residual=chidden, rows_per_gate=context.shape[1]),
+                                    x.dtype, panels=False)
+    return out.view(x.shape), cout.view(context.shape)
 
 
 def flux_single_mlp_int4(x: torch.Tensor, norm_hidden: torch.Tensor, attn_output: torch.Tensor, gate: torch.Tensor,
@@ -159,4 +176,4 @@ def flux_double_block_int4(x: torch.Tensor, context: torch.Tensor, temb: torch.T
     attn, cattn = attention(_w4a4_3d(w.to_qkv, n), _w4a4_3d(w.to_added_qkv, nc))
     a_out = _w4a4_3d(w.to_out, attn.contiguous())
     c_out = _w4a4_3d(w.to_add_out, cattn.contiguous())
-    return flux_attn_post_int4(x, a_out, msa, w.ff), flux_attn_post_int4(context, c_out, cmsa, w.ff_context)
+    return flux_attn_post_int4_pair(x, a_out, msa, w.ff, context, c_out, cmsa, w.ff_context)

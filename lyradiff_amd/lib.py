@@ -78,6 +78,7 @@ SYMBOLS = {
     "lq_gemm_fp8": (_I, [_P, _I, _P, _P, _P, _P, _P, _I, _P, _F, _I, _I, _I, _P]),
     "lq_gemm_fp8_ex": (_I, [_P, _I, _P, _P, _P, _P, _P, _I, _P, _F, _I, _I, _I, _P, _P, _P, _P]),
     "lq_gemm_fp8_gated": (_I, [_P, _I, _P, _P, _P, _P, _P, _P, _Z, _P, _I, _I, _I, _P]),
+    "lq_gemm_fp8_pair": (_I, [_P, _I, _I, _I, _I, _I, _P]),
     "lq_gemm_fp8_codes": (_I, [_P, _Z, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "lq_fp8_scale_cast_2d": (_I, [_P, _Z, _P, _Z, _I, _P, _I, _Z, _Z, _P]),
     "lq_gemm_w4a4": (_I, [_P, _I, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P]),
@@ -132,6 +133,12 @@ SYMBOLS = {
     "lq_mfma_fp8_probe": (_I, [_P, _P, C.c_size_t, _I, _P, _P]),
 }
 
+
+
+class Fp8Half(C.Structure):
+    """lq_fp8_half_t of include/lyraquant.h."""
+    _fields_ = [("C", _P), ("A", _P), ("B_rows32", _P), ("a_scale", _P), ("b_scale", _P), ("bias", _P), ("C_fp8", _P), ("C_fp8_scale", _P),
+                ("gate", _P), ("rows_per_gate", _Z), ("residual", _P), ("m", _I)]
 
 
 class Epilogue(C.Structure):

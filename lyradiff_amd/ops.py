@@ -9,6 +9,7 @@ torch.ops.lyradiff.* custom operators.
 from __future__ import annotations
 
 import ctypes as C
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -747,6 +748,60 @@ def fp8_linear_codes_panels(a_panels, w_rows32, a_scale, b_scale, bias, out_fp8_
                                                 _ptr(w_rows32), _ptr(a_scale), _ptr(b_scale), _ptr(bias), int(gelu), m, n, k, _stream()),
              "lq_gemm_fp8_codes_panels")
     return out
+
+
+class FP8Half(NamedTuple):
+    """One of the two problems of fp8_linear_pair: k-panels [K/64, M, 64] (or row-major codes [M, K]), the linear, and what its output is."""
+    codes: torch.Tensor
+    w_rows32: torch.Tensor
+    a_scale: torch.Tensor
+    b_scale: torch.Tensor
+    bias: Optional[torch.Tensor] = None
+    out_fp8_scale: Optional[torch.Tensor] = None  # e4m3 codes with this scale instead of a 16-bit output
+    gate: Optional[torch.Tensor] = None
+    residual: Optional[torch.Tensor] = None
+    rows_per_gate: int = 0
+
+
+def fp8_linear_pair(first: FP8Half, second: FP8Half, dtype, gelu: int = 0, panels: bool = True):
+    """Two FP8 linears of one N and K in one launch where that is faster: fp8_linear_panels, fp8_linear_codes_panels (gelu, out_fp8_scale)
+    or fp8_linear_gated_panels (gate, residual) of each, the same kind for both; with panels=False their row-major forms.  Returns both
+    outputs."""
+    if dtype not in (torch.float16, torch.bfloat16):
+        raise TypeError("dtype must be float16 or bfloat16")
+    n = first.w_rows32.shape[0]
+    k = first.w_rows32.shape[1]
+    args, outs = (_l.Fp8Half * 2)(), []
+    for h, a in zip((first, second), args):
+        _chk(h.codes, "codes", (torch.uint8,))
+        _chk(h.w_rows32, "w_rows32", (torch.uint8,))
+        for name, t, dt in (("a_scale", h.a_scale, torch.float32), ("b_scale", h.b_scale, torch.float32), ("bias", h.bias, dtype),
+                            ("out_fp8_scale", h.out_fp8_scale, torch.float32), ("gate", h.gate, dtype), ("residual", h.residual, dtype)):
+            if t is not None:
+                _chk(t, name, (dt,))
+        if tuple(h.w_rows32.shape) != (n, k) or (h.bias is not None and h.bias.numel() != n):
+            raise ValueError("both linears must be [N, K], a bias [N]")
+        if panels and (h.codes.dim() != 3 or h.codes.shape[0] * 64 != k or h.codes.shape[2] != 64):
+            raise ValueError("codes must be k-panels [K/64, M, 64]")
+        if not panels and (h.codes.dim() != 2 or h.codes.shape[1] != k):
+            raise ValueError("codes must be [M, K]")
+        m = h.codes.shape[1] if panels else h.codes.shape[0]
+        if (h.gate is None) != (h.residual is None):
+            raise ValueError("gate and residual go together")
+        if h.gate is not None and (h.residual.numel() != m * n or h.rows_per_gate <= 0 or
+                                   h.gate.numel() != ((m + h.rows_per_gate - 1) // h.rows_per_gate) * n):
+            raise ValueError("residual must be [M,N] and gate [ceil(M/rows_per_gate), N]")
+        if h.out_fp8_scale is None:
+            out = torch.empty((m, n), dtype=dtype, device=h.codes.device)
+            a.C = out.data_ptr()
+        else:
+            out = torch.empty((n // 64, m, 64) if panels else (m, n), dtype=torch.uint8, device=h.codes.device)
+            a.C_fp8, a.C_fp8_scale = out.data_ptr(), h.out_fp8_scale.data_ptr()
+        outs.append(out)
+        a.A, a.B_rows32, a.a_scale, a.b_scale, a.bias = h.codes.data_ptr(), h.w_rows32.data_ptr(), h.a_scale.data_ptr(), h.b_scale.data_ptr(), _ptr(h.bias)
+        a.gate, a.rows_per_gate, a.residual, a.m = _ptr(h.gate), int(h.rows_per_gate), _ptr(h.residual), m
+    _l.check(_l.load().lq_gemm_fp8_pair(C.addressof(args), _DT[dtype], int(gelu), int(panels), n, k, _stream()), "lq_gemm_fp8_pair")
+    return outs[0], outs[1]
 
 
 def fp8_scale_cast_into(x, scale, out, col_offset: int = 0, invert: bool = True):

@@ -158,17 +158,37 @@ struct FP8Linear {
            "lq_gemm_fp8_gated_panels");
         return y;
     }
-    // `gate` [B, n] and `residual` [m, n]:  T(T(T(y) * gate) + residual) in the epilogue; row-major codes (written by the W4A4
-    // GEMM's epilogue in the INT4 blocks)
-    at::Tensor from_codes_gated(const at::Tensor& q, int64_t m, const at::Tensor& gate, int64_t rows_per_gate,
-                                const at::Tensor& residual) const {
-        at::Tensor y = at::empty({m, n}, residual.options());
-        ok(lq_gemm_fp8_gated(P(y), lq_dt(residual.scalar_type()), P8(q), P8(w_rows32), PF(in_scale), PF(w_scale), P(bias), P(gate),
-                             (size_t)rows_per_gate, P(residual), (int)m, (int)n, (int)k, cur_stream()),
-           "lq_gemm_fp8_gated");
-        return y;
-    }
 };
+
+// One half of an FP8 pair (lq_gemm_fp8_pair): the codes of its [m, K] input; the caller adds what the output is
+lq_fp8_half_t half_of(const FP8Linear& l, const at::Tensor& q, int64_t m) {
+    lq_fp8_half_t h = {};
+    h.A = P8(q), h.B_rows32 = P8(l.w_rows32), h.a_scale = PF(l.in_scale), h.b_scale = PF(l.w_scale), h.bias = P(l.bias), h.m = (int)m;
+    return h;
+}
+void gemm_pair(const lq_fp8_half_t& a, const lq_fp8_half_t& b, at::ScalarType T, int gelu, int panels, int64_t n, int64_t k) {
+    const lq_fp8_half_t halves[2] = {a, b};
+    ok(lq_gemm_fp8_pair(halves, lq_dt(T), gelu, panels, (int)n, (int)k, cur_stream()), "lq_gemm_fp8_pair");
+}
+// two linears of one shape on codes in k-panels, in one launch where that is faster: [m, n] each
+std::pair<at::Tensor, at::Tensor> linear_pair(const FP8Linear& la, const at::Tensor& qa, int64_t ma, const FP8Linear& lb, const at::Tensor& qb,
+                                              int64_t mb, at::ScalarType T) {
+    at::Tensor ya = at::empty({ma, la.n}, on_gpu(T)), yb = at::empty({mb, lb.n}, on_gpu(T));
+    lq_fp8_half_t a = half_of(la, qa, ma), b = half_of(lb, qb, mb);
+    a.C = P(ya), b.C = P(yb);
+    gemm_pair(a, b, T, 0, 1, la.n, la.k);
+    return {ya, yb};
+}
+// the gated output projections behind the activations of both halves: gate [B, n], residual [B, S, n] -> [B, S, n]
+std::vector<at::Tensor> gated_pair(const FP8Linear& la, const at::Tensor& qa, const at::Tensor& gate_a, const at::Tensor& res_a, const FP8Linear& lb,
+                                   const at::Tensor& qb, const at::Tensor& gate_b, const at::Tensor& res_b, int panels) {
+    at::Tensor ya = at::empty_like(res_a), yb = at::empty_like(res_b);
+    lq_fp8_half_t a = half_of(la, qa, res_a.size(0) * res_a.size(1)), b = half_of(lb, qb, res_b.size(0) * res_b.size(1));
+    a.C = P(ya), a.gate = P(gate_a), a.rows_per_gate = (size_t)res_a.size(1), a.residual = P(res_a);
+    b.C = P(yb), b.gate = P(gate_b), b.rows_per_gate = (size_t)res_b.size(1), b.residual = P(res_b);
+    gemm_pair(a, b, res_a.scalar_type(), 0, panels, la.n, la.k);
+    return {ya, yb};
+}
 
 // W4A4 group-64 linear with its low-rank branch (W4A4GemmWeight.cc:65-83, W4A4Gemm.cc:113-169)
 // Large problems run on one e4m3 byte per value, laid out from the packed weight in each call (lq_w4a4_weight_codes): same results, no
@@ -278,29 +298,37 @@ at::Tensor attention_core(const at::Tensor& qkv, const at::Tensor& ctx_qkv, cons
     return o;
 }
 
-// FluxAttnPostFP8Processor::forward (FluxAttnPostFP8Processor.cc:93-240) in three launches
+// FluxAttnPostFP8Processor (FluxAttnPostFP8Processor.cc:93-240)
 struct AttnPostFP8 {
     FP8Linear gelu_proj, ff_linear;
     void load(const Source& src, const std::string& prefix, int64_t dim, at::ScalarType T) {
         gelu_proj.load(src, prefix + "net.0.proj", 4 * dim, dim, T);
         ff_linear.load(src, prefix + "net.2", dim, 4 * dim, T);
     }
-    at::Tensor forward(const at::Tensor& x, const at::Tensor& attn, const at::Tensor& msa) const {
-        const int64_t b = x.size(0), s = x.size(1), d = x.size(2), m = b * s;
-        const lq_dtype_t dt = lq_dt(x.scalar_type());
-        at::Tensor q1 = at::empty({d / 64, m, 64}, on_gpu(at::kByte)), hidden = at::empty_like(x);
-        ok(lq_gate_residual_layernorm_mod_fp8_panels(P8(q1), P(hidden), P(attn), P(msa[2]), P(x), P(msa[4]), P(msa[3]), dt,
+    // gate + residual + adaLN + cast: {codes for gelu_proj as k-panels, hidden}
+    std::pair<at::Tensor, at::Tensor> gated_norm(const at::Tensor& x, const at::Tensor& attn, const at::Tensor& msa) const {
+        const int64_t b = x.size(0), s = x.size(1), d = x.size(2);
+        at::Tensor q1 = at::empty({d / 64, b * s, 64}, on_gpu(at::kByte)), hidden = at::empty_like(x);
+        ok(lq_gate_residual_layernorm_mod_fp8_panels(P8(q1), P(hidden), P(attn), P(msa[2]), P(x), P(msa[4]), P(msa[3]), lq_dt(x.scalar_type()),
                                                      PF(gelu_proj.in_scale), (size_t)b, (size_t)s, (size_t)d, 1e-6f, cur_stream()),
            "lq_gate_residual_layernorm_mod_fp8_panels");
-        at::Tensor q2 = at::empty({4 * d / 64, m, 64}, on_gpu(at::kByte));
-        ok(lq_gemm_fp8_codes_panels(P8(q2), PF(ff_linear.in_scale), dt, P8(q1), P8(gelu_proj.w_rows32), PF(gelu_proj.in_scale),
-                                    PF(gelu_proj.w_scale), P(gelu_proj.bias), 1, (int)m, (int)(4 * d), (int)d, cur_stream()),
-           "lq_gemm_fp8_codes_panels");
-        return ff_linear.from_panels_gated(q2, m, msa[5], s, hidden).view({b, s, d});
+        return {q1, hidden};
     }
 };
+// FluxAttnPostFP8Processor::forward of the image and of the text half, their linears two to a launch
+std::vector<at::Tensor> attn_post_pair(const AttnPostFP8& w, const at::Tensor& x, const at::Tensor& attn, const at::Tensor& msa,
+                                       const AttnPostFP8& wc, const at::Tensor& c, const at::Tensor& cattn, const at::Tensor& cmsa) {
+    const auto a = w.gated_norm(x, attn, msa), b = wc.gated_norm(c, cattn, cmsa);
+    const int64_t ma = x.size(0) * x.size(1), mb = c.size(0) * c.size(1), f = w.gelu_proj.n;
+    at::Tensor qa = at::empty({f / 64, ma, 64}, on_gpu(at::kByte)), qb = at::empty({f / 64, mb, 64}, on_gpu(at::kByte));
+    lq_fp8_half_t ha = half_of(w.gelu_proj, a.first, ma), hb = half_of(wc.gelu_proj, b.first, mb);
+    ha.C_fp8 = P8(qa), ha.C_fp8_scale = PF(w.ff_linear.in_scale);
+    hb.C_fp8 = P8(qb), hb.C_fp8_scale = PF(wc.ff_linear.in_scale);
+    gemm_pair(ha, hb, x.scalar_type(), 1, 1, f, w.gelu_proj.k);
+    return gated_pair(w.ff_linear, qa, msa[5], a.second, wc.ff_linear, qb, cmsa[5], b.second, 1);
+}
 
-// FluxAttnPostInt4Processor::forward (FluxAttnPostInt4Processor.cc:103-215)
+// FluxAttnPostInt4Processor (FluxAttnPostInt4Processor.cc:103-215)
 struct AttnPostInt4 {
     W4A4Linear gelu_proj;
     FP8Linear ff_linear;
@@ -308,7 +336,8 @@ struct AttnPostInt4 {
         gelu_proj.load(src, prefix + "net.0.proj.", 4 * dim, dim, true, T);
         ff_linear.load(src, prefix + "net.2", dim, 4 * dim, T);
     }
-    at::Tensor forward(const at::Tensor& x, const at::Tensor& attn, const at::Tensor& msa) const {
+    // everything up to ff_linear: {its input's codes [B*S, 4D], hidden}
+    std::pair<at::Tensor, at::Tensor> activation(const at::Tensor& x, const at::Tensor& attn, const at::Tensor& msa) const {
         const int64_t b = x.size(0), s = x.size(1), d = x.size(2), m = b * s;
         at::Tensor norm = at::empty_like(x), hidden = at::empty_like(x);
         ok(lq_gate_residual_layernorm_mod(P(norm), P(hidden), P(attn), P(msa[2]), P(x), P(msa[4]), P(msa[3]), lq_dt(x.scalar_type()),
@@ -317,9 +346,15 @@ struct AttnPostInt4 {
         at::Tensor q2 = at::empty({m, 4 * d}, on_gpu(at::kByte));
         lq_epilogue_t epi = {2, nullptr, nullptr, 1, nullptr, P8(q2), (size_t)(4 * d), PF(ff_linear.in_scale)};
         gelu_proj.run(norm.view({m, d}), &epi, false);
-        return ff_linear.from_codes_gated(q2, m, msa[5], s, hidden).view({b, s, d});
+        return {q2, hidden};
     }
 };
+// FluxAttnPostInt4Processor::forward of both halves, their FP8 output projections two to a launch
+std::vector<at::Tensor> attn_post_pair(const AttnPostInt4& w, const at::Tensor& x, const at::Tensor& attn, const at::Tensor& msa,
+                                       const AttnPostInt4& wc, const at::Tensor& c, const at::Tensor& cattn, const at::Tensor& cmsa) {
+    const auto a = w.activation(x, attn, msa), b = wc.activation(c, cattn, cmsa);
+    return gated_pair(w.ff_linear, a.first, msa[5], a.second, wc.ff_linear, b.first, cmsa[5], b.second, 0);
+}
 
 void check_input(const at::Tensor& t, const char* name, at::ScalarType T) {  // CHECK_TH_CUDA, CHECK_CONTIGUOUS, th_utils.h:14-33
     TORCH_CHECK(t.is_cuda(), name, " must be a CUDA tensor");
@@ -450,18 +485,18 @@ struct FluxTransformerBlockOp : th::CustomClassHolder {
             qkv = to_qkv4.run(adaln_16(x, msa).view({b * s, d}), nullptr, true).view({b, s, 3 * d});
             cqkv = to_added_qkv4.run(adaln_16(c, cmsa).view({b * sc, d}), nullptr, true).view({b, sc, 3 * d});
         } else {
-            qkv = to_qkv.from_panels(adaln_codes(x, msa, to_qkv.in_scale), b * s, cfg.T).view({b, s, 3 * d});
-            cqkv = to_added_qkv.from_panels(adaln_codes(c, cmsa, to_added_qkv.in_scale), b * sc, cfg.T).view({b, sc, 3 * d});
+            const auto both = linear_pair(to_qkv, adaln_codes(x, msa, to_qkv.in_scale), b * s, to_added_qkv,
+                                          adaln_codes(c, cmsa, to_added_qkv.in_scale), b * sc, cfg.T);
+            qkv = both.first.view({b, s, 3 * d}), cqkv = both.second.view({b, sc, 3 * d});
         }
         at::Tensor o = attention_core(qkv, cqkv, norm_qk, norm_added_qk, rope_emb, cfg.heads);
         at::Tensor attn = o.slice(1, sc, sc + s).contiguous().view({b * s, d}), cattn = o.slice(1, 0, sc).contiguous().view({b * sc, d});
         if (cfg.int4) {
             at::Tensor a_out = to_out4.run(attn, nullptr, true).view({b, s, d}), c_out = to_add_out4.run(cattn, nullptr, true).view({b, sc, d});
-            return {ff4.forward(x, a_out, msa), ff_context4.forward(c, c_out, cmsa)};
+            return attn_post_pair(ff4, x, a_out, msa, ff_context4, c, c_out, cmsa);
         }
-        at::Tensor a_out = to_out.from_panels(to_out.cast_input(attn), b * s, cfg.T).view({b, s, d});
-        at::Tensor c_out = to_add_out.from_panels(to_add_out.cast_input(cattn), b * sc, cfg.T).view({b, sc, d});
-        return {ff.forward(x, a_out, msa), ff_context.forward(c, c_out, cmsa)};
+        const auto out = linear_pair(to_out, to_out.cast_input(attn), b * s, to_add_out, to_add_out.cast_input(cattn), b * sc, cfg.T);
+        return attn_post_pair(ff, x, out.first.view({b, s, d}), msa, ff_context, c, out.second.view({b, sc, d}), cmsa);
     }
 };
 
