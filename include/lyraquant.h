@@ -565,6 +565,11 @@ int lq_rmsnorm_rope(void* out, const void* qkv, const void* context_qkv, const v
                     const void* rope, size_t rope_batch_stride, lq_dtype_t dtype, int batch, int seq, int context_seq,
                     int heads, int head_dim, float eps, lq_stream_t stream);
 
+/* lq_rmsnorm_rope in place on the concatenated tensor: qkv [batch, seq, 3, heads, head_dim], its first context_seq tokens the text.  v
+ * stays where it is; q and k have the bits of lq_rmsnorm_rope. */
+int lq_rmsnorm_rope_inplace(void* qkv, const void* norm_qk, const void* norm_added_qk, const void* rope, size_t rope_batch_stride,
+                            lq_dtype_t dtype, int batch, int seq, int context_seq, int heads, int head_dim, float eps, lq_stream_t stream);
+
 /* Softmax attention without mask: out[b, i, h, :] = sum_j softmax_j(scale * q[b, i, h, :] . k[b, j, h, :]) v[b, j, h, :], fp32
  * scores and accumulation (the flash attention the reference's attention processors call,
  * layers/flux_attention_processor/FluxAttentionFP8Processor.cc:246-291,
@@ -575,6 +580,28 @@ int lq_rmsnorm_rope(void* out, const void* qkv, const void* context_qkv, const v
 int lq_attention(void* out, const void* q, size_t q_row, size_t q_batch, const void* k, size_t k_row, size_t k_batch, const void* v,
                  size_t v_row, size_t v_batch, lq_dtype_t dtype, int batch, int seq_q, int seq_k, int heads, int head_dim, float scale,
                  lq_stream_t stream);
+
+/* lq_attention with the quantisation of its output folded in.  Exactly one kind of output, the others zero:
+ *     out       [batch, seq_q, heads, head_dim] of T, as lq_attention
+ *     out_fp8   e4m3 codes of T(result) / scale as k-panels [heads * head_dim / 64][batch * (seq_q - context)][64], and context_fp8
+ *               [..][batch * context][64] with a scale of its own (lq_fp8_scale_cast_panels of the two parts; same bits)
+ *     out_int8  int8 codes [batch, seq_q, heads, head_dim] of T(result) * int8_pre[channel] (NULL: 1) / int8_scale (lq_sq_input_quant with
+ *               a static scale; same bits) */
+typedef struct {
+    void* out;
+    const void *q, *k, *v;
+    size_t q_row, q_batch, k_row, k_batch, v_row, v_batch;
+    lq_dtype_t dtype;
+    int batch, seq_q, seq_k, heads, head_dim;
+    float scale;
+    int context; /* leading tokens of a batch whose codes go to context_fp8 */
+    uint8_t *out_fp8, *context_fp8;
+    const float *out_fp8_scale, *context_fp8_scale;
+    int8_t* out_int8;
+    const float *int8_pre, *int8_scale;
+} lq_attention_t;
+int lq_attention_ex(const lq_attention_t* args, lq_stream_t stream);
+
 
 /* dst[i] = T( dst[i] + T( src[i] * T(alpha) ) ): merges a full-rank LoRA delta into a 16-bit (or fp32) weight
  * (invokeLoadLora, kernels/lora/load_lora.h + load_lora.cu:6-14,92-96).  An FP8 weight is re-quantised after the

@@ -38,6 +38,12 @@ struct AttnParams {
     int batch, heads, sq, sk;
     int q_blocks;                       // ceil(sq / (32 * NW))
     float scale_log2;                   // softmax scale * log2(e)
+    int context;                        // leading tokens of a batch that have codes of their own (text tokens)
+    // codes in place of `out`: e4m3 as k-panels [heads * DH / 64][rows][64], the context's rows into a tensor of their own; or int8 rows
+    uint8_t *fp8, *fp8_context;
+    const float *fp8_scale, *fp8_context_scale;
+    int8_t* int8;
+    const float *int8_pre, *int8_scale;
 };
 
 typedef __bf16 attn_bf8 __attribute__((ext_vector_type(8)));
@@ -356,12 +362,53 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
             *reinterpret_cast<uint2*>(strip + lr * PITCH + (d * 32 + 8 * q4 + 4 * lh) * 2) =
                 make_uint2(attn_pack<Tag>(o[d][4 * q4] * inv, o[d][4 * q4 + 1] * inv), attn_pack<Tag>(o[d][4 * q4 + 2] * inv, o[d][4 * q4 + 3] * inv));
     const size_t o_row = (size_t)p.heads * DH;
+    // a row of the strip is the output rounded to T; codes are made from that, as the casts behind the attention make them
+    auto strip_row = [&](int r) { return *reinterpret_cast<const uint4*>(strip + r * PITCH + d_ch * 16); };
+    if (p.fp8 != nullptr) {
+        const float inv_rest = 1.0f / p.fp8_scale[0], inv_ctx = p.context > 0 ? 1.0f / p.fp8_context_scale[0] : 0.0f;
+        const size_t panel = (size_t)head * (DH / 64) + d_ch / 8;
+#pragma unroll
+        for (int i = 0; i < 32 / RPD; ++i) {
+            const int r = i * RPD + d_row, token = q0 + r;
+            const bool ctx = token < p.context;
+            const float f = ctx ? inv_ctx : inv_rest;
+            const int rows = ctx ? p.context : p.sq - p.context;
+            float y[8];
+            unpack8<Tag>(strip_row(r), y);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] *= f;
+            uint8_t* dst = (ctx ? p.fp8_context : p.fp8) + (panel * ((size_t)p.batch * rows) + (size_t)b * rows + (ctx ? token : token - p.context)) * 64 + (d_ch % 8) * 8;
+            if (token < p.sq) *reinterpret_cast<uint2*>(dst) = make_uint2(e4m3x4(y[0], y[1], y[2], y[3]), e4m3x4(y[4], y[5], y[6], y[7]));
+        }
+        return;
+    }
+    if (p.int8 != nullptr) {
+        const float sc = p.int8_scale[0], rcp = fast_recip(sc);
+        const bool slow = scale_out_of_range(sc);
+        float pre[8];
+        const float* pp = p.int8_pre + (size_t)head * DH + d_ch * 8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pre[e] = p.int8_pre != nullptr ? pp[e] : 1.0f;
+        int8_t* dst = p.int8 + (size_t)b * p.sq * o_row + (size_t)head * DH + d_ch * 8;
+#pragma unroll
+        for (int i = 0; i < 32 / RPD; ++i) {
+            const int r = i * RPD + d_row;
+            float y[8];
+            unpack8<Tag>(strip_row(r), y);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) y[e] = y[e] * pre[e];
+            int q[8];
+            quant8<-128, 127>(y, sc, rcp, slow, q);
+            if (q0 + r < p.sq)
+                *reinterpret_cast<uint2*>(dst + (size_t)(q0 + r) * o_row) = make_uint2(pack4_s8(q[0], q[1], q[2], q[3]), pack4_s8(q[4], q[5], q[6], q[7]));
+        }
+        return;
+    }
     unsigned short* op = p.out + (size_t)b * p.sq * o_row + (size_t)head * DH;
 #pragma unroll
     for (int i = 0; i < 32 / RPD; ++i) {
         const int r = i * RPD + d_row;
-        const uint4 w = *reinterpret_cast<const uint4*>(strip + r * PITCH + d_ch * 16);
-        if (q0 + r < p.sq) *reinterpret_cast<uint4*>(op + (size_t)(q0 + r) * o_row + d_ch * 8) = w;
+        if (q0 + r < p.sq) *reinterpret_cast<uint4*>(op + (size_t)(q0 + r) * o_row + d_ch * 8) = strip_row(r);
     }
 }
 
@@ -395,31 +442,60 @@ template <typename Tag> static int attention_typed(const AttnParams& p, int head
 
 using namespace lq;
 
+static int attention_entry(const char* what, const lq_attention_t& a, lq_stream_t stream) {
+    LQ_REQUIRE(a.dtype == LQ_F16 || a.dtype == LQ_BF16, LQ_ERR_UNSUPPORTED, "%s: tensors must be F16 or BF16", what);
+    LQ_REQUIRE(a.batch >= 0 && a.heads > 0 && a.seq_q >= 0 && a.seq_k > 0 && (a.head_dim == 64 || a.head_dim == 128), LQ_ERR_SHAPE,
+               "%s: need head_dim 64 or 128 and at least one key (batch=%d heads=%d seq_q=%d seq_k=%d head_dim=%d)", what, a.batch, a.heads,
+               a.seq_q, a.seq_k, a.head_dim);
+    LQ_REQUIRE(a.scale > 0.0f, LQ_ERR_ARG, "%s: the softmax scale must be positive", what);  // the largest score is taken before scaling
+    LQ_REQUIRE(a.context >= 0 && a.context <= a.seq_q, LQ_ERR_SHAPE, "%s: context=%d of %d queries", what, a.context, a.seq_q);
+    if (a.batch == 0 || a.seq_q == 0) return LQ_OK;
+    const int outputs = (a.out != nullptr) + (a.out_fp8 != nullptr || a.context_fp8 != nullptr) + (a.out_int8 != nullptr);
+    LQ_REQUIRE(outputs == 1 && a.q && a.k && a.v, LQ_ERR_ARG, "%s: null pointer", what);
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
+                           reinterpret_cast<uintptr_t>(a.v) | ((a.q_row | a.k_row | a.v_row | a.q_batch | a.k_batch | a.v_batch) * 2);
+    LQ_REQUIRE(bits % 16 == 0, LQ_ERR_ARG, "%s: tensors and their row and batch strides must be multiples of 16 bytes", what);
+    const size_t width = (size_t)a.heads * a.head_dim, longest = a.k_row > a.v_row ? a.k_row : a.v_row;
+    LQ_REQUIRE(a.q_row >= width && a.k_row >= width && a.v_row >= width, LQ_ERR_SHAPE, "%s: a row stride is shorter than heads * head_dim", what);
+    // a lane's offset inside one batch of K or V is 32 bits, a product of two 24-bit numbers
+    LQ_REQUIRE(longest < ((size_t)1 << 23) && a.seq_k < (1 << 24) && (size_t)a.seq_k * longest < ((size_t)1 << 31) &&
+                   (long long)a.batch * a.heads * ((a.seq_q + 127) / 128) <= 0x7fffffffLL,
+               LQ_ERR_SHAPE, "%s: tensors too large (seq_k=%d, row stride %zu)", what, a.seq_k, longest);
+    if (a.out_fp8 != nullptr || a.context_fp8 != nullptr) {
+        LQ_REQUIRE((a.context == a.seq_q || (a.out_fp8 && a.out_fp8_scale)) && (a.context == 0 || (a.context_fp8 && a.context_fp8_scale)), LQ_ERR_ARG,
+                   "%s: codes need a destination and a scale for each part of the tokens", what);
+        LQ_REQUIRE((reinterpret_cast<uintptr_t>(a.out_fp8) | reinterpret_cast<uintptr_t>(a.context_fp8)) % 8 == 0, LQ_ERR_ARG,
+                   "%s: codes must be 8-byte aligned", what);
+    }
+    LQ_REQUIRE(a.out_int8 == nullptr || (a.int8_scale != nullptr && reinterpret_cast<uintptr_t>(a.out_int8) % 8 == 0), LQ_ERR_ARG,
+               "%s: int8 codes need a scale and 8-byte alignment", what);
+    auto us = [](const void* x) { return static_cast<const unsigned short*>(x); };
+    AttnParams p{};
+    p.q = us(a.q); p.k = us(a.k); p.v = us(a.v);
+    p.out = static_cast<unsigned short*>(a.out);
+    p.q_row = a.q_row; p.k_row = a.k_row; p.v_row = a.v_row;
+    p.q_batch = a.q_batch; p.k_batch = a.k_batch; p.v_batch = a.v_batch;
+    p.batch = a.batch; p.heads = a.heads; p.sq = a.seq_q; p.sk = a.seq_k;
+    p.scale_log2 = a.scale * 1.4426950408889634f;
+    p.context = a.context;
+    // the kernel looks at fp8 to know that codes are wanted; tokens of a part that is empty never come up
+    p.fp8 = a.out_fp8 != nullptr ? a.out_fp8 : a.context_fp8;
+    p.fp8_context = a.context_fp8;
+    p.fp8_scale = a.out_fp8_scale != nullptr ? a.out_fp8_scale : a.context_fp8_scale; p.fp8_context_scale = a.context_fp8_scale;
+    p.int8 = a.out_int8; p.int8_pre = a.int8_pre; p.int8_scale = a.int8_scale;
+    return a.dtype == LQ_BF16 ? attention_typed<BF16Tag>(p, a.head_dim, as_stream(stream)) : attention_typed<F16Tag>(p, a.head_dim, as_stream(stream));
+}
+
 extern "C" int lq_attention(void* out, const void* q, size_t q_row, size_t q_batch, const void* k, size_t k_row, size_t k_batch, const void* v,
                             size_t v_row, size_t v_batch, lq_dtype_t dtype, int batch, int seq_q, int seq_k, int heads, int head_dim,
                             float scale, lq_stream_t stream) {
-    LQ_REQUIRE(dtype == LQ_F16 || dtype == LQ_BF16, LQ_ERR_UNSUPPORTED, "lq_attention: tensors must be F16 or BF16");
-    LQ_REQUIRE(batch >= 0 && heads > 0 && seq_q >= 0 && seq_k > 0 && (head_dim == 64 || head_dim == 128), LQ_ERR_SHAPE,
-               "lq_attention: need head_dim 64 or 128 and at least one key (batch=%d heads=%d seq_q=%d seq_k=%d head_dim=%d)", batch, heads,
-               seq_q, seq_k, head_dim);
-    LQ_REQUIRE(scale > 0.0f, LQ_ERR_ARG, "lq_attention: the softmax scale must be positive");  // the largest score is taken before scaling
-    if (batch == 0 || seq_q == 0) return LQ_OK;
-    LQ_REQUIRE(out && q && k && v, LQ_ERR_ARG, "lq_attention: null pointer");
-    const uintptr_t bits = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
-                           reinterpret_cast<uintptr_t>(v) | ((q_row | k_row | v_row | q_batch | k_batch | v_batch) * 2);
-    LQ_REQUIRE(bits % 16 == 0, LQ_ERR_ARG, "lq_attention: tensors and their row and batch strides must be multiples of 16 bytes");
-    const size_t width = (size_t)heads * head_dim, longest = k_row > v_row ? k_row : v_row;
-    LQ_REQUIRE(q_row >= width && k_row >= width && v_row >= width, LQ_ERR_SHAPE, "lq_attention: a row stride is shorter than heads * head_dim");
-    // a lane's offset inside one batch of K or V is 32 bits, a product of two 24-bit numbers
-    LQ_REQUIRE(longest < ((size_t)1 << 23) && seq_k < (1 << 24) && (size_t)seq_k * longest < ((size_t)1 << 31) &&
-                   (long long)batch * heads * ((seq_q + 127) / 128) <= 0x7fffffffLL,
-               LQ_ERR_SHAPE, "lq_attention: tensors too large (seq_k=%d, row stride %zu)", seq_k, longest);
-    AttnParams p{};
-    p.q = static_cast<const unsigned short*>(q); p.k = static_cast<const unsigned short*>(k); p.v = static_cast<const unsigned short*>(v);
-    p.out = static_cast<unsigned short*>(out);
-    p.q_row = q_row; p.k_row = k_row; p.v_row = v_row;
-    p.q_batch = q_batch; p.k_batch = k_batch; p.v_batch = v_batch;
-    p.batch = batch; p.heads = heads; p.sq = seq_q; p.sk = seq_k;
-    p.scale_log2 = scale * 1.4426950408889634f;
-    return dtype == LQ_BF16 ? attention_typed<BF16Tag>(p, head_dim, as_stream(stream)) : attention_typed<F16Tag>(p, head_dim, as_stream(stream));
+    lq_attention_t a = {};
+    a.out = out; a.q = q; a.q_row = q_row; a.q_batch = q_batch; a.k = k; a.k_row = k_row; a.k_batch = k_batch; a.v = v; a.v_row = v_row; a.v_batch = v_batch;
+    a.dtype = dtype; a.batch = batch; a.seq_q = seq_q; a.seq_k = seq_k; a.heads = heads; a.head_dim = head_dim; a.scale = scale;
+    return attention_entry("lq_attention", a, stream);
+}
+
+extern "C" int lq_attention_ex(const lq_attention_t* a, lq_stream_t stream) {
+    LQ_REQUIRE(a, LQ_ERR_ARG, "lq_attention_ex: null pointer");
+    return attention_entry("lq_attention_ex", *a, stream);
 }

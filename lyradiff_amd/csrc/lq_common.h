@@ -366,6 +366,47 @@ __device__ __forceinline__ float gelu_fast(float x) {
     return x * __builtin_amdgcn_rcpf(1.0f + e);            // x, resp. -0
 }
 
+// RMSNorm and rotary embedding of one rotation pair, every product and sum rounded to T as the reference's T arithmetic does
+// (kernels/rope/flux_apply_rope.cu:74-156): n = T(x * inv) * w, then the 2x2 matrix of words r0 = (r00, r01), r1 = (r10, r11).
+// x: the pair as floats, w: its two norm weights as a word; returns the rotated pair as a word.
+template <typename Tag> __device__ __forceinline__ u32 norm_rope_pair(float x0, float x1, float inv, u32 w, u32 r0, u32 r1) {
+    float n0 = x0 * inv, n1 = x1 * inv;
+    round_through2<Tag>(n0, n1);
+    n0 = n0 * Elem<Tag>::load(w & 0xFFFFu);
+    n1 = n1 * Elem<Tag>::load(w >> 16);
+    round_through2<Tag>(n0, n1);
+    float a0 = n0 * Elem<Tag>::load(r0 & 0xFFFFu), a1 = n1 * Elem<Tag>::load(r0 >> 16);
+    float c0 = n0 * Elem<Tag>::load(r1 & 0xFFFFu), c1 = n1 * Elem<Tag>::load(r1 >> 16);
+    round_through2<Tag>(a0, a1);
+    round_through2<Tag>(c0, c1);
+    float y0 = a0 + a1, y1 = c0 + c1;
+    asm volatile("" : "+v"(y0), "+v"(y1));  // the sums are rounded to fp32 before the conversion to T
+    return Elem<Tag>::store(y0) | (Elem<Tag>::store(y1) << 16);
+}
+
+// saturate-to-finite RNE conversion of two floats into the low or high half of a dword
+// (finite inputs and infinities; NaN lanes are patched by the caller)
+__device__ __forceinline__ u32 cvt2_e4m3(float a, float b, u32 old, bool hi) {
+    float ca = __builtin_amdgcn_fmed3f(a, 448.0f, -448.0f);
+    float cb = __builtin_amdgcn_fmed3f(b, 448.0f, -448.0f);
+    return hi ? (u32)__builtin_amdgcn_cvt_pk_fp8_f32(ca, cb, (int)old, true)
+              : (u32)__builtin_amdgcn_cvt_pk_fp8_f32(ca, cb, (int)old, false);
+}
+__device__ __forceinline__ u32 nan_code(float v) { return 0x7Fu | ((__float_as_uint(v) >> 24) & 0x80u); }
+// four floats -> four e4m3 codes; NaN -> 0x7F with the sign of the NaN (rare: one unordered
+// compare per pair decides whether the patch-up path runs at all)
+__device__ __forceinline__ u32 e4m3x4(float a, float b, float c, float d) {
+    u32 w = cvt2_e4m3(a, b, 0u, false);
+    w = cvt2_e4m3(c, d, w, true);
+    if (__builtin_expect(__builtin_isunordered(a, b) || __builtin_isunordered(c, d), 0)) {
+        if (a != a) w = (w & 0xFFFFFF00u) | nan_code(a);
+        if (b != b) w = (w & 0xFFFF00FFu) | (nan_code(b) << 8);
+        if (c != c) w = (w & 0xFF00FFFFu) | (nan_code(c) << 16);
+        if (d != d) w = (w & 0x00FFFFFFu) | (nan_code(d) << 24);
+    }
+    return w;
+}
+
 static inline hipStream_t as_stream(lq_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 }  // namespace lq

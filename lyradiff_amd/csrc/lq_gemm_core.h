@@ -172,17 +172,6 @@ template <typename OutTag> __device__ __forceinline__ void publish_out_max(float
     }
 }
 
-// Four floats -> four e4m3 codes, round-to-nearest-even, saturating to +-448, NaN -> 0x7F | sign (the cast kernel's rule).
-__device__ __forceinline__ u32 e4m3x4(float a, float b, float c, float d) {
-    const float v[4] = {a, b, c, d};
-    u32 w = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(a, 448.0f, -448.0f), __builtin_amdgcn_fmed3f(b, 448.0f, -448.0f), 0, false);
-    w = (u32)__builtin_amdgcn_cvt_pk_fp8_f32(__builtin_amdgcn_fmed3f(c, 448.0f, -448.0f), __builtin_amdgcn_fmed3f(d, 448.0f, -448.0f), (int)w, true);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (v[i] != v[i]) w = (w & ~(0xFFu << (8 * i))) | ((0x7Fu | ((__float_as_uint(v[i]) >> 24) & 0x80u)) << (8 * i));
-    return w;
-}
-
 // One 16-byte-per-lane global -> LDS transfer without passing through registers: lane l of the
 // wavefront fetches 16 bytes at gbase + voff and the hardware writes them to LDS byte address
 // lds_addr + 16*l (lds_addr is wavefront-uniform, carried in M0).  Issued as inline assembly

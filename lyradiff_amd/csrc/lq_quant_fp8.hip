@@ -75,29 +75,7 @@ template <int E, int KC = 1> struct PanelWalk {  // blocks of RB rows x KC 64-el
     __device__ __forceinline__ size_t dst_byte(const PanelMap& pm) const { return ((size_t)(kc + sub) * pm.rows + row()) * 64 + part * E; }
 };
 
-// saturate-to-finite RNE conversion of two floats into the low or high half of a dword
-// (finite inputs and infinities; NaN lanes are patched by the caller)
-__device__ __forceinline__ u32 cvt2_e4m3(float a, float b, u32 old, bool hi) {
-    float ca = __builtin_amdgcn_fmed3f(a, 448.0f, -448.0f);
-    float cb = __builtin_amdgcn_fmed3f(b, 448.0f, -448.0f);
-    return hi ? (u32)__builtin_amdgcn_cvt_pk_fp8_f32(ca, cb, (int)old, true)
-              : (u32)__builtin_amdgcn_cvt_pk_fp8_f32(ca, cb, (int)old, false);
-}
-__device__ __forceinline__ u32 nan_code(float v) { return 0x7Fu | ((__float_as_uint(v) >> 24) & 0x80u); }
-// four floats -> four e4m3 codes; NaN -> 0x7F with the sign of the NaN (rare: one unordered
-// compare per pair decides whether the patch-up path runs at all)
-__device__ __forceinline__ u32 cvt4_e4m3(float a, float b, float c, float d) {
-    u32 w = cvt2_e4m3(a, b, 0u, false);
-    w = cvt2_e4m3(c, d, w, true);
-    if (__builtin_expect(__builtin_isunordered(a, b) || __builtin_isunordered(c, d), 0)) {
-        if (a != a) w = (w & 0xFFFFFF00u) | nan_code(a);
-        if (b != b) w = (w & 0xFFFF00FFu) | (nan_code(b) << 8);
-        if (c != c) w = (w & 0xFF00FFFFu) | (nan_code(c) << 16);
-        if (d != d) w = (w & 0x00FFFFFFu) | (nan_code(d) << 24);
-    }
-    return w;
-}
-__device__ __forceinline__ u32 cvt1_e4m3(float a) { return cvt4_e4m3(a, 0.0f, 0.0f, 0.0f) & 0xFFu; }
+__device__ __forceinline__ u32 cvt1_e4m3(float a) { return e4m3x4(a, 0.0f, 0.0f, 0.0f) & 0xFFu; }
 
 // Non-negative floats order like their bit patterns, so an integer atomic max works.  Thousands of
 // same-address atomics serialise in L2, so a workgroup first looks at the current value and only
@@ -148,7 +126,7 @@ __global__ __launch_bounds__(256) void fp8_cast_kernel(uint8_t* __restrict__ dst
         u32 w[4];
 #pragma unroll
         for (int i = 0; i < E / 4; ++i)
-            w[i] = cvt4_e4m3(v[4 * i] * r, v[4 * i + 1] * r, v[4 * i + 2] * r, v[4 * i + 3] * r);
+            w[i] = e4m3x4(v[4 * i] * r, v[4 * i + 1] * r, v[4 * i + 2] * r, v[4 * i + 3] * r);
         if constexpr (E == 16) *reinterpret_cast<uint4*>(o) = make_uint4(w[0], w[1], w[2], w[3]);
         else *reinterpret_cast<uint2*>(o) = make_uint2(w[0], w[1]);
     };
@@ -214,7 +192,7 @@ __global__ __launch_bounds__(256) void fp8_gelu_cast_kernel(uint8_t* __restrict_
         u32 w[4];
 #pragma unroll
         for (int i = 0; i < E / 4; ++i)
-            w[i] = cvt4_e4m3(v[4 * i] * r, v[4 * i + 1] * r, v[4 * i + 2] * r, v[4 * i + 3] * r);
+            w[i] = e4m3x4(v[4 * i] * r, v[4 * i + 1] * r, v[4 * i + 2] * r, v[4 * i + 3] * r);
         if constexpr (E == 16) *reinterpret_cast<uint4*>(o) = make_uint4(w[0], w[1], w[2], w[3]);
         else *reinterpret_cast<uint2*>(o) = make_uint2(w[0], w[1]);
     };
@@ -257,7 +235,7 @@ __global__ __launch_bounds__(256) void fp8_cast_2d_kernel(uint8_t* __restrict__ 
         u32 w[4];
 #pragma unroll
         for (int i = 0; i < E / 4; ++i)
-            w[i] = cvt4_e4m3(v[4 * i] * r, v[4 * i + 1] * r, v[4 * i + 2] * r, v[4 * i + 3] * r);
+            w[i] = e4m3x4(v[4 * i] * r, v[4 * i + 1] * r, v[4 * i + 2] * r, v[4 * i + 3] * r);
         uint8_t* o = dst + row * dst_ld + cc * E;
         if constexpr (E == 16) *reinterpret_cast<uint4*>(o) = make_uint4(w[0], w[1], w[2], w[3]);
         else *reinterpret_cast<uint2*>(o) = make_uint2(w[0], w[1]);
@@ -569,9 +547,9 @@ __global__ __launch_bounds__(kCoopThreads) void fp8_amax_cast_coop_kernel(uint8_
         float f[8];
         if constexpr (E2 == 8) unpack8<Tag>(v, f);
         else { f[0] = __uint_as_float(v.x); f[1] = __uint_as_float(v.y); f[2] = __uint_as_float(v.z); f[3] = __uint_as_float(v.w); }
-        const u32 w0 = cvt4_e4m3(f[0] * r, f[1] * r, f[2] * r, f[3] * r);
+        const u32 w0 = e4m3x4(f[0] * r, f[1] * r, f[2] * r, f[3] * r);
         if constexpr (E2 == 8) {
-            const u32x2_t w = {w0, cvt4_e4m3(f[4] * r, f[5] * r, f[6] * r, f[7] * r)};
+            const u32x2_t w = {w0, e4m3x4(f[4] * r, f[5] * r, f[6] * r, f[7] * r)};
             if (stream_out) __builtin_nontemporal_store(w, reinterpret_cast<u32x2_t*>(o));
             else *reinterpret_cast<u32x2_t*>(o) = w;
         } else {

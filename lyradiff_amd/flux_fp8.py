@@ -178,16 +178,23 @@ def flux_single_mlp_fp8(x: torch.Tensor, norm_hidden, attn_output: torch.Tensor,
     q1 = norm_hidden if norm_hidden.dtype == torch.uint8 else ops.fp8_scale_cast_panels(norm_hidden.view(m, d), w.proj_mlp.input_scale)
     q2 = torch.empty(((d + f) // 64, m, 64), dtype=torch.uint8, device=x.device)
     ops.fp8_scale_cast_panels(attn_output.view(m, d), w.proj_out.input_scale, out=q2, col_offset=0)
+    return _single_tail(x, q1, q2, gate, w)
+
+
+def _single_tail(x, q1, q2, gate, w: FluxSingleMlpFP8Weights) -> torch.Tensor:
+    """proj_mlp and proj_out: q1 the codes for proj_mlp, q2 those for proj_out whose first D columns (the attention output) are there."""
+    b, s, d = x.shape
     ops.fp8_linear_codes_panels(q1, w.proj_mlp.weight_rows32, w.proj_mlp.input_scale, w.proj_mlp.weight_scale,
                                 w.proj_mlp.bias, w.proj_out.input_scale, gelu=2, round_dtype=x.dtype, out=q2, col_offset=d)
     out = ops.fp8_linear_gated_panels(q2, w.proj_out.weight_rows32, w.proj_out.input_scale, w.proj_out.weight_scale,
-                                      w.proj_out.bias, gate, x.view(m, d), rows_per_gate=s)
+                                      w.proj_out.bias, gate, x.view(b * s, d), rows_per_gate=s)
     return out.view(b, s, d)
 
 
 # ---- whole blocks around a caller-supplied attention --------------------------------------------------------------------
 # Everything the reference's FP8 blocks run through a quantized linear is here; `attention` is the caller's function
-# for the part in between (q/k RMSNorm, rotary embedding, scaled-dot-product attention), which is not quantized.
+# for the part in between (q/k RMSNorm, rotary embedding, scaled-dot-product attention), which is not quantized.  The block ops pass a
+# `core` instead (flux_ops.AttentionCore): this library's kernels for that part, whose output leaves the attention as codes.
 
 @dataclass
 class FluxSingleBlockFP8Weights:
@@ -236,24 +243,35 @@ def _linear_from_panels(lin: FP8Linear, panels: torch.Tensor, batch: int, dtype)
     return y.view(batch, y.shape[0] // batch, y.shape[1])
 
 
-def flux_single_block_fp8(x: torch.Tensor, temb: torch.Tensor, w: FluxSingleBlockFP8Weights, attention) -> torch.Tensor:
+def flux_single_block_fp8(x: torch.Tensor, temb: torch.Tensor, w: FluxSingleBlockFP8Weights, attention=None, core=None) -> torch.Tensor:
     """FluxSingleTransformerFP8Block<T>::forward (FluxSingleTransformerFP8Block.cc:163-291).  x [B, S, D], temb [B, D]
     (SiLU already applied); attention(qkv [B, S, 3D]) -> [B, S, D].  One adaLN read yields the codes for to_qkv and for
-    proj_mlp; five launches besides the attention."""
+    proj_mlp; five launches besides the attention, four with a core."""
+    b, s, d = x.shape
     (c_qkv, c_mlp), msa = ada_fp8_layernorm(x, temb, w.norm, 3, (w.to_qkv.input_scale, w.mlp.proj_mlp.input_scale), panels=True)
-    attn_out = attention(_linear_from_panels(w.to_qkv, c_qkv, x.shape[0], x.dtype))
-    return flux_single_mlp_fp8(x, c_mlp, attn_out.contiguous(), msa[2].contiguous(), w.mlp, norm_in_panels=True)
+    qkv = _linear_from_panels(w.to_qkv, c_qkv, b, x.dtype)
+    gate = msa[2].contiguous()
+    if core is None:
+        return flux_single_mlp_fp8(x, c_mlp, attention(qkv).contiguous(), gate, w.mlp, norm_in_panels=True)
+    q2 = torch.empty((w.mlp.proj_out.weight_rows32.shape[1] // 64, b * s, 64), dtype=torch.uint8, device=x.device)
+    core.codes(core.rotate(qkv), w.mlp.proj_out.input_scale, out=q2[: d // 64])
+    return _single_tail(x, c_mlp, q2, gate, w.mlp)
 
 
-def flux_double_block_fp8(x: torch.Tensor, context: torch.Tensor, temb: torch.Tensor, w: FluxDoubleBlockFP8Weights, attention):
+def flux_double_block_fp8(x: torch.Tensor, context: torch.Tensor, temb: torch.Tensor, w: FluxDoubleBlockFP8Weights, attention=None, core=None):
     """FluxTransformerFP8Block<T>::forward (FluxTransformerFP8Block.cc:159-262) with FluxAttentionFP8Processor
     (FluxAttentionFP8Processor.cc:165-360).  attention(qkv [B, S, 3D], context_qkv [B, Sc, 3D]) -> (attn [B, S, D],
     context_attn [B, Sc, D]).  Returns (output, context_output)."""
     c, msa = ada_fp8_layernorm(x, temb, w.norm1, 6, (w.to_qkv.input_scale,), panels=True)
     cc, cmsa = ada_fp8_layernorm(context, temb, w.norm1_context, 6, (w.to_added_qkv.input_scale,), panels=True)
-    qkv, cqkv = ops.fp8_linear_pair(fp8_half(w.to_qkv, c), fp8_half(w.to_added_qkv, cc), x.dtype)
-    attn, cattn = attention(qkv.view(*x.shape[:2], -1), cqkv.view(*context.shape[:2], -1))
-    rows = lambda t: t.contiguous().view(-1, t.shape[-1])
-    a_out, c_out = ops.fp8_linear_pair(fp8_half(w.to_out, ops.fp8_scale_cast_panels(rows(attn), w.to_out.input_scale)),
-                                       fp8_half(w.to_add_out, ops.fp8_scale_cast_panels(rows(cattn), w.to_add_out.input_scale)), x.dtype)
+    parts = core.joint_qkv(x, context) if core is not None else None  # both halves side by side, where the batch lets them
+    qkv, cqkv = ops.fp8_linear_pair(fp8_half(w.to_qkv, c, out=parts and parts[0]), fp8_half(w.to_added_qkv, cc, out=parts and parts[1]), x.dtype)
+    if core is not None:
+        cat = core.rotate(parts[2], context.shape[1]) if parts else core.rotate_two(qkv.view(*x.shape[:2], -1), cqkv.view(*context.shape[:2], -1))
+        q, cq = core.codes(cat, w.to_out.input_scale, context.shape[1], w.to_add_out.input_scale)
+    else:
+        attn, cattn = attention(qkv.view(*x.shape[:2], -1), cqkv.view(*context.shape[:2], -1))
+        q, cq = (ops.fp8_scale_cast_panels(t.contiguous().view(-1, t.shape[-1]), lin.input_scale)
+                 for t, lin in ((attn, w.to_out), (cattn, w.to_add_out)))
+    a_out, c_out = ops.fp8_linear_pair(fp8_half(w.to_out, q), fp8_half(w.to_add_out, cq), x.dtype)
     return flux_attn_post_fp8_pair(x, a_out.view(x.shape), msa, w.ff, context, c_out.view(context.shape), cmsa, w.ff_context)

@@ -153,27 +153,35 @@ def load_flux_double_block_int4(src, prefix: str, dim: int, full: bool = True, d
                                       load_flux_attn_post_int4(src, prefix + "ff_context.", dim, dtype, device, lora_rank))
 
 
-def _w4a4_3d(lin: W4A4Linear, x: torch.Tensor) -> torch.Tensor:
-    y = lin.run(x.reshape(-1, x.shape[-1]))
+def _w4a4_3d(lin: W4A4Linear, x: torch.Tensor, out=None) -> torch.Tensor:
+    y = lin.run(x.reshape(-1, x.shape[-1]), out=out)
     return y.view(*x.shape[:-1], y.shape[-1])
 
 
-def flux_single_block_int4(x: torch.Tensor, temb: torch.Tensor, w: FluxSingleBlockInt4Weights, attention) -> torch.Tensor:
+def flux_single_block_int4(x: torch.Tensor, temb: torch.Tensor, w: FluxSingleBlockInt4Weights, attention=None, core=None) -> torch.Tensor:
     """FluxSingleTransformerInt4Block<T>::forward (FluxSingleTransformerInt4Block.cc:178-316): adaLN, W4A4 QKV projection
-    (its bias added in the GEMM epilogue; the reference adds it in a pass of its own), attention(qkv [B, S, 3D]) -> [B, S, D],
-    then the feed-forward tail."""
+    (its bias added in the GEMM epilogue; the reference adds it in a pass of its own), attention(qkv [B, S, 3D]) -> [B, S, D]
+    (or the block ops' core, flux_ops.AttentionCore), then the feed-forward tail."""
     norm, msa = ada_layernorm_int4(x, temb, w.norm, 3)
-    attn_out = attention(_w4a4_3d(w.to_qkv, norm))
+    qkv = _w4a4_3d(w.to_qkv, norm)
+    attn_out = attention(qkv) if core is None else core.output(core.rotate(qkv))
     return flux_single_mlp_int4(x, norm, attn_out.contiguous(), msa[2].contiguous(), w.mlp)
 
 
-def flux_double_block_int4(x: torch.Tensor, context: torch.Tensor, temb: torch.Tensor, w: FluxDoubleBlockInt4Weights, attention):
+def flux_double_block_int4(x: torch.Tensor, context: torch.Tensor, temb: torch.Tensor, w: FluxDoubleBlockInt4Weights, attention=None, core=None):
     """FluxTransformerInt4Block<T>::forward (FluxTransformerInt4Block.cc:159-246) with FluxAttentionInt4Processor
     (FluxAttentionInt4Processor.cc:206-331).  attention(qkv, context_qkv) -> (attn [B, S, D], context_attn [B, Sc, D]).
     Returns (output, context_output)."""
     n, msa = ada_layernorm_int4(x, temb, w.norm1, 6)
     nc, cmsa = ada_layernorm_int4(context, temb, w.norm1_context, 6)
-    attn, cattn = attention(_w4a4_3d(w.to_qkv, n), _w4a4_3d(w.to_added_qkv, nc))
+    parts = core.joint_qkv(x, context) if core is not None else None
+    qkv, cqkv = _w4a4_3d(w.to_qkv, n, parts and parts[0]), _w4a4_3d(w.to_added_qkv, nc, parts and parts[1])
+    if core is None:
+        attn, cattn = attention(qkv, cqkv)
+    else:
+        sc = context.shape[1]
+        o = core.output(core.rotate(parts[2], sc) if parts else core.rotate_two(qkv, cqkv))
+        attn, cattn = o[:, sc:], o[:, :sc]
     a_out = _w4a4_3d(w.to_out, attn.contiguous())
     c_out = _w4a4_3d(w.to_add_out, cattn.contiguous())
     return flux_attn_post_int4_pair(x, a_out, msa, w.ff, context, c_out, cmsa, w.ff_context)

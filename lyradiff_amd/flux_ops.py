@@ -49,20 +49,53 @@ def flux_attention_core(qkv: torch.Tensor, norm_q: torch.Tensor, norm_k: torch.T
     projections: q/k RMSNorm per head, rotary embedding and the [text, image] concatenation in one HIP kernel
     (ops.rmsnorm_rope = invokeFusedRmsNormCatAndRope), then softmax attention on its [B, S, 3, H, Dh] output.
     With `context_qkv` (image [B, S, D], text [B, Sc, D]) is returned; without it a single [B, S, D] tensor."""
-    added = None if context_qkv is None else torch.cat([norm_added_q, norm_added_k])
-    return _attention_core(qkv, torch.cat([norm_q, norm_k]), rope_emb, heads, context_qkv, added)
-
-
-def _attention_core(qkv, norm_qk, rope_emb, heads, context_qkv=None, norm_added_qk=None):
-    """flux_attention_core with the norm weights as [2 * Dh] (q then k), as the block classes keep them."""
-    b, s, d3 = qkv.shape
-    sc = 0 if context_qkv is None else context_qkv.shape[1]
-    cat = ops.rmsnorm_rope(qkv.contiguous(), norm_qk, rope_emb.contiguous(), heads,
-                           None if context_qkv is None else context_qkv.contiguous(), norm_added_qk)
-    o = ops.softmax_attention(cat[:, :, 0], cat[:, :, 1], cat[:, :, 2]).reshape(b, sc + s, d3 // 3)
+    core = AttentionCore(torch.cat([norm_q, norm_k]), rope_emb, heads, None if context_qkv is None else torch.cat([norm_added_q, norm_added_k]))
+    o = core.output(core.rotate_two(qkv, context_qkv))
     if context_qkv is None:
         return o
+    sc = context_qkv.shape[1]
     return o[:, sc:], o[:, :sc]
+
+
+class AttentionCore:
+    """The part between the QKV and the output projections of one forward pass; norm weights as [2 * Dh] (q then k)."""
+
+    def __init__(self, norm_qk: torch.Tensor, rope_emb: torch.Tensor, heads: int, norm_added_qk: Optional[torch.Tensor] = None):
+        self.norm_qk, self.rope, self.heads, self.norm_added_qk = norm_qk, rope_emb.contiguous(), heads, norm_added_qk
+
+    def joint_qkv(self, x: torch.Tensor, context: torch.Tensor):
+        """Views for the image and the text half's QKV [S, 3D] and [Sc, 3D], and the tensor [1, Sc + S, 3D] they are parts of, so that
+        nothing has to be concatenated; None for a batch of several, whose halves are not contiguous there."""
+        if x.shape[0] != 1:
+            return None
+        sc = context.shape[1]
+        both = torch.empty((1, sc + x.shape[1], 3 * x.shape[2]), dtype=x.dtype, device=x.device)
+        return both[0, sc:], both[0, :sc], both
+
+    def rotate(self, qkv: torch.Tensor, context: int = 0) -> torch.Tensor:
+        """q/k RMSNorm and rotary embedding in place: qkv [B, S, 3D], text first -> [B, S, 3, H, Dh]."""
+        return ops.rmsnorm_rope_inplace(qkv, self.norm_qk, self.rope, self.heads, context, self.norm_added_qk)
+
+    def rotate_two(self, qkv: torch.Tensor, context_qkv: Optional[torch.Tensor]) -> torch.Tensor:
+        """The same with the concatenation [text, image] into a new tensor."""
+        return ops.rmsnorm_rope(qkv.contiguous(), self.norm_qk, self.rope, self.heads, None if context_qkv is None else context_qkv.contiguous(),
+                                self.norm_added_qk)
+
+    def output(self, cat: torch.Tensor) -> torch.Tensor:
+        """Softmax attention: [B, S, 3, H, Dh] -> [B, S, D]."""
+        return ops.softmax_attention(cat[:, :, 0], cat[:, :, 1], cat[:, :, 2]).reshape(cat.shape[0], cat.shape[1], -1)
+
+    def codes(self, cat: torch.Tensor, scale: torch.Tensor, context: int = 0, context_scale: Optional[torch.Tensor] = None, out=None):
+        """The attention's output as e4m3 codes in k-panels; with a context_scale those of the text tokens behind them."""
+        q, k, v = cat[:, :, 0], cat[:, :, 1], cat[:, :, 2]
+        if ops.attention_supported(q, k, v):
+            return ops.attention_codes(q, k, v, None, context, scale, context_scale, out)
+        o = self.output(cat)
+        rows = lambda t: t.reshape(-1, t.shape[-1])
+        if out is not None:
+            return ops.fp8_scale_cast_panels(rows(o), scale, out=out)
+        main = ops.fp8_scale_cast_panels(rows(o[:, context:]), scale)
+        return main if context_scale is None else (main, ops.fp8_scale_cast_panels(rows(o[:, :context]), context_scale))
 
 
 class _BlockOpBase:
@@ -172,9 +205,9 @@ class FluxTransformerBlockOp(_BlockOpBase):
         for n, t in (("hidden_states", hidden_states), ("encoder_hidden_states", encoder_hidden_states),
                      ("rope_emb", rope_emb), ("temb_emb", temb_emb)):
             self._check(n, t)
-        core = lambda qkv, cqkv: _attention_core(qkv, self.norm_qk, rope_emb, self.heads, cqkv, self.norm_added_qk)
+        core = AttentionCore(self.norm_qk, rope_emb, self.heads, self.norm_added_qk)
         block = I4.flux_double_block_int4 if self.int4 else F.flux_double_block_fp8
-        out, ctx = block(hidden_states, encoder_hidden_states, temb_emb, w, core)
+        out, ctx = block(hidden_states, encoder_hidden_states, temb_emb, w, core=core)
         return [out, ctx]
 
 
@@ -212,4 +245,4 @@ class FluxSingleTransformerBlockOp(_BlockOpBase):
         for n, t in (("hidden_states", hidden_states), ("rope_emb", rope_emb), ("temb_emb", temb_emb)):
             self._check(n, t)
         block = I4.flux_single_block_int4 if self.int4 else F.flux_single_block_fp8
-        return block(hidden_states, temb_emb, w, lambda qkv: _attention_core(qkv, self.norm_qk, rope_emb, self.heads))
+        return block(hidden_states, temb_emb, w, core=AttentionCore(self.norm_qk, rope_emb, self.heads))

@@ -117,6 +117,8 @@ SYMBOLS = {
     "lq_w4a4_quantize_lora_down": (_I, [_P, _P, _I, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _P]),
     "lq_rmsnorm_rope": (_I, [_P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _F, _P]),
     "lq_attention": (_I, [_P, _P, _Z, _Z, _P, _Z, _Z, _P, _Z, _Z, _I, _I, _I, _I, _I, _I, _F, _P]),
+    "lq_attention_ex": (_I, [_P, _P]),
+    "lq_rmsnorm_rope_inplace": (_I, [_P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _F, _P]),
     "lq_cast_f32": (_I, [_P, _I, _P, _Z, _P]),
     "lq_load_lora": (_I, [_P, _P, _I, _Z, _F, _P]),
     "lq_gemm_set_tactic": (_I, [_I, _I]),
@@ -139,6 +141,14 @@ class Fp8Half(C.Structure):
     """lq_fp8_half_t of include/lyraquant.h."""
     _fields_ = [("C", _P), ("A", _P), ("B_rows32", _P), ("a_scale", _P), ("b_scale", _P), ("bias", _P), ("C_fp8", _P), ("C_fp8_scale", _P),
                 ("gate", _P), ("rows_per_gate", _Z), ("residual", _P), ("m", _I)]
+
+
+class Attention(C.Structure):
+    """lq_attention_t of include/lyraquant.h."""
+    _fields_ = [("out", _P), ("q", _P), ("k", _P), ("v", _P), ("q_row", _Z), ("q_batch", _Z), ("k_row", _Z), ("k_batch", _Z), ("v_row", _Z),
+                ("v_batch", _Z), ("dtype", _I), ("batch", _I), ("seq_q", _I), ("seq_k", _I), ("heads", _I), ("head_dim", _I), ("scale", _F),
+                ("context", _I), ("out_fp8", _P),
+                ("context_fp8", _P), ("out_fp8_scale", _P), ("context_fp8_scale", _P), ("out_int8", _P), ("int8_pre", _P), ("int8_scale", _P)]
 
 
 class Epilogue(C.Structure):

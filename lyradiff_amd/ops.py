@@ -761,6 +761,7 @@ class FP8Half(NamedTuple):
     gate: Optional[torch.Tensor] = None
     residual: Optional[torch.Tensor] = None
     rows_per_gate: int = 0
+    out: Optional[torch.Tensor] = None  # where a 16-bit output goes
 
 
 def fp8_linear_pair(first: FP8Half, second: FP8Half, dtype, gelu: int = 0, panels: bool = True):
@@ -792,7 +793,9 @@ def fp8_linear_pair(first: FP8Half, second: FP8Half, dtype, gelu: int = 0, panel
                                    h.gate.numel() != ((m + h.rows_per_gate - 1) // h.rows_per_gate) * n):
             raise ValueError("residual must be [M,N] and gate [ceil(M/rows_per_gate), N]")
         if h.out_fp8_scale is None:
-            out = torch.empty((m, n), dtype=dtype, device=h.codes.device)
+            out = torch.empty((m, n), dtype=dtype, device=h.codes.device) if h.out is None else _chk(h.out, "out", (dtype,))
+            if out.numel() != m * n:
+                raise ValueError("out must be [M, N]")
             a.C = out.data_ptr()
         else:
             out = torch.empty((n // 64, m, 64) if panels else (m, n), dtype=torch.uint8, device=h.codes.device)
@@ -1110,6 +1113,78 @@ def attention(q, k, v, scale=None):
     out = torch.empty((b, sq, h, dh), dtype=q.dtype, device=q.device)
     _l.check(_l.load().lq_attention(_ptr(out), _ptr(q), q.stride(1), batch(q), _ptr(k), k.stride(1), batch(k), _ptr(v), v.stride(1), batch(v),
                                     _DT[q.dtype], b, sq, sk, h, dh, float(dh ** -0.5 if scale is None else scale), _stream()), "lq_attention")
+    return out
+
+
+def rmsnorm_rope_inplace(qkv, norm_qk, rope, heads: int, context: int = 0, norm_added_qk=None, eps: float = 1e-6):
+    """rmsnorm_rope in place on the concatenated qkv [B, S, 3*H*Dh], its first `context` tokens the text: q and k as there, v untouched.
+    Returns qkv as [B, S, 3, H, Dh]."""
+    _chk(qkv, "qkv", (torch.float16, torch.bfloat16))
+    b, s, d3 = qkv.shape
+    if d3 % (3 * heads):
+        raise ValueError("the last dimension of qkv must be 3 * heads * head_dim")
+    dh = d3 // (3 * heads)
+    for name, t in (("norm_qk", norm_qk), ("rope", rope), ("norm_added_qk", norm_added_qk)):
+        if t is not None:
+            _chk(t, name, (qkv.dtype,))
+    if norm_qk.numel() != 2 * dh or (norm_added_qk is not None and norm_added_qk.numel() != 2 * dh):
+        raise ValueError("norm weights must hold 2 * head_dim elements (q then k)")
+    if not 0 <= context <= s or (context > 0 and norm_added_qk is None):
+        raise ValueError("context must lie within the tokens and needs norm_added_qk")
+    per_batch = s * dh * 2
+    if rope.numel() not in (per_batch, b * per_batch):
+        raise ValueError("rope must be [B or 1, S, head_dim / 2, 2, 2]")
+    _l.check(_l.load().lq_rmsnorm_rope_inplace(_ptr(qkv), _ptr(norm_qk), _ptr(norm_added_qk), _ptr(rope), per_batch if rope.numel() != per_batch else 0,
+                                               _DT[qkv.dtype], b, s, context, heads, dh, eps, _stream()), "lq_rmsnorm_rope_inplace")
+    return qkv.view(b, s, 3, heads, dh)
+
+
+def attention_codes(q, k, v, scale=None, context: int = 0, fp8_scale=None, context_fp8_scale=None, fp8_out=None, int8_scale=None,
+                    int8_pre=None):
+    """attention whose result, rounded to the type of q, is quantised on the way out.  One of
+      fp8_scale, context_fp8_scale e4m3 codes as k-panels: [H*Dh/64, B*(Sq - context), 64] (written to fp8_out if given), and with a
+                                   context_fp8_scale a pair with [H*Dh/64, B*context, 64], the first tokens of a batch, behind it
+      int8_scale, int8_pre [H*Dh]  int8 codes [B, Sq, H*Dh] of a static scale
+    Same bits as fp8_scale_cast_panels or sq_quant of the result."""
+    if k.shape != v.shape or k.shape[0] != q.shape[0] or k.shape[2:] != q.shape[2:]:
+        raise ValueError("attention: q must be [B, Sq, H, Dh], k and v [B, Sk, H, Dh]")
+    if not attention_supported(q, k, v):
+        raise ValueError("attention: needs fp16 / bf16 device tensors of 64- or 128-wide heads, dense within a token, 16-byte aligned")
+    b, sq, h, dh = q.shape
+    if not 0 <= context <= sq:
+        raise ValueError("context must lie within the queries")
+    if (fp8_scale is None) == (int8_scale is None):
+        raise ValueError("one of fp8_scale and int8_scale")
+    for name, t, n, dt in (("fp8_scale", fp8_scale, 1, torch.float32), ("context_fp8_scale", context_fp8_scale, 1, torch.float32),
+                           ("int8_scale", int8_scale, 1, torch.float32), ("int8_pre", int8_pre, h * dh, torch.float32)):
+        if t is not None:
+            _chk(t, name, (dt,))
+            if n is not None and t.numel() != n:
+                raise ValueError(f"{name} must hold {n} elements")
+    a = _l.Attention()
+    a.q, a.k, a.v, a.dtype = q.data_ptr(), k.data_ptr(), v.data_ptr(), _DT[q.dtype]
+    a.q_row, a.k_row, a.v_row = q.stride(1), k.stride(1), v.stride(1)
+    if b > 1:
+        a.q_batch, a.k_batch, a.v_batch = q.stride(0), k.stride(0), v.stride(0)
+    a.batch, a.seq_q, a.seq_k, a.heads, a.head_dim, a.context = b, sq, k.shape[1], h, dh, context
+    a.scale = float(dh ** -0.5 if scale is None else scale)
+    if fp8_scale is not None:
+        panels = lambda rows: torch.empty((h * dh // 64, b * rows, 64), dtype=torch.uint8, device=q.device)
+        if fp8_out is not None:
+            _chk(fp8_out, "fp8_out", (torch.uint8,))
+            if tuple(fp8_out.shape) != (h * dh // 64, b * (sq - context), 64):
+                raise ValueError("fp8_out must be [H*Dh/64, B*(Sq - context), 64]")
+        out = panels(sq - context) if fp8_out is None else fp8_out
+        a.out_fp8, a.out_fp8_scale = out.data_ptr(), fp8_scale.data_ptr()
+        if context and context_fp8_scale is None:
+            raise ValueError("context tokens need context_fp8_scale")
+        if context_fp8_scale is not None:
+            out = out, panels(context)
+            a.context_fp8, a.context_fp8_scale = out[1].data_ptr(), context_fp8_scale.data_ptr()
+    else:
+        out = torch.empty((b, sq, h * dh), dtype=torch.int8, device=q.device)
+        a.out_int8, a.int8_pre, a.int8_scale = out.data_ptr(), _ptr(int8_pre), int8_scale.data_ptr()
+    _l.check(_l.load().lq_attention_ex(C.addressof(a), _stream()), "lq_attention_ex")
     return out
 
 

@@ -94,10 +94,14 @@ def _gemm_int8(q8: torch.Tensor, lin: Int8Linear, dtype, bias=None) -> torch.Ten
     return y.view(*q8.shape[:-1], y.shape[-1])
 
 
-def _attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int) -> torch.Tensor:
+def _attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, heads: int, to_out=None) -> torch.Tensor:
+    """Softmax attention [B, S, D], or the codes an INT8 `to_out` takes (invokeSqInputQuant) straight from the attention kernel."""
     b, s, d = q.shape
     split = lambda t: t.view(b, t.shape[1], heads, d // heads)
-    return ops.softmax_attention(split(q), split(k), split(v)).reshape(b, s, d)
+    q, k, v = split(q), split(k), split(v)
+    if isinstance(to_out, Int8Linear) and ops.attention_supported(q, k, v):
+        return ops.attention_codes(q, k, v, int8_scale=to_out.input_quant_scale, int8_pre=to_out.pre_quant_scale)
+    return ops.softmax_attention(q, k, v).reshape(b, s, d)
 
 
 def _ln16(x, gb, eps):
@@ -105,10 +109,11 @@ def _ln16(x, gb, eps):
 
 
 def _to_out_and_norm(attn: torch.Tensor, residual: torch.Tensor, lin, bias, norm, consumer: Optional[Int8Linear], eps):
-    """Output projection of an attention, residual + bias, and the LayerNorm in front of the next linear.
+    """Output projection of an attention (its input as _attention leaves it), residual + bias, and the LayerNorm in front of the next linear.
     Returns (codes for `consumer` or the 16-bit normalised tensor when consumer is None, new hidden state)."""
-    if isinstance(lin, Int8Linear):  # level 3: quantise, GEMM without bias, then residual + bias + LayerNorm + quantisation fused
-        y = _gemm_int8(ops.sq_quant(attn, lin.pre_quant_scale, lin.input_quant_scale), lin, attn.dtype)
+    if isinstance(lin, Int8Linear):  # level 3: codes, GEMM without bias, then residual + bias + LayerNorm + quantisation fused
+        q8 = attn if attn.dtype == torch.int8 else ops.sq_quant(attn, lin.pre_quant_scale, lin.input_quant_scale)
+        y = _gemm_int8(q8, lin, residual.dtype)
         q8, _, hidden = ops.layernorm_int8(y, norm[0], norm[1], consumer.pre_quant_scale, consumer.input_quant_scale, residual, bias, eps)
         return q8, hidden
     hidden = torch.nn.functional.linear(attn, lin.weight, bias) + residual  # GemmWithResidualAndBias, beta = 1
@@ -130,13 +135,13 @@ def basic_transformer_int8_block(x: torch.Tensor, encoder_hidden_states: torch.T
     else:
         qkv = w.attn1_qkv.forward(_ln16(x, w.norm1, eps))
     q, k, v = qkv.split(d, dim=-1)
-    a1 = _attention(q, k, v, heads).contiguous()
+    a1 = _attention(q, k, v, heads, w.attn1_to_out).contiguous()
     # to_out + residual + norm2 (+ quantisation for attn2.to_q at level 3)
     q2_consumer = w.attn2_q if isinstance(w.attn2_q, Int8Linear) else None
     n2, h1 = _to_out_and_norm(a1, x, w.attn1_to_out, w.attn1_to_out_bias, w.norm2, q2_consumer, eps)
     # cross-attention
     q = _gemm_int8(n2, w.attn2_q, x.dtype) if q2_consumer is not None else w.attn2_q.forward(n2)
-    a2 = _attention(q, w.attn2_k.forward(encoder_hidden_states), w.attn2_v.forward(encoder_hidden_states), heads).contiguous()
+    a2 = _attention(q, w.attn2_k.forward(encoder_hidden_states), w.attn2_v.forward(encoder_hidden_states), heads, w.attn2_to_out).contiguous()
     # to_out + residual + norm3 + quantisation for the GEGLU projection (INT8 at every level)
     q8, h2 = _to_out_and_norm(a2, h1, w.attn2_to_out, w.attn2_to_out_bias, w.norm3, w.geglu, eps)
     # feed-forward

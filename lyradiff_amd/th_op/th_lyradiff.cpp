@@ -170,14 +170,11 @@ void gemm_pair(const lq_fp8_half_t& a, const lq_fp8_half_t& b, at::ScalarType T,
     const lq_fp8_half_t halves[2] = {a, b};
     ok(lq_gemm_fp8_pair(halves, lq_dt(T), gelu, panels, (int)n, (int)k, cur_stream()), "lq_gemm_fp8_pair");
 }
-// two linears of one shape on codes in k-panels, in one launch where that is faster: [m, n] each
-std::pair<at::Tensor, at::Tensor> linear_pair(const FP8Linear& la, const at::Tensor& qa, int64_t ma, const FP8Linear& lb, const at::Tensor& qb,
-                                              int64_t mb, at::ScalarType T) {
-    at::Tensor ya = at::empty({ma, la.n}, on_gpu(T)), yb = at::empty({mb, lb.n}, on_gpu(T));
-    lq_fp8_half_t a = half_of(la, qa, ma), b = half_of(lb, qb, mb);
+// two linears of one shape on codes in k-panels, in one launch where that is faster, into ya and yb ([.., n])
+void linear_pair(const FP8Linear& la, const at::Tensor& qa, const at::Tensor& ya, const FP8Linear& lb, const at::Tensor& qb, const at::Tensor& yb) {
+    lq_fp8_half_t a = half_of(la, qa, qa.size(1)), b = half_of(lb, qb, qb.size(1));
     a.C = P(ya), b.C = P(yb);
-    gemm_pair(a, b, T, 0, 1, la.n, la.k);
-    return {ya, yb};
+    gemm_pair(a, b, ya.scalar_type(), 0, 1, la.n, la.k);
 }
 // the gated output projections behind the activations of both halves: gate [B, n], residual [B, S, n] -> [B, S, n]
 std::vector<at::Tensor> gated_pair(const FP8Linear& la, const at::Tensor& qa, const at::Tensor& gate_a, const at::Tensor& res_a, const FP8Linear& lb,
@@ -209,13 +206,12 @@ struct W4A4Linear {
         if (has_bias) bias = src.get(prefix + "bias", {n}, T).to(at::kCUDA);
     }
     // quantise + low-rank down + GEMM with the epilogue options of lq_epilogue_t; returns the 16-bit output (undefined
-    // when only codes are asked for)
-    at::Tensor run(const at::Tensor& x2, const lq_epilogue_t* epi, bool want_output) const {
+    // when only codes are asked for), written to y if that is given
+    at::Tensor run(const at::Tensor& x2, const lq_epilogue_t* epi, bool want_output, at::Tensor y = at::Tensor()) const {
         const int64_t m = x2.size(0);
         const at::ScalarType T = x2.scalar_type();
         at::Tensor act = at::empty({m, rank}, on_gpu(T));
-        at::Tensor y;
-        if (want_output) y = at::empty({m, n}, on_gpu(T));
+        if (want_output && !y.defined()) y = at::empty({m, n}, on_gpu(T));
         if (lq_w4a4_prefers_codes((int)m, (int)n, (int)k)) {
             at::Tensor q = at::empty({m, k}, on_gpu(at::kByte)), s = at::empty({k / 64, m}, on_gpu(at::kFloat));
             at::Tensor w = at::empty({n, k}, on_gpu(at::kByte)), ws = at::empty({k / 64, n}, on_gpu(at::kFloat));
@@ -275,27 +271,57 @@ at::Tensor adaln_16(const at::Tensor& x, const at::Tensor& msa) {
     return y;
 }
 
-// q/k RMSNorm + rotary embedding + [text, image] concatenation in one kernel (invokeFusedRmsNormCatAndRope,
-// kernels/rope/flux_apply_rope.cu:74-156), then softmax attention (lq_attention) on its [B, Sc + S, 3, H, Dh] output.
-// Returns [B, Sc + S, D] with the text tokens first.
-at::Tensor attention_core(const at::Tensor& qkv, const at::Tensor& ctx_qkv, const at::Tensor& norm_qk, const at::Tensor& norm_added_qk,
-                          const at::Tensor& rope, int64_t heads) {
-    const int64_t b = qkv.size(0), s = qkv.size(1), d = qkv.size(2) / 3, dh = d / heads;
-    const int64_t sc = ctx_qkv.defined() ? ctx_qkv.size(1) : 0;
-    const int64_t per_batch = (sc + s) * dh * 2;
-    TORCH_CHECK(rope.numel() == per_batch || rope.numel() == b * per_batch, "rope_emb must be [B or 1, ", sc + s, ", ", dh / 2, ", 2, 2]");
-    at::Tensor cat = at::empty({b, sc + s, 3, heads, dh}, qkv.options());
-    ok(lq_rmsnorm_rope(P(cat), P(qkv), P(ctx_qkv), P(norm_qk), P(norm_added_qk), P(rope), rope.numel() != per_batch ? (size_t)per_batch : 0,
-                       lq_dt(qkv.scalar_type()), (int)b, (int)s, (int)sc, (int)heads, (int)dh, 1e-6f, cur_stream()),
+// ---- between the QKV and the output projections ----------------------------------------------------------------------
+// elements between the rotary tables of two batches: rope_emb is [B or 1, tokens, Dh / 2, 2, 2]
+size_t rope_stride(const at::Tensor& rope, int64_t b, int64_t tokens, int64_t dh) {
+    const int64_t per_batch = tokens * dh * 2;
+    TORCH_CHECK(rope.numel() == per_batch || rope.numel() == b * per_batch, "rope_emb must be [B or 1, ", tokens, ", ", dh / 2, ", 2, 2]");
+    return rope.numel() != per_batch ? (size_t)per_batch : 0;
+}
+// q/k RMSNorm + rotary embedding in place on qkv [B, S, 3D] whose first sc tokens are the text (invokeFusedRmsNormCatAndRope,
+// kernels/rope/flux_apply_rope.cu:74-156)
+void rotate(const at::Tensor& qkv, int64_t sc, const at::Tensor& norm_qk, const at::Tensor& norm_added_qk, const at::Tensor& rope, int64_t heads) {
+    const int64_t b = qkv.size(0), s = qkv.size(1), dh = qkv.size(2) / 3 / heads;
+    ok(lq_rmsnorm_rope_inplace(P(qkv), P(norm_qk), P(norm_added_qk), P(rope), rope_stride(rope, b, s, dh), lq_dt(qkv.scalar_type()), (int)b,
+                               (int)s, (int)sc, (int)heads, (int)dh, 1e-6f, cur_stream()),
+       "lq_rmsnorm_rope_inplace");
+}
+// the same with the concatenation [text, image] into a new tensor [B, Sc + S, 3D]
+at::Tensor rotate_two(const at::Tensor& qkv, const at::Tensor& ctx_qkv, const at::Tensor& norm_qk, const at::Tensor& norm_added_qk,
+                      const at::Tensor& rope, int64_t heads) {
+    const int64_t b = qkv.size(0), s = qkv.size(1), sc = ctx_qkv.size(1), dh = qkv.size(2) / 3 / heads;
+    at::Tensor cat = at::empty({b, sc + s, qkv.size(2)}, qkv.options());
+    ok(lq_rmsnorm_rope(P(cat), P(qkv), P(ctx_qkv), P(norm_qk), P(norm_added_qk), P(rope), rope_stride(rope, b, sc + s, dh), lq_dt(qkv.scalar_type()),
+                       (int)b, (int)s, (int)sc, (int)heads, (int)dh, 1e-6f, cur_stream()),
        "lq_rmsnorm_rope");
-    // q, k and v are strided parts of `cat`; dh is 64 or 128 here, lq_rmsnorm_rope takes no other
+    return cat;
+}
+// softmax attention of cat [B, S, 3D] (q, k and v are strided parts of it); the caller adds the outputs
+lq_attention_t attention_of(const at::Tensor& cat, int64_t heads) {
+    const int64_t b = cat.size(0), s = cat.size(1), d = cat.size(2) / 3, dh = d / heads;  // dh is 64 or 128 here, the rotation takes no other
     const char* parts = static_cast<const char*>(P(cat));
-    const size_t row = (size_t)(3 * d), batch = row * (size_t)(sc + s), part = (size_t)d * cat.element_size();
-    at::Tensor o = at::empty({b, sc + s, d}, qkv.options());
-    ok(lq_attention(P(o), parts, row, batch, parts + part, row, batch, parts + 2 * part, row, batch, lq_dt(qkv.scalar_type()), (int)b,
-                    (int)(sc + s), (int)(sc + s), (int)heads, (int)dh, 1.0f / std::sqrt((float)dh), cur_stream()),
-       "lq_attention");
+    const size_t part = (size_t)d * cat.element_size();
+    lq_attention_t a = {};
+    a.q = parts, a.k = parts + part, a.v = parts + 2 * part;
+    a.q_row = a.k_row = a.v_row = (size_t)(3 * d);
+    a.q_batch = a.k_batch = a.v_batch = (size_t)(3 * d * s);
+    a.dtype = lq_dt(cat.scalar_type()), a.batch = (int)b, a.seq_q = a.seq_k = (int)s, a.heads = (int)heads, a.head_dim = (int)dh;
+    a.scale = 1.0f / std::sqrt((float)dh);
+    return a;
+}
+at::Tensor attention_out(const at::Tensor& cat, int64_t heads) {  // [B, S, D]
+    at::Tensor o = at::empty({cat.size(0), cat.size(1), cat.size(2) / 3}, cat.options());
+    lq_attention_t a = attention_of(cat, heads);
+    a.out = P(o);
+    ok(lq_attention_ex(&a, cur_stream()), "lq_attention_ex");
     return o;
+}
+// the output as e4m3 codes in k-panels: the image's to `codes`, those of the first sc tokens to `ctx_codes`
+void attention_codes(const at::Tensor& cat, int64_t heads, uint8_t* codes, const float* scale, int64_t sc = 0, uint8_t* ctx_codes = nullptr,
+                     const float* ctx_scale = nullptr) {
+    lq_attention_t a = attention_of(cat, heads);
+    a.out_fp8 = codes, a.out_fp8_scale = scale, a.context = (int)sc, a.context_fp8 = ctx_codes, a.context_fp8_scale = ctx_scale;
+    ok(lq_attention_ex(&a, cur_stream()), "lq_attention_ex");
 }
 
 // FluxAttnPostFP8Processor (FluxAttnPostFP8Processor.cc:93-240)
@@ -480,23 +506,33 @@ struct FluxTransformerBlockOp : th::CustomClassHolder {
         const int64_t b = x.size(0), s = x.size(1), sc = c.size(1), d = cfg.dim;
         at::Tensor temb = temb_emb.reshape({b, d});
         at::Tensor msa = norm1.msa(temb, 6), cmsa = norm1_context.msa(temb, 6);
-        at::Tensor qkv, cqkv;
-        if (cfg.int4) {
-            qkv = to_qkv4.run(adaln_16(x, msa).view({b * s, d}), nullptr, true).view({b, s, 3 * d});
-            cqkv = to_added_qkv4.run(adaln_16(c, cmsa).view({b * sc, d}), nullptr, true).view({b, sc, 3 * d});
+        // one batch: both halves' QKV side by side, text first, so that nothing has to be concatenated
+        at::Tensor cat, qkv, cqkv;
+        if (b == 1) {
+            cat = at::empty({1, sc + s, 3 * d}, x.options());
+            qkv = cat[0].slice(0, sc, sc + s), cqkv = cat[0].slice(0, 0, sc);
         } else {
-            const auto both = linear_pair(to_qkv, adaln_codes(x, msa, to_qkv.in_scale), b * s, to_added_qkv,
-                                          adaln_codes(c, cmsa, to_added_qkv.in_scale), b * sc, cfg.T);
-            qkv = both.first.view({b, s, 3 * d}), cqkv = both.second.view({b, sc, 3 * d});
+            qkv = at::empty({b * s, 3 * d}, x.options()), cqkv = at::empty({b * sc, 3 * d}, x.options());
         }
-        at::Tensor o = attention_core(qkv, cqkv, norm_qk, norm_added_qk, rope_emb, cfg.heads);
-        at::Tensor attn = o.slice(1, sc, sc + s).contiguous().view({b * s, d}), cattn = o.slice(1, 0, sc).contiguous().view({b * sc, d});
         if (cfg.int4) {
+            to_qkv4.run(adaln_16(x, msa).view({b * s, d}), nullptr, true, qkv);
+            to_added_qkv4.run(adaln_16(c, cmsa).view({b * sc, d}), nullptr, true, cqkv);
+        } else {
+            linear_pair(to_qkv, adaln_codes(x, msa, to_qkv.in_scale), qkv, to_added_qkv, adaln_codes(c, cmsa, to_added_qkv.in_scale), cqkv);
+        }
+        if (b == 1) rotate(cat, sc, norm_qk, norm_added_qk, rope_emb, cfg.heads);
+        else cat = rotate_two(qkv.view({b, s, 3 * d}), cqkv.view({b, sc, 3 * d}), norm_qk, norm_added_qk, rope_emb, cfg.heads);
+        if (cfg.int4) {
+            at::Tensor o = attention_out(cat, cfg.heads);
+            at::Tensor attn = o.slice(1, sc, sc + s).contiguous().view({b * s, d}), cattn = o.slice(1, 0, sc).contiguous().view({b * sc, d});
             at::Tensor a_out = to_out4.run(attn, nullptr, true).view({b, s, d}), c_out = to_add_out4.run(cattn, nullptr, true).view({b, sc, d});
             return attn_post_pair(ff4, x, a_out, msa, ff_context4, c, c_out, cmsa);
         }
-        const auto out = linear_pair(to_out, to_out.cast_input(attn), b * s, to_add_out, to_add_out.cast_input(cattn), b * sc, cfg.T);
-        return attn_post_pair(ff, x, out.first.view({b, s, d}), msa, ff_context, c, out.second.view({b, sc, d}), cmsa);
+        at::Tensor q = at::empty({d / 64, b * s, 64}, on_gpu(at::kByte)), cq = at::empty({d / 64, b * sc, 64}, on_gpu(at::kByte));
+        attention_codes(cat, cfg.heads, P8(q), PF(to_out.in_scale), sc, P8(cq), PF(to_add_out.in_scale));
+        at::Tensor a_out = at::empty({b, s, d}, x.options()), c_out = at::empty({b, sc, d}, x.options());
+        linear_pair(to_out, q, a_out, to_add_out, cq, c_out);
+        return attn_post_pair(ff, x, a_out, msa, ff_context, c, c_out, cmsa);
     }
 };
 
@@ -575,8 +611,9 @@ struct FluxSingleTransformerBlockOp : th::CustomClassHolder {
         at::Tensor gate = msa[2].contiguous(), none;
         if (cfg.int4) {
             at::Tensor nh = adaln_16(x, msa).view({m, d});
-            at::Tensor attn = attention_core(to_qkv4.run(nh, nullptr, true).view({b, s, 3 * d}), none, norm_qk, none, rope_emb, cfg.heads)
-                                  .contiguous().view({m, d});
+            at::Tensor qkv = to_qkv4.run(nh, nullptr, true).view({b, s, 3 * d});
+            rotate(qkv, 0, norm_qk, none, rope_emb, cfg.heads);
+            at::Tensor attn = attention_out(qkv, cfg.heads).view({m, d});
             lq_epilogue_t gelu = {2, nullptr, nullptr, 1, nullptr, nullptr, 0, nullptr};
             at::Tensor mlp = proj_mlp4.run(nh, &gelu, true);
             at::Tensor h1 = proj_out_1.run(attn, nullptr, true);
@@ -588,14 +625,13 @@ struct FluxSingleTransformerBlockOp : th::CustomClassHolder {
         ok(lq_layernorm_mod_fp8_dual_panels(P8(c_qkv), PF(to_qkv.in_scale), P8(c_mlp), PF(proj_mlp.in_scale), P(x), P(msa[1]), P(msa[0]),
                                             dt, (size_t)b, (size_t)s, (size_t)d, 1e-6f, cur_stream()),
            "lq_layernorm_mod_fp8_dual_panels");
-        at::Tensor attn = attention_core(to_qkv.from_panels(c_qkv, m, cfg.T).view({b, s, 3 * d}), none, norm_qk, none, rope_emb, cfg.heads)
-                              .contiguous();
+        at::Tensor qkv = to_qkv.from_panels(c_qkv, m, cfg.T).view({b, s, 3 * d});
+        rotate(qkv, 0, norm_qk, none, rope_emb, cfg.heads);
         // proj_out's input [attn | gelu(mlp)] as e4m3 codes in k-panels [(D + F)/64, M, 64]: a block of columns is a run of whole
-        // panels, so the attention columns are a cast into the first D/64 panels and the mlp columns come straight from the
-        // proj_mlp GEMM's epilogue into the rest (FluxSingleTransformerFP8Block.cc:216-253)
+        // panels, so the attention writes the first D/64 panels and the proj_mlp GEMM's epilogue the rest
+        // (FluxSingleTransformerFP8Block.cc:216-253)
         at::Tensor q2 = at::empty({(d + f) / 64, m, 64}, on_gpu(at::kByte));
-        ok(lq_fp8_scale_cast_panels(P8(q2), P(attn), dt, PF(proj_out.in_scale), 1, (size_t)m, (size_t)d, cur_stream()),
-           "lq_fp8_scale_cast_panels");
+        attention_codes(qkv, cfg.heads, P8(q2), PF(proj_out.in_scale));
         ok(lq_gemm_fp8_codes_panels(P8(q2) + (size_t)(d / 64) * (size_t)m * 64, PF(proj_out.in_scale), dt, P8(c_mlp), P8(proj_mlp.w_rows32),
                                     PF(proj_mlp.in_scale), PF(proj_mlp.w_scale), P(proj_mlp.bias), 2, (int)m, (int)f, (int)d, cur_stream()),
            "lq_gemm_fp8_codes_panels");

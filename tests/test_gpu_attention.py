@@ -193,6 +193,57 @@ def test_attention_on_a_side_stream_and_replayed_from_a_graph(dev, sq, h, dh):
         torch.cuda.synchronize()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,sq,h,dh", [(2, 77, 3, 64), (2, 300, 2, 128), (1, 1443, 24, 128)])  # the three forms of the kernel, ragged
+def test_attention_codes_are_the_casts_of_its_output(dev, b, sq, h, dh, dt):
+    """e4m3 k-panels of both parts and int8 codes: bit for bit the separate quantisers', NaN, saturation and untouched neighbours included."""
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(sq + dh)
+    qkv = torch.randn(b, sq, 3, h, dh, generator=g, device=dev).to(dt)
+    qkv[0, 5, 2, 0, 7] = float("inf")  # a value: its column saturates
+    qkv[-1, 3, 0, h - 1] = float("nan")  # a query: its row is NaN
+    q, k, v = qkv.unbind(2)
+    o = ops.attention(q, k, v)
+    assert o[0, :, 0, 7].isinf().any() and o[-1, 3, h - 1].isnan().all()
+    sa, sb = torch.full((1,), 1e-3, device=dev), torch.full((1,), 3e-4, device=dev)
+    rows = lambda t: t.reshape(-1, h * dh).contiguous()
+    assert torch.equal(ops.attention_codes(q, k, v, fp8_scale=sa), ops.fp8_scale_cast_panels(rows(o), sa))
+    for context in (0, 1, 33, sq):
+        got, ctx = ops.attention_codes(q, k, v, None, context, sa, sb)
+        assert torch.equal(ctx, ops.fp8_scale_cast_panels(rows(o[:, :context]), sb)), context
+        assert torch.equal(got, ops.fp8_scale_cast_panels(rows(o[:, context:]), sa)), context
+    wide = torch.full((h * dh // 64 + 2, b * sq, 64), 0xAB, dtype=torch.uint8, device=dev)
+    ops.attention_codes(q, k, v, fp8_scale=sa, fp8_out=wide[1:-1])
+    assert torch.equal(wide[1:-1], ops.fp8_scale_cast_panels(rows(o), sa)) and (wide[0] == 0xAB).all() and (wide[-1] == 0xAB).all()
+    pre = 0.5 + torch.rand(h * dh, generator=g, device=dev)
+    for scale in (sa, torch.full((1,), 2.0 ** -120, device=dev)):
+        assert torch.equal(ops.attention_codes(q, k, v, int8_scale=scale, int8_pre=pre), ops.sq_quant(o.reshape(b, sq, h * dh), pre, scale))
+    assert torch.equal(ops.attention_codes(q, k, v, int8_scale=sa), ops.sq_quant(o.reshape(b, sq, h * dh), None, sa))
+    with pytest.raises(ValueError):
+        ops.attention_codes(q, k, v, None, 1, sa)
+    with pytest.raises(ValueError):
+        ops.attention_codes(q, k, v)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,s,sc,h,dh", [(1, 97, 0, 24, 128), (1, 40, 33, 3, 64), (2, 21, 21, 5, 128), (2, 9, 4, 1, 64)])
+def test_rmsnorm_rope_in_place(dev, b, s, sc, h, dh, dt):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(s + h)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device=dev).to(dt)
+    qkv, norm, added = draw(b, s, 3 * h * dh), draw(2 * dh), draw(2 * dh)
+    for tables in (1, b):
+        rope = draw(tables, s, dh // 2, 2, 2)
+        want = ops.rmsnorm_rope(qkv[:, sc:].contiguous(), norm, rope, h, qkv[:, :sc].contiguous() if sc else None, added if sc else None)
+        got = qkv.clone()
+        assert torch.equal(ops.rmsnorm_rope_inplace(got, norm, rope, h, sc, added if sc else None), want)
+        assert torch.equal(got.view(b, s, 3, h, dh)[:, :, 2], qkv.view(b, s, 3, h, dh)[:, :, 2])
+
+
 def test_attention_argument_errors_do_not_reach_the_gpu():
     from lyradiff_amd import lib as L
 
