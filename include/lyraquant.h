@@ -30,6 +30,7 @@ typedef enum { LQ_F32 = 0, LQ_F16 = 1, LQ_BF16 = 2, LQ_I32 = 3 } lq_dtype_t;
 
 typedef enum {
     LQ_OK = 0,
+    LQ_NOT_TAKEN = 1,        /* the entry point's documented alternative is to be used; nothing was done */
     LQ_ERR_ARG = -1,         /* null pointer, bad enum */
     LQ_ERR_SHAPE = -2,       /* shape not supported by the kernels (message says which rule) */
     LQ_ERR_HIP = -3,         /* a HIP runtime call failed */
@@ -327,6 +328,19 @@ int lq_gate_residual_layernorm_mod_fp8_panels(uint8_t* dst_panels, void* hidden_
 int lq_gemm_fp8_gated(void* C, lq_dtype_t out_dtype, const uint8_t* A, const uint8_t* B_rows32,
                       const float* a_scale, const float* b_scale, const void* bias, const void* gate,
                       size_t rows_per_gate, const void* residual, int m, int n, int k, lq_stream_t stream);
+
+/* lq_fp8_scale_cast followed by lq_gemm_fp8 (scales and bias) for few rows, in one launch: x [m, k] of T, C [m, n] of T, a_scale the static
+ * input scale.  Same bits.  With C2 (B2_rows32, a_scale2, b_scale2, bias2) a second linear of the same shape on the same x in that launch.
+ * LQ_NOT_TAKEN (and nothing done) where the two calls are the better or the only way. */
+int lq_linear_fp8_rows(void* C, void* C2, const void* x, lq_dtype_t dtype, const uint8_t* B_rows32, const uint8_t* B2_rows32,
+                       const float* a_scale, const float* a_scale2, const float* b_scale, const float* b_scale2, const void* bias,
+                       const void* bias2, int m, int n, int k, lq_stream_t stream);
+
+/* A plain 16-bit linear of few rows: y [m, n] = x [m, k] . w [n, k]^T + bias [n] (or NULL), fp32 sums, T in {F16, BF16}; with y2, w2 (and
+ * bias2) a second one of the same shape on the same input in the same launch.  n % 4 == 0, k % 64 == 0.  (AdaLayerNorm.cc's modulation,
+ * the text key and value projections of BasicTransformerInt8Block.cc.) */
+int lq_linear16_rows(void* y, void* y2, const void* x, const void* w, const void* w2, const void* bias, const void* bias2, lq_dtype_t dtype,
+                     int m, int n, int k, lq_stream_t stream);
 
 /* Two FP8 linears of one n and k (the image and the text half of a double-stream block, FluxTransformerFP8Block.cc:159-262), in one
  * launch where that is faster.  Per half one of

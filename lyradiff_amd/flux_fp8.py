@@ -94,22 +94,44 @@ def load_ada_layernorm(src, prefix: str, dim: int, n_chunks: int, full: bool, dt
                        get(prefix + "linear.bias", (n_chunks * dim,), dtype).to(device))
 
 
+def _modulation_rows(temb: torch.Tensor, linear: Union[FP8Linear, AdaLinear16], dtype) -> torch.Tensor:
+    if isinstance(linear, AdaLinear16):
+        return ops.linear16(temb, linear.weight, linear.bias)
+    flat = ops.fp8_linear_rows(temb, (linear.weight_rows32, linear.input_scale, linear.weight_scale, linear.bias)) if temb.dtype == dtype else None
+    if flat is None:
+        q = ops.fp8_scale_cast(temb, linear.input_scale)
+        flat = ops.fp8_linear(q, linear.weight_rows32, linear.input_scale, linear.weight_scale, linear.bias, out_dtype=dtype)
+    return flat
+
+
+def ada_modulation(temb: torch.Tensor, linear: Union[FP8Linear, AdaLinear16], n_chunks: int, dtype, second=None):
+    """msa [n_chunks, B, D] of the (already SiLU'd) time embedding temb [B, D]; with `second` (the other half's adaLN linear) a pair, in one
+    launch where few rows let it.  16-bit linears are no quantized linears: a plain 16-bit matmul (AdaLayerNorm.cc)."""
+    b, d = temb.shape
+    lins = [linear] if second is None else [linear, second]
+    flat = None
+    if second is not None and all(isinstance(lin, AdaLinear16) for lin in lins):
+        flat = ops.linear16_pair(temb, linear.weight, second.weight, linear.bias, second.bias)
+    elif second is not None and temb.dtype == dtype and all(isinstance(lin, FP8Linear) for lin in lins):
+        flat = ops.fp8_linear_rows(temb, *((lin.weight_rows32, lin.input_scale, lin.weight_scale, lin.bias) for lin in lins))
+    if flat is None:
+        flat = [_modulation_rows(temb, lin, dtype) for lin in lins]
+    chunks = lambda f: f.view(b, n_chunks, d).transpose(0, 1).contiguous() if b > 1 else f.view(n_chunks, 1, d)  # invokeTranspose102
+    return chunks(flat[0]) if second is None else (chunks(flat[0]), chunks(flat[1]))
+
+
 def ada_fp8_layernorm(x: torch.Tensor, temb: torch.Tensor, linear: Union[FP8Linear, AdaLinear16], n_chunks: int, code_scales=(),
-                      switch_scale: bool = False, eps: float = 1e-6, panels: bool = False):
+                      switch_scale: bool = False, eps: float = 1e-6, panels: bool = False, msa=None):
     """AdaFP8LayerNorm<T>::forward (layers/ada_layer_norm/AdaFP8LayerNorm.cc:93-205): msa = FP8 linear of the
     (already SiLU'd) time embedding, stored [n_chunks, B, D]; output = (1 + msa[1]) * LayerNorm(x) + msa[0]
-    (msa[0]/msa[1] swapped with switch_scale).  x [B, S, D], temb [B, D].
+    (msa[0]/msa[1] swapped with switch_scale).  x [B, S, D], temb [B, D]; msa given: that one instead.
     code_scales: () -> the 16-bit normalised tensor as the reference writes it; one or two fp32 [1] input scales ->
     the e4m3 codes for the FP8 linears that consume it instead (cast fused, no 16-bit tensor); with panels=True the codes
     are k-panels [D/64, B*S, 64] (ops.fp8_quant_panels) instead of [B, S, D].
     Returns (norm | codes | (codes_a, codes_b), msa)."""
     b, s, d = x.shape
-    if isinstance(linear, AdaLinear16):  # not a quantized linear: a plain 16-bit matmul (AdaLayerNorm.cc)
-        flat = torch.nn.functional.linear(temb.reshape(b, d), linear.weight, linear.bias)
-    else:
-        q = ops.fp8_scale_cast(temb.reshape(b, d), linear.input_scale)
-        flat = ops.fp8_linear(q, linear.weight_rows32, linear.input_scale, linear.weight_scale, linear.bias, out_dtype=x.dtype)
-    msa = flat.view(b, n_chunks, d).transpose(0, 1).contiguous() if b > 1 else flat.view(n_chunks, 1, d)  # invokeTranspose102
+    if msa is None:
+        msa = ada_modulation(temb.reshape(b, d), linear, n_chunks, x.dtype)
     shift, scale = (msa[1], msa[0]) if switch_scale else (msa[0], msa[1])
     if len(code_scales) == 0:
         return ops.gate_residual_layernorm_mod(x, scale, shift, eps=eps), msa
@@ -262,8 +284,9 @@ def flux_double_block_fp8(x: torch.Tensor, context: torch.Tensor, temb: torch.Te
     """FluxTransformerFP8Block<T>::forward (FluxTransformerFP8Block.cc:159-262) with FluxAttentionFP8Processor
     (FluxAttentionFP8Processor.cc:165-360).  attention(qkv [B, S, 3D], context_qkv [B, Sc, 3D]) -> (attn [B, S, D],
     context_attn [B, Sc, D]).  Returns (output, context_output)."""
-    c, msa = ada_fp8_layernorm(x, temb, w.norm1, 6, (w.to_qkv.input_scale,), panels=True)
-    cc, cmsa = ada_fp8_layernorm(context, temb, w.norm1_context, 6, (w.to_added_qkv.input_scale,), panels=True)
+    msa, cmsa = ada_modulation(temb.reshape(x.shape[0], x.shape[2]), w.norm1, 6, x.dtype, w.norm1_context)
+    c, _ = ada_fp8_layernorm(x, temb, w.norm1, 6, (w.to_qkv.input_scale,), panels=True, msa=msa)
+    cc, _ = ada_fp8_layernorm(context, temb, w.norm1_context, 6, (w.to_added_qkv.input_scale,), panels=True, msa=cmsa)
     parts = core.joint_qkv(x, context) if core is not None else None  # both halves side by side, where the batch lets them
     qkv, cqkv = ops.fp8_linear_pair(fp8_half(w.to_qkv, c, out=parts and parts[0]), fp8_half(w.to_added_qkv, cc, out=parts and parts[1]), x.dtype)
     if core is not None:

@@ -27,7 +27,7 @@ from typing import Union
 import torch
 
 from . import ops
-from .flux_fp8 import AdaLinear16, ada_fp8_layernorm, fp8_half, load_ada_layernorm
+from .flux_fp8 import AdaLinear16, ada_fp8_layernorm, ada_modulation, fp8_half, load_ada_layernorm
 from .weights import FP8Linear, W4A4Linear, load_fp8_linear, load_w4a4_linear
 
 
@@ -172,8 +172,9 @@ def flux_double_block_int4(x: torch.Tensor, context: torch.Tensor, temb: torch.T
     """FluxTransformerInt4Block<T>::forward (FluxTransformerInt4Block.cc:159-246) with FluxAttentionInt4Processor
     (FluxAttentionInt4Processor.cc:206-331).  attention(qkv, context_qkv) -> (attn [B, S, D], context_attn [B, Sc, D]).
     Returns (output, context_output)."""
-    n, msa = ada_layernorm_int4(x, temb, w.norm1, 6)
-    nc, cmsa = ada_layernorm_int4(context, temb, w.norm1_context, 6)
+    msa, cmsa = ada_modulation(temb.reshape(x.shape[0], x.shape[2]), w.norm1, 6, x.dtype, w.norm1_context)
+    n, _ = ada_fp8_layernorm(x, temb, w.norm1, 6, msa=msa)
+    nc, _ = ada_fp8_layernorm(context, temb, w.norm1_context, 6, msa=cmsa)
     parts = core.joint_qkv(x, context) if core is not None else None
     qkv, cqkv = _w4a4_3d(w.to_qkv, n, parts and parts[0]), _w4a4_3d(w.to_added_qkv, nc, parts and parts[1])
     if core is None:

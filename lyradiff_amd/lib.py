@@ -78,6 +78,8 @@ SYMBOLS = {
     "lq_gemm_fp8": (_I, [_P, _I, _P, _P, _P, _P, _P, _I, _P, _F, _I, _I, _I, _P]),
     "lq_gemm_fp8_ex": (_I, [_P, _I, _P, _P, _P, _P, _P, _I, _P, _F, _I, _I, _I, _P, _P, _P, _P]),
     "lq_gemm_fp8_gated": (_I, [_P, _I, _P, _P, _P, _P, _P, _P, _Z, _P, _I, _I, _I, _P]),
+    "lq_linear_fp8_rows": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
+    "lq_linear16_rows": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "lq_gemm_fp8_pair": (_I, [_P, _I, _I, _I, _I, _I, _P]),
     "lq_gemm_fp8_codes": (_I, [_P, _Z, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "lq_fp8_scale_cast_2d": (_I, [_P, _Z, _P, _Z, _I, _P, _I, _Z, _Z, _P]),

@@ -750,6 +750,74 @@ def fp8_linear_codes_panels(a_panels, w_rows32, a_scale, b_scale, bias, out_fp8_
     return out
 
 
+def fp8_linear_rows(x, first, second=None):
+    """fp8_scale_cast and fp8_linear of few rows in one launch: x [M, K] fp16 / bf16 -> [M, N] of its type, same bits.  first: (w_rows32,
+    static input scale, weight scale, bias or None); second: another linear of that shape on the same x, whose result then comes as a second
+    output.  None where the separate calls are the better or the only way."""
+    _chk(x, "x", (torch.float16, torch.bfloat16))
+    m, k = x.shape
+    n = first[0].shape[0]
+    for w, a_scale, b_scale, bias in (first, second) if second is not None else (first,):
+        _chk(w, "w_rows32", (torch.uint8,))
+        _chk(a_scale, "a_scale", (torch.float32,))
+        _chk(b_scale, "b_scale", (torch.float32,))
+        if bias is not None:
+            _chk(bias, "bias", (x.dtype,))
+        if tuple(w.shape) != (n, k):
+            raise ValueError("K mismatch between activation and weight" if second is None else "both weights must be [N, K]")
+    y = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    y2 = torch.empty((m, n), dtype=x.dtype, device=x.device) if second is not None else None
+    w2, a2, s2, b2 = second if second is not None else (None,) * 4
+    rc = _l.load().lq_linear_fp8_rows(_ptr(y), _ptr(y2), _ptr(x), _DT[x.dtype], _ptr(first[0]), _ptr(w2), _ptr(first[1]), _ptr(a2), _ptr(first[2]),
+                                      _ptr(s2), _ptr(first[3]), _ptr(b2), m, n, k, _stream())
+    if rc == 1:
+        return None
+    _l.check(rc, "lq_linear_fp8_rows")
+    return y if second is None else (y, y2)
+
+
+_LINEAR16_ROWS = 256
+
+
+def linear16_supported(x, *tensors) -> bool:
+    """True when linear16 and linear16_pair take x [.., K] and the weights and biases `tensors`: few rows, dense 16-bit GPU tensors of one type,
+    aligned, no gradient recorded."""
+    k = x.shape[-1]
+    if x.dtype not in (torch.float16, torch.bfloat16) or k == 0 or k % 64 or x.numel() > _LINEAR16_ROWS * k or x.numel() == 0:
+        return False
+    grad = torch.is_grad_enabled()
+    for t in (x, *tensors):
+        if t is None:
+            continue
+        if not t.is_cuda or t.dtype != x.dtype or not t.is_contiguous() or t.data_ptr() % 16 or (grad and t.requires_grad) or \
+                (t is not x and t.shape[0] % 4):
+            return False
+    return True
+
+
+def linear16(x, weight, bias=None):
+    """A plain 16-bit linear x [.., K] . weight [N, K]^T + bias with fp32 sums, for few rows (linear16_supported); PyTorch's elsewhere."""
+    if not linear16_supported(x, weight, bias) or weight.dim() != 2 or weight.shape[1] != x.shape[-1] or (bias is not None and bias.numel() != weight.shape[0]):
+        return torch.nn.functional.linear(x, weight, bias)
+    n, k = weight.shape
+    y = torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device)
+    _l.check(_l.load().lq_linear16_rows(_ptr(y), None, _ptr(x), _ptr(weight), None, _ptr(bias), None, _DT[x.dtype], x.numel() // k, n, k, _stream()),
+             "lq_linear16_rows")
+    return y
+
+
+def linear16_pair(x, weight, weight2, bias=None, bias2=None):
+    """linear16 of one input with two weights of one shape (and biases), in one launch where linear16_supported takes them."""
+    if not linear16_supported(x, weight, weight2, bias, bias2) or weight.dim() != 2 or weight.shape != weight2.shape or \
+            weight.shape[1] != x.shape[-1] or any(b is not None and b.numel() != weight.shape[0] for b in (bias, bias2)):
+        return torch.nn.functional.linear(x, weight, bias), torch.nn.functional.linear(x, weight2, bias2)
+    n, k = weight.shape
+    y, y2 = (torch.empty((*x.shape[:-1], n), dtype=x.dtype, device=x.device) for _ in range(2))
+    _l.check(_l.load().lq_linear16_rows(_ptr(y), _ptr(y2), _ptr(x), _ptr(weight), _ptr(weight2), _ptr(bias), _ptr(bias2), _DT[x.dtype],
+                                        x.numel() // k, n, k, _stream()), "lq_linear16_rows")
+    return y, y2
+
+
 class FP8Half(NamedTuple):
     """One of the two problems of fp8_linear_pair: k-panels [K/64, M, 64] (or row-major codes [M, K]), the linear, and what its output is."""
     codes: torch.Tensor

@@ -41,7 +41,7 @@ class Linear16:
     bias: Optional[torch.Tensor] = None
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return torch.nn.functional.linear(x, self.weight, self.bias)
+        return ops.linear16(x, self.weight, self.bias)
 
 
 @dataclass
@@ -141,7 +141,8 @@ def basic_transformer_int8_block(x: torch.Tensor, encoder_hidden_states: torch.T
     n2, h1 = _to_out_and_norm(a1, x, w.attn1_to_out, w.attn1_to_out_bias, w.norm2, q2_consumer, eps)
     # cross-attention
     q = _gemm_int8(n2, w.attn2_q, x.dtype) if q2_consumer is not None else w.attn2_q.forward(n2)
-    a2 = _attention(q, w.attn2_k.forward(encoder_hidden_states), w.attn2_v.forward(encoder_hidden_states), heads, w.attn2_to_out).contiguous()
+    tk, tv = ops.linear16_pair(encoder_hidden_states, w.attn2_k.weight, w.attn2_v.weight, w.attn2_k.bias, w.attn2_v.bias)
+    a2 = _attention(q, tk, tv, heads, w.attn2_to_out).contiguous()
     # to_out + residual + norm3 + quantisation for the GEGLU projection (INT8 at every level)
     q8, h2 = _to_out_and_norm(a2, h1, w.attn2_to_out, w.attn2_to_out_bias, w.norm3, w.geglu, eps)
     # feed-forward

@@ -248,10 +248,31 @@ struct AdaLinear {
         bias = src.get(prefix + "linear.bias", {chunks * dim}, T).to(at::kCUDA);
     }
     // msa [chunks, B, D] from the (already SiLU'd) time embedding [B, D]  (AdaFP8LayerNorm.cc:100-175, invokeTranspose102)
-    at::Tensor msa(const at::Tensor& temb, int64_t chunks) const {
-        const int64_t b = temb.size(0), d = temb.size(1);
-        at::Tensor flat = fp8 ? q.from_panels(q.cast_input(temb), b, temb.scalar_type()) : at::linear(temb, weight, bias);
+    static at::Tensor chunked(const at::Tensor& flat, int64_t chunks, int64_t d) {
+        const int64_t b = flat.size(0);
         return b > 1 ? flat.view({b, chunks, d}).transpose(0, 1).contiguous() : flat.view({chunks, 1, d});
+    }
+    at::Tensor msa(const at::Tensor& temb, int64_t chunks) const { return msa_of(temb, chunks, nullptr).first; }
+    // with `other`, the adaLN linear of the other half of a double-stream block (same temb), both: in one launch where few rows let it
+    std::pair<at::Tensor, at::Tensor> msa_of(const at::Tensor& temb, int64_t chunks, const AdaLinear* other) const {
+        const int64_t b = temb.size(0), d = temb.size(1), n = chunks * d;
+        const lq_dtype_t dt = lq_dt(temb.scalar_type());
+        at::Tensor y = at::empty({b, n}, temb.options()), y2;
+        if (other != nullptr) y2 = at::empty({b, n}, temb.options());
+        int rc = LQ_NOT_TAKEN;
+        if (fp8)
+            rc = lq_linear_fp8_rows(P(y), P(y2), P(temb), dt, P8(q.w_rows32), other ? P8(other->q.w_rows32) : nullptr, PF(q.in_scale),
+                                    other ? PF(other->q.in_scale) : nullptr, PF(q.w_scale), other ? PF(other->q.w_scale) : nullptr, P(q.bias),
+                                    other ? P(other->q.bias) : nullptr, (int)b, (int)n, (int)d, cur_stream());
+        else if (b <= 256 && d % 64 == 0 && reinterpret_cast<uintptr_t>(P(temb)) % 16 == 0 && !(at::GradMode::is_enabled() && temb.requires_grad()))
+            rc = lq_linear16_rows(P(y), P(y2), P(temb), P(weight), other ? P(other->weight) : nullptr, P(bias), other ? P(other->bias) : nullptr, dt,
+                                  (int)b, (int)n, (int)d, cur_stream());
+        if (rc < 0) ok(rc, "adaLN linear");
+        if (rc == LQ_NOT_TAKEN) {
+            if (other != nullptr) return {msa_of(temb, chunks, nullptr).first, other->msa_of(temb, chunks, nullptr).first};
+            y = fp8 ? q.from_panels(q.cast_input(temb), b, temb.scalar_type()) : at::linear(temb, weight, bias);
+        }
+        return {chunked(y, chunks, d), other != nullptr ? chunked(y2, chunks, d) : at::Tensor()};
     }
 };
 
@@ -505,7 +526,8 @@ struct FluxTransformerBlockOp : th::CustomClassHolder {
         const at::Tensor &x = hidden_states, &c = encoder_hidden_states;
         const int64_t b = x.size(0), s = x.size(1), sc = c.size(1), d = cfg.dim;
         at::Tensor temb = temb_emb.reshape({b, d});
-        at::Tensor msa = norm1.msa(temb, 6), cmsa = norm1_context.msa(temb, 6);
+        const auto both_msa = norm1.msa_of(temb, 6, &norm1_context);
+        const at::Tensor &msa = both_msa.first, &cmsa = both_msa.second;
         // one batch: both halves' QKV side by side, text first, so that nothing has to be concatenated
         at::Tensor cat, qkv, cqkv;
         if (b == 1) {

@@ -145,6 +145,10 @@ class FP8Linear:
 
     def forward(self, x: torch.Tensor, gelu: bool = False, residual=None, beta: float = 0.0, dynamic: bool = False) -> torch.Tensor:
         x2 = _rows(x)
+        if not dynamic and not gelu and residual is None and x2.shape[0] <= 8 and x2.dtype != torch.float32:
+            y = ops.fp8_linear_rows(x2, (self.weight_rows32, self.input_scale, self.weight_scale, self.bias))
+            if y is not None:
+                return _shaped(y, x)
         if not gelu and residual is None and x2.shape[1] % 64 == 0 and x2.numel() < 2 ** 32:
             # scales and bias only: the codes travel as k-panels, which the GEMM fetches in whole cache lines (same bits)
             q, s = ops.fp8_quant_panels(x2) if dynamic else (ops.fp8_scale_cast_panels(x2, self.input_scale), self.input_scale)
