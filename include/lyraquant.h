@@ -89,6 +89,13 @@ int lq_geglu_int8(int8_t* dst, const void* hidden, const void* bias, lq_dtype_t 
                   const float* pre_quant_scale, const float* input_quant_scale, size_t rows, size_t dim,
                   lq_stream_t stream);
 
+/* lq_gemm_int8 (static scale alpha_row[0], no bias, rounded to `dtype`) and lq_geglu_int8 on its output in one kernel, the same bits
+ * without the [m, 2 * inner] tensor: A [m, k] int8, B_rows32 of 2 * inner rows, alpha_col [2 * inner], bias [2 * inner] of dtype or NULL,
+ * pre_quant_scale [inner] or NULL, out [m, inner].  dtype in {F16, BF16}; inner % 64 == 0, k % 64 == 0, k >= 256. */
+int lq_gemm_int8_geglu(int8_t* out, const int8_t* A, const int8_t* B_rows32, const float* alpha_col, const float* alpha_row, const void* bias,
+                       lq_dtype_t dtype, const float* pre_quant_scale, const float* input_quant_scale, int m, int inner, int k,
+                       lq_stream_t stream);
+
 /* Same with the dynamic per-token scale of lq_sq_dynamic_quant (scale_out[rows]). */
 int lq_geglu_int8_dynamic(int8_t* dst, float* scale_out, const void* hidden, const void* bias,
                           lq_dtype_t dtype, const float* pre_quant_scale, size_t rows, size_t dim,

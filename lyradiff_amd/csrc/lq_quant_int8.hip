@@ -12,6 +12,7 @@
 #include <atomic>
 
 #include "lq_common.h"
+#include "lq_gate_table.h"
 #include <type_traits>
 
 namespace lq {
@@ -416,9 +417,6 @@ template <typename Tag> __device__ __forceinline__ float geglu_gate(float g) {
     const float cdf = 0.5f * (1.0f + tanh_basic(0.7978845608028654f * (g + 0.044715f * cube)));
     return round_through<Tag>(g * round_through<Tag>(cdf));
 }
-template <typename Tag> struct GateTable;
-template <> struct GateTable<F16Tag> { static constexpr u32 LO = 0x0C00u, COUNT = 0x4800u - 0x0C00u; };   // 2^-12 .. 8
-template <> struct GateTable<BF16Tag> { static constexpr u32 LO = 0x3980u, COUNT = 0x4100u - 0x3980u; };
 __device__ __attribute__((aligned(16))) unsigned short g_gate_table_f16[2 * GateTable<F16Tag>::COUNT];
 __device__ __attribute__((aligned(16))) unsigned short g_gate_table_bf16[2 * GateTable<BF16Tag>::COUNT];
 template <typename Tag> __device__ __forceinline__ unsigned short* gate_table() {
@@ -498,10 +496,8 @@ __global__ __launch_bounds__(THREADS, (SW == 2 && THREADS == 512) ? 4 : 1) void 
                     }
                     if (__builtin_expect(!all_in, 0)) {  // rare: outside the table the inner factor is a constant
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) {
-                            const float c = fabsf(g[i]) < 1.0f ? 0.5f : (g[i] < 0.0f ? 0.0f : 1.0f);  // below the table : beyond it
-                            if (!in[i]) gel[i] = round_through<Tag>(g[i] * c);
-                        }
+                        for (int i = 0; i < 8; ++i)
+                            if (!in[i]) gel[i] = Elem<Tag>::load(gate_outside_table<Tag>(Elem<Tag>::store(g[i])));
                     }
                 } else {
 #pragma unroll
@@ -573,6 +569,23 @@ template <typename Tag> static int ensure_gate_table(hipStream_t st) {
         return LQ_ERR_HIP;
     }
     built.fetch_or(bit, std::memory_order_release);
+    return LQ_OK;
+}
+
+int gate_table_on_device(bool f16, hipStream_t st, const unsigned short** table) {
+    static std::atomic<const unsigned short*> known[2][32];  // per device: a device symbol stays where it is
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) dev = 32;
+    if (int rc = f16 ? ensure_gate_table<F16Tag>(st) : ensure_gate_table<BF16Tag>(st); rc != LQ_OK) return rc;
+    if (dev < 32 && (*table = known[f16][dev].load(std::memory_order_relaxed)) != nullptr) return LQ_OK;
+    void* at = nullptr;
+    const hipError_t e = f16 ? hipGetSymbolAddress(&at, HIP_SYMBOL(g_gate_table_f16)) : hipGetSymbolAddress(&at, HIP_SYMBOL(g_gate_table_bf16));
+    if (e != hipSuccess) {
+        set_error("gate table: %s", hipGetErrorString(e));
+        return LQ_ERR_HIP;
+    }
+    *table = static_cast<const unsigned short*>(at);
+    if (dev < 32) known[f16][dev].store(*table, std::memory_order_relaxed);
     return LQ_OK;
 }
 

@@ -163,6 +163,29 @@ def geglu_int8(hidden, bias, pre_quant_scale, input_quant_scale):
     return q
 
 
+def int8_linear_geglu(a_q, w_rows32, alpha_col, alpha_row, bias, pre_quant_scale, input_quant_scale, dtype):
+    """geglu_int8(int8_linear(a_q, w_rows32, alpha_col, alpha_row, None, dtype), bias, ...) with a static alpha_row: a_q int8 [M, K],
+    w_rows32 int8 [2D, K] (rows32) -> int8 [M, D].  One kernel for 16-bit types, D % 64 == 0 and K >= 256, else those two."""
+    m, k = a_q.shape
+    n = w_rows32.shape[0]
+    if dtype not in (torch.float16, torch.bfloat16) or n % 128 or k % 64 or k < 256 or alpha_row.numel() != 1:
+        return geglu_int8(int8_linear(a_q, w_rows32, alpha_col, alpha_row, None, dtype), bias, pre_quant_scale, input_quant_scale)
+    for t, name, dt in ((a_q, "a_q", torch.int8), (w_rows32, "w_rows32", torch.int8), (alpha_col, "alpha_col", torch.float32),
+                        (alpha_row, "alpha_row", torch.float32), (input_quant_scale, "input_quant_scale", torch.float32)):
+        _chk(t, name, (dt,))
+    if bias is not None:
+        _chk(bias, "bias", (dtype,))
+    if pre_quant_scale is not None:
+        _chk(pre_quant_scale, "pre_quant_scale", (torch.float32,))
+    if w_rows32.shape[1] != k or alpha_col.numel() != n or (bias is not None and bias.numel() != n) or \
+            (pre_quant_scale is not None and pre_quant_scale.numel() != n // 2):
+        raise ValueError("int8_linear_geglu: a_q [M, K], w_rows32 [2D, K], alpha_col and bias [2D], pre_quant_scale [D]")
+    q = torch.empty(m, n // 2, dtype=torch.int8, device=a_q.device)
+    _l.check(_l.load().lq_gemm_int8_geglu(_ptr(q), _ptr(a_q), _ptr(w_rows32), _ptr(alpha_col), _ptr(alpha_row), _ptr(bias), _DT[dtype],
+                                          _ptr(pre_quant_scale), _ptr(input_quant_scale), m, n // 2, k, _stream()), "lq_gemm_int8_geglu")
+    return q
+
+
 def geglu_int8_dynamic(hidden, bias=None, pre_quant_scale=None):
     _chk(hidden, "hidden", _FLOATS)
     if bias is not None:

@@ -146,6 +146,6 @@ def basic_transformer_int8_block(x: torch.Tensor, encoder_hidden_states: torch.T
     # to_out + residual + norm3 + quantisation for the GEGLU projection (INT8 at every level)
     q8, h2 = _to_out_and_norm(a2, h1, w.attn2_to_out, w.attn2_to_out_bias, w.norm3, w.geglu, eps)
     # feed-forward
-    up = _gemm_int8(q8, w.geglu, x.dtype)
-    q8 = ops.geglu_int8(up, w.geglu_bias, w.ffn.pre_quant_scale, w.ffn.input_quant_scale)
+    q8 = ops.int8_linear_geglu(q8.view(b * s, d), w.geglu.weight_rows32, w.geglu.weight_scale, w.geglu.input_quant_scale, w.geglu_bias,
+                               w.ffn.pre_quant_scale, w.ffn.input_quant_scale, x.dtype).view(b, s, -1)
     return _gemm_int8(q8, w.ffn, x.dtype, w.ffn.bias) + h2

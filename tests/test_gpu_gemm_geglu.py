@@ -1,0 +1,46 @@
+"""The INT8 up projection with GEGLU and the next linear's codes in its epilogue against the two kernels it stands for, which
+tests/test_gpu_gemm.py and tests/test_gpu_quant.py hold against the oracle: the arithmetic is the same, so every code has to be."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# rows, outputs, k: one row, tiles of 128 and 256 rows less / exactly / more than full, the fewest and more k-tiles, fewer tiles than
+# CUs, one per CU and several (2049 x 2560 is 360 tiles of 256 rows, 700 x 2560 240 of 128)
+SHAPES = [(1, 64, 256), (127, 64, 320), (128, 128, 256), (129, 192, 640), (700, 2560, 640), (1024, 5120, 1280), (2049, 2560, 640), (8192, 2560, 640)]
+
+
+@pytest.mark.parametrize("m,inner,k", SHAPES)
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_same_codes_as_gemm_then_geglu(dev, m, inner, k, dt):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(m + inner + k)
+    rnd = lambda *s: torch.rand(*s, generator=g, device=dev)
+    codes = lambda *s: torch.randint(-128, 128, s, generator=g, device=dev, dtype=torch.int8)
+    a, w = codes(m, k), ops.repack_weight(codes(2 * inner, k))
+    # results of the size of a few units; a column of tiny gates, one of large ones and one of infinities leave the gate's table
+    col = (0.5 + rnd(2 * inner)) * (2.0 / (73.0 * 73.0 * k ** 0.5))
+    col[inner + 3], col[inner + 8], col[inner + 40] = 1e-9, 1.0, 3e38
+    row, scale, pre = torch.full((1,), 1.1, device=dev), torch.full((1,), 0.03, device=dev), 0.7 + 0.6 * rnd(inner)
+    bias = torch.randn(2 * inner, generator=g, device=dev).to(dt)
+    bias[inner + 3] = 0.0
+    for b, p in ((bias, pre), (bias, None), (None, pre)):
+        want = ops.geglu_int8(ops.int8_linear(a, w, col, row, None, dt), b, p, scale)
+        got = ops.int8_linear_geglu(a, w, col, row, b, p, scale, dt)
+        assert torch.equal(got, want), (m, inner, k, b is None, p is None, int((got != want).sum()))
+    zero = torch.zeros(1, device=dev)  # a scale without a reciprocal
+    assert torch.equal(ops.int8_linear_geglu(a, w, col, row, bias, pre, zero, dt), ops.geglu_int8(ops.int8_linear(a, w, col, row, None, dt), bias, pre, zero))
+
+
+def test_other_forms_keep_to_the_two_kernels(dev):
+    from lyradiff_amd import ops
+
+    a, w = torch.ones(40, 128, device=dev, dtype=torch.int8), ops.repack_weight(torch.ones(64, 128, device=dev, dtype=torch.int8))
+    col, row, scale = torch.full((64,), 1e-2, device=dev), torch.ones(1, device=dev), torch.full((1,), 0.05, device=dev)
+    want = ops.geglu_int8(ops.int8_linear(a, w, col, row, None, torch.float16), None, None, scale)
+    assert torch.equal(ops.int8_linear_geglu(a, w, col, row, None, None, scale, torch.float16), want)
+    with pytest.raises(ValueError):
+        wide = ops.repack_weight(torch.ones(128, 256, device=dev, dtype=torch.int8))
+        ops.int8_linear_geglu(torch.ones(4, 256, device=dev, dtype=torch.int8), wide, torch.ones(128, device=dev), row, torch.zeros(64, device=dev, dtype=torch.float16),
+                              None, scale, torch.float16)
