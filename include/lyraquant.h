@@ -215,6 +215,10 @@ int lq_unpack_rows32(uint8_t* dst, const uint8_t* src, size_t n, size_t row_byte
 int lq_gemm_int8(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_t* B_rows32,
                  const float* alpha_col, const float* alpha_row, int per_token, const void* bias,
                  int m, int n, int k, lq_stream_t stream);
+/* Same with a static scale (alpha_row[0]) and a tensor of T joined to the rounded result: C = T( T(y) + addend ).  addend [m, n], 16-byte
+ * aligned, may be C; out_dtype F16 or BF16. */
+int lq_gemm_int8_add(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_t* B_rows32, const float* alpha_col, const float* alpha_row,
+                     const void* bias, const void* addend, int m, int n, int k, lq_stream_t stream);
 
 /* C[m,n] = T( act( (a_scale[0]*b_scale[0]) * sum_k A[m,k]*B[n,k] + f32(bias[n]) ) + beta*f32(residual[m,n]) )
  * on e4m3 operands with fp32 accumulation; act = tanh-GELU when gelu != 0.  bias and residual are

@@ -72,7 +72,7 @@ struct GemmParams {
     // followed by an elementwise multiply and add in T; requires residual, ignores beta
     const void* gate;
     size_t gate_rows;
-    // addend (optional, [m, n] of T): y = T( T(y) + addend ) before the gate/residual step -- the sum of two linears'
+    // addend (optional, [m, n] of T; INT8: with a static scale only): y = T( T(y) + addend ) before the gate/residual step -- the sum of two linears'
     // outputs as the reference forms it with invokeFusedBiasAndResidual
     const void* addend;
     // w4a4
@@ -738,7 +738,8 @@ struct GemmKernel {
         char* strip = smem_all + wave_all * (32 * PITCH);
         const int out_row = lane / LPR, out_n = n0 + wn * TN + (lane % LPR) * 4;
         const bool n_ok = out_n < p.n;
-        float alpha = 1.0f, bias4[4] = {0.f, 0.f, 0.f, 0.f}, acol4[4] = {0.f, 0.f, 0.f, 0.f}, arow_l[MT];
+        // without a bias -0 is added, which changes nothing (and takes no select)
+        float alpha = 1.0f, bias4[4] = {-0.f, -0.f, -0.f, -0.f}, acol4[4] = {0.f, 0.f, 0.f, 0.f}, arow_l[MT];
         float out_amax = 0.0f, out_pmax = 0.0f, c8_inv = 0.0f, gate4[4] = {0.f, 0.f, 0.f, 0.f};
         bool gate_uniform = true;  // every row of the wavefront's tile uses the same gate vector
         // the FP8 and W4A4 linears of the FLUX blocks share the activation / re-quantisation / gate epilogues
@@ -761,10 +762,14 @@ struct GemmKernel {
                 if (n_ok) {
                     float4 ac = *reinterpret_cast<const float4*>(p.alpha_col + out_n);
                     acol4[0] = ac.x; acol4[1] = ac.y; acol4[2] = ac.z; acol4[3] = ac.w;
+                    if (!p.per_token) {  // one factor per column, formed here
+                        const float ar = p.alpha_row[0];
+                        acol4[0] *= ar; acol4[1] *= ar; acol4[2] *= ar; acol4[3] *= ar;
+                    }
                 }
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
-                    arow_l[i] = p.alpha_row[p.per_token ? min(m0 + wm * TM + i * 32 + lr, p.m - 1) : 0];
+                    if (p.per_token) arow_l[i] = p.alpha_row[min(m0 + wm * TM + i * 32 + lr, p.m - 1)];
             }
         }
         // The row loop exists in a few specialisations, chosen once per workgroup: which optional steps run
@@ -772,7 +777,8 @@ struct GemmKernel {
         // instead of C; GATED: gate and residual; GENERAL: every option, checked at run time) and whether the tile lies
         // entirely inside C (no bounds checks).  Strip rows are read four at a time so that their LDS latencies
         // overlap, and the specialisations keep the per-row code free of branches.
-        constexpr int E_PLAIN = 0, E_ACT = 1, E_CODES = 2, E_GATED = 3, E_GENERAL = 4;
+        // INT8: PLAIN has a scale per row, STATIC one for all of them; ADD joins a residual to that.
+        constexpr int E_PLAIN = 0, E_ACT = 1, E_CODES = 2, E_GATED = 3, E_GENERAL = 4, E_STATIC = 5, E_STATIC_ADD = 6;
         constexpr bool kSpecialise = kExtras && ESZ == 2;  // fp32 outputs take the general path only (build time)
         int emode = kExtras ? E_GENERAL : E_PLAIN;
         if constexpr (kSpecialise) {
@@ -783,7 +789,6 @@ struct GemmKernel {
                      p.gelu == 0 && p.out_scale == nullptr) emode = E_GATED;
         }
         const bool tile_full = m0 + BM <= p.m && n0 + BN <= p.n;
-        const bool has_bias = p.bias != nullptr;
         auto band_rows = [&](auto i_c, auto mode_c, auto full_c) {
             constexpr int i = decltype(i_c)::value;
             constexpr int MODE = decltype(mode_c)::value;
@@ -796,12 +801,16 @@ struct GemmKernel {
 #pragma unroll
             for (int tb = 0; tb < NITER; tb += NB) {
                 v4i raw[NB];
-                float arv[NB];
+                float arv[NB], joined[NB][4];
 #pragma unroll
                 for (int u = 0; u < NB; ++u) {
                     const int row = (tb + u) * RPI + out_row;
                     raw[u] = *reinterpret_cast<const v4i*>(strip + row * PITCH + (lane % LPR) * 16);
-                    if constexpr (KIND == K_INT8 && !kI32) arv[u] = *reinterpret_cast<const float*>(strip + row * PITCH + TN * 4);
+                    if constexpr (KIND == K_INT8 && !kI32 && MODE == E_PLAIN) arv[u] = *reinterpret_cast<const float*>(strip + row * PITCH + TN * 4);
+                    if constexpr (!kI32) {
+                        if constexpr (MODE == E_STATIC_ADD)
+                            if (FULL || (mrow0 + (tb + u) * RPI < p.m && n_ok)) OutStore<OutTag>::load4(p.addend, idx0 + (size_t)(tb + u) * rstep, joined[u]);
+                    }
                 }
 #pragma unroll
                 for (int u = 0; u < NB; ++u) {
@@ -816,15 +825,15 @@ struct GemmKernel {
                         if constexpr (KIND == K_INT8) {
 #pragma unroll
                             for (int e = 0; e < 4; ++e) {
-                                y[e] = (float)raw[u][e] * (acol4[e] * arv[u]);
-                                if (has_bias) y[e] = y[e] + bias4[e];
+                                y[e] = (float)raw[u][e] * (MODE == E_PLAIN ? acol4[e] * arv[u] : acol4[e]) + bias4[e];
+                                if constexpr (MODE == E_STATIC_ADD) y[e] = round_through<OutTag>(y[e]) + joined[u][e];
                             }
                         } else {
 #pragma unroll
                             for (int e = 0; e < 4; ++e) {
                                 const float vf = __int_as_float(raw[u][e]);
                                 y[e] = (KIND == K_FP8) ? vf * alpha : vf;
-                                if (has_bias) y[e] = y[e] + bias4[e];
+                                y[e] = y[e] + bias4[e];
                             }
                         }
                         if constexpr (kExtras && (MODE == E_ACT || MODE == E_CODES || GEN)) {
@@ -908,7 +917,7 @@ struct GemmKernel {
                             *reinterpret_cast<int4*>(spot) = make_int4(acc[i][j][q4 * 4], acc[i][j][q4 * 4 + 1],
                                                                        acc[i][j][q4 * 4 + 2], acc[i][j][q4 * 4 + 3]);
                     }
-                if constexpr (KIND == K_INT8 && !kI32) {
+                if constexpr (KIND == K_INT8 && !kI32 && decltype(mode_c)::value == E_PLAIN) {
                     if (lh == 0) *reinterpret_cast<float*>(strip + lr * PITCH + TN * 4) = arow_l[i];
                 }
                 // strip -> registers with rows contiguous, math, store (the wavefront's own LDS accesses
@@ -939,8 +948,17 @@ struct GemmKernel {
             } else if constexpr (kExtras) {
                 all_bands(integral_constant<int, E_GENERAL>{}, std::false_type{});
             } else {
-                if (tile_full) all_bands(integral_constant<int, E_PLAIN>{}, std::true_type{});
-                else all_bands(integral_constant<int, E_PLAIN>{}, std::false_type{});
+                auto plain = [&](auto full_c) {
+                    if constexpr (KIND == K_INT8 && !kI32) {
+                        if (p.per_token) all_bands(integral_constant<int, E_PLAIN>{}, full_c);
+                        else if (p.addend == nullptr) all_bands(integral_constant<int, E_STATIC>{}, full_c);
+                        else all_bands(integral_constant<int, E_STATIC_ADD>{}, full_c);
+                    } else {
+                        all_bands(integral_constant<int, E_PLAIN>{}, full_c);
+                    }
+                };
+                if (tile_full) plain(std::true_type{});
+                else plain(std::false_type{});
             }
         }
         if constexpr (kExtras) {

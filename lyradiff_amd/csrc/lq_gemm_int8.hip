@@ -27,7 +27,9 @@ template <typename OutTag> static int run_int8(GemmParams p, hipStream_t st) {
         // other's MFMA work)
         const long last256 = t256 % 256;
         t = t256 >= 192 ? ((last256 == 0 || last256 >= 128) ? 6 : 4) : (t128 >= 128 ? 2 : 3);  // 128x128 tiles from half a round up (4096x640x2560: 14.5 against 16.3 us with 64x64)
-        if (p.k <= 1024 && t128 >= 192) t = 2;  // short K: prologue and epilogue dominate, smaller tiles overlap them better
+        // short K: prologue and epilogue dominate, smaller tiles overlap them better -- until eight rounds of them per CU make the
+        // operands' way from L2 count (k = 640, 128x128 / 128x256 tiles: 8192 x 5120 45.8 / 40.3 us, 4096 x 5120 24.1 / 24.6)
+        if (p.k <= 1024 && t128 >= 192) t = t128 >= 2048 ? 4 : 2;
         // more full 256x256 tiles than CUs: the persistent form (4608x12288x3072: 153-160 us against 162-165 with 128x256 tiles)
         if (t256 > device_cu_count() && p.m % 256 == 0 && p.n % 256 == 0 && p.kb % 128 == 0 && p.k > 1024 &&
             (out_enum<OutTag>() == LQ_F16 || out_enum<OutTag>() == LQ_BF16))
@@ -62,22 +64,29 @@ template <typename OutTag> static int run_int8(GemmParams p, hipStream_t st) {
 using namespace lq;
 
 static int gemm_int8(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_t* B_rows32, const float* alpha_col,
-                     const float* alpha_row, int per_token, const void* bias, int m, int n, int k, int a_panel, lq_stream_t stream);
+                     const float* alpha_row, int per_token, const void* bias, const void* addend, int m, int n, int k, int a_panel, lq_stream_t stream);
 
 extern "C" int lq_gemm_int8(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_t* B_rows32,
                             const float* alpha_col, const float* alpha_row, int per_token, const void* bias, int m,
                             int n, int k, lq_stream_t stream) {
-    return gemm_int8(C, out_dtype, A, B_rows32, alpha_col, alpha_row, per_token, bias, m, n, k, 0, stream);
+    return gemm_int8(C, out_dtype, A, B_rows32, alpha_col, alpha_row, per_token, bias, nullptr, m, n, k, 0, stream);
 }
 
 extern "C" int lq_gemm_int8_panels(void* C, lq_dtype_t out_dtype, const int8_t* A_panels, const int8_t* B_rows32,
                                    const float* alpha_col, const float* alpha_row, int per_token, const void* bias, int m,
                                    int n, int k, lq_stream_t stream) {
-    return gemm_int8(C, out_dtype, A_panels, B_rows32, alpha_col, alpha_row, per_token, bias, m, n, k, 1, stream);
+    return gemm_int8(C, out_dtype, A_panels, B_rows32, alpha_col, alpha_row, per_token, bias, nullptr, m, n, k, 1, stream);
+}
+
+extern "C" int lq_gemm_int8_add(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_t* B_rows32, const float* alpha_col, const float* alpha_row,
+                                const void* bias, const void* addend, int m, int n, int k, lq_stream_t stream) {
+    LQ_REQUIRE(addend && reinterpret_cast<uintptr_t>(addend) % 16 == 0, LQ_ERR_ARG, "lq_gemm_int8_add: addend must be a 16-byte aligned pointer");
+    LQ_REQUIRE(out_dtype == LQ_F16 || out_dtype == LQ_BF16, LQ_ERR_UNSUPPORTED, "lq_gemm_int8_add: F16 and BF16 only");
+    return gemm_int8(C, out_dtype, A, B_rows32, alpha_col, alpha_row, 0, bias, addend, m, n, k, 0, stream);
 }
 
 static int gemm_int8(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_t* B_rows32, const float* alpha_col,
-                     const float* alpha_row, int per_token, const void* bias, int m, int n, int k, int a_panel, lq_stream_t stream) {
+                     const float* alpha_row, int per_token, const void* bias, const void* addend, int m, int n, int k, int a_panel, lq_stream_t stream) {
     LQ_REQUIRE(C && A && B_rows32, LQ_ERR_ARG, "lq_gemm_int8: null pointer");
     LQ_REQUIRE(out_dtype == LQ_I32 || (alpha_col && alpha_row), LQ_ERR_ARG, "lq_gemm_int8: scale pointers are required");
     LQ_REQUIRE(m >= 0 && n > 0 && k > 0 && n % 32 == 0 && k % 64 == 0, LQ_ERR_SHAPE,
@@ -89,7 +98,7 @@ static int gemm_int8(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_
     if (m == 0) return LQ_OK;
     GemmParams p = {};
     p.C = C; p.A = reinterpret_cast<const uint8_t*>(A); p.B = reinterpret_cast<const uint8_t*>(B_rows32);
-    p.bias = bias; p.alpha_col = alpha_col; p.alpha_row = alpha_row; p.per_token = per_token;
+    p.bias = bias; p.addend = addend; p.alpha_col = alpha_col; p.alpha_row = alpha_row; p.per_token = per_token;
     p.m = m; p.n = n; p.k = k; p.kb = k;
     p.a_panel = a_panel;
     hipStream_t st = as_stream(stream);

@@ -437,8 +437,9 @@ def unpack_weight(packed):
 
 # ---- GEMMs -----------------------------------------------------------------------------------------
 
-def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.float16):
-    """runGemmInt8 + fused bias: a_q int8 [M,K], w_rows32 int8 [N,K] (rows32), returns [M,N]."""
+def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.float16, addend=None):
+    """runGemmInt8 + fused bias: a_q int8 [M,K], w_rows32 int8 [N,K] (rows32), returns [M,N].  addend [M,N]: joined to the rounded result,
+    in the same kernel with 16-bit outputs and one alpha_row."""
     _chk(a_q, "a_q", (torch.int8,))
     _chk(w_rows32, "w_rows32", (torch.int8,))
     m, k = a_q.shape
@@ -456,6 +457,16 @@ def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.
         per_token = int(alpha_row.numel() == m and m != 1)
     if bias is not None:
         _chk(bias, "bias", (out_dtype,))
+    if addend is not None:
+        if addend.shape != (m, n):
+            raise ValueError("addend must be [M, N]")
+        if per_token or m * n == 0 or out_dtype not in (torch.float16, torch.bfloat16) or addend.dtype != out_dtype or addend.data_ptr() % 16 or \
+                not addend.is_contiguous():
+            return int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias, out_dtype) + addend
+        c = torch.empty(m, n, dtype=out_dtype, device=a_q.device)
+        _l.check(_l.load().lq_gemm_int8_add(_ptr(c), _DT[out_dtype], _ptr(a_q), _ptr(w_rows32), _ptr(alpha_col), _ptr(alpha_row), _ptr(bias),
+                                            _ptr(addend), m, n, k, _stream()), "lq_gemm_int8_add")
+        return c
     c = torch.empty(m, n, dtype=out_dtype, device=a_q.device)
     _l.check(_l.load().lq_gemm_int8(_ptr(c), _DT[out_dtype], _ptr(a_q), _ptr(w_rows32), _ptr(alpha_col),
                                     _ptr(alpha_row), per_token, _ptr(bias), m, n, k, _stream()), "lq_gemm_int8")

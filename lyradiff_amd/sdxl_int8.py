@@ -87,10 +87,11 @@ def load_basic_transformer_int8(src, prefix: str, dim: int, cross_dim: int, leve
                                        i8("ff.net.0.proj", 8 * dim, dim), t16("ff.net.0.proj.bias", (8 * dim,)), ffn)
 
 
-def _gemm_int8(q8: torch.Tensor, lin: Int8Linear, dtype, bias=None) -> torch.Tensor:
-    """runGemmInt8 on codes that are already quantised with lin's static scale."""
+def _gemm_int8(q8: torch.Tensor, lin: Int8Linear, dtype, bias=None, addend=None) -> torch.Tensor:
+    """runGemmInt8 on codes that are already quantised with lin's static scale; addend [..., N]: joined to the rounded result."""
     m = q8.numel() // q8.shape[-1]
-    y = ops.int8_linear(q8.view(m, q8.shape[-1]), lin.weight_rows32, lin.weight_scale, lin.input_quant_scale, bias, dtype)
+    y = ops.int8_linear(q8.view(m, q8.shape[-1]), lin.weight_rows32, lin.weight_scale, lin.input_quant_scale, bias, dtype,
+                        None if addend is None else addend.reshape(m, -1))
     return y.view(*q8.shape[:-1], y.shape[-1])
 
 
@@ -148,4 +149,4 @@ def basic_transformer_int8_block(x: torch.Tensor, encoder_hidden_states: torch.T
     # feed-forward
     q8 = ops.int8_linear_geglu(q8.view(b * s, d), w.geglu.weight_rows32, w.geglu.weight_scale, w.geglu.input_quant_scale, w.geglu_bias,
                                w.ffn.pre_quant_scale, w.ffn.input_quant_scale, x.dtype).view(b, s, -1)
-    return _gemm_int8(q8, w.ffn, x.dtype, w.ffn.bias) + h2
+    return _gemm_int8(q8, w.ffn, x.dtype, w.ffn.bias, h2)

@@ -44,3 +44,23 @@ def test_other_forms_keep_to_the_two_kernels(dev):
         wide = ops.repack_weight(torch.ones(128, 256, device=dev, dtype=torch.int8))
         ops.int8_linear_geglu(torch.ones(4, 256, device=dev, dtype=torch.int8), wide, torch.ones(128, device=dev), row, torch.zeros(64, device=dev, dtype=torch.float16),
                               None, scale, torch.float16)
+
+
+# every configuration that the rule picks (64x64, k shared, 128x128, 128x256, 256x256 tiles), full and ragged tiles
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (130, 96, 192), (200, 640, 2560), (1024, 1280, 1280), (4096, 640, 2560), (4100, 1280, 640), (2048, 5120, 2048), (8192, 5120, 64)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_int8_linear_with_a_residual_is_the_sum(dev, m, n, k, dt):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    codes = lambda *s: torch.randint(-128, 128, s, generator=g, device=dev, dtype=torch.int8)
+    a, w = codes(m, k), ops.repack_weight(codes(n, k))
+    col, row = 1e-4 * torch.rand(n, generator=g, device=dev), torch.full((1,), 0.9, device=dev)
+    bias, add = torch.randn(n, generator=g, device=dev).to(dt), torch.randn(m, n, generator=g, device=dev).to(dt)
+    for b in (bias, None):
+        plain = ops.int8_linear(a, w, col, row, b, dt)
+        if m > 1:  # the same scale given per row
+            assert torch.equal(plain, ops.int8_linear(a, w, col, row.repeat(m), b, dt))
+        assert torch.equal(ops.int8_linear(a, w, col, row, b, dt, addend=add), plain + add)
+    strided = torch.randn(n, m, generator=g, device=dev).to(dt).t()
+    assert torch.equal(ops.int8_linear(a, w, col, row, bias, dt, addend=strided), ops.int8_linear(a, w, col, row, bias, dt) + strided)
