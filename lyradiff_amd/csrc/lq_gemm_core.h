@@ -779,6 +779,10 @@ struct GemmKernel {
         // overlap, and the specialisations keep the per-row code free of branches.
         // INT8: PLAIN has a scale per row, STATIC one for all of them; ADD joins a residual to that.
         constexpr int E_PLAIN = 0, E_ACT = 1, E_CODES = 2, E_GATED = 3, E_GENERAL = 4, E_STATIC = 5, E_STATIC_ADD = 6;
+        // CODES of full tiles, by activation (E_CODES_FULL + p.gelu).  The epilogue of such a GEMM is bound by vector instructions, beside the
+        // other workgroup's matrix ones: four rows go through it a step at a time, sixteen values of every step without a branch between
+        // them, rounded in pairs, one test for NaN for all of them, and a row's address is one addition.
+        constexpr int E_CODES_FULL = 8;
         constexpr bool kSpecialise = kExtras && ESZ == 2;  // fp32 outputs take the general path only (build time)
         int emode = kExtras ? E_GENERAL : E_PLAIN;
         if constexpr (kSpecialise) {
@@ -798,6 +802,9 @@ struct GemmKernel {
             static_assert(NITER % NB == 0, "strip rows are processed four at a time");
             const int mrow0 = m0 + wm * TM + i * 32 + out_row;
             const size_t idx0 = (size_t)mrow0 * p.n + out_n, rstep = (size_t)RPI * p.n;
+            constexpr bool CODES_FULL = MODE >= E_CODES_FULL;
+            const size_t c8_pitch = CODES_FULL ? (p.c8_panel ? 64 : p.ldc8) : 0;
+            uint8_t* const c8_row0 = !CODES_FULL ? nullptr : p.C8 + (p.c8_panel ? (size_t)(out_n >> 6) * p.m * 64 + (out_n & 63) : (size_t)out_n) + (size_t)mrow0 * c8_pitch;
 #pragma unroll
             for (int tb = 0; tb < NITER; tb += NB) {
                 v4i raw[NB];
@@ -811,6 +818,41 @@ struct GemmKernel {
                         if constexpr (MODE == E_STATIC_ADD)
                             if (FULL || (mrow0 + (tb + u) * RPI < p.m && n_ok)) OutStore<OutTag>::load4(p.addend, idx0 + (size_t)(tb + u) * rstep, joined[u]);
                     }
+                }
+                if constexpr (CODES_FULL) {
+                    float y[NB][4];
+                    auto each = [&](auto&& step) {
+#pragma unroll
+                        for (int u = 0; u < NB; ++u)
+#pragma unroll
+                            for (int e = 0; e < 4; e += 2) step(u, e);
+                    };
+                    each([&](int u, int e) {
+#pragma unroll
+                        for (int x = e; x < e + 2; ++x) {
+                            const float vf = __int_as_float(raw[u][x]);
+                            y[u][x] = ((KIND == K_FP8) ? vf * alpha : vf) + bias4[x];
+                        }
+                    });
+                    if constexpr (MODE == E_CODES_FULL + 2) each([&](int u, int e) { round_through2<OutTag>(y[u][e], y[u][e + 1]); });
+                    if constexpr (MODE > E_CODES_FULL) each([&](int u, int e) { y[u][e] = gelu_fast(y[u][e]); y[u][e + 1] = gelu_fast(y[u][e + 1]); });
+                    bool nan = false;
+                    each([&](int u, int e) {
+                        round_through2<OutTag>(y[u][e], y[u][e + 1]);
+                        y[u][e] *= c8_inv;
+                        y[u][e + 1] *= c8_inv;
+                        nan |= __builtin_isunordered(y[u][e], y[u][e + 1]);
+                    });
+                    u32 w[NB];
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) w[u] = cvt2_e4m3(y[u][2], y[u][3], cvt2_e4m3(y[u][0], y[u][1], 0u, false), true);
+                    if (__builtin_expect(nan, 0)) {
+#pragma unroll
+                        for (int u = 0; u < NB; ++u) w[u] = e4m3x4(y[u][0], y[u][1], y[u][2], y[u][3]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) *reinterpret_cast<u32*>(c8_row0 + (size_t)((tb + u) * RPI) * c8_pitch) = w[u];
+                    continue;
                 }
 #pragma unroll
                 for (int u = 0; u < NB; ++u) {
@@ -937,8 +979,10 @@ struct GemmKernel {
                 else if (tile_full) {
                     if (emode == E_PLAIN) all_bands(integral_constant<int, E_PLAIN>{}, std::true_type{});
                     else if (emode == E_ACT) all_bands(integral_constant<int, E_ACT>{}, std::true_type{});
-                    else if (emode == E_CODES) all_bands(integral_constant<int, E_CODES>{}, std::true_type{});
-                    else all_bands(integral_constant<int, E_GATED>{}, std::true_type{});
+                    else if (emode != E_CODES) all_bands(integral_constant<int, E_GATED>{}, std::true_type{});
+                    else if (p.gelu == 0) all_bands(integral_constant<int, E_CODES_FULL>{}, std::true_type{});
+                    else if (p.gelu == 1) all_bands(integral_constant<int, E_CODES_FULL + 1>{}, std::true_type{});
+                    else all_bands(integral_constant<int, E_CODES_FULL + 2>{}, std::true_type{});
                 } else {
                     if (emode == E_PLAIN) all_bands(integral_constant<int, E_PLAIN>{}, std::false_type{});
                     else if (emode == E_ACT) all_bands(integral_constant<int, E_ACT>{}, std::false_type{});

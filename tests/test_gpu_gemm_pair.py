@@ -60,3 +60,22 @@ def test_fp8_pair_with_an_empty_half_and_bad_arguments(dev):
         ops.fp8_linear_pair(ops.FP8Half(x, w, one, one), ops.FP8Half(x, w[:32], one, one), torch.float16)
     with pytest.raises(RuntimeError):  # outputs of two kinds
         ops.fp8_linear_pair(ops.FP8Half(x, w, one, one), ops.FP8Half(x, w, one, one, None, one), torch.float16)
+
+
+# codes of full tiles (four rows a step) against those of partial ones (value by value): the same problem with one row less; 64x64, 128x128
+# and 256-wide tiles, k shared between wavefront groups
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(64, 64, 128), (1024, 2048, 256), (256, 768, 2048), (4096, 3072, 1152), (4352, 3072, 1152)])
+@pytest.mark.parametrize("gelu", [0, 1, 2])
+def test_codes_of_full_and_of_partial_tiles_are_the_same(dev, m, n, k, dt, gelu):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    a, w = (torch.randn(r, k, generator=g, device=dev).clamp_(-4, 4).to(torch.float8_e4m3fn).view(torch.uint8) for r in (m, n))
+    bias = torch.randn(n, generator=g, device=dev)
+    bias[5], bias[n // 2], bias[n - 3] = float("inf"), float("-inf"), float("nan")
+    lin = (ops.repack_weight(w), torch.full((1,), k ** -0.5, device=dev), torch.ones(1, device=dev), bias.to(dt), torch.full((1,), 0.02, device=dev))
+    codes = lambda rows: ops.fp8_panels_to_rows(ops.fp8_linear_codes_panels(a[:rows].view(rows, k // 64, 64).transpose(0, 1).contiguous(), *lin, gelu=gelu,
+                                                                            round_dtype=dt))
+    full, part = codes(m), codes(m - 1)
+    assert torch.equal(full[:-1], part) and bool(((full[:, n - 3] & 0x7F) == 0x7F).all())
