@@ -781,7 +781,8 @@ struct GemmKernel {
         constexpr int E_PLAIN = 0, E_ACT = 1, E_CODES = 2, E_GATED = 3, E_GENERAL = 4, E_STATIC = 5, E_STATIC_ADD = 6;
         // CODES of full tiles, by activation (E_CODES_FULL + p.gelu).  The epilogue of such a GEMM is bound by vector instructions, beside the
         // other workgroup's matrix ones: four rows go through it a step at a time, sixteen values of every step without a branch between
-        // them, rounded in pairs, one test for NaN for all of them, and a row's address is one addition.
+        // them, rounded in pairs, one test for NaN for all of them, and a row's address is one addition.  us: 6912x12288x3072 with GELU
+        // 253 -> 229 under the tracer, double block 863 -> 851.
         constexpr int E_CODES_FULL = 8;
         constexpr bool kSpecialise = kExtras && ESZ == 2;  // fp32 outputs take the general path only (build time)
         int emode = kExtras ? E_GENERAL : E_PLAIN;
@@ -805,6 +806,15 @@ struct GemmKernel {
             constexpr bool CODES_FULL = MODE >= E_CODES_FULL;
             const size_t c8_pitch = CODES_FULL ? (p.c8_panel ? 64 : p.ldc8) : 0;
             uint8_t* const c8_row0 = !CODES_FULL ? nullptr : p.C8 + (p.c8_panel ? (size_t)(out_n >> 6) * p.m * 64 + (out_n & 63) : (size_t)out_n) + (size_t)mrow0 * c8_pitch;
+            // GATED of full tiles: a band's rows of the residual are requested at once.  One row at a time, each behind the store of the one in
+            // front of it (which the compiler has to take for the same memory), is a chain of round trips to memory.  us, whole FLUX blocks
+            // (FP8): double 832 -> 822, single at 6912 tokens 1344 -> 1330.
+            constexpr bool GATED_FULL = MODE == E_GATED && FULL && ESZ == 2;
+            uint2 residual[GATED_FULL ? NITER : 1];
+            if constexpr (GATED_FULL) {
+#pragma unroll
+                for (int t = 0; t < NITER; ++t) residual[t] = *reinterpret_cast<const uint2*>(static_cast<const unsigned short*>(p.residual) + idx0 + (size_t)t * rstep);
+            }
 #pragma unroll
             for (int tb = 0; tb < NITER; tb += NB) {
                 v4i raw[NB];
@@ -898,7 +908,13 @@ struct GemmKernel {
                         if constexpr (kExtras && (MODE == E_GATED || GEN)) {
                             if ((MODE == E_GATED || p.residual != nullptr) && ok) {
                                 float rr[4];
-                                OutStore<OutTag>::load4(p.residual, idx, rr);
+                                if constexpr (GATED_FULL) {
+                                    const u32 w[2] = {residual[t].x, residual[t].y};
+#pragma unroll
+                                    for (int e = 0; e < 4; ++e) rr[e] = Elem<OutTag>::load(e & 1 ? w[e / 2] >> 16 : w[e / 2] & 0xFFFFu);
+                                } else {
+                                    OutStore<OutTag>::load4(p.residual, idx, rr);
+                                }
                                 if (MODE == E_GATED || p.gate != nullptr) {
                                     if (!gate_uniform) OutStore<OutTag>::load4(p.gate, ((size_t)mo / p.gate_rows) * (size_t)p.n + out_n, gate4);
 #pragma unroll
