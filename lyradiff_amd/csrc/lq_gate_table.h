@@ -11,12 +11,10 @@ template <typename Tag> struct GateTable;
 template <> struct GateTable<F16Tag> { static constexpr u32 LO = 0x0C00u, COUNT = 0x4800u - 0x0C00u; };   // 2^-12 .. 8
 template <> struct GateTable<BF16Tag> { static constexpr u32 LO = 0x3980u, COUNT = 0x4100u - 0x3980u; };
 
-// the factor of a value without an entry, as bits of T: below the table the inner factor is 0.5, beyond it 0 or 1
-template <typename Tag> __device__ __forceinline__ u32 gate_outside_table(u32 bits) {
-    const float g = Elem<Tag>::load(bits), c = fabsf(g) < 1.0f ? 0.5f : (g < 0.0f ? 0.0f : 1.0f);
-    float y = g * c;
-    asm volatile("" : "+v"(y));
-    return Elem<Tag>::store(y);
+// the factor of a value without an entry, rounded to T: below the table the inner factor is 0.5, beyond it 0 or 1
+template <typename Tag> __device__ __forceinline__ float gate_outside_table(float g) {
+    const float c = fabsf(g) < 1.0f ? 0.5f : (g < 0.0f ? 0.0f : 1.0f);
+    return round_through<Tag>(g * c);
 }
 
 // The table of the current device, built before the stream's next kernel (lq_quant_int8.hip).

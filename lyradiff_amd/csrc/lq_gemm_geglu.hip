@@ -71,7 +71,7 @@ template <typename Tag, int MT> struct GegluGemm {
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         const u32 bits = (__builtin_bit_cast(u32, g[i]) >> (16 * e)) & 0xFFFFu;
-                        if ((bits & 0x7FFFu) - LO >= COUNT) gel[i][e] = __builtin_bit_cast(_Float16, (unsigned short)gate_outside_table<Tag>(bits));
+                        if ((bits & 0x7FFFu) - LO >= COUNT) gel[i][e] = (_Float16)gate_outside_table<Tag>((float)g[i][e]);
                     }
             }
 #pragma unroll
@@ -110,7 +110,7 @@ template <typename Tag, int MT> struct GegluGemm {
             if (__builtin_expect(far >= COUNT, 0)) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i)
-                    if ((gb[i] & 0x7FFFu) - LO >= COUNT) gel[i] = Elem<Tag>::load(gate_outside_table<Tag>(gb[i]));
+                    if ((gb[i] & 0x7FFFu) - LO >= COUNT) gel[i] = gate_outside_table<Tag>(Elem<Tag>::load(gb[i]));
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {

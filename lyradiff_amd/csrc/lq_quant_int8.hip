@@ -497,7 +497,7 @@ __global__ __launch_bounds__(THREADS, (SW == 2 && THREADS == 512) ? 4 : 1) void 
                     if (__builtin_expect(!all_in, 0)) {  // rare: outside the table the inner factor is a constant
 #pragma unroll
                         for (int i = 0; i < 8; ++i)
-                            if (!in[i]) gel[i] = Elem<Tag>::load(gate_outside_table<Tag>(Elem<Tag>::store(g[i])));
+                            if (!in[i]) gel[i] = gate_outside_table<Tag>(g[i]);
                     }
                 } else {
 #pragma unroll
