@@ -460,6 +460,8 @@ def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.
     if addend is not None:
         if addend.shape != (m, n):
             raise ValueError("addend must be [M, N]")
+        if not addend.is_cuda or addend.device != a_q.device:  # its pointer is read on the device
+            raise ValueError("addend must be on the device of a_q")
         if per_token or m * n == 0 or out_dtype not in (torch.float16, torch.bfloat16) or addend.dtype != out_dtype or addend.data_ptr() % 16 or \
                 not addend.is_contiguous():
             return int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias, out_dtype) + addend
