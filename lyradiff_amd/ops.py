@@ -801,6 +801,8 @@ def fp8_linear_rows(x, first, second=None):
             _chk(bias, "bias", (x.dtype,))
         if tuple(w.shape) != (n, k):
             raise ValueError("K mismatch between activation and weight" if second is None else "both weights must be [N, K]")
+        if a_scale.numel() != 1 or b_scale.numel() != 1 or (bias is not None and bias.numel() != n):
+            raise ValueError("a_scale and b_scale must hold one element, a bias [N]")
     y = torch.empty((m, n), dtype=x.dtype, device=x.device)
     y2 = torch.empty((m, n), dtype=x.dtype, device=x.device) if second is not None else None
     w2, a2, s2, b2 = second if second is not None else (None,) * 4
