@@ -342,7 +342,9 @@ int lq_gemm_fp8_gated(void* C, lq_dtype_t out_dtype, const uint8_t* A, const uin
 
 /* lq_fp8_scale_cast followed by lq_gemm_fp8 (scales and bias) for few rows, in one launch: x [m, k] of T, C [m, n] of T, a_scale the static
  * input scale.  Same bits.  With C2 (B2_rows32, a_scale2, b_scale2, bias2) a second linear of the same shape on the same x in that launch.
- * LQ_NOT_TAKEN (and nothing done) where the two calls are the better or the only way. */
+ * LQ_NOT_TAKEN (and nothing done) where the two calls are the better or the only way: where lq_linear_fp8_rows_takes is 0, which a caller
+ * can ask before it allocates the outputs, or x is not 16-byte aligned. */
+int lq_linear_fp8_rows_takes(int m, int n, int k);
 int lq_linear_fp8_rows(void* C, void* C2, const void* x, lq_dtype_t dtype, const uint8_t* B_rows32, const uint8_t* B2_rows32,
                        const float* a_scale, const float* a_scale2, const float* b_scale, const float* b_scale2, const void* bias,
                        const void* bias2, int m, int n, int k, lq_stream_t stream);

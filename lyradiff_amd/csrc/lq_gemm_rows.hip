@@ -145,6 +145,11 @@ int run_fp8_rows(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st) {
 
 using namespace lq;
 
+extern "C" int lq_linear_fp8_rows_takes(int m, int n, int k) {
+    const bool few_tiles = ((long)m + 255) / 256 * (((long)n + 255) / 256) < 192;  // where run_fp8_as turns to the rows kernel
+    return m >= 0 && m <= kCastRows && (long)m * k <= kCastElems && k > 1024 && k % 256 == 0 && few_tiles && requested_tactic(g_tactic_fp8, LQ_W_FP8, m, n, k) < 0;
+}
+
 extern "C" int lq_linear_fp8_rows(void* C, void* C2, const void* x, lq_dtype_t dtype, const uint8_t* B_rows32, const uint8_t* B2_rows32,
                                   const float* a_scale, const float* a_scale2, const float* b_scale, const float* b_scale2, const void* bias,
                                   const void* bias2, int m, int n, int k, lq_stream_t stream) {
@@ -154,10 +159,7 @@ extern "C" int lq_linear_fp8_rows(void* C, void* C2, const void* x, lq_dtype_t d
     if (m == 0) return LQ_OK;
     const bool two = C2 != nullptr;
     LQ_REQUIRE(C && x && B_rows32 && a_scale && b_scale && (!two || (B2_rows32 && a_scale2 && b_scale2)), LQ_ERR_ARG, "lq_linear_fp8_rows: null pointer");
-    const bool few_tiles = ((long)m + 255) / 256 * (((long)n + 255) / 256) < 192;  // where run_fp8_as turns to the rows kernel
-    if (m > kCastRows || (long)m * k > kCastElems || k <= 1024 || k % 256 != 0 || !few_tiles || reinterpret_cast<uintptr_t>(x) % 16 != 0 ||
-        tl_forced_tactic >= 0 || requested_tactic(g_tactic_fp8, LQ_W_FP8, m, n, k) >= 0)
-        return LQ_NOT_TAKEN;
+    if (!lq_linear_fp8_rows_takes(m, n, k) || reinterpret_cast<uintptr_t>(x) % 16 != 0) return LQ_NOT_TAKEN;
     LQ_REQUIRE((reinterpret_cast<uintptr_t>(B_rows32) | reinterpret_cast<uintptr_t>(C) | reinterpret_cast<uintptr_t>(B2_rows32) |
                 reinterpret_cast<uintptr_t>(C2)) % 16 == 0 && (reinterpret_cast<uintptr_t>(bias) | reinterpret_cast<uintptr_t>(bias2)) % 8 == 0,
                LQ_ERR_ARG, "lq_linear_fp8_rows: B and C must be 16-byte aligned, bias 8-byte aligned");

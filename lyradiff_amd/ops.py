@@ -786,6 +786,11 @@ def fp8_linear_codes_panels(a_panels, w_rows32, a_scale, b_scale, bias, out_fp8_
     return out
 
 
+def fp8_linear_rows_takes(m: int, n: int, k: int) -> bool:
+    """True for the sizes that fp8_linear_rows has a kernel for (lq_linear_fp8_rows_takes)."""
+    return m <= 8 and bool(_l.load().lq_linear_fp8_rows_takes(m, n, k))
+
+
 def fp8_linear_rows(x, first, second=None):
     """fp8_scale_cast and fp8_linear of few rows in one launch: x [M, K] fp16 / bf16 -> [M, N] of its type, same bits.  first: (w_rows32,
     static input scale, weight scale, bias or None); second: another linear of that shape on the same x, whose result then comes as a second
@@ -793,6 +798,8 @@ def fp8_linear_rows(x, first, second=None):
     _chk(x, "x", (torch.float16, torch.bfloat16))
     m, k = x.shape
     n = first[0].shape[0]
+    if not fp8_linear_rows_takes(m, n, k):
+        return None
     for w, a_scale, b_scale, bias in (first, second) if second is not None else (first,):
         _chk(w, "w_rows32", (torch.uint8,))
         _chk(a_scale, "a_scale", (torch.float32,))

@@ -257,14 +257,17 @@ struct AdaLinear {
     std::pair<at::Tensor, at::Tensor> msa_of(const at::Tensor& temb, int64_t chunks, const AdaLinear* other) const {
         const int64_t b = temb.size(0), d = temb.size(1), n = chunks * d;
         const lq_dtype_t dt = lq_dt(temb.scalar_type());
-        at::Tensor y = at::empty({b, n}, temb.options()), y2;
-        if (other != nullptr) y2 = at::empty({b, n}, temb.options());
+        const bool rows = fp8 ? lq_linear_fp8_rows_takes((int)b, (int)n, (int)d) != 0
+                              : b <= 256 && d % 64 == 0 && reinterpret_cast<uintptr_t>(P(temb)) % 16 == 0 && !(at::GradMode::is_enabled() && temb.requires_grad());
+        at::Tensor y, y2;
         int rc = LQ_NOT_TAKEN;
-        if (fp8)
+        if (rows) y = at::empty({b, n}, temb.options());
+        if (rows && other != nullptr) y2 = at::empty({b, n}, temb.options());
+        if (rows && fp8)
             rc = lq_linear_fp8_rows(P(y), P(y2), P(temb), dt, P8(q.w_rows32), other ? P8(other->q.w_rows32) : nullptr, PF(q.in_scale),
                                     other ? PF(other->q.in_scale) : nullptr, PF(q.w_scale), other ? PF(other->q.w_scale) : nullptr, P(q.bias),
                                     other ? P(other->q.bias) : nullptr, (int)b, (int)n, (int)d, cur_stream());
-        else if (b <= 256 && d % 64 == 0 && reinterpret_cast<uintptr_t>(P(temb)) % 16 == 0 && !(at::GradMode::is_enabled() && temb.requires_grad()))
+        else if (rows)
             rc = lq_linear16_rows(P(y), P(y2), P(temb), P(weight), other ? P(other->weight) : nullptr, P(bias), other ? P(other->bias) : nullptr, dt,
                                   (int)b, (int)n, (int)d, cur_stream());
         if (rc < 0) ok(rc, "adaLN linear");

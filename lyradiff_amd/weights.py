@@ -145,7 +145,8 @@ class FP8Linear:
 
     def forward(self, x: torch.Tensor, gelu: bool = False, residual=None, beta: float = 0.0, dynamic: bool = False) -> torch.Tensor:
         x2 = _rows(x)
-        if not dynamic and not gelu and residual is None and x2.shape[0] <= 8 and x2.dtype != torch.float32:
+        if not dynamic and not gelu and residual is None and x2.dtype != torch.float32 and \
+                ops.fp8_linear_rows_takes(x2.shape[0], self.weight_rows32.shape[0], x2.shape[1]):
             y = ops.fp8_linear_rows(x2, (self.weight_rows32, self.input_scale, self.weight_scale, self.bias))
             if y is not None:
                 return _shaped(y, x)

@@ -1,16 +1,31 @@
 """What the Python wrappers refuse, and which route they take, before anything is enqueued (no GPU: a call that reaches the library fails
 the test)."""
+import ctypes as C
+
 import pytest
 import torch
 
 
+class _Rules:
+    """The library's functions that answer a question on the host; any other fails the test."""
+
+    def __init__(self, lib):
+        self.lib = lib
+
+    def __getattr__(self, name):
+        if not name.endswith("_takes"):
+            pytest.fail(f"{name} was called")
+        return getattr(self.lib, name)
+
+
 @pytest.fixture
 def ops(monkeypatch):
-    """ops whose operands count as device tensors and whose library must not be called."""
+    """ops whose operands count as device tensors and whose library answers questions only."""
     from lyradiff_amd import ops as _ops
 
+    rules = _Rules(_ops._l.load())
     monkeypatch.setattr(_ops, "_chk", lambda t, name, dtypes=None: t)
-    monkeypatch.setattr(_ops._l, "load", lambda: pytest.fail("the call reached the library"))
+    monkeypatch.setattr(_ops._l, "load", lambda: rules)
     return _ops
 
 
@@ -31,3 +46,36 @@ def test_fp8_linear_rows_refuses_short_scales_and_biases(ops, which, bad):
         ops.fp8_linear_rows(x, *((wrong, tuple(lin)) if which == 0 else (tuple(lin), wrong)))
     with pytest.raises(ValueError, match="one element"):
         ops.fp8_linear_rows(x, wrong)
+
+
+SIZES = [(m, n, k) for m in (1, 2, 4, 5, 8, 9) for n in (64, 9216, 32 * 1536) for k in (1024, 1280, 1344, 1536, 3072, 12288)]
+
+
+def test_fp8_rows_rule_is_that_of_the_entry_point():
+    """A misaligned weight is refused behind the rule and in front of any launch."""
+    from lyradiff_amd import lib as L, ops as _ops
+
+    lib, at, odd = L.load(), C.c_void_p(16), C.c_void_p(8)
+    taken = 0
+    for m, n, k in SIZES:
+        takes = _ops.fp8_linear_rows_takes(m, n, k)
+        assert lib.lq_linear_fp8_rows(at, None, at, L.LQ_F16, odd, None, at, None, at, None, None, None, m, n, k, None) == (-1 if takes else 1), (m, n, k)
+        assert takes == (m <= 8 and m * k <= 12288 and k > 1024 and k % 256 == 0 and n < 32 * 1536), (m, n, k)
+        taken += takes
+        with _ops.gemm_thread_tactic(2):
+            assert not _ops.fp8_linear_rows_takes(m, n, k)
+    assert taken > 0
+
+
+@pytest.mark.parametrize("m", [5, 8, 9])
+def test_fp8_linears_of_a_few_more_rows_go_straight_to_the_two_calls(ops, monkeypatch, m):
+    from lyradiff_amd import weights
+
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: pytest.fail("an output was allocated"))
+    x, w, one = torch.zeros(m, 3072, dtype=torch.float16), torch.zeros(64, 3072, dtype=torch.uint8), torch.ones(1)
+    lin = (w, one, one, None)
+    assert ops.fp8_linear_rows(x, lin) is None and ops.fp8_linear_rows(x, lin, lin) is None
+    monkeypatch.setattr(ops, "fp8_linear_rows", lambda *a: pytest.fail("the few-rows route was tried"))
+    monkeypatch.setattr(ops, "fp8_scale_cast_panels", lambda x, scale: "codes")
+    monkeypatch.setattr(ops, "fp8_linear_panels", lambda q, *a: torch.zeros(m, 64))
+    assert weights.FP8Linear(w, one, one).forward(x).shape == (m, 64)
