@@ -377,6 +377,7 @@ typedef struct {
     const void* residual;
     int m;
 } lq_fp8_half_t;
+int lq_gemm_fp8_pair_takes(int m, int m2, int n, int k, int plain); /* 1: one launch (plain: outputs of the first kind), 0: one after the other */
 int lq_gemm_fp8_pair(const lq_fp8_half_t* halves, lq_dtype_t dtype, int gelu, int panels, int n, int k, lq_stream_t stream);
 
 /* lq_gemm_fp8 that writes only e4m3 codes of its output, into a destination whose rows are `ldc` bytes apart:

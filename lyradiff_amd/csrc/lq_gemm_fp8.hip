@@ -161,28 +161,47 @@ extern "C" int lq_gemm_fp8_codes_panels(uint8_t* C_fp8_panels, const float* C_fp
                           m, n, k, 1, stream);
 }
 
-// The form for both problems in one launch, by the tiles of the two together and the lines of run_fp8_as; -1: one after the other.
-// The second problem's tiles by themselves leave most of the chip idle for a whole walk over k.  Measured (us, bf16, k-panels, two
-// launches / one), 4096 + 512 rows: 9216x3072 119 / 114, 3072x3072 48 / 39, 12288x3072 with GELU to codes 179 / 165, 3072x12288 with
-// gate 159 / 138; 1200 + 512 rows: 58 / 43, 27 / 23, 86 / 75, 80 / 79; 400 + 100 rows: 30 / 23, 16 / 10, 47 / 35, 47 / 31.
-static int pair_form(const GemmParams& a, const GemmParams& b) {
-    if (a.m <= 32 || b.m <= 32) return -1;  // few rows have a kernel of their own
-    for (const GemmParams* p : {&a, &b})
-        if (tl_forced_tactic >= 0 || requested_tactic(g_tactic_fp8, LQ_W_FP8, p->m, p->n, p->k) >= 0) return -1;  // tactics stand
-    auto tiles = [&](int rows, int cols) { return ((long)(a.m + rows - 1) / rows + (b.m + rows - 1) / rows) * ((a.n + cols - 1) / cols); };
-    const long t256 = tiles(256, 256), t128 = tiles(128, 128);
-    if (a.k <= 1024) return t128 >= 128 ? 2 : 3;
-    if (t256 < 192) {  // where the tiles of the second only open another round, two launches are ahead (2500 + 200 rows, 3072x12288: 115 against 126 us)
-        float both, first, second;
-        const int form = few_tiles_form(a.m, b.m, a.n, a.k, &both);
-        few_tiles_form(a.m, 0, a.n, a.k, &first);
-        few_tiles_form(b.m, 0, b.n, b.k, &second);
-        return both < first + second ? form : -1;
+static long pair_tiles(int m, int m2, int n, int rows, int cols) {
+    return (((long)m + rows - 1) / rows + ((long)m2 + rows - 1) / rows) * (((long)n + cols - 1) / cols);
+}
+
+// The form of one launch over m and m2 rows and its time (us at k = 3072), by the lines of run_fp8_as; persist: 256x256 tiles that are all
+// full run in the persistent form there.  A round of 256 256x256 tiles or of 512 128x256 tiles takes 38, of the persistent form 35, and
+// up to 256 128x256 tiles behind full rounds 18.
+static int launch_form(int m, int m2, int n, int k, bool plain, bool persist, float* cost) {
+    const long t256 = pair_tiles(m, m2, n, 256, 256), last256 = t256 % 256;
+    if (t256 < 192) return few_tiles_form(m, m2, n, k, cost);
+    *cost = (float)((t256 + 255) / 256) * (persist && t256 > 256 ? 35.0f : 38.0f);
+    const bool wide = (last256 != 0 && last256 < 128) || (!plain && t256 > 256);
+    if (!wide || (persist && t256 > 256)) return plain ? 6 : 0;
+    const long t4 = pair_tiles(m, m2, n, 128, 256), left = t4 % 512;
+    *cost = (float)(t4 / 512) * 38.0f + (left == 0 ? 0.0f : left <= 256 ? 18.0f : 38.0f);
+    return 4;
+}
+
+// The form for both problems in one launch; -1: one after the other.  The second problem's tiles by themselves leave most of the chip idle
+// for a whole walk over k; behind the first one's they cost nothing where its last round has room for them, and most of a round where it
+// has not: the times of the rounds decide.  Measured (us, bf16, k-panels, two launches / one), 4096 + 512 rows: 9216x3072 121 / 114,
+// 3072x3072 48 / 39, 12288x3072 with GELU to codes 161 / 153, 3072x12288 with gate 160 / 141; 6400 + 512: 176 / 160, 80 / 60, 244 / 236,
+// 252 / 231; 400 + 100: 30 / 23, 16 / 10, 47 / 35, 47 / 31.  Two launches are ahead where the second only opens another round: 5120 + 512
+// rows 3072x3072 51 / 57, 3072x12288 with gate 180 / 205; 8192 + 512 rows 3072x12288 277 / 297; 6144 + 64 rows 9216x3072 151 / 154 (the
+// persistent form), 12288x3072 to codes 209 / 218; 4096 + 77 rows 12288x3072 147 / 153; 2500 + 200 rows 3072x12288 115 / 126.
+static int pair_form(int m, int m2, int n, int k, bool plain) {
+    if (m <= 32 || m2 <= 32) return -1;  // few rows have a kernel of their own
+    for (int rows : {m, m2})
+        if (requested_tactic(g_tactic_fp8, LQ_W_FP8, rows, n, k) >= 0) return -1;  // tactics stand
+    if (k <= 1024) return pair_tiles(m, m2, n, 128, 128) >= 128 ? 2 : 3;
+    float both, alone[2];
+    const int form = launch_form(m, m2, n, k, plain, false, &both);
+    for (int i = 0; i < 2; ++i) {
+        const int rows = i ? m2 : m;
+        launch_form(rows, 0, n, k, plain, plain && rows % 256 == 0 && n % 256 == 0 && k % 128 == 0, &alone[i]);
     }
-    const bool plain = a.gelu == 0 && a.C8 == nullptr && a.gate == nullptr;
-    const long last256 = t256 % 256;
-    if (last256 != 0 && last256 < 128) return 4;
-    return plain ? 6 : (t256 > 256 ? 4 : 0);
+    return both < alone[0] + alone[1] ? form : -1;
+}
+
+extern "C" int lq_gemm_fp8_pair_takes(int m, int m2, int n, int k, int plain) {
+    return m > 0 && m2 > 0 && n > 0 && k > 0 && pair_form(m, m2, n, k, plain != 0) >= 0;
 }
 
 extern "C" int lq_gemm_fp8_pair(const lq_fp8_half_t* halves, lq_dtype_t dtype, int gelu, int panels, int n, int k, lq_stream_t stream) {
@@ -216,7 +235,7 @@ extern "C" int lq_gemm_fp8_pair(const lq_fp8_half_t* halves, lq_dtype_t dtype, i
         const GemmParams &a = pair.p[0], &b = pair.p[1];
         LQ_REQUIRE((a.C8 == nullptr) == (b.C8 == nullptr) && (a.gate == nullptr) == (b.gate == nullptr), LQ_ERR_ARG,
                    "lq_gemm_fp8_pair: both halves need the same outputs");
-        const int form = pair_form(a, b);
+        const int form = pair_form(a.m, b.m, n, k, a.gelu == 0 && a.C8 == nullptr && a.gate == nullptr);
         if (form >= 0) return dtype == LQ_BF16 ? run_fp8_pair_bf16(pair, form, as_stream(stream)) : run_fp8_pair_f16(pair, form, as_stream(stream));
     }
     for (int i = 0; i < problems; ++i) {

@@ -79,3 +79,16 @@ def test_fp8_linears_of_a_few_more_rows_go_straight_to_the_two_calls(ops, monkey
     monkeypatch.setattr(ops, "fp8_scale_cast_panels", lambda x, scale: "codes")
     monkeypatch.setattr(ops, "fp8_linear_panels", lambda q, *a: torch.zeros(m, 64))
     assert weights.FP8Linear(w, one, one).forward(x).shape == (m, 64)
+
+
+# rows of both, n, k, scales and bias only; 1: measured ahead in one launch, 0: ahead one after the other (lq_gemm_fp8.hip has the times)
+@pytest.mark.parametrize("m,m2,n,k,plain,one", [
+    (4096, 512, 9216, 3072, 1, 1), (6400, 512, 3072, 3072, 1, 1), (6400, 512, 12288, 3072, 0, 1), (6400, 512, 3072, 12288, 0, 1), (400, 100, 3072, 12288, 0, 1),
+    (5120, 512, 3072, 3072, 1, 0), (5120, 512, 3072, 12288, 0, 0), (8192, 512, 3072, 12288, 0, 0), (6144, 64, 9216, 3072, 1, 0),
+    (6144, 64, 12288, 3072, 0, 0), (4096, 77, 12288, 3072, 0, 0), (2500, 200, 3072, 12288, 0, 0), (4096, 32, 3072, 3072, 1, 0)])
+def test_fp8_pairs_share_a_launch_where_that_is_faster(m, m2, n, k, plain, one):
+    from lyradiff_amd import lib as L, ops as _ops
+
+    assert L.load().lq_gemm_fp8_pair_takes(m, m2, n, k, plain) == one
+    with _ops.gemm_thread_tactic(2):
+        assert L.load().lq_gemm_fp8_pair_takes(m, m2, n, k, plain) == 0
