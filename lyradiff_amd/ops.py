@@ -12,6 +12,7 @@ import ctypes as C
 from typing import NamedTuple, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import lib as _l
 
@@ -47,6 +48,27 @@ def _stream():
 
 
 _FLOATS = (torch.float32, torch.float16, torch.bfloat16)
+
+_transforms = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", None)
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
+
+
+def _plain(*tensors) -> bool:
+    """True when a kernel may stand in for PyTorch operations on the tensors (None is passed over): ordinary dense tensors on the current
+    device in eager mode, no gradient recorded, no forward-mode tangent, and nothing around the call that has to see the operations
+    (vmap and the other function transforms, tracing, compilation, dispatch modes such as fake tensors)."""
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or (_transforms is not None and _transforms() is not None) or \
+            (_dispatch_modes is not None and _dispatch_modes()):
+        return False
+    grad, duals = torch.is_grad_enabled(), forward_ad._current_level >= 0
+    for t in tensors:
+        if t is None:
+            continue
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.layout is not torch.strided or (grad and t.requires_grad) or \
+                (duals and forward_ad.unpack_dual(t).tangent is not None) or \
+                (t.is_cuda and t.get_device() != (torch.cuda.current_device() if _raw_device is None else _raw_device())):
+            return False
+    return True
 
 
 # ---- INT8 SmoothQuant ---------------------------------------------------------------------------
@@ -462,8 +484,8 @@ def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.
             raise ValueError("addend must be [M, N]")
         if not addend.is_cuda or addend.device != a_q.device:  # its pointer is read on the device
             raise ValueError("addend must be on the device of a_q")
-        if per_token or m * n == 0 or out_dtype not in (torch.float16, torch.bfloat16) or addend.dtype != out_dtype or addend.data_ptr() % 16 or \
-                not addend.is_contiguous():
+        if per_token or m * n == 0 or out_dtype not in (torch.float16, torch.bfloat16) or addend.dtype != out_dtype or not _plain(addend) or \
+                not addend.is_contiguous() or addend.data_ptr() % 16:
             return int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias, out_dtype) + addend
         c = torch.empty(m, n, dtype=out_dtype, device=a_q.device)
         _l.check(_l.load().lq_gemm_int8_add(_ptr(c), _DT[out_dtype], _ptr(a_q), _ptr(w_rows32), _ptr(alpha_col), _ptr(alpha_row), _ptr(bias),

@@ -64,3 +64,24 @@ def test_int8_linear_with_a_residual_is_the_sum(dev, m, n, k, dt):
         assert torch.equal(ops.int8_linear(a, w, col, row, b, dt, addend=add), plain + add)
     strided = torch.randn(n, m, generator=g, device=dev).to(dt).t()
     assert torch.equal(ops.int8_linear(a, w, col, row, bias, dt, addend=strided), ops.int8_linear(a, w, col, row, bias, dt) + strided)
+
+
+def test_a_residual_that_pytorch_has_to_see_is_added_by_pytorch(dev):
+    """A sum that records a gradient, carries a tangent or runs under vmap, as it was with a sum behind the linear."""
+    from torch.autograd import forward_ad
+
+    from lyradiff_amd import ops
+
+    a, w = torch.ones(8, 64, device=dev, dtype=torch.int8), ops.repack_weight(torch.ones(32, 64, device=dev, dtype=torch.int8))
+    call = lambda r: ops.int8_linear(a, w, torch.full((32,), 1e-2, device=dev), torch.ones(1, device=dev), None, torch.float16, addend=r)
+    res = torch.randn(3, 8, 32, device=dev).half()
+    want = torch.stack([call(r) for r in res])
+    leaf = res[0].clone().requires_grad_()
+    call(leaf).backward(res[1])
+    assert torch.equal(leaf.grad, res[1])
+    with torch.no_grad():
+        assert torch.equal(call(leaf), want[0])
+    with forward_ad.dual_level():
+        y, tangent = forward_ad.unpack_dual(call(forward_ad.make_dual(res[0], res[1])))
+        assert torch.equal(y, want[0]) and torch.equal(tangent, res[1])
+    assert torch.equal(torch.vmap(call)(res), want)
