@@ -848,18 +848,18 @@ _LINEAR16_ROWS = 256
 
 def linear16_supported(x, *tensors) -> bool:
     """True when linear16 and linear16_pair take x [.., K] and the weights and biases `tensors`: few rows, dense 16-bit GPU tensors of one type,
-    aligned, no gradient recorded."""
-    k = x.shape[-1]
-    if x.dtype not in (torch.float16, torch.bfloat16) or k == 0 or k % 64 or x.numel() > _LINEAR16_ROWS * k or x.numel() == 0:
+    aligned, in a call that PyTorch need not see (_plain) and would not cast (autocast)."""
+    if x.dtype not in (torch.float16, torch.bfloat16) or x.dim() == 0 or not _plain(x, *tensors):
         return False
-    grad = torch.is_grad_enabled()
+    k = x.shape[-1]
+    if k == 0 or k % 64 or x.numel() > _LINEAR16_ROWS * k or x.numel() == 0:
+        return False
     for t in (x, *tensors):
         if t is None:
             continue
-        if not t.is_cuda or t.dtype != x.dtype or not t.is_contiguous() or t.data_ptr() % 16 or (grad and t.requires_grad) or \
-                (t is not x and t.shape[0] % 4):
+        if not t.is_cuda or t.dtype != x.dtype or not t.is_contiguous() or t.data_ptr() % 16 or (t is not x and (t.dim() == 0 or t.shape[0] % 4)):
             return False
-    return True
+    return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype
 
 
 def linear16(x, weight, bias=None):

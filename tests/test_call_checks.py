@@ -92,3 +92,26 @@ def test_fp8_pairs_share_a_launch_where_that_is_faster(m, m2, n, k, plain, one):
     assert L.load().lq_gemm_fp8_pair_takes(m, m2, n, k, plain) == one
     with _ops.gemm_thread_tactic(2):
         assert L.load().lq_gemm_fp8_pair_takes(m, m2, n, k, plain) == 0
+
+
+def test_plain_calls_are_told_from_those_that_pytorch_has_to_see():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.autograd import forward_ad
+
+    from lyradiff_amd import ops as _ops
+
+    x, seen = torch.zeros(2, 4), []
+    look = lambda t: (seen.append(_ops._plain(t)), t)[1]
+    leaf = x.clone().requires_grad_()
+    assert _ops._plain(x, None, torch.nn.Parameter(x, requires_grad=False)) and not _ops._plain(x, leaf) and not _ops._plain(x.to_sparse())
+    with torch.no_grad():
+        assert _ops._plain(leaf)
+    torch.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    torch.jit.trace(look, (x,), check_trace=False)
+    with FakeTensorMode() as mode:
+        look(mode.from_tensor(x))
+    with forward_ad.dual_level():
+        look(forward_ad.make_dual(x, x))
+        assert _ops._plain(x)
+    assert len(seen) >= 5 and not any(seen)

@@ -87,3 +87,33 @@ def test_linear16_takes_batches_and_leaves_the_rest_to_pytorch(dev):
         assert ops.linear16_supported(leaf, w)
     with pytest.raises(RuntimeError):
         ops.linear16(r(2, 128), r(64, 192))
+
+
+def test_linear16_is_pytorchs_where_pytorch_has_to_see_it(dev):
+    """Forward-mode tangents, vmap, function transforms, fake tensors, dispatch modes, tracing and autocast, through the layer that uses it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.autograd import forward_ad
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from lyradiff_amd import ops, sdxl_int8
+
+    F = torch.nn.functional
+    r = lambda *s: torch.randn(*s, device=dev, generator=torch.Generator(device=dev).manual_seed(sum(s))).half()
+    x, w, b = r(3, 8, 128), r(64, 128), r(64)
+    lin = sdxl_int8.Linear16(w, b).forward
+    with forward_ad.dual_level():
+        assert ops.linear16_supported(x, w)  # a level without a tangent changes nothing
+        dual = forward_ad.make_dual(x, 2 * x)
+        got, want = (forward_ad.unpack_dual(f(dual)) for f in (lin, lambda t: F.linear(t, w, b)))
+        assert torch.equal(got.primal, want.primal) and torch.equal(got.tangent, want.tangent)
+        assert all(forward_ad.unpack_dual(y).tangent is not None for y in ops.linear16_pair(dual, w, w))
+    assert torch.equal(torch.vmap(lin)(x), torch.vmap(lambda t: F.linear(t, w, b))(x))
+    assert all(torch.equal(g, e) for g, e in zip(torch.func.jvp(lin, (x,), (x,)), torch.func.jvp(lambda t: F.linear(t, w, b), (x,), (x,))))
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        assert lin(mode.from_tensor(x)).shape == (3, 8, 64)
+    with FlopCounterMode(display=False) as flops:
+        lin(x)
+    assert flops.get_total_flops() == 2 * x.numel() * 64
+    assert torch.equal(torch.jit.trace(lin, (x[:1],))(x), F.linear(x, w, b))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert lin(x).dtype == torch.bfloat16
