@@ -252,13 +252,16 @@ struct AdaLinear {
         const int64_t b = flat.size(0);
         return b > 1 ? flat.view({b, chunks, d}).transpose(0, 1).contiguous() : flat.view({chunks, 1, d});
     }
+    static bool aligned(const at::Tensor& t, uintptr_t bytes) { return reinterpret_cast<uintptr_t>(P(t)) % bytes == 0; }
+    bool rows16() const { return aligned(weight, 16) && aligned(bias, 8); }  // a view into a larger buffer need not be: at::linear takes it
     at::Tensor msa(const at::Tensor& temb, int64_t chunks) const { return msa_of(temb, chunks, nullptr).first; }
     // with `other`, the adaLN linear of the other half of a double-stream block (same temb), both: in one launch where few rows let it
     std::pair<at::Tensor, at::Tensor> msa_of(const at::Tensor& temb, int64_t chunks, const AdaLinear* other) const {
         const int64_t b = temb.size(0), d = temb.size(1), n = chunks * d;
         const lq_dtype_t dt = lq_dt(temb.scalar_type());
         const bool rows = fp8 ? lq_linear_fp8_rows_takes((int)b, (int)n, (int)d) != 0
-                              : b <= 256 && d % 64 == 0 && reinterpret_cast<uintptr_t>(P(temb)) % 16 == 0 && !(at::GradMode::is_enabled() && temb.requires_grad());
+                              : b <= 256 && d % 64 == 0 && aligned(temb, 16) && rows16() && (other == nullptr || other->rows16()) &&
+                                    !(at::GradMode::is_enabled() && temb.requires_grad());
         at::Tensor y, y2;
         int rc = LQ_NOT_TAKEN;
         if (rows) y = at::empty({b, n}, temb.options());

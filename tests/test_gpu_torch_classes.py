@@ -137,6 +137,31 @@ def test_fp8_block_classes_equal_the_python_ops_and_match_the_fp64_restatement(c
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("names", [("norm1.linear.weight",), ("norm1_context.linear.weight", "norm1_context.linear.bias"), ("norm1.linear.bias",)])
+def test_16_bit_modulation_weights_may_be_views_at_any_offset(classes, ops, dev, names):
+    """Parts of one flat device buffer, as a checkpoint loaded in one piece leaves them; the few-rows kernel asks for 16 and 8 bytes."""
+    from lyradiff_amd import flux_ops as FO
+
+    b, s, sc, heads, dh = 1, 96, 32, 4, 64
+    d = heads * dh
+    sd = _block_state(d, dh, 405, ("t.",))
+    args = [_fp8_inputs(dev, b, s, sc, heads, dh, 506)[i] for i in (0, 1, 3, 2)]
+
+    def forward(cls):
+        op = cls("bf16", d, heads, dh, 4, 1)
+        op.reload_model_from_state_dict("t.", sd, "cpu")
+        return op.forward(*args)
+
+    want = forward(classes.FluxTransformerBlockOp)
+    for n in names:
+        t, off = sd["t." + n], 4 if n.endswith("weight") else 2
+        sd["t." + n] = torch.cat([t.new_zeros(off), t.flatten()]).to(dev)[off:].view(t.shape)
+    got = forward(classes.FluxTransformerBlockOp)
+    for y, p, w in zip(got, forward(FO.FluxTransformerBlockOp), want):
+        assert torch.equal(y, p) and _rel(y, w) < 0.02
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("file_dtype", ["fp32", "bf16"])
 def test_fp8_block_classes_reload_model_from_bin(classes, ops, dev, tmp_path, file_dtype):
     """reload_model_from_bin(model_path, model_dtype) (FluxTransformerBlockOp.h:239-258): raw files model_path + name + ".bin";
