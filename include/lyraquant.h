@@ -91,7 +91,10 @@ int lq_geglu_int8(int8_t* dst, const void* hidden, const void* bias, lq_dtype_t 
 
 /* lq_gemm_int8 (static scale alpha_row[0], no bias, rounded to `dtype`) and lq_geglu_int8 on its output in one kernel, the same bits
  * without the [m, 2 * inner] tensor: A [m, k] int8, B_rows32 of 2 * inner rows, alpha_col [2 * inner], bias [2 * inner] of dtype or NULL,
- * pre_quant_scale [inner] or NULL, out [m, inner].  dtype in {F16, BF16}; inner % 64 == 0, k % 64 == 0, k >= 256. */
+ * pre_quant_scale [inner] or NULL, out [m, inner].  dtype in {F16, BF16}; inner % 64 == 0, k % 64 == 0, k >= 256.
+ * lq_gemm_int8_geglu_takes: 1 where a caller does well to use it, 0 for other sizes and where a tactic is forced or cached for the GEMM of
+ * 2 * inner columns, which has one tile configuration here and all of them there. */
+int lq_gemm_int8_geglu_takes(int m, int inner, int k);
 int lq_gemm_int8_geglu(int8_t* out, const int8_t* A, const int8_t* B_rows32, const float* alpha_col, const float* alpha_row, const void* bias,
                        lq_dtype_t dtype, const float* pre_quant_scale, const float* input_quant_scale, int m, int inner, int k,
                        lq_stream_t stream);

@@ -290,6 +290,11 @@ template <typename Tag> static int geglu_gemm_typed(GegluParams p, hipStream_t s
 
 using namespace lq;
 
+extern "C" int lq_gemm_int8_geglu_takes(int m, int inner, int k) {
+    return m >= 0 && inner > 0 && inner % 64 == 0 && inner < (1 << 29) && k >= 256 && k % 64 == 0 &&
+           requested_tactic(g_tactic_int8, LQ_W_INT8, m, 2 * inner, k) < 0;  // tactics stand
+}
+
 extern "C" int lq_gemm_int8_geglu(int8_t* out, const int8_t* A, const int8_t* B_rows32, const float* alpha_col, const float* alpha_row, const void* bias,
                                   lq_dtype_t dtype, const float* pre_quant_scale, const float* input_quant_scale, int m, int inner, int k,
                                   lq_stream_t stream) {

@@ -60,6 +60,7 @@ SYMBOLS = {
     "lq_sq_output_dequant": (_I, [_P, _I, _P, _P, _P, _I, _Z, _Z, _P]),
     "lq_int8_weight_quant": (_I, [_P, _P, _P, _I, _P, _Z, _Z, _P]),
     "lq_geglu_int8": (_I, [_P, _P, _P, _I, _P, _P, _Z, _Z, _P]),
+    "lq_gemm_int8_geglu_takes": (_I, [_I, _I, _I]),
     "lq_gemm_int8_geglu": (_I, [_P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _I, _P]),
     "lq_geglu_int8_dynamic": (_I, [_P, _P, _P, _P, _I, _P, _Z, _Z, _P]),
     "lq_fp8_amax_scale": (_I, [_P, _P, _I, _Z, _P]),

@@ -187,10 +187,11 @@ def geglu_int8(hidden, bias, pre_quant_scale, input_quant_scale):
 
 def int8_linear_geglu(a_q, w_rows32, alpha_col, alpha_row, bias, pre_quant_scale, input_quant_scale, dtype):
     """geglu_int8(int8_linear(a_q, w_rows32, alpha_col, alpha_row, None, dtype), bias, ...) with a static alpha_row: a_q int8 [M, K],
-    w_rows32 int8 [2D, K] (rows32) -> int8 [M, D].  One kernel for 16-bit types, D % 64 == 0 and K >= 256, else those two."""
+    w_rows32 int8 [2D, K] (rows32) -> int8 [M, D].  One kernel for 16-bit types, D % 64 == 0 and K >= 256, else those two, as where the GEMM has
+    a forced or cached tactic."""
     m, k = a_q.shape
     n = w_rows32.shape[0]
-    if dtype not in (torch.float16, torch.bfloat16) or n % 128 or k % 64 or k < 256 or alpha_row.numel() != 1:
+    if dtype not in (torch.float16, torch.bfloat16) or n % 128 or alpha_row.numel() != 1 or not _l.load().lq_gemm_int8_geglu_takes(m, n // 2, k):
         return geglu_int8(int8_linear(a_q, w_rows32, alpha_col, alpha_row, None, dtype), bias, pre_quant_scale, input_quant_scale)
     for t, name, dt in ((a_q, "a_q", torch.int8), (w_rows32, "w_rows32", torch.int8), (alpha_col, "alpha_col", torch.float32),
                         (alpha_row, "alpha_row", torch.float32), (input_quant_scale, "input_quant_scale", torch.float32)):

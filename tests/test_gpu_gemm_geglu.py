@@ -46,6 +46,27 @@ def test_other_forms_keep_to_the_two_kernels(dev):
                               None, scale, torch.float16)
 
 
+def test_tactics_of_the_up_projection_stand(dev, monkeypatch):
+    from lyradiff_amd import lib, ops
+
+    m, inner, k = 64, 128, 256
+    a, w = torch.ones(m, k, device=dev, dtype=torch.int8), ops.repack_weight(torch.ones(2 * inner, k, device=dev, dtype=torch.int8))
+    args = (a, w, torch.full((2 * inner,), 1e-2, device=dev), torch.ones(1, device=dev), None, None, torch.full((1,), 0.05, device=dev), torch.float16)
+    want, calls = ops.int8_linear_geglu(*args), []
+    plain = ops.int8_linear
+    monkeypatch.setattr(ops, "int8_linear", lambda *a: (calls.append(1), plain(*a))[1])
+    assert torch.equal(ops.int8_linear_geglu(*args), want) and not calls
+    with ops.gemm_thread_tactic(2):
+        assert torch.equal(ops.int8_linear_geglu(*args), want) and len(calls) == 1
+    try:
+        ops.gemm_shape_tactic("int8", m, 2 * inner, k, 3)
+        assert torch.equal(ops.int8_linear_geglu(*args), want) and len(calls) == 2
+    finally:
+        ops.gemm_shape_tactic("int8", m, 2 * inner, k, -1)
+    takes = lib.load().lq_gemm_int8_geglu_takes
+    assert takes(m, inner, k) and not takes(m, inner, 192) and not takes(m, inner, 288) and not takes(m, 96, k) and not takes(-1, inner, k)
+
+
 # every configuration that the rule picks (64x64, k shared, 128x128, 128x256, 256x256 tiles), full and ragged tiles
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (130, 96, 192), (200, 640, 2560), (1024, 1280, 1280), (4096, 640, 2560), (4100, 1280, 640), (2048, 5120, 2048), (8192, 5120, 64)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
