@@ -756,20 +756,28 @@ struct GemmKernel {
                 }
             }
         }
+        if constexpr (KIND == K_INT8 && !kI32) {
+            if (n_ok) {
+                const float4 ac = *reinterpret_cast<const float4*>(p.alpha_col + out_n);
+                acol4[0] = ac.x; acol4[1] = ac.y; acol4[2] = ac.z; acol4[3] = ac.w;
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i) arow_l[i] = p.alpha_row[p.per_token ? min(m0 + wm * TM + i * 32 + lr, p.m - 1) : 0];
+        }
         if constexpr (!kI32) {
             if (p.bias != nullptr && n_ok) OutStore<OutTag>::load4(p.bias, out_n, bias4);
-            if constexpr (KIND == K_INT8) {
-                if (n_ok) {
-                    float4 ac = *reinterpret_cast<const float4*>(p.alpha_col + out_n);
-                    acol4[0] = ac.x; acol4[1] = ac.y; acol4[2] = ac.z; acol4[3] = ac.w;
-                    if (!p.per_token) {  // one factor per column, formed here
-                        const float ar = p.alpha_row[0];
-                        acol4[0] *= ar; acol4[1] *= ar; acol4[2] *= ar; acol4[3] *= ar;
-                    }
-                }
+        }
+        if constexpr (KIND == K_INT8 && !kI32) {
+            // All of them have arrived here, once: first needed behind a branch of the row loop they would be waited for at every row of a
+            // partial tile, and with them the store of the row in front (us, per-token scales: 1334x5120x640 13.0 -> 12.3, 1334x640x2560
+            // 10.9 -> 10.4).
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
-                    if (p.per_token) arow_l[i] = p.alpha_row[min(m0 + wm * TM + i * 32 + lr, p.m - 1)];
+            for (int e = 0; e < 4; ++e) asm volatile("" : "+v"(acol4[e]));
+#pragma unroll
+            for (int i = 0; i < MT; ++i) asm volatile("" : "+v"(arow_l[i]));
+            if (!p.per_token) {  // one factor per column, formed here
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acol4[e] *= arow_l[0];
             }
         }
         // The row loop exists in a few specialisations, chosen once per workgroup: which optional steps run
