@@ -28,8 +28,11 @@ template <typename OutTag> static int run_int8(GemmParams p, hipStream_t st) {
         const long last256 = t256 % 256;
         t = t256 >= 192 ? ((last256 == 0 || last256 >= 128) ? 6 : 4) : (t128 >= 128 ? 2 : 3);  // 128x128 tiles from half a round up (4096x640x2560: 14.5 against 16.3 us with 64x64)
         // short K: prologue and epilogue dominate, smaller tiles overlap them better -- until eight rounds of them per CU make the
-        // operands' way from L2 count (k = 640, 128x128 / 128x256 tiles: 8192 x 5120 45.8 / 40.3 us, 4096 x 5120 24.1 / 24.6)
-        if (p.k <= 1024 && t128 >= 192) t = t128 >= 2048 ? 4 : 2;
+        // operands' way from L2 count, which takes some k (us, 128x128 / 128x256 tiles, static scale: k = 640 8192x5120 44.7 / 42.7,
+        // 16384x5120 101 / 87, 32768x1280 51 / 47, 3300x10240 39.2 / 38.6; k = 1024 64 / 54, 136 / 116, 68 / 63, 56 / 51; with per-token scales
+        // or k-panels much the same.  k = 256: 29.0 / 29.3, 53.5 / 53.7, 34 / 33, 25 / 27; k = 512 with ragged tiles 3300x10240 34.5 / 36.5,
+        // 18432x1920 37 / 39.  Below 2048 tiles at k = 640: 16384x1920 37.5 / 37.7, 32768x640 27.6 / 28.1)
+        if (p.k <= 1024 && t128 >= 192) t = t128 >= 2048 && p.k >= 640 ? 4 : 2;
         // more full 256x256 tiles than CUs: the persistent form (4608x12288x3072: 153-160 us against 162-165 with 128x256 tiles)
         if (t256 > device_cu_count() && p.m % 256 == 0 && p.n % 256 == 0 && p.kb % 128 == 0 && p.k > 1024 &&
             (out_enum<OutTag>() == LQ_F16 || out_enum<OutTag>() == LQ_BF16))
