@@ -354,7 +354,9 @@ int lq_linear_fp8_rows(void* C, void* C2, const void* x, lq_dtype_t dtype, const
 
 /* A plain 16-bit linear of few rows: y [m, n] = x [m, k] . w [n, k]^T + bias [n] (or NULL), fp32 sums, T in {F16, BF16}; with y2, w2 (and
  * bias2) a second one of the same shape on the same input in the same launch.  n % 4 == 0, k % 64 == 0.  (AdaLayerNorm.cc's modulation,
- * the text key and value projections of BasicTransformerInt8Block.cc.) */
+ * the text key and value projections of BasicTransformerInt8Block.cc.)  lq_linear16_rows_takes: 1 for the sizes at which it was measured
+ * ahead of a library GEMM, 0 where that is the better or the only way. */
+int lq_linear16_rows_takes(int m, int n, int k);
 int lq_linear16_rows(void* y, void* y2, const void* x, const void* w, const void* w2, const void* bias, const void* bias2, lq_dtype_t dtype,
                      int m, int n, int k, lq_stream_t stream);
 

@@ -3,8 +3,9 @@
 // (154 x 640 x 2048, two of them: latency).  They are plain linears of the models (AdaLayerNorm.cc, BasicTransformerInt8Block.cc), one
 // launch and 20 us or 2 x 10 us each in the vendor's library.
 //
-// Up to four rows (linear16_gemv_kernel): a stream of weights, each wavefront four rows of them, a kilobyte of a row per request, with
-// three requests per row in flight; vector arithmetic, 64 partial sums per output added in one tree.
+// One row (linear16_gemv_kernel): a stream of weights, each wavefront four rows of them, a kilobyte of a row per request, with
+// three requests per row in flight; vector arithmetic, 64 partial sums per output added in one tree.  Two to four rows in that form are behind
+// the other one (us from memory, this form / the other: 4x640x640 4.9 / 3.6, 4x9216x3072 17.1 / 16.0, 4x18432x3072 25.6 / 24.2).
 // More rows (linear16_kernel): a workgroup of eight wavefronts owns 32 x 32 outputs and shares k out; wavefront g takes the 64-element pieces
 // g, g + 8, ... of both operands.  Eight neighbouring lanes fetch one 128-byte line of a row (lanes that fetch 16 bytes of 32 rows each, the
 // matrix operand's own order, make four times the requests: 154x1280x2048 twice: 23.6 us in that form, 9.6 now, the host's time for the call), and the piece reaches operand order through an LDS block
@@ -28,62 +29,50 @@ typedef _Float16 l16_h8 __attribute__((ext_vector_type(8)));
 
 constexpr int kGemvRows = 4;  // weight rows per wavefront
 
-template <typename Tag, int M> __global__ __launch_bounds__(256) void linear16_gemv_kernel(Linear16Params p) {
+template <typename Tag> __global__ __launch_bounds__(256) void linear16_gemv_kernel(Linear16Params p) {
     constexpr int R = kGemvRows, U = 3;
     const int lane = threadIdx.x & 63, which = blockIdx.z;
     const int n0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)) * R);
     if (n0 >= p.n) return;  // n is a multiple of R
     const unsigned short* w = p.w[which] + (size_t)n0 * p.k;
-    float sum[M][R];
+    float sum[R];
 #pragma unroll
-    for (int m = 0; m < M; ++m)
-#pragma unroll
-        for (int r = 0; r < R; ++r) sum[m][r] = 0.0f;
+    for (int r = 0; r < R; ++r) sum[r] = 0.0f;
     for (int k0 = lane * 8; k0 < p.k; k0 += 512 * U) {
-        uint4 wv[U][R], xv[U][M];
+        uint4 wv[U][R], xv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int at = k0 + 512 * u;
 #pragma unroll
             for (int r = 0; r < R; ++r) wv[u][r] = at < p.k ? *reinterpret_cast<const uint4*>(w + (size_t)r * p.k + at) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int m = 0; m < M; ++m) xv[u][m] = at < p.k && m < p.m ? *reinterpret_cast<const uint4*>(p.x + (size_t)m * p.k + at) : make_uint4(0, 0, 0, 0);
+            xv[u] = at < p.k ? *reinterpret_cast<const uint4*>(p.x + at) : make_uint4(0, 0, 0, 0);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            float xf[M][8];
-#pragma unroll
-            for (int m = 0; m < M; ++m) unpack8<Tag>(xv[u][m], xf[m]);
+            float xf[8];
+            unpack8<Tag>(xv[u], xf);
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 float wf[8];
                 unpack8<Tag>(wv[u][r], wf);
 #pragma unroll
-                for (int m = 0; m < M; ++m)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) sum[m][r] = __builtin_fmaf(wf[e], xf[m][e], sum[m][r]);
+                for (int e = 0; e < 8; ++e) sum[r] = __builtin_fmaf(wf[e], xf[e], sum[r]);
             }
         }
     }
 #pragma unroll
-    for (int m = 0; m < M; ++m)
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) sum[m][r] += __shfl_xor(sum[m][r], off, 64);
+        for (int off = 32; off > 0; off >>= 1) sum[r] += __shfl_xor(sum[r], off, 64);
     if (lane != 0) return;
     uint2 b = make_uint2(0, 0);
     const bool has_bias = p.bias[which] != nullptr;
     if (has_bias) b = *reinterpret_cast<const uint2*>(p.bias[which] + n0);
     const u32 bw[4] = {b.x & 0xFFFFu, b.x >> 16, b.y & 0xFFFFu, b.y >> 16};
+    u32 o[4];
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-        if (m >= p.m) break;
-        u32 o[4];
-#pragma unroll
-        for (int r = 0; r < R; ++r) o[r] = Elem<Tag>::store(has_bias ? sum[m][r] + Elem<Tag>::load(bw[r]) : sum[m][r]);
-        *reinterpret_cast<uint2*>(p.y[which] + (size_t)m * p.n + n0) = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
-    }
+    for (int r = 0; r < R; ++r) o[r] = Elem<Tag>::store(has_bias ? sum[r] + Elem<Tag>::load(bw[r]) : sum[r]);
+    *reinterpret_cast<uint2*>(p.y[which] + n0) = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
 }
 
 template <typename Tag> __global__ __launch_bounds__(512, 2) void linear16_kernel(Linear16Params p) {
@@ -181,6 +170,17 @@ template <typename Tag> __global__ __launch_bounds__(512, 2) void linear16_kerne
 
 using namespace lq;
 
+// Every 32 rows stream the weight again, and a workgroup's eight wavefronts share one k: large weights are the library's from 17 rows up, and
+// long sums, too, where its split of k has more workgroups (us from memory, library / this): 16x9216x3072 20.5 / 17.1, 32x 17.3 / 19.6,
+// 128x 25.0 / 36.2; 16x18432x3072 63.9 / 25.7, 32x 29.7 / 29.1, 64x 33.9 / 39.3; 128x10240x1280 17.2 / 17.6; 16x4096x4096 15.8 / 13.2, 32x
+// 13.7 / 14.3.  Smaller weights: 256x5120x1280 18.7 / 15.0, 256x3840x1280 13.9 / 12.0, 256x1280x1280 7.2 / 6.9, 256x640x640 6.3 / 4.1,
+// 154x1280x2048 twice 20.4 / 9.7.  16x1280x5120 10.1 / 14.5, 8x3072x12288 19.1 / 27.0.  One row: 640x640 6.4 / 3.2, 18432x3072 67 / 22, 3072x12288
+// 20.3 / 19.9, 3072x15360 22.8 / 23.7.
+extern "C" int lq_linear16_rows_takes(int m, int n, int k) {
+    if (m <= 0 || n <= 0 || k <= 0 || n % 4 != 0 || k % 64 != 0) return 0;
+    return (m == 1 && k <= 12288) || (m <= 256 && k <= 4096 && (m <= 16 || (long)n * k <= (1L << 23)));
+}
+
 extern "C" int lq_linear16_rows(void* y, void* y2, const void* x, const void* w, const void* w2, const void* bias, const void* bias2,
                                 lq_dtype_t dtype, int m, int n, int k, lq_stream_t stream) {
     LQ_REQUIRE(dtype == LQ_F16 || dtype == LQ_BF16, LQ_ERR_UNSUPPORTED, "lq_linear16_rows: dtype must be F16 or BF16");
@@ -197,15 +197,10 @@ extern "C" int lq_linear16_rows(void* y, void* y2, const void* x, const void* w,
     Linear16Params p = {{static_cast<unsigned short*>(y), static_cast<unsigned short*>(y2)}, {us(w), us(w2)}, {us(bias), us(bias2)}, us(x), m, n, k};
     const unsigned both = y2 != nullptr ? 2 : 1;
     hipStream_t st = as_stream(stream);
-    if (m <= 4) {
+    if (m == 1) {
         const dim3 grid((unsigned)((n / kGemvRows + 3) / 4), 1, both), block(256);
-        if (dtype == LQ_BF16) {
-            if (m == 1) hipLaunchKernelGGL((linear16_gemv_kernel<BF16Tag, 1>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((linear16_gemv_kernel<BF16Tag, 4>), grid, block, 0, st, p);
-        } else {
-            if (m == 1) hipLaunchKernelGGL((linear16_gemv_kernel<F16Tag, 1>), grid, block, 0, st, p);
-            else hipLaunchKernelGGL((linear16_gemv_kernel<F16Tag, 4>), grid, block, 0, st, p);
-        }
+        if (dtype == LQ_BF16) hipLaunchKernelGGL((linear16_gemv_kernel<BF16Tag>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((linear16_gemv_kernel<F16Tag>), grid, block, 0, st, p);
         return check_launch("lq_linear16_rows");
     }
     const dim3 grid((unsigned)n_tiles, (unsigned)m_tiles, both), block(512);

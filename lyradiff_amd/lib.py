@@ -82,6 +82,7 @@ SYMBOLS = {
     "lq_gemm_fp8_gated": (_I, [_P, _I, _P, _P, _P, _P, _P, _P, _Z, _P, _I, _I, _I, _P]),
     "lq_linear_fp8_rows_takes": (_I, [_I, _I, _I]),
     "lq_linear_fp8_rows": (_I, [_P, _P, _P, _I, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
+    "lq_linear16_rows_takes": (_I, [_I, _I, _I]),
     "lq_linear16_rows": (_I, [_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "lq_gemm_fp8_pair_takes": (_I, [_I, _I, _I, _I, _I]),
     "lq_gemm_fp8_pair": (_I, [_P, _I, _I, _I, _I, _I, _P]),

@@ -9,6 +9,7 @@ torch.ops.lyradiff.* custom operators.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 from typing import NamedTuple, Optional
 
 import torch
@@ -49,25 +50,33 @@ def _stream():
 
 _FLOATS = (torch.float32, torch.float16, torch.bfloat16)
 
-_transforms = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", None)
-_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", None)
+_tracing = torch._C._is_tracing if hasattr(torch._C, "_is_tracing") else torch.jit.is_tracing
+_transforms = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack", lambda: None)
+_dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 0)
+_autocast = torch.is_autocast_enabled
+_strided, _Parameter, _Tensor = torch.strided, torch.nn.Parameter, torch.Tensor
 
 
 def _plain(*tensors) -> bool:
     """True when a kernel may stand in for PyTorch operations on the tensors (None is passed over): ordinary dense tensors on the current
     device in eager mode, no gradient recorded, no forward-mode tangent, and nothing around the call that has to see the operations
     (vmap and the other function transforms, tracing, compilation, dispatch modes such as fake tensors)."""
-    if torch.jit.is_tracing() or torch.compiler.is_compiling() or (_transforms is not None and _transforms() is not None) or \
-            (_dispatch_modes is not None and _dispatch_modes()):
+    if _tracing() or _transforms() is not None or _dispatch_modes() or torch.compiler.is_compiling():
         return False
-    grad, duals = torch.is_grad_enabled(), forward_ad._current_level >= 0
+    grad, duals, device = torch.is_grad_enabled(), forward_ad._current_level >= 0, None
     for t in tensors:
         if t is None:
             continue
-        if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.layout is not torch.strided or (grad and t.requires_grad) or \
-                (duals and forward_ad.unpack_dual(t).tangent is not None) or \
-                (t.is_cuda and t.get_device() != (torch.cuda.current_device() if _raw_device is None else _raw_device())):
+        kind = type(t)
+        if (kind is not _Tensor and kind is not _Parameter) or (grad and t.requires_grad) or t.layout is not _strided:
             return False
+        if duals and forward_ad.unpack_dual(t).tangent is not None:
+            return False
+        if t.is_cuda:
+            if device is None:
+                device = torch.cuda.current_device() if _raw_device is None else _raw_device()
+            if t.get_device() != device:
+                return False
     return True
 
 
@@ -844,23 +853,25 @@ def fp8_linear_rows(x, first, second=None):
     return y if second is None else (y, y2)
 
 
-_LINEAR16_ROWS = 256
+@functools.lru_cache(maxsize=512)
+def _linear16_rows_takes(m: int, n: int, k: int) -> bool:
+    return m < 1 << 31 and bool(_l.load().lq_linear16_rows_takes(m, n, k))
 
 
 def linear16_supported(x, *tensors) -> bool:
-    """True when linear16 and linear16_pair take x [.., K] and the weights and biases `tensors`: few rows, dense 16-bit GPU tensors of one type,
-    aligned, in a call that PyTorch need not see (_plain) and would not cast (autocast)."""
+    """True when linear16 and linear16_pair take x [.., K] and the weights and biases `tensors`, a weight first: sizes at which they are the faster
+    way (lq_linear16_rows_takes), dense 16-bit GPU tensors of one type, aligned, in a call that PyTorch need not see (_plain) and would not cast (autocast)."""
     if x.dtype not in (torch.float16, torch.bfloat16) or x.dim() == 0 or not _plain(x, *tensors):
         return False
     k = x.shape[-1]
-    if k == 0 or k % 64 or x.numel() > _LINEAR16_ROWS * k or x.numel() == 0:
+    if k == 0 or not _linear16_rows_takes(x.numel() // k, tensors[0].shape[0] if tensors and tensors[0].dim() else 4, k):
         return False
     for t in (x, *tensors):
         if t is None:
             continue
         if not t.is_cuda or t.dtype != x.dtype or not t.is_contiguous() or t.data_ptr() % 16 or (t is not x and (t.dim() == 0 or t.shape[0] % 4)):
             return False
-    return not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype
+    return not _autocast("cuda") or torch.get_autocast_dtype("cuda") == x.dtype
 
 
 def linear16(x, weight, bias=None):

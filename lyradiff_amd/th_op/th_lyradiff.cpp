@@ -260,7 +260,7 @@ struct AdaLinear {
         const int64_t b = temb.size(0), d = temb.size(1), n = chunks * d;
         const lq_dtype_t dt = lq_dt(temb.scalar_type());
         const bool rows = fp8 ? lq_linear_fp8_rows_takes((int)b, (int)n, (int)d) != 0
-                              : b <= 256 && d % 64 == 0 && aligned(temb, 16) && rows16() && (other == nullptr || other->rows16()) &&
+                              : lq_linear16_rows_takes((int)b, (int)n, (int)d) != 0 && aligned(temb, 16) && rows16() && (other == nullptr || other->rows16()) &&
                                     !(at::GradMode::is_enabled() && temb.requires_grad());
         at::Tensor y, y2;
         int rc = LQ_NOT_TAKEN;

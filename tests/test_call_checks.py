@@ -81,6 +81,17 @@ def test_fp8_linears_of_a_few_more_rows_go_straight_to_the_two_calls(ops, monkey
     assert weights.FP8Linear(w, one, one).forward(x).shape == (m, 64)
 
 
+# rows, n, k; 1: measured ahead of the library's GEMM, 0: behind it, or a size the kernel does not take (lq_linear16.hip has the times)
+@pytest.mark.parametrize("m,n,k,one", [
+    (1, 640, 640, 1), (1, 18432, 3072, 1), (2, 9216, 3072, 1), (16, 18432, 3072, 1), (17, 18432, 3072, 0), (17, 9216, 3072, 0), (64, 18432, 3072, 0),
+    (256, 9216, 3072, 0), (256, 640, 640, 1), (256, 3840, 1280, 1), (154, 1280, 2048, 1), (257, 640, 640, 0), (16, 1280, 5120, 0), (8, 3072, 12288, 0),
+    (1, 3072, 12288, 1), (1, 3072, 15360, 0), (128, 10240, 1280, 0), (0, 640, 640, 0), (4, 642, 640, 0), (4, 640, 100, 0)])
+def test_16_bit_linears_of_few_rows_are_taken_where_that_is_faster(m, n, k, one):
+    from lyradiff_amd import lib as L
+
+    assert L.load().lq_linear16_rows_takes(m, n, k) == one
+
+
 # rows of both, n, k, scales and bias only; 1: measured ahead in one launch, 0: ahead one after the other (lq_gemm_fp8.hip has the times)
 @pytest.mark.parametrize("m,m2,n,k,plain,one", [
     (4096, 512, 9216, 3072, 1, 1), (6400, 512, 3072, 3072, 1, 1), (6400, 512, 12288, 3072, 0, 1), (6400, 512, 3072, 12288, 0, 1), (400, 100, 3072, 12288, 0, 1),

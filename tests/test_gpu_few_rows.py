@@ -48,7 +48,7 @@ def test_fp8_rows_leaves_the_rest_to_the_two_calls(dev):
         ops.fp8_linear_rows(x(1, 1280), lin(64, 1536))
 
 
-# one to four rows stream the weight; 64-element pieces fewer than the eight wavefronts, a remainder of 32 rows and columns, the most rows
+# one row streams the weight; 64-element pieces fewer than the eight wavefronts, a remainder of 32 rows and columns, the most rows
 @pytest.mark.parametrize("dt", DTS)
 @pytest.mark.parametrize("m,n,k", [(1, 4, 64), (1, 9216, 3072), (3, 36, 576), (4, 1280, 1600), (5, 36, 64), (33, 100, 448), (154, 640, 2048), (256, 1284, 1088)])
 def test_linear16(dev, dt, m, n, k):
