@@ -5,9 +5,12 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# rows, outputs, k: one row, tiles of 128 and 256 rows less / exactly / more than full, the fewest and more k-tiles, fewer tiles than
-# CUs, one per CU and several (2049 x 2560 is 360 tiles of 256 rows, 700 x 2560 240 of 128)
-SHAPES = [(1, 64, 256), (127, 64, 320), (128, 128, 256), (129, 192, 640), (700, 2560, 640), (1024, 5120, 1280), (2049, 2560, 640), (8192, 2560, 640)]
+# rows, outputs, k: one row, tiles of 128 and 256 rows less / exactly / more than full, the fewest and more k-tiles; at most one tile per
+# workgroup (700 x 2560: 240 tiles of 128 rows) and several, where the transfers run on across tiles (1024 and 897 x 2560: 320 tiles of 128
+# rows; 2049 x 2560: 360 of 256), also with k = 256, where a tile is as long as the pipeline and the next one's columns are requested in the
+# first step behind an epilogue
+SHAPES = [(1, 64, 256), (127, 64, 320), (128, 128, 256), (129, 192, 640), (700, 2560, 640), (1024, 5120, 1280), (2049, 2560, 640), (8192, 2560, 640),
+          (1024, 2560, 640), (897, 2560, 256), (2049, 2560, 256)]
 
 
 @pytest.mark.parametrize("m,inner,k", SHAPES)
@@ -67,8 +70,10 @@ def test_tactics_of_the_up_projection_stand(dev, monkeypatch):
     assert takes(m, inner, k) and not takes(m, inner, 192) and not takes(m, inner, 288) and not takes(m, 96, k) and not takes(-1, inner, k)
 
 
-# every configuration that the rule picks (64x64, k shared, 128x128, 128x256, 256x256 tiles), full and ragged tiles
-@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (130, 96, 192), (200, 640, 2560), (1024, 1280, 1280), (4096, 640, 2560), (4100, 1280, 640), (2048, 5120, 2048), (8192, 5120, 64)])
+# every configuration that the rule picks (64x64, k shared, 128x128, 128x256, 256x256 tiles), full and ragged tiles.  4352x4096x1152 is 272
+# whole tiles of 256x256: the plain product takes the persistent form, which declines a residual, and the sum the plain 256x256 tiles
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (130, 96, 192), (200, 640, 2560), (1024, 1280, 1280), (4096, 640, 2560), (4100, 1280, 640), (2048, 5120, 2048), (8192, 5120, 64),
+                                   (4100, 10240, 640), (4352, 4096, 1152), (4100, 3072, 1152)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_int8_linear_with_a_residual_is_the_sum(dev, m, n, k, dt):
     from lyradiff_amd import ops

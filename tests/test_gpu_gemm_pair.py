@@ -79,3 +79,25 @@ def test_codes_of_full_and_of_partial_tiles_are_the_same(dev, m, n, k, dt, gelu)
                                                                             round_dtype=dt))
     full, part = codes(m), codes(m - 1)
     assert torch.equal(full[:-1], part) and bool(((full[:, n - 3] & 0x7F) == 0x7F).all())
+
+
+# gates of full tiles (a band's rows of the residual in registers) and of partial ones, with gates that change inside a tile and on its edge
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k,rows", [(64, 64, 128, 24), (1024, 2048, 256, 100), (1024, 2048, 256, 512), (256, 768, 2048, 37), (4096, 3072, 1152, 1000), (4352, 3072, 1152, 17)])
+def test_gates_that_change_inside_a_tile(dev, m, n, k, rows, dt):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(m + n + k + rows)
+    a, w = (torch.randn(r, k, generator=g, device=dev).clamp_(-4, 4).to(torch.float8_e4m3fn).view(torch.uint8) for r in (m, n))
+    lin = (ops.repack_weight(w), torch.full((1,), k ** -0.5, device=dev), torch.ones(1, device=dev), torch.randn(n, generator=g, device=dev).to(dt))
+    gate, res = (torch.randn(r, n, generator=g, device=dev).to(dt) for r in (-(-m // rows), m))
+    panels = lambda count: a[:count].view(count, k // 64, 64).transpose(0, 1).contiguous()
+    for count in (m, m - 1):
+        got = ops.fp8_linear_gated_panels(panels(count), *lin, gate[: -(-count // rows)], res[:count], rows_per_gate=rows)
+        want = ops.fp8_linear_panels(panels(count), *lin, None, dt) * gate.repeat_interleave(rows, 0)[:count] + res[:count]
+        assert torch.equal(got, want), (count, int((got != want).sum()))
+    # in place: the residual is the output
+    half = ops.FP8Half(panels(m), *lin, gate=gate, residual=res, rows_per_gate=rows, out=res)
+    want = ops.fp8_linear_panels(panels(m), *lin, None, dt) * gate.repeat_interleave(rows, 0)[:m] + res
+    empty = ops.FP8Half(panels(0), *lin, gate=gate[:0], residual=res[:0], rows_per_gate=rows)
+    assert torch.equal(ops.fp8_linear_pair(half, empty, dt)[0], want)
