@@ -816,7 +816,7 @@ struct GemmKernel {
             uint8_t* const c8_row0 = !CODES_FULL ? nullptr : p.C8 + (p.c8_panel ? (size_t)(out_n >> 6) * p.m * 64 + (out_n & 63) : (size_t)out_n) + (size_t)mrow0 * c8_pitch;
             // GATED of full tiles: a band's rows of the residual are requested at once.  One row at a time, each behind the store of the one in
             // front of it (which the compiler has to take for the same memory), is a chain of round trips to memory.  us, whole FLUX blocks
-            // (FP8): double 832 -> 822, single at 6912 tokens 1344 -> 1330.
+            // (FP8): double 819 -> 810, single at 6912 tokens 1372 -> 1356, at 4608 796 -> 782.
             constexpr bool GATED_FULL = MODE == E_GATED && FULL && ESZ == 2;
             uint2 residual[GATED_FULL ? NITER : 1];
             if constexpr (GATED_FULL) {
@@ -835,6 +835,15 @@ struct GemmKernel {
                     if constexpr (!kI32) {
                         if constexpr (MODE == E_STATIC_ADD)
                             if (FULL || (mrow0 + (tb + u) * RPI < p.m && n_ok)) OutStore<OutTag>::load4(p.addend, idx0 + (size_t)(tb + u) * rstep, joined[u]);
+                    }
+                }
+                if constexpr (!FULL) {
+                    // of a partial tile too the four rows are read at once: the compiler would move a read behind its row's bounds check, where
+                    // its latency stands alone (us, static FP8 linear with its cast: 1334x12288x3072 60.4 -> 59.4, 700x9216x3072 26.8 -> 26.6)
+#pragma unroll
+                    for (int u = 0; u < NB; ++u) {
+                        asm volatile("" : "+v"(raw[u]));
+                        if constexpr (KIND == K_INT8 && !kI32 && MODE == E_PLAIN) asm volatile("" : "+v"(arv[u]));
                     }
                 }
                 if constexpr (CODES_FULL) {
