@@ -13,7 +13,7 @@
 // 8-byte loads of up to four slot groups are in flight together.  The sum of squares is reduced across the lanes of a head in
 // a fixed order; 1/sqrt is the IEEE one (the reference uses the approximate rsqrt).
 // What bounds it: memory.  In place it leaves v alone, a third of the bytes (us, bf16, 24 heads of 128, into a second tensor / in place):
-// 4608 tokens 33.5 / 25.8 (4.4 TB/s), 6912 tokens 43.8 / 35.1.  Folding q's share into the attention's prologue measured the same sum
+// 4608 tokens 33.5 / 25.8 (4.4 TB/s), 6912 tokens 43.8 / 35.1 by themselves; in a traced block 35.6 / 31.7 and 49.5 / 42.7.  Folding q's share into the attention's prologue measured the same sum
 // (4608 tokens: 16.0 for k and 11.4 more in the attention).
 #include "lq_common.h"
 

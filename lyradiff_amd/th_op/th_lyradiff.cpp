@@ -9,8 +9,9 @@
 //
 // Quant levels 1, 2 (FP8_W8A8, FP8_W8A8_FULL) and 7, 8 (INT4_W4A4, INT4_W4A4_FULL) are built, the levels whose blocks
 // consist of quantized linears.  Every quantized linear, adaLN / gate / residual step, activation quantisation, the q/k
-// RMSNorm, the rotary embedding and the softmax attention run on liblyraquant.so through its C ABI; PyTorch supplies device
-// memory, the current stream and the 16-bit adaLN matmul of the non-FULL levels.
+// RMSNorm, the rotary embedding and the softmax attention run on liblyraquant.so through its C ABI, and so does the 16-bit adaLN matmul of
+// the non-FULL levels for the row counts that lq_linear16_rows_takes; PyTorch supplies device memory, the current stream and that matmul for
+// other sizes and alignments.
 // This file holds no device code and is compiled with the host compiler.
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
