@@ -19,11 +19,17 @@
 //     apart by the workgroup barriers; left to themselves two wavefronts of a SIMD drift into step and both pipes idle half the
 //     time.  NW == 4: two or more workgroups per CU run freely, one barrier per tile; a head dimension of 64 leaves registers
 //     for three wavefronts per SIMD, which cover for each other without phases.
-// Measured (settled, random operands, bf16; in parentheses the library attention that stood here before): 24 heads of 128,
-// 4608 tokens 261 us = 1.0 PFLOP/s (506), 6912 tokens 583 us (908), 1600 tokens 45 us (135), 1000 tokens 24 us; 2 x 10 heads of 64,
-// 4096 tokens 120 us (190).  NW == 4 at 24 x 4608 tokens of 128: 299 us; NW == 8 at 64: 147 us.  The row sum of the fp32
-// probabilities takes as long as one of the rounded ones (262 / 583 / 24 / 120 us against 261 / 583 / 26 / 123), and makes the error
-// against 64 bits that of the library attention (bf16, 4608 tokens, 2-norm: 2.264e-3 both).
+//   * Vector instructions are counted: beside a matrix wavefront that keeps its pipe full each takes 6.7 cycles (5.0 alone), an exponential
+//     11.8 (9.0), so the row maximum is v_maximum3 (fmaxf quietens its operands first), m * c is formed when m changes, and V lies below K in
+//     LDS, where its reads need no address arithmetic beyond their offsets: 243 vector instructions per tile of 64 keys, 270 without these.
+// Measured (settled, random operands, bf16; in parentheses before the last paragraph's changes, same run, then the library attention):
+// 24 heads of 128, 4608 tokens 257 us = 1.0 PFLOP/s (264; 506), 6912 tokens 576 us (596; 908), 1600 tokens 44.7 us (45.9; 135), 1000 tokens
+// 23.7 us (24.2); 2 x 10 heads of 64, 4096 tokens 122.7 us (125.5; 190).  NW == 4 at 24 x 4608 tokens of 128: 299 us; NW == 8 at 64: 147 us.
+// What was measured and is not here (4608 tokens, beside 257 us): a rescaled output only where the maximum grew by more than 2^8, 239 us, but
+// the error against 64 bits goes from 1.93e-3 to 2.31e-3, since the largest probabilities are then rounded; the rescaling moved between the
+// matrix instructions, 252; softmax and matrix instructions mixed in one wavefront's stream, 286; tiles of 128 keys, 254.
+// The row sum of the fp32 probabilities takes as long as one of the rounded ones, and makes the error against 64 bits that of the library
+// attention (bf16, 4608 tokens, 2-norm: 2.264e-3 both).
 #include "lq_common.h"
 
 namespace lq {
@@ -60,6 +66,10 @@ template <typename Tag> __device__ __forceinline__ v16f attn_mfma(attn_s8 a, att
 template <typename Tag> __device__ __forceinline__ u32 attn_pack(float a, float b) {
     if constexpr (std::is_same<Tag, BF16Tag>::value) return pack2_bf16(a, b);
     else return pack2_f16(a, b);
+}
+// v_maximum3.  NaN where an operand is one: a row with such a score is NaN throughout, whatever its maximum.
+__device__ __forceinline__ float attn_max(float a, float b, float c) {
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
 }
 // 16 bytes per lane from global memory to LDS byte address lds_addr + 16 * lane, awaited with attn_wait_vmcnt
 __device__ __forceinline__ void attn_dma16(const void* gbase, u32 voff, u32 lds_addr) {
@@ -113,8 +123,8 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
         ck[i] = (d_ch ^ (CH == 16 ? (r & 15) : ((r >> 1) & 7))) * 16;
         cv[i] = (d_ch ^ (CH == 16 ? ((r & 3) << 2) : (((r >> 1) & 1) << 2))) * 16;
     }
-    auto k_tile = [&](int t) { return (t % NSTAGE) * TILE_B; };
-    auto v_tile = [&](int t) { return (NSTAGE + t % NSTAGE) * TILE_B; };
+    auto k_tile = [&](int t) { return (NSTAGE + t % NSTAGE) * TILE_B; };
+    auto v_tile = [&](int t) { return (t % NSTAGE) * TILE_B; };
     // tiles and rows past the end repeat the last ones: the number of transfers in flight stays a compile-time constant
     auto src_row = [&](int t, int i) { return (u32)min(min(t, ntiles - 1) * KT + (wave * DMA + i) * RPD + d_row, p.sk - 1); };
     auto issue_k = [&](int t, int i) {
@@ -179,6 +189,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
     // would make (-inf) - (-inf) of it.
     float m_run = -__FLT_MAX__, l_run[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const float c = p.scale_log2;
+    float mc = fmaxf(m_run * c, -__FLT_MAX__);
     // Probabilities of a tile, in fp32 and, two keys per word, in T: words 4 * kk .. 4 * kk + 3 are the operand of PV step kk.  The row
     // sum takes the former, beside the matrix instructions (SUM_LATE); at a head dimension of 64 the 32 registers would cost the third
     // wavefront per SIMD, and the sum is formed with the exponentials.
@@ -228,20 +239,21 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
         // four independent chains, here and below: nobody else fills the latency of a dependent vector instruction
         float mq[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) mq[e] = fmaxf(fmaxf(s[0][e], s[1][e]), s[0][4 + e]);
+        for (int e = 0; e < 4; ++e) mq[e] = attn_max(s[0][e], s[1][e], s[0][4 + e]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) mq[e] = fmaxf(fmaxf(mq[e], s[1][4 + e]), s[0][8 + e]);
+        for (int e = 0; e < 4; ++e) mq[e] = attn_max(mq[e], s[1][4 + e], s[0][8 + e]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) mq[e] = fmaxf(fmaxf(mq[e], s[1][8 + e]), s[0][12 + e]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) mq[e] = fmaxf(mq[e], s[1][12 + e]);
+        for (int e = 0; e < 4; ++e) mq[e] = attn_max(mq[e], s[1][8 + e], s[0][12 + e]);
+        mq[0] = attn_max(mq[0], mq[1], s[1][12]);
+        mq[2] = attn_max(mq[2], mq[3], s[1][13]);
         float lo, hi;
-        attn_halves(fmaxf(fmaxf(mq[0], mq[1]), fmaxf(mq[2], mq[3])), lo, hi);
-        const float mx = fmaxf(lo, hi);
+        attn_halves(attn_max(mq[0], mq[2], __builtin_elementwise_maximum(s[1][14], s[1][15])), lo, hi);
+        const float mx = __builtin_elementwise_maximum(lo, hi);
         if (__any(mx > m_run)) {
-            const float m_new = fmaxf(m_run, mx);
+            const float m_new = mx > m_run ? mx : m_run;
             const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c);
             m_run = m_new;
+            mc = fmaxf(m_run * c, -__FLT_MAX__);  // finite too: c > 1 would make -inf of the start, and NaN of a score of -inf
 #pragma unroll
             for (int i = 0; i < 4; ++i) l_run[i] *= alpha;
 #pragma unroll
@@ -249,7 +261,6 @@ __global__ __launch_bounds__(NW * 64, 2) void attention_kernel(AttnParams p) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
         }
-        const float mc = fmaxf(m_run * c, -__FLT_MAX__);  // finite too: c > 1 would make -inf of the start, and NaN of a score of -inf
 #pragma unroll
         for (int i = 0; i < 32; ++i) e[i] = __builtin_fmaf(s[i >> 4][i & 15], c, -mc);
         __builtin_amdgcn_sched_barrier(0);
