@@ -64,7 +64,7 @@ struct GemmParams {
     // A is stored as k-panels [kb / 64][m][64] instead of row-major [m][kb]: the 64 bytes a k-tile takes from each of a
     // tile's rows are then contiguous (256 rows = 16 KiB, whole 128-byte cache lines), where a row-major operand gives half
     // a line per row and every line is requested from L2 twice, one k-tile apart (TCP_TCC_READ_REQ per launch at
-    // 4608x3072x12288: 16.2 M row-major, 10.6 M = the operand bytes / 128 in panels).  Kernels with 64-byte k-tiles only.
+    // 4608x3072x12288: 16.2 M row-major, 10.6 M = the operand bytes / 128 in panels).
     int a_panel;
     // gelu: 0 none, 1 on the fp32 value, 2 on the value rounded to T first (the activation applied by a separate
     // kernel to a stored T tensor)
@@ -231,7 +231,10 @@ struct GemmKernel {
     static_assert(PER_TILE * NSTAGE < 64, "vmcnt is a 6-bit counter");
     using AccT = typename std::conditional<KIND == K_FP8 || W4C, v16f, v16i>::type;
     using FragT = typename std::conditional<KIND == K_FP8 || W4C, v8i, v4i>::type;
-    static constexpr int KSTEP = (KIND == K_FP8 || W4C) ? 64 : 32;  // operand bytes per MFMA k-step
+    // INT8, 96x32 wavefront tile: its three matrix instructions are over before the next k-step's fragments arrive; two steps are one (us,
+    // 8192x640x2560 20.3 -> 18.9; square wavefront tiles level)
+    static constexpr bool PAIRED = KIND == K_INT8 && BKB == 128 && MT * NT == 3;
+    static constexpr int KSTEP = (KIND == K_FP8 || W4C || PAIRED) ? 64 : 32;  // operand bytes per MFMA k-step
     static constexpr int KS = BKB / KSTEP;
 
     // between the k-tiles of a group: a wavefront whose stages are its own only has to be done with its reads
@@ -257,8 +260,9 @@ struct GemmKernel {
         const u32 smem_base = (u32)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
 
         // ---- global -> LDS transfer plan (per lane offsets are fixed; the bases advance with k) ----
-        const u32 a_pitch = p.a_panel ? (u32)BKB : (u32)kb;                      // bytes between two rows of A
+        const u32 a_pitch = p.a_panel ? 64u : (u32)kb;                           // bytes between two rows of A
         const size_t a_kstep = (p.a_panel ? (size_t)p.m * BKB : (size_t)BKB) * KW;  // bytes between two k-tiles of a row
+        const u32 a_half = BKB == 128 && p.a_panel ? (u32)p.m * 64u - 64u : 0u;  // a 128-byte k-tile is two panels: what its second half lies further off
         const uint8_t* a_base = p.A + (size_t)m0 * a_pitch + (size_t)kg * (a_kstep / KW);
         const uint8_t* b_base = p.B + (size_t)(n0 / 32) * b_block_stride + (size_t)kg * (BKB * 32);
         u32 a_voff[A_DMA], b_voff[B_DMA];
@@ -267,7 +271,7 @@ struct GemmKernel {
         for (int i = 0; i < A_DMA; ++i) {
             int slot = (wave * A_DMA + i) * 64 + lane;  // 16-byte slot inside the A stage
             int row = slot / CH, c = (slot % CH) ^ chunk_swizzle<CH>(row);
-            a_voff[i] = (u32)min(row, row_last) * a_pitch + c * 16;
+            a_voff[i] = (u32)min(row, row_last) * a_pitch + c * 16 + (BKB == 128 && c >= 4 ? a_half : 0u);
         }
 #pragma unroll
         for (int i = 0; i < B_DMA; ++i) {
@@ -523,7 +527,7 @@ struct GemmKernel {
         if constexpr (!W4) {
             // Operand fragments as 16-byte pieces (an fp8 fragment is two pieces), so that the LDS reads
             // of the next k-step can be interleaved one by one with the MFMAs of the current step.
-            constexpr int PPF = (KIND == K_FP8) ? 2 : 1;
+            constexpr int PPF = (KIND == K_FP8 || PAIRED) ? 2 : 1;
             constexpr int KCH = KSTEP / 16;  // chunks per k-step
             constexpr int NPIECE = (NT + MT) * PPF;
             constexpr int NMFMA = MT * NT;
@@ -546,7 +550,8 @@ struct GemmKernel {
                     v8i x = __builtin_shufflevector(xp[buf][i][0], xp[buf][i][PPF - 1], 0, 1, 2, 3, 4, 5, 6, 7);
                     acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w, x, acc[i][j], 0, 0, 0, 0, 0, 0);
                 } else {
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wp[buf][j][0], xp[buf][i][0], acc[i][j], 0, 0, 0);
+#pragma unroll
+                    for (int h = 0; h < PPF; ++h) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wp[buf][j][h], xp[buf][i][h], acc[i][j], 0, 0, 0);
                 }
             };
             // With three or more stages a tile's transfers are not issued in one burst behind the barrier
@@ -1094,10 +1099,6 @@ template <int BM, int BN, int BKB, int KW> static int plan_tiles(GemmParams& p) 
         set_error("gemm: row length %d bytes is not a multiple of the %d-byte k-tile", p.kb, BKB * KW);
         return LQ_ERR_SHAPE;
     }
-    if (p.a_panel && BKB != 64) {
-        set_error("gemm: an activation in 64-byte k-panels needs a configuration with 64-byte k-tiles");
-        return LQ_ERR_ARG;
-    }
     p.tiles_m = (p.m + BM - 1) / BM;
     p.tiles_n = (p.n + BN - 1) / BN;
     return LQ_OK;
@@ -1147,8 +1148,8 @@ static int launch_gemm_pair(GemmPair pair, hipStream_t st) {
 int launch_persist_fp8(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st);
 int launch_persist_int8(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st);
 // Forms for problems of few tiles (lq_gemm_small.hip); numbered behind the tactics, which can be forced and cached: these cannot.
-enum SmallForm { SMALL_32x32_K4 = 64, SMALL_32x64_K4, SMALL_64x128_K2, SMALL_128x128_K2 };
-// the tactic or form for fewer than 192 tiles of 256x256, k > 1024 and 16-bit outputs; m2: rows of a second problem in the same launch;
+enum SmallForm { SMALL_32x32_K4 = 64, SMALL_32x64_K4, SMALL_64x128_K2, SMALL_128x128, SMALL_192x128 };
+// the tactic or form for fewer than 192 tiles of 256x256 and 16-bit outputs (k <= 1024: -1 where none of the forms leads); m2: rows of a second problem in the same launch;
 // cost_out: its time by the table that it goes by
 int few_tiles_form(int m, int m2, int n, int k, float* cost_out = nullptr);
 int run_small(GemmKind kind, const GemmParams& p, lq_dtype_t out_dtype, int form, hipStream_t st);

@@ -38,11 +38,11 @@ template <typename OutTag> static int run_int8(GemmParams p, hipStream_t st) {
             (out_enum<OutTag>() == LQ_F16 || out_enum<OutTag>() == LQ_BF16))
             t = 7;
     }
-    // Too few 256x256 tiles: the form whose rounds of workgroups cost least.  A forced or cached tactic stands.  k <= 1024: a
-    // workgroup's ten or sixteen k-tiles leave nothing to share (1024x640x640: 4.7 us with 64x64 tiles, 4.9 with k shared).
-    if (requested < 0 && out16 && p.k > 1024 && (long)((p.m + 255) / 256) * ((p.n + 255) / 256) < 192) {
-        t = few_tiles_form(p.m, 0, p.n, p.k);
-        if (t >= SMALL_32x32_K4) return run_small(K_INT8, p, out_enum<OutTag>(), t, st);
+    // Too few 256x256 tiles: the form whose rounds of workgroups cost least.  A forced or cached tactic stands.
+    if (requested < 0 && out16 && (long)((p.m + 255) / 256) * ((p.n + 255) / 256) < 192) {
+        const int form = few_tiles_form(p.m, 0, p.n, p.k);
+        if (form >= SMALL_32x32_K4) return run_small(K_INT8, p, out_enum<OutTag>(), form, st);
+        if (form >= 0) t = form;
     }
     if (t == 1 && (p.kb % 128 != 0 || p.a_panel)) t = 0;  // the 128-byte k-tile needs k % 128 == 0 and a row-major activation
     if (t == 7) {  // the persistent form of tactic 6 where it applies, tactic 6 itself elsewhere

@@ -1,11 +1,18 @@
 // 8-bit GEMMs whose tiles leave most of the chip idle: the forms of GemmKernel whose wavefront groups share k out.
 //
 // What bounds them: a workgroup alone on a CU takes 0.17 us (64x64) to 0.3 us (128x256) per 64-byte k-tile whatever it computes --
-// the barrier, the LDS round trip of the fragments and the matrix instructions follow each other -- and walks k by itself.  With
-// k shared between two or four groups of wavefronts the chain is that much shorter and the CU has as many more chains to switch
-// between; the partial sums meet in LDS (at most 128 KiB, about 1 us), not in memory.  Measured (us, FP8 to bf16, before -> now):
-// 154x9216x3072 14.8 -> 9.9, 512x3072x3072 11.6 -> 8.8, 512x3072x12288 42 -> 29; INT8 1024x1280x1280 8.4 -> 6.5, 333x1280x5120 16 ->
-// 10.  FP8 of few rows with no more than scales and bias goes to lq_gemm_rows.hip instead.
+// the barrier, the LDS round trip of the fragments, the transfers' issue and the matrix instructions follow each other -- and walks k by
+// itself.  Two remedies:
+//   * k shared between two or four groups of wavefronts (_K2, _K4), where tiles fill at most half of the chip: the chain is that much
+//     shorter and the CU has as many more chains to switch between; the partial sums meet in LDS (at most 64 KiB), not in memory.
+//   * k-tiles of 128 bytes and eight wavefronts, one workgroup per CU, where up to 256 tiles of 128x128 or of 192x128 make one round: half
+//     the barriers, whole 128-byte lines of a row-major activation, a second wavefront on each SIMD beside the one that waits.  128x128
+//     with k shared by two groups of four stood here before (us, then the general tiles / that / now, FP8: 333x9216x3072 16.5 / 14.7 /
+//     12.9, 1024x3072x3072 15.9 / 14.6 / 12.6, 1024x3072x12288 52 / 43 / 38; INT8: 2048x1280x1280 8.8 / 8.8 / 7.9, 2048x1280x5120 26.5 /
+//     22.6 / 19.4, 4096x640x2560 13.7 / 12.4 / 11.4).  192x128, general / now: FP8 512x9216x3072 20.3 / 16.7, 700x12288x3072 34.5 / 30.4 (two
+//     rounds); INT8 8192x640x2560 21.2 / 17.1, 4096x1280x5120 33.4 / 29.6.  Three or four stages, four wavefronts of 64x64 in place of
+//     eight of 64x32, level; 256x128 tiles 20.7 where 192x128 take 17.1.
+// FP8 of few rows with no more than scales and bias goes to lq_gemm_rows.hip instead.
 #pragma once
 
 #include "lq_gemm_core.h"
@@ -17,7 +24,8 @@ template <int KIND, typename OutTag> static int run_small_as(const GemmParams& p
         case SMALL_32x32_K4: return launch_gemm<KIND, OutTag, 32, 32, 64, 1, 1, 3, 4>(p, st);
         case SMALL_32x64_K4: return launch_gemm<KIND, OutTag, 32, 64, 64, 1, 2, 3, 4>(p, st);
         case SMALL_64x128_K2: return launch_gemm<KIND, OutTag, 64, 128, 64, 1, 2, 4, 2>(p, st);
-        case SMALL_128x128_K2: return launch_gemm<KIND, OutTag, 128, 128, 64, 2, 2, 3, 2>(p, st);
+        case SMALL_128x128: return launch_gemm<KIND, OutTag, 128, 128, 128, 2, 4, 4>(p, st);
+        case SMALL_192x128: return launch_gemm<KIND, OutTag, 192, 128, 128, 2, 4, 3>(p, st);
         default: set_error("gemm: unknown form %d", form); return LQ_ERR_ARG;
     }
 }

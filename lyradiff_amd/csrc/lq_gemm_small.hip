@@ -4,24 +4,31 @@
 namespace lq {
 
 int few_tiles_form(int m, int m2, int n, int k, float* cost_out) {
+    auto tiles_of = [&](int bm, int bn) { return (((long)m + bm - 1) / bm + ((long)m2 + bm - 1) / bm) * (((long)n + bn - 1) / bn); };
+    // Short k: prologue and epilogue are most of the time, and only the forms of eight wavefronts and 128-byte k-tiles lead, by one
+    // round against the 1.25 or the half that 128x128 tiles of four wavefronts make (INT8, k = 640, us, those / this: 640 outputs, 4096 rows
+    // 6.7 / 6.3, 6000 7.6 / 7.0, 8192 9.5 / 8.4; 2048 rows, 80 tiles, 5.8 / 5.9).
+    if (k <= 1024) {
+        if (k < 640 || k % 128 != 0) return -1;
+        const long t128 = tiles_of(128, 128);
+        return t128 > 256 && tiles_of(192, 128) <= 256 ? SMALL_192x128 : t128 > 128 && t128 <= 256 ? SMALL_128x128 : -1;
+    }
     // Time of a launch by the number of workgroups each CU of 256 has to hold (us at k = 3072): up to 256 of them, up to 512, ...; more
-    // than fit make whole rounds.  128x128 tiles share k from k = 2048 up: below, adding up two halves costs what the shorter walk
-    // saves (us, one walk / shared, 128 to 256 tiles -- FP8 k = 1152: 7.0-7.7 / 7.6-8.7, 1792: 8.5-11.4 / 8.9-10.8, 2048: 9.2-12.5 /
-    // 9.4-12.1, 2560: 10.6-15.3 / 10.5-14.3, 3072: 13.1-17.7 / 12.6-16.4; INT8 k = 1280: 8.7-10.0 / 8.5-9.9, 2048: 11.1-13.7 /
-    // 10.4-12.7, 3072: 15.6-19.5 / 14.0-18.1).
-    struct Cost { int form, bm, bn, per_round, groups; float us[4]; };
-    static const Cost table[] = {{2, 128, 128, 512, 1, {16, 26}},
-                                 {4, 128, 256, 512, 1, {21, 42}},
-                                 {3, 64, 64, 1024, 1, {9.5f, 13, 19, 19}},
-                                 {SMALL_128x128_K2, 128, 128, 256, 2, {14}},
-                                 {SMALL_64x128_K2, 64, 128, 256, 2, {9}},
-                                 {SMALL_32x64_K4, 32, 64, 512, 4, {6.2f, 10}},
-                                 {SMALL_32x32_K4, 32, 32, 768, 4, {5, 7.5f, 11.5f}}};
+    // than fit make whole rounds.  k is a multiple of k_unit.
+    struct Cost { int form, bm, bn, per_round, k_unit; float us[4]; };
+    static const Cost table[] = {{2, 128, 128, 512, 64, {16, 26}},
+                                 {4, 128, 256, 512, 64, {21, 42}},
+                                 {3, 64, 64, 1024, 64, {9.5f, 13, 19, 19}},
+                                 {SMALL_128x128, 128, 128, 256, 128, {12.6f}},
+                                 {SMALL_192x128, 192, 128, 256, 128, {16.5f}},
+                                 {SMALL_64x128_K2, 64, 128, 256, 128, {9}},
+                                 {SMALL_32x64_K4, 32, 64, 512, 256, {6.2f, 10}},
+                                 {SMALL_32x32_K4, 32, 32, 768, 256, {5, 7.5f, 11.5f}}};
     int best = 2;
     float least = 0.0f;
     for (const Cost& c : table) {
-        if (k % (64 * c.groups) != 0 || (c.form == SMALL_128x128_K2 && k < 2048)) continue;
-        const long tiles = (((long)m + c.bm - 1) / c.bm + ((long)m2 + c.bm - 1) / c.bm) * (((long)n + c.bn - 1) / c.bn), left = tiles % c.per_round;
+        if (k % c.k_unit != 0) continue;
+        const long tiles = tiles_of(c.bm, c.bn), left = tiles % c.per_round;
         const float cost = (float)(tiles / c.per_round) * c.us[(c.per_round + 255) / 256 - 1] + (left == 0 ? 0.0f : c.us[(left - 1) / 256]);
         if (least == 0.0f || cost < least) { best = c.form; least = cost; }
     }
