@@ -222,6 +222,11 @@ int lq_gemm_int8(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_t* B
  * aligned, may be C; out_dtype F16 or BF16. */
 int lq_gemm_int8_add(void* C, lq_dtype_t out_dtype, const int8_t* A, const int8_t* B_rows32, const float* alpha_col, const float* alpha_row,
                      const void* bias, const void* addend, int m, int n, int k, lq_stream_t stream);
+/* A SmoothQuant linear in one call: lq_sq_input_quant with input_quant_scale[0], or lq_sq_dynamic_quant where that is NULL, of X [m, k], and
+ * lq_gemm_int8 on the codes with the scale or scales; C and bias have X's dtype.  workspace, 16-byte aligned: m * k bytes of codes, with
+ * NULL followed by m scales. */
+int lq_sq_linear(void* C, const void* X, lq_dtype_t dtype, const float* pre_quant_scale, const float* input_quant_scale, void* workspace,
+                 const int8_t* B_rows32, const float* weight_scale, const void* bias, int m, int n, int k, lq_stream_t stream);
 
 /* C[m,n] = T( act( (a_scale[0]*b_scale[0]) * sum_k A[m,k]*B[n,k] + f32(bias[n]) ) + beta*f32(residual[m,n]) )
  * on e4m3 operands with fp32 accumulation; act = tanh-GELU when gelu != 0.  bias and residual are

@@ -148,3 +148,23 @@ extern "C" int lq_gemm_tactics_deserialize(const void* data, size_t bytes) {
     lq::g_shape_entries.store((int)lq::g_shape_tactics.size(), std::memory_order_relaxed);
     return LQ_OK;
 }
+
+extern "C" int lq_sq_linear(void* C, const void* X, lq_dtype_t dtype, const float* pre_quant_scale, const float* input_quant_scale, void* workspace,
+                            const int8_t* B_rows32, const float* weight_scale, const void* bias, int m, int n, int k, lq_stream_t stream) {
+    if (m < 0 || n <= 0 || n % 32 != 0 || k <= 0 || k % 64 != 0) {
+        lq::set_error("lq_sq_linear: need n %% 32 == 0 and k %% 64 == 0 (m=%d n=%d k=%d)", m, n, k);
+        return LQ_ERR_SHAPE;
+    }
+    if (workspace == nullptr || reinterpret_cast<uintptr_t>(workspace) % 16 != 0) {
+        lq::set_error("lq_sq_linear: workspace must be a 16-byte aligned pointer");
+        return LQ_ERR_ARG;
+    }
+    int8_t* codes = static_cast<int8_t*>(workspace);
+    if (input_quant_scale != nullptr) {
+        const int rc = lq_sq_input_quant(codes, X, dtype, pre_quant_scale, input_quant_scale, 0, (size_t)m, (size_t)k, stream);
+        return rc != LQ_OK ? rc : lq_gemm_int8(C, dtype, codes, B_rows32, weight_scale, input_quant_scale, 0, bias, m, n, k, stream);
+    }
+    float* scales = reinterpret_cast<float*>(codes + (size_t)m * k);
+    const int rc = lq_sq_dynamic_quant(codes, scales, X, dtype, pre_quant_scale, (size_t)m, (size_t)k, stream);
+    return rc != LQ_OK ? rc : lq_gemm_int8(C, dtype, codes, B_rows32, weight_scale, scales, m != 1, bias, m, n, k, stream);
+}

@@ -117,6 +117,7 @@ SYMBOLS = {
     "lq_gemm_fp8_codes_panels": (_I, [_P, _P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
     "lq_fp8_scale_cast_panels": (_I, [_P, _P, _I, _P, _I, _Z, _Z, _P]),
     "lq_sq_dynamic_quant_panels": (_I, [_P, _P, _P, _I, _P, _Z, _Z, _P]),
+    "lq_sq_linear": (_I, [_P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "lq_gemm_int8_add": (_I, [_P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "lq_gemm_int8_panels": (_I, [_P, _I, _P, _P, _P, _P, _I, _P, _I, _I, _I, _P]),
     "lq_fp8_gelu_cast_panels": (_I, [_P, _P, _P, _I, _Z, _Z, _P, _P, _P]),

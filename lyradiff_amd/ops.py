@@ -507,6 +507,34 @@ def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.
     return c
 
 
+def sq_linear(x, pre_quant_scale, input_quant_scale, w_rows32, weight_scale, bias=None):
+    """sq_quant (sq_quant_dynamic where input_quant_scale is None) of x [M, K], and int8_linear on the codes.  What both take of 16-bit
+    tensors goes through one call of the library: 1024x1280x1280 with per-token scales 15.5 -> 11.3 us, all of it on the GPU.
+    Anything else is left to the two functions, refusals included."""
+    dt = x.dtype
+    m, k = x.shape
+    if (x.is_cuda and x.is_contiguous() and (dt is torch.float16 or dt is torch.bfloat16) and m > 0 and k > 0 and k % 64 == 0
+            and isinstance(w_rows32, _Tensor) and isinstance(weight_scale, _Tensor) and isinstance(pre_quant_scale, _Tensor)
+            and (bias is None or isinstance(bias, _Tensor)) and (input_quant_scale is None or isinstance(input_quant_scale, _Tensor))
+            and w_rows32.dim() == 2 and (n := w_rows32.shape[0]) > 0 and w_rows32.shape[1] == k and w_rows32.dtype is torch.int8 and w_rows32.is_cuda and w_rows32.is_contiguous()
+            and weight_scale.dtype is torch.float32 and weight_scale.is_cuda and weight_scale.is_contiguous() and weight_scale.numel() == n
+            and pre_quant_scale.dtype is torch.float32 and pre_quant_scale.is_cuda
+            and pre_quant_scale.is_contiguous() and pre_quant_scale.numel() == k
+            and (bias is None or (bias.dtype is dt and bias.is_cuda and bias.is_contiguous()))
+            and (input_quant_scale is None or (input_quant_scale.dtype is torch.float32 and input_quant_scale.is_cuda
+                                               and input_quant_scale.is_contiguous() and input_quant_scale.numel() == 1))):
+        c = torch.empty(m, n, dtype=dt, device=x.device)
+        work = torch.empty(m * k if input_quant_scale is not None else m * (k + 4), dtype=torch.int8, device=x.device)
+        _l.check(_l.load().lq_sq_linear(c.data_ptr(), x.data_ptr(), _DT[dt], pre_quant_scale.data_ptr(), _ptr(input_quant_scale), work.data_ptr(),
+                                        w_rows32.data_ptr(), weight_scale.data_ptr(), _ptr(bias), m, n, k, _stream()), "lq_sq_linear")
+        return c
+    if input_quant_scale is None:
+        q, input_quant_scale = sq_quant_dynamic(x, pre_quant_scale)
+    else:
+        q = sq_quant(x, pre_quant_scale, input_quant_scale)
+    return int8_linear(q, w_rows32, weight_scale, input_quant_scale, bias, dt)
+
+
 def fp8_linear(a_q, w_rows32, a_scale, b_scale, bias=None, gelu: bool = False, residual=None, beta: float = 0.0,
                out_dtype=torch.bfloat16, out_scale=None, out_fp8_scale=None, want_output: bool = True):
     """FP8 GemmWithResidualAndBias: a_q uint8 e4m3 [M,K], w_rows32 uint8 e4m3 [N,K] (rows32).

@@ -104,12 +104,8 @@ class Int8Linear:
     bias: Optional[torch.Tensor] = None
 
     def forward(self, x: torch.Tensor, dynamic: bool = False) -> torch.Tensor:
-        x2 = _rows(x)
-        if dynamic:  # per-token scales computed on the fly instead of the calibrated one
-            q, s = ops.sq_quant_dynamic(x2, self.pre_quant_scale)
-        else:
-            q, s = ops.sq_quant(x2, self.pre_quant_scale, self.input_quant_scale), self.input_quant_scale
-        y = ops.int8_linear(q, self.weight_rows32, self.weight_scale, s, self.bias, x.dtype)
+        # dynamic: per-token scales computed on the fly instead of the calibrated one
+        y = ops.sq_linear(_rows(x), self.pre_quant_scale, None if dynamic else self.input_quant_scale, self.weight_rows32, self.weight_scale, self.bias)
         return _shaped(y, x)
 
 

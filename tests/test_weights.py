@@ -56,6 +56,29 @@ def test_int8_linear_from_bin_files(dev, tmp_path):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dynamic", [False, True])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16, torch.float32])
+def test_int8_linear_is_its_two_operations(dev, dt, dynamic):
+    """The quantiser and the GEMM behind it in one call where both take the tensors, else one after the other: the same bits either way."""
+    from lyradiff_amd import ops, weights as W
+
+    for m, n, k, bias in ((1, 32, 64, True), (65, 96, 320, False), (300, 640, 640, True)):
+        g = torch.Generator(device=dev).manual_seed(m + n + k)
+        w = ops.repack_weight(torch.randint(-127, 128, (n, k), generator=g, device=dev, dtype=torch.int8))
+        rnd = lambda *s: torch.rand(*s, generator=g, device=dev)
+        lin = W.Int8Linear(w, 1e-3 + 1e-2 * rnd(n), torch.full((1,), 0.03, device=dev), 0.5 + rnd(k), rnd(n).to(dt) if bias else None)
+        x = torch.randn(m, k, generator=g, device=dev).to(dt)
+        q, s = ops.sq_quant_dynamic(x, lin.pre_quant_scale) if dynamic else (ops.sq_quant(x, lin.pre_quant_scale, lin.input_quant_scale), lin.input_quant_scale)
+        want = ops.int8_linear(q, w, lin.weight_scale, s, lin.bias, dt)
+        y = lin.forward(x, dynamic=dynamic)
+        assert y.dtype == dt and torch.equal(y, want), (m, n, k)
+        for name, bad, error in (("pre_quant_scale", lin.pre_quant_scale[:-1], ValueError), ("weight_scale", lin.weight_scale.half(), TypeError),
+                                 ("weight_rows32", w.t(), ValueError), ("bias", lin.weight_scale.double(), TypeError), ("weight_scale", None, TypeError)):
+            with pytest.raises(error):
+                W.Int8Linear(**{**vars(lin), name: bad}).forward(x, dynamic=dynamic)
+
+
+@pytest.mark.gpu
 def test_fp8_linear_from_state_dict(dev):
     from lyradiff_amd import weights as W
 
