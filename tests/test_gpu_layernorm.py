@@ -70,6 +70,31 @@ def test_fused_residual_bias_layernorm_int8(ops, dev, dt, with_bias):
     close_codes(q.cpu().numpy(), q_ref, "fused residual layernorm int8")
 
 
+# rows that share a wavefront: fewer than wavefronts, one more than they are, a last turn that only some have; the four widths that are walked
+# this way and, behind the last, one that is not
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,dim", [(1, 640), (2049, 640), (4100, 768), (3, 1152), (2050, 1280), (5, 1024)])
+@pytest.mark.parametrize("dynamic", [False, True])
+@pytest.mark.parametrize("residual", ["none", "residual", "bias"])
+def test_layernorm_int8_several_rows_a_wavefront(ops, dev, dt, rows, dim, dynamic, residual):
+    g = rng_t(3 * rows + dim)
+    t = TORCH_DT[dt]
+    x, res = (torch.randn(rows, dim, generator=g) * 2 + 0.3).to(t), torch.randn(rows, dim, generator=g).to(t)
+    gamma, beta, bias = ((a + 0.1 * torch.randn(dim, generator=g)).to(t) for a in (1.0, 0.0, 0.0))
+    pre = (0.5 + torch.rand(dim, generator=g)).float()
+    s_in = torch.tensor([0.031], dtype=torch.float32)
+    r, b = (res if residual != "none" else None), (bias if residual == "bias" else None)
+    on = lambda v: None if v is None else v.to(dev)
+    q, s, h = ops.layernorm_int8(on(x), on(gamma), on(beta), on(pre), None if dynamic else on(s_in), on(r), on(b))
+    as_np = lambda v: None if v is None else to_np_f32(v)
+    q_ref, s_ref, h_ref = O.layernorm_int8(to_np_f32(x), as_np(r), as_np(b), to_np_f32(gamma), to_np_f32(beta), pre.numpy(),
+                                           None if dynamic else s_in.numpy(), dt)
+    assert (h is None) if r is None else np.array_equal(to_np_f32(h), h_ref)
+    close_codes(q.cpu().numpy(), q_ref, "layernorm int8")
+    if dynamic:
+        assert np.all(np.abs(s.cpu().numpy() - s_ref) <= 2.0 ** (-10 if dt == "f16" else -7) * s_ref)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("batch,seq,dim", [(2, 2304, 3072), (1, 512, 3072), (3, 50, 768), (2, 37, 2568)])
 def test_layernorm_mod_fp8(ops, dev, dt, batch, seq, dim):
