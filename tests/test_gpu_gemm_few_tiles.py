@@ -87,3 +87,36 @@ def test_a_cached_tactic_stands(dev):
         finally:
             ops.gemm_shape_tactic("fp8", rows, n, k, -1)
     assert torch.equal(run(), shared)
+
+
+# tiles of 128x128 and 192x128 in 128-byte k-tiles: one round of either, one tile less and more than a round of the former, k from where INT8
+# takes them on, rows and columns that leave tiles partly filled
+@pytest.mark.parametrize("m,n,k", [(6000, 640, 640), (8191, 608, 768), (8192, 640, 1024), (2040, 2048, 1280), (2049, 2048, 1280), (1345, 3040, 1152)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_forms_of_eight_wavefronts(dev, m, n, k, dt):
+    from lyradiff_amd import ops
+
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    a, w = (torch.randint(-127, 128, (r, k), generator=g, device=dev, dtype=torch.int8) for r in (m, n))
+    col, row = (1e-4 * (0.5 + torch.rand(r, generator=g, device=dev)) for r in (n, m))
+    bias, add = torch.randn(n, generator=g, device=dev).to(dt), torch.randn(m, n, generator=g, device=dev).to(dt)
+    acc = (a.double() @ w.double().t()).float()  # integers below 2^24: the 32-bit sums, exactly
+    want = lambda s: (acc * (col[None] * s) + bias.float()).to(dt)
+    w32, panels = ops.repack_weight(w), a.view(m, k // 64, 64).transpose(0, 1).contiguous()
+    assert torch.equal(ops.int8_linear(a, w32, col, row, bias, dt), want(row[:, None]))
+    assert torch.equal(ops.int8_linear_panels(panels, w32, col, row, bias, dt), want(row[:, None]))
+    assert torch.equal(ops.int8_linear(a, w32, col, row[:1], bias, dt, add), want(row[:1]) + add)
+
+    # e4m3: as above, a 13-bit sum of a matrix instruction's products and 24 bits for the running one
+    a, w = _fp8((m, k), g, dev), _fp8((n, k), g, dev)
+    one, w32 = torch.ones(1, device=dev), ops.repack_weight(w.view(torch.uint8))
+    ref = a.double() @ w.double().t() + bias.double()
+    terms = a.double().abs() @ w.double().abs().t()
+    half_ulp = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+    bound = 1.01 * half_ulp * ref.abs() + (k // 64) * 64 * 16.0 * 2.0 ** -13 + (k // 64 + 4) * 2.0 ** -24 * terms
+    codes = a.view(torch.uint8)
+    y = ops.fp8_linear(codes, w32, one, one, bias, out_dtype=dt)
+    assert bool(((y.double() - ref).abs() <= bound).all())
+    assert torch.equal(ops.fp8_linear_panels(codes.view(m, k // 64, 64).transpose(0, 1).contiguous(), w32, one, one, bias, None, dt), y)
+    gate, res = torch.randn(1, n, generator=g, device=dev).to(dt), torch.randn(m, n, generator=g, device=dev).to(dt)
+    assert torch.equal(ops.fp8_linear_gated(codes, w32, one, one, bias, gate, res, m), y * gate + res)
