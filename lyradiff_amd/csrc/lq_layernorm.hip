@@ -15,7 +15,10 @@
 // activation is read once and only the 1-byte codes (and dst2) are written.  Mean and variance are two-pass
 // fp32 sums over the registers (the reference runs Welford updates, in T for the INT8 kernels), reduced across
 // the 64 lanes in a fixed order; rstd = 1 / sqrt(var + eps) with IEEE sqrt and division.
+#include <algorithm>
+
 #include "lq_common.h"
+#include "lq_walk.h"
 
 namespace lq {
 
@@ -296,104 +299,48 @@ __global__ __launch_bounds__(SPLIT ? 384 : 256) void ln_quant_rows_kernel(uint8_
     }
 }
 
-// INT8, rows of 512 * NF + 64 * TAIL columns: a lane holds eight columns of each pass and TAIL of the rest, where the kernel above has a last
-// pass that most lanes spend on nothing; a wavefront walks over rows with the vectors in registers, and requests the next row ahead of
+// INT8, rows that a wavefront holds as a whole (lq_walk.h): it walks over rows with the vectors in registers, and requests the next row ahead of
 // this one's statistics.  What bounds it: vector instructions, beside the way of the first row (a sum of two tensors of 8192 x 640 takes
 // 4.0 us on this card, an empty launch 2.1).
-// us, the kernel above / this, f16: 8192 x 640 7.9 / 6.8, with residual and bias 12.0 / 8.4; 2048 x 1280 5.1 / 4.7, 6.7 / 5.8; 1024 x 1280 4.7 / 3.6,
-// 5.8 / 4.1.  The residual's sums as packed f16: 9.1 -> 8.4.
-template <int N> __device__ __forceinline__ void ln_quant_s8(const float* t, float s, float r, bool slow, u32* words) {
-    float rq[N], dev = 0.0f;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const float qa = t[i] * r;
-        rq[i] = __builtin_rintf(qa);
-        dev = fmaxf(dev, fabsf(qa - rq[i]));
-    }
-    if (__builtin_expect(slow | !(dev <= 0.5f - tie_margin<127>()), 0)) {  // see quant8_round
-#pragma unroll
-        for (int i = 0; i < N; ++i) rq[i] = __builtin_rintf(t[i] / s);
-    }
-    int q[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const int v = cvt_i32_sat(rq[i]);
-        q[i] = v < -128 ? -128 : (v > 127 ? 127 : v);
-    }
-#pragma unroll
-    for (int i = 0; i < N; i += 4) words[i / 4] = pack4_s8(q[i], q[i + 1], i + 2 < N ? q[i + 2 < N ? i + 2 : 0] : 0, i + 3 < N ? q[i + 3 < N ? i + 3 : 0] : 0);
-}
+// us, the kernel above / this, f16: 8192 x 640 7.9 / 6.6, with residual and bias 11.9 / 8.3; 2048 x 1280 5.2 / 4.7, 6.6 / 5.7; 1024 x 1280 4.6 / 3.6,
+// 5.9 / 4.2; 8192 x 1280 10.8 / 10.1, 18.1 / 13.6.  The residual's sums as packed f16: 9.1 -> 8.4.
 template <typename Tag, int NF, int TAIL, int QMODE, int RESID>
 __global__ __launch_bounds__(256) void ln_int8_walk_kernel(uint8_t* __restrict__ dst, void* __restrict__ dst2, float* __restrict__ scale_out,
                                                            const void* __restrict__ src, const void* __restrict__ residual,
                                                            const void* __restrict__ bias, const void* __restrict__ gamma,
                                                            const void* __restrict__ beta, const float* __restrict__ pre,
                                                            const float* __restrict__ in_scale, u32 rows, float eps, float rdim) {
-    constexpr int E = 8 * NF + TAIL, DIM = 64 * E;
+    using Row = WalkRow<Tag, NF, TAIL>;
+    constexpr int E = Row::E, DIM = Row::DIM;
     const int lane = threadIdx.x & 63;
     const u32 nw = gridDim.x * 4;
     u32 row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (row >= rows) return;
-    struct Raw { uint4 full[NF]; u32 tail[TAIL / 2]; };
-    auto load = [&](const void* base, size_t r) {
-        const unsigned short* p = static_cast<const unsigned short*>(base) + r * DIM;
-        Raw o;
-#pragma unroll
-        for (int i = 0; i < NF; ++i) o.full[i] = *reinterpret_cast<const uint4*>(p + i * 512 + lane * 8);
-        if constexpr (TAIL == 2) o.tail[0] = *reinterpret_cast<const u32*>(p + NF * 512 + lane * 2);
-        else {
-            const uint2 v = *reinterpret_cast<const uint2*>(p + NF * 512 + lane * 4);
-            o.tail[0] = v.x; o.tail[1] = v.y;
-        }
-        return o;
-    };
-    auto unpack = [&](const Raw& r, float* o) {
-#pragma unroll
-        for (int i = 0; i < NF; ++i) unpack8<Tag>(r.full[i], o + 8 * i);
-#pragma unroll
-        for (int i = 0; i < TAIL / 2; ++i) {
-            o[8 * NF + 2 * i] = Elem<Tag>::load(r.tail[i] & 0xFFFFu);
-            o[8 * NF + 2 * i + 1] = Elem<Tag>::load(r.tail[i] >> 16);
-        }
-    };
-    Raw x = load(src, row), res;
-    if constexpr (RESID == 1) res = load(residual, row);
+    Row x, res, vec;
+    x.load(src, row, lane);
+    if constexpr (RESID == 1) res.load(residual, row, lane);
     float g[E], b[E], pv[E];
     u32 bw[RESID == 1 ? E / 2 : 1];
-    unpack(load(gamma, 0), g);
-    unpack(load(beta, 0), b);
-    auto words = [&](const Raw& r, u32* w) {
-#pragma unroll
-        for (int i = 0; i < NF; ++i) w[4 * i] = r.full[i].x, w[4 * i + 1] = r.full[i].y, w[4 * i + 2] = r.full[i].z, w[4 * i + 3] = r.full[i].w;
-#pragma unroll
-        for (int i = 0; i < TAIL / 2; ++i) w[4 * NF + i] = r.tail[i];
-    };
+    vec.load(gamma, 0, lane);
+    vec.unpack(g);
+    vec.load(beta, 0, lane);
+    vec.unpack(b);
     if constexpr (RESID == 1) {
 #pragma unroll
         for (int i = 0; i < E / 2; ++i) bw[i] = 0x80008000u;  // -0 changes nothing
-        if (bias != nullptr) words(load(bias, 0), bw);
-    }
-#pragma unroll
-    for (int i = 0; i < E; ++i) pv[i] = 1.0f;
-    if (pre != nullptr) {
-#pragma unroll
-        for (int i = 0; i < 8 * NF; i += 4) {
-            const float4 v = *reinterpret_cast<const float4*>(pre + (i / 8) * 512 + lane * 8 + i % 8);
-            pv[i] = v.x; pv[i + 1] = v.y; pv[i + 2] = v.z; pv[i + 3] = v.w;
-        }
-#pragma unroll
-        for (int i = 0; i < TAIL; i += 2) {
-            const float2 v = *reinterpret_cast<const float2*>(pre + NF * 512 + lane * TAIL + i);
-            pv[8 * NF + i] = v.x; pv[8 * NF + i + 1] = v.y;
+        if (bias != nullptr) {
+            vec.load(bias, 0, lane);
+            vec.words(bw);
         }
     }
+    Row::load_f32(pre, lane, pv);
     const float s_in = QMODE == 0 ? in_scale[0] : 1.0f;
     for (;;) {
         float h[E];
         if constexpr (RESID == 1) {
             u32 w[E / 2], r[E / 2];
-            words(x, w);
-            words(res, r);
+            x.words(w);
+            res.words(r);
 #pragma unroll
             for (int i = 0; i < E / 2; ++i) {
                 if constexpr (std::is_same<Tag, F16Tag>::value) {  // two values an instruction, each sum rounded once: what 32 bits and a rounding make too
@@ -407,19 +354,15 @@ __global__ __launch_bounds__(256) void ln_int8_walk_kernel(uint8_t* __restrict__
                 h[2 * i] = Elem<Tag>::load(w[i] & 0xFFFFu);
                 h[2 * i + 1] = Elem<Tag>::load(w[i] >> 16);
             }
-            unsigned short* o = static_cast<unsigned short*>(dst2) + (size_t)row * DIM;
-#pragma unroll
-            for (int i = 0; i < NF; ++i) *reinterpret_cast<uint4*>(o + i * 512 + lane * 8) = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
-            if constexpr (TAIL == 2) *reinterpret_cast<u32*>(o + NF * 512 + lane * 2) = w[4 * NF];
-            else *reinterpret_cast<uint2*>(o + NF * 512 + lane * 4) = make_uint2(w[4 * NF], w[4 * NF + 1]);
+            Row::store_words(dst2, row, lane, w);
         } else {
-            unpack(x, h);
+            x.unpack(h);
         }
         const u32 next = row + nw;
         const bool more = next < rows;
         if (more) {
-            x = load(src, next);
-            if constexpr (RESID == 1) res = load(residual, next);
+            x.load(src, next, lane);
+            if constexpr (RESID == 1) res.load(residual, next, lane);
         }
         // two chains each: nobody else fills the latency of a dependent instruction
         float s0 = h[0], s1 = h[1];
@@ -451,19 +394,7 @@ __global__ __launch_bounds__(256) void ln_int8_walk_kernel(uint8_t* __restrict__
             if (amax <= 5.9604644775390625e-08f) s = 1.0f;
             if (lane == 0) scale_out[row] = s;
         }
-        const float r = fast_recip(s);
-        const bool slow = scale_out_of_range(s);
-        uint8_t* o = dst + (size_t)row * DIM;
-#pragma unroll
-        for (int i = 0; i < NF; ++i) {
-            u32 w[2];
-            ln_quant_s8<8>(h + 8 * i, s, r, slow, w);
-            *reinterpret_cast<uint2*>(o + i * 512 + lane * 8) = make_uint2(w[0], w[1]);
-        }
-        u32 w;
-        ln_quant_s8<TAIL>(h + 8 * NF, s, r, slow, &w);
-        if constexpr (TAIL == 2) *reinterpret_cast<unsigned short*>(o + NF * 512 + lane * 2) = (unsigned short)w;
-        else *reinterpret_cast<u32*>(o + NF * 512 + lane * 4) = w;
+        Row::store_codes(dst, row, lane, h, s, fast_recip(s), scale_out_of_range(s));
         if (!more) break;
         row = next;
     }
@@ -476,8 +407,7 @@ struct LnArgs {
 };
 
 template <typename Tag, int NF, int TAIL, int QMODE, int RESID> static int launch_ln_walk(const LnArgs& a, hipStream_t st) {
-    // at most two wavefronts per SIMD of 256 CUs: eight times as many, a row each, measured 9.7 us where this takes 9.1 (8192 x 640)
-    const size_t each = (a.rows + 2047) / 2048, waves = (a.rows + each - 1) / each;
+    const size_t waves = std::min<size_t>(a.rows, 4096);  // four per SIMD of 256 CUs; with two 3000 x 1280 takes 6.5 us, the kernel above 6.0, this 5.6
     hipLaunchKernelGGL((ln_int8_walk_kernel<Tag, NF, TAIL, QMODE, RESID>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, a.dst, a.dst2, a.scale_out,
                        a.src, a.residual, a.bias, a.gamma, a.beta, a.pre, a.in_scale, (u32)a.rows, a.eps, 1.0f / (float)a.dim);
     return check_launch("layernorm_quant");

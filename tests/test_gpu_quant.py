@@ -34,6 +34,23 @@ def test_sq_dynamic_quant(ops, dev, dt, m, k):
     assert np.array_equal(s2.cpu().numpy(), s2_ref) and np.array_equal(q2.cpu().numpy(), q2_ref)
 
 
+# widths that a wavefront holds as a whole: one row, as many as wavefronts and one more, a second turn that some of them have
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("m,k", [(1, 640), (4097, 640), (5000, 768), (4096, 1152), (70, 1280)])
+def test_sq_quant_rows_of_whole_wavefronts(ops, dev, dt, m, k):
+    x = make_outlier_acts(m, k, 8, 20.0, TORCH_DT[dt], 2000 + m + k)
+    pre = (torch.rand(k, generator=rng_t(9)) * 1.5 + 0.25).float()
+    one, each = torch.tensor([0.031]), 0.01 + 0.1 * torch.rand(m, generator=rng_t(10))
+    for p in (pre, None):
+        on, p_np = (None if p is None else p.to(dev)), (None if p is None else p.numpy())
+        q, s = ops.sq_quant_dynamic(x.to(dev), on)
+        q_ref, s_ref = O.sq_dynamic_quant(to_np_f32(x), p_np)
+        assert np.array_equal(s.cpu().numpy(), s_ref) and np.array_equal(q.cpu().numpy(), q_ref)
+        for scale, per_token in ((one, False), (each, True)):
+            q = ops.sq_quant(x.to(dev), on, scale.to(dev), per_token)
+            assert np.array_equal(q.cpu().numpy(), O.sq_input_quant(to_np_f32(x), p_np, scale.numpy(), per_token))
+
+
 @pytest.mark.parametrize("k", [64, 2080])
 def test_sq_dynamic_nan_and_inf_rows(ops, dev, k):
     """NaN never enters the row maximum and quantises to 0; a row holding an infinity gets an infinite scale,
