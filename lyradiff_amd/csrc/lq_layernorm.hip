@@ -302,8 +302,9 @@ __global__ __launch_bounds__(SPLIT ? 384 : 256) void ln_quant_rows_kernel(uint8_
 // INT8, rows that a wavefront holds as a whole (lq_walk.h): it walks over rows with the vectors in registers, and requests the next row ahead of
 // this one's statistics.  What bounds it: vector instructions, beside the way of the first row (a sum of two tensors of 8192 x 640 takes
 // 4.0 us on this card, an empty launch 2.1).
-// us, the kernel above / this, f16: 8192 x 640 7.9 / 6.6, with residual and bias 11.9 / 8.3; 2048 x 1280 5.2 / 4.7, 6.6 / 5.7; 1024 x 1280 4.6 / 3.6,
-// 5.9 / 4.2; 8192 x 1280 10.8 / 10.1, 18.1 / 13.6.  The residual's sums as packed f16: 9.1 -> 8.4.
+// us, the kernel above / this, f16, static scale: 8192 x 640 7.6 / 6.7, with residual and bias 11.5 / 8.4; 8192 x 768 7.8 / 7.5, 12.2 / 9.5; 4096 x 1152
+// 6.6 / 6.3, 9.7 / 8.0; 2048 x 1280 5.0 / 4.7, 6.5 / 5.8; 1024 x 1280 4.7 / 3.7, 5.9 / 4.3; 8192 x 1280 10.7 / 10.4, 18.1 / 14.1.  The sums in an order of
+// this layout's own, without the way through LDS: 8192 x 640 6.4, 8.1.  The residual's sums as packed f16: 9.1 -> 8.4.
 template <typename Tag, int NF, int TAIL, int QMODE, int RESID>
 __global__ __launch_bounds__(256) void ln_int8_walk_kernel(uint8_t* __restrict__ dst, void* __restrict__ dst2, float* __restrict__ scale_out,
                                                            const void* __restrict__ src, const void* __restrict__ residual,
@@ -335,8 +336,13 @@ __global__ __launch_bounds__(256) void ln_int8_walk_kernel(uint8_t* __restrict__
     }
     Row::load_f32(pre, lane, pv);
     const float s_in = QMODE == 0 ? in_scale[0] : 1.0f;
+    // The statistics are those of the kernel above to the bit: its last pass has eight columns in each of the first 8 * TAIL lanes, and the
+    // rest of the row takes that form through LDS, for the two sums alone.
+    __shared__ __attribute__((aligned(16))) u32 s_rest[4][32 * TAIL];
+    u32* const rest = s_rest[threadIdx.x >> 6];
     for (;;) {
         float h[E];
+        u32 tail[TAIL / 2];
         if constexpr (RESID == 1) {
             u32 w[E / 2], r[E / 2];
             x.words(w);
@@ -355,28 +361,49 @@ __global__ __launch_bounds__(256) void ln_int8_walk_kernel(uint8_t* __restrict__
                 h[2 * i + 1] = Elem<Tag>::load(w[i] >> 16);
             }
             Row::store_words(dst2, row, lane, w);
+#pragma unroll
+            for (int i = 0; i < TAIL / 2; ++i) tail[i] = w[4 * NF + i];
         } else {
             x.unpack(h);
+#pragma unroll
+            for (int i = 0; i < TAIL / 2; ++i) tail[i] = x.tail[i];
         }
+        if constexpr (TAIL == 2) rest[lane] = tail[0];
+        else *reinterpret_cast<uint2*>(rest + 2 * lane) = make_uint2(tail[0], tail[1]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // a wavefront's LDS accesses complete in order: this binds the compiler
+        __builtin_amdgcn_wave_barrier();
+        const uint4 rest8 = *reinterpret_cast<const uint4*>(rest + 4 * (lane & (8 * TAIL - 1)));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         const u32 next = row + nw;
         const bool more = next < rows;
         if (more) {
             x.load(src, next, lane);
             if constexpr (RESID == 1) res.load(residual, next, lane);
         }
-        // two chains each: nobody else fills the latency of a dependent instruction
-        float s0 = h[0], s1 = h[1];
+        const bool has_rest = lane < 8 * TAIL;
+        float hr[8], sum = 0.0f;
+        unpack8<Tag>(rest8, hr);
 #pragma unroll
-        for (int i = 2; i < E; i += 2) s0 += h[i], s1 += h[i + 1];
+        for (int i = 0; i < 8 * NF; ++i) sum += h[i];
+        float sum_r = sum;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum_r += hr[i];
         auto row_total = [&](float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wave_sum_lane63(v)), 63)); };
-        const float mean = div_small_int(row_total(s0 + s1), (float)DIM, rdim);
-        s0 = s1 = 0.0f;
+        const float mean = div_small_int(row_total(has_rest ? sum_r : sum), (float)DIM, rdim);
+        float sq = 0.0f;
 #pragma unroll
-        for (int i = 0; i < E; i += 2) {
-            h[i] -= mean, h[i + 1] -= mean;
-            s0 = __builtin_fmaf(h[i], h[i], s0), s1 = __builtin_fmaf(h[i + 1], h[i + 1], s1);
+        for (int i = 0; i < E; ++i) {
+            h[i] -= mean;
+            if (i < 8 * NF) sq = __builtin_fmaf(h[i], h[i], sq);
         }
-        const float var = div_small_int(row_total(s0 + s1), (float)DIM, rdim);
+        float sq_r = sq;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float d = hr[i] - mean;
+            sq_r = __builtin_fmaf(d, d, sq_r);
+        }
+        const float var = div_small_int(row_total(has_rest ? sq_r : sq), (float)DIM, rdim);
         const float rstd = 1.0f / __builtin_sqrtf(var + eps);
 #pragma unroll
         for (int i = 0; i < E; i += 2) {

@@ -95,6 +95,25 @@ def test_layernorm_int8_several_rows_a_wavefront(ops, dev, dt, rows, dim, dynami
         assert np.all(np.abs(s.cpu().numpy() - s_ref) <= 2.0 ** (-10 if dt == "f16" else -7) * s_ref)
 
 
+# A row's statistics do not depend on the kernel that forms them: with no scale and shift, the modulated LayerNorm leaves the values that the
+# INT8 one quantises, and its kernel does not walk over rows.  More rows than the 4096 wavefronts of a walk.
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("rows,dim", [(8200, 640), (4099, 768), (4100, 1152), (4300, 1280), (513, 1024)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_layernorm_int8_has_the_modulated_layernorms_statistics(ops, dev, dt, rows, dim, residual):
+    g = torch.Generator(device=dev).manual_seed(rows + dim)
+    t = TORCH_DT[dt]
+    x, res = ((torch.randn(rows, dim, generator=g, device=dev) * 2 + 0.3).to(t) for _ in range(2))
+    pre, s_in = 0.5 + torch.rand(dim, generator=g, device=dev), torch.full((1,), 0.031, device=dev)
+    one, zero = torch.ones(dim, dtype=t, device=dev), torch.zeros(1, dim, dtype=t, device=dev)
+    q, _, h = ops.layernorm_int8(x, one, zero[0], pre, s_in, res if residual else None)
+    qd, sd, _ = ops.layernorm_int8(x, one, zero[0], pre, None, res if residual else None)
+    y = ops.gate_residual_layernorm_mod((h if residual else x)[None], zero, zero)[0]
+    assert torch.equal(q, ops.sq_quant(y, pre, s_in))
+    want, scale = ops.sq_quant_dynamic(y, pre)
+    assert torch.equal(qd, want) and torch.equal(sd, scale)
+
+
 @pytest.mark.parametrize("dt", ["bf16", "f16"])
 @pytest.mark.parametrize("batch,seq,dim", [(2, 2304, 3072), (1, 512, 3072), (3, 50, 768), (2, 37, 2568)])
 def test_layernorm_mod_fp8(ops, dev, dt, batch, seq, dim):
