@@ -38,7 +38,7 @@ template <typename OutTag> static int run_fp8_as(GemmParams p, hipStream_t st) {
     // Too few 256x256 tiles: the form whose rounds of workgroups cost least.  A forced or cached tactic stands.  k <= 1024: a
     // workgroup's ten or sixteen k-tiles leave nothing to share (1024x640x640: 4.7 us with 64x64 tiles, 4.9 with k shared).
     if (requested < 0 && out16 && p.k > 1024 && (long)((p.m + 255) / 256) * ((p.n + 255) / 256) < 192) {
-        t = few_tiles_form(p.m, 0, p.n, p.k);
+        t = few_tiles_form(p.m, 0, p.n, p.k, p.a_panel == 0 && (plain_epilogue || p.k >= 2560));
         if (t >= SMALL_32x32_K4) return run_small(K_FP8, p, out_enum<OutTag>(), t, st);
     }
     if (t == 1 && (p.kb % 128 != 0 || p.a_panel)) t = 0;  // the 128-byte k-tile needs k % 128 == 0 and a row-major activation

@@ -12,6 +12,11 @@
 //     22.6 / 19.4, 4096x640x2560 13.7 / 12.4 / 11.4).  192x128, general / now: FP8 512x9216x3072 20.3 / 16.7, 700x12288x3072 34.5 / 30.4 (two
 //     rounds); INT8 8192x640x2560 21.2 / 17.1, 4096x1280x5120 33.4 / 29.6.  Three or four stages, four wavefronts of 64x64 in place of
 //     eight of 64x32, level; 256x128 tiles 20.7 where 192x128 take 17.1.
+// More than one round of the second kind: for a row-major activation, with a residual, an activation function, gates or codes in the epilogue
+// from k = 2560 up.  Two workgroups of four wavefronts per CU overlap one's epilogue with the other's walk, and k-panels take the cache
+// lines' advantage away (us, four wavefronts / two rounds of these -- row-major, scales and bias: FP8 1024x9216x3072 37.9 / 32.7, x1152 18.4 /
+// 17.4, INT8 1700x5120x5120 65 / 54; gated, FP8 900x9216x3072 40.4 / 37.4, x1152 20.7 / 23.4, k = 2048 0.93 to 1.04 times; INT8 with a
+// residual x3072 43.1 / 39.6, x1152 21.3 / 23.5; k-panels, gated FP8 34.0 / 37.2, x1152 18.2 / 23.4, scales and bias 31.1 / 31.5, x1152 15.8 / 16.9).
 // FP8 of few rows with no more than scales and bias goes to lq_gemm_rows.hip instead.
 #pragma once
 

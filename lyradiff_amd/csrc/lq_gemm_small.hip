@@ -3,7 +3,7 @@
 
 namespace lq {
 
-int few_tiles_form(int m, int m2, int n, int k, float* cost_out) {
+int few_tiles_form(int m, int m2, int n, int k, bool rounds, float* cost_out) {
     auto tiles_of = [&](int bm, int bn) { return (((long)m + bm - 1) / bm + ((long)m2 + bm - 1) / bm) * (((long)n + bn - 1) / bn); };
     // Short k: prologue and epilogue are most of the time, and only the forms of eight wavefronts and 128-byte k-tiles lead, by one
     // round against the 1.25 or the half that 128x128 tiles of four wavefronts make (INT8, k = 640, us, those / this: 640 outputs, 4096 rows
@@ -29,6 +29,7 @@ int few_tiles_form(int m, int m2, int n, int k, float* cost_out) {
     for (const Cost& c : table) {
         if (k % c.k_unit != 0) continue;
         const long tiles = tiles_of(c.bm, c.bn), left = tiles % c.per_round;
+        if ((c.form == SMALL_128x128 || c.form == SMALL_192x128) && tiles > c.per_round && !rounds) continue;
         const float cost = (float)(tiles / c.per_round) * c.us[(c.per_round + 255) / 256 - 1] + (left == 0 ? 0.0f : c.us[(left - 1) / 256]);
         if (least == 0.0f || cost < least) { best = c.form; least = cost; }
     }
