@@ -1149,10 +1149,10 @@ int launch_persist_fp8(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st
 int launch_persist_int8(const GemmParams& p, lq_dtype_t out_dtype, hipStream_t st);
 // Forms for problems of few tiles (lq_gemm_small.hip); numbered behind the tactics, which can be forced and cached: these cannot.
 enum SmallForm { SMALL_32x32_K4 = 64, SMALL_32x64_K4, SMALL_64x128_K2, SMALL_128x128, SMALL_192x128 };
-// the tactic or form for fewer than 192 tiles of 256x256 and 16-bit outputs (k <= 1024: -1 where none of the forms leads); m2: rows of a second problem in the same launch;
-// cost_out: its time by the table that it goes by
-// rounds: whether the forms of eight wavefronts may take more than one round (lq_gemm_small.h)
+// The tactic or form for fewer than 192 tiles of 256x256, k > 1024 and 16-bit outputs; m2: rows of a second problem in the same launch;
+// rounds: whether the forms of eight wavefronts may take more than one round (lq_gemm_small.h); cost_out: its time by the table that it goes by.
 int few_tiles_form(int m, int m2, int n, int k, bool rounds, float* cost_out = nullptr);
+int short_k_form(int m, int n, int k);  // the same for k <= 1024, or -1 where none of the forms leads
 int run_small(GemmKind kind, const GemmParams& p, lq_dtype_t out_dtype, int form, hipStream_t st);
 int run_small_fp8_bf16(const GemmParams& p, int form, hipStream_t st);  // lq_gemm_small_{bf16,f16}.hip
 int run_small_fp8_f16(const GemmParams& p, int form, hipStream_t st);

@@ -40,7 +40,8 @@ template <typename OutTag> static int run_int8(GemmParams p, hipStream_t st) {
     }
     // Too few 256x256 tiles: the form whose rounds of workgroups cost least.  A forced or cached tactic stands.
     if (requested < 0 && out16 && (long)((p.m + 255) / 256) * ((p.n + 255) / 256) < 192) {
-        const int form = few_tiles_form(p.m, 0, p.n, p.k, p.a_panel == 0 && (p.addend == nullptr || p.k >= 2560));
+        const int form = p.k <= 1024 ? short_k_form(p.m, p.n, p.k)
+                                     : few_tiles_form(p.m, 0, p.n, p.k, p.a_panel == 0 && (p.addend == nullptr || p.k >= 2560));
         if (form >= SMALL_32x32_K4) return run_small(K_INT8, p, out_enum<OutTag>(), form, st);
         if (form >= 0) t = form;
     }

@@ -3,16 +3,21 @@
 
 namespace lq {
 
+static long tiles_of(int m, int m2, int n, int bm, int bn) {
+    return (((long)m + bm - 1) / bm + ((long)m2 + bm - 1) / bm) * (((long)n + bn - 1) / bn);
+}
+
+// Short k: prologue and epilogue are most of the time, and only the forms of eight wavefronts and 128-byte k-tiles lead, by one round
+// against the 1.25 or the half that 128x128 tiles of four wavefronts make (INT8, us, those / this: k = 640, 640 outputs, 4096 rows 6.7 / 6.3,
+// 6000 7.6 / 7.0, 8192 9.5 / 8.4, 2048 rows, 80 tiles, 5.8 / 5.9; 1024x5120 11.1 / 10.0, 1500x1920 8.4 / 7.6; k = 768 1345x3040 11.7 / 9.9; k = 896
+// 2048x1920 9.3 / 8.8; k = 1024 8192x640 13.2 / 11.6, 1024x5120 13.1 / 11.3).
+int short_k_form(int m, int n, int k) {
+    if (k < 640 || k % 128 != 0) return -1;
+    const long t128 = tiles_of(m, 0, n, 128, 128);
+    return t128 > 256 && tiles_of(m, 0, n, 192, 128) <= 256 ? SMALL_192x128 : t128 > 128 && t128 <= 256 ? SMALL_128x128 : -1;
+}
+
 int few_tiles_form(int m, int m2, int n, int k, bool rounds, float* cost_out) {
-    auto tiles_of = [&](int bm, int bn) { return (((long)m + bm - 1) / bm + ((long)m2 + bm - 1) / bm) * (((long)n + bn - 1) / bn); };
-    // Short k: prologue and epilogue are most of the time, and only the forms of eight wavefronts and 128-byte k-tiles lead, by one
-    // round against the 1.25 or the half that 128x128 tiles of four wavefronts make (INT8, k = 640, us, those / this: 640 outputs, 4096 rows
-    // 6.7 / 6.3, 6000 7.6 / 7.0, 8192 9.5 / 8.4; 2048 rows, 80 tiles, 5.8 / 5.9).
-    if (k <= 1024) {
-        if (k < 640 || k % 128 != 0) return -1;
-        const long t128 = tiles_of(128, 128);
-        return t128 > 256 && tiles_of(192, 128) <= 256 ? SMALL_192x128 : t128 > 128 && t128 <= 256 ? SMALL_128x128 : -1;
-    }
     // Time of a launch by the number of workgroups each CU of 256 has to hold (us at k = 3072): up to 256 of them, up to 512, ...; more
     // than fit make whole rounds.  k is a multiple of k_unit.
     struct Cost { int form, bm, bn, per_round, k_unit; float us[4]; };
@@ -28,7 +33,7 @@ int few_tiles_form(int m, int m2, int n, int k, bool rounds, float* cost_out) {
     float least = 0.0f;
     for (const Cost& c : table) {
         if (k % c.k_unit != 0) continue;
-        const long tiles = tiles_of(c.bm, c.bn), left = tiles % c.per_round;
+        const long tiles = tiles_of(m, m2, n, c.bm, c.bn), left = tiles % c.per_round;
         if ((c.form == SMALL_128x128 || c.form == SMALL_192x128) && tiles > c.per_round && !rounds) continue;
         const float cost = (float)(tiles / c.per_round) * c.us[(c.per_round + 255) / 256 - 1] + (left == 0 ? 0.0f : c.us[(left - 1) / 256]);
         if (least == 0.0f || cost < least) { best = c.form; least = cost; }
