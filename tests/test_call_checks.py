@@ -36,6 +36,18 @@ def test_int8_linear_refuses_a_residual_in_host_memory(ops, per_token):
         ops.int8_linear(a, w, torch.ones(32), torch.ones(4 if per_token else 1), None, torch.float16, addend=torch.zeros(4, 32, dtype=torch.float16))
 
 
+def test_int8_linear_without_a_calibrated_scale_is_refused_unless_dynamic(monkeypatch):
+    from lyradiff_amd import ops as _ops, weights
+
+    lin = weights.Int8Linear(torch.zeros(32, 64, dtype=torch.int8), torch.ones(32), None, torch.ones(64))
+    x, seen = torch.zeros(4, 64, dtype=torch.float16), []
+    monkeypatch.setattr(_ops, "sq_quant_dynamic", lambda *a: pytest.fail("quantised per token"))
+    with pytest.raises(TypeError, match="input_quant_scale"):
+        lin.forward(x)
+    monkeypatch.setattr(_ops, "sq_linear", lambda x, pre, scale, *a: (seen.append(scale), x)[1])
+    assert lin.forward(x, dynamic=True) is x and seen == [None]
+
+
 @pytest.mark.parametrize("which", [0, 1])
 @pytest.mark.parametrize("bad", [{1: torch.ones(0)}, {2: torch.ones(0)}, {2: torch.ones(64)}, {3: torch.zeros(32, dtype=torch.float16)}])
 def test_fp8_linear_rows_refuses_short_scales_and_biases(ops, which, bad):
