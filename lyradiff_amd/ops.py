@@ -32,6 +32,14 @@ def _chk(t: torch.Tensor, name: str, dtypes=None) -> torch.Tensor:
     return t
 
 
+def _chk_bias(bias, dtype, n: int, m: int) -> None:
+    """bias of a linear of N outputs, or None; a longer one has its first N values used.  A kernel would read a shorter one past its end."""
+    if bias is not None:
+        _chk(bias, "bias", (dtype,))
+        if bias.numel() < n and m:
+            raise ValueError("bias must have N elements")
+
+
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
@@ -478,6 +486,7 @@ def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.
     n = w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
+    _chk_bias(bias, out_dtype, n if out_dtype != torch.int32 else 0, m)  # 32-bit sums come without
     per_token = 0
     if out_dtype != torch.int32:
         _chk(alpha_col, "alpha_col", (torch.float32,))
@@ -487,8 +496,6 @@ def int8_linear(a_q, w_rows32, alpha_col, alpha_row, bias=None, out_dtype=torch.
         if alpha_row.numel() not in (1, m):
             raise ValueError("alpha_row must have 1 or M elements")
         per_token = int(alpha_row.numel() == m and m != 1)
-    if bias is not None:
-        _chk(bias, "bias", (out_dtype,))
     if addend is not None:
         if addend.shape != (m, n):
             raise ValueError("addend must be [M, N]")
@@ -520,7 +527,7 @@ def sq_linear(x, pre_quant_scale, input_quant_scale, w_rows32, weight_scale, bia
             and weight_scale.dtype is torch.float32 and weight_scale.is_cuda and weight_scale.is_contiguous() and weight_scale.numel() == n
             and pre_quant_scale.dtype is torch.float32 and pre_quant_scale.is_cuda
             and pre_quant_scale.is_contiguous() and pre_quant_scale.numel() == k
-            and (bias is None or (bias.dtype is dt and bias.is_cuda and bias.is_contiguous()))
+            and (bias is None or (bias.dtype is dt and bias.is_cuda and bias.is_contiguous() and bias.numel() >= n))
             and (input_quant_scale is None or (input_quant_scale.dtype is torch.float32 and input_quant_scale.is_cuda
                                                and input_quant_scale.is_contiguous() and input_quant_scale.numel() == 1))):
         c = torch.empty(m, n, dtype=dt, device=x.device)
@@ -549,8 +556,7 @@ def fp8_linear(a_q, w_rows32, a_scale, b_scale, bias=None, gelu: bool = False, r
     n = w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
-    if bias is not None:
-        _chk(bias, "bias", (out_dtype,))
+    _chk_bias(bias, out_dtype, n, m)
     if residual is not None:
         _chk(residual, "residual", (out_dtype,))
     for name, t in (("out_scale", out_scale), ("out_fp8_scale", out_fp8_scale)):
@@ -580,8 +586,7 @@ def fp8_linear_max(a_q, w_rows32, a_scale, b_scale, bias, out_max, out_dtype=tor
     n = w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
-    if bias is not None:
-        _chk(bias, "bias", (out_dtype,))
+    _chk_bias(bias, out_dtype, n, m)
     c = torch.empty(m, n, dtype=out_dtype, device=a_q.device)
     _l.check(_l.load().lq_gemm_fp8_max(_ptr(c), _DT[out_dtype], _ptr(a_q), _ptr(w_rows32), _ptr(a_scale), _ptr(b_scale),
                                        _ptr(bias), m, n, k, _ptr(out_max), _stream()), "lq_gemm_fp8_max")
@@ -685,8 +690,7 @@ def fp8_linear_panels(a_panels, w_rows32, a_scale, b_scale, bias, out_max=None, 
     n = w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
-    if bias is not None:
-        _chk(bias, "bias", (out_dtype,))
+    _chk_bias(bias, out_dtype, n, m)
     c = torch.empty(m, n, dtype=out_dtype, device=a_panels.device)
     _l.check(_l.load().lq_gemm_fp8_panels(_ptr(c), _DT[out_dtype], _ptr(a_panels), _ptr(w_rows32), _ptr(a_scale), _ptr(b_scale),
                                           _ptr(bias), m, n, k, _ptr(out_max), _stream()), "lq_gemm_fp8_panels")
@@ -721,6 +725,7 @@ def int8_linear_panels(a_panels, w_rows32, alpha_col, alpha_row, bias=None, out_
     n = w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
+    _chk_bias(bias, out_dtype, n if out_dtype != torch.int32 else 0, m)  # 32-bit sums come without
     per_token = 0
     if out_dtype != torch.int32:
         _chk(alpha_col, "alpha_col", (torch.float32,))
@@ -730,8 +735,6 @@ def int8_linear_panels(a_panels, w_rows32, alpha_col, alpha_row, bias=None, out_
         if alpha_row.numel() not in (1, m):
             raise ValueError("alpha_row must have 1 or M elements")
         per_token = int(alpha_row.numel() == m and m != 1)
-    if bias is not None:
-        _chk(bias, "bias", (out_dtype,))
     c = torch.empty(m, n, dtype=out_dtype, device=a_panels.device)
     _l.check(_l.load().lq_gemm_int8_panels(_ptr(c), _DT[out_dtype], _ptr(a_panels), _ptr(w_rows32), _ptr(alpha_col),
                                            _ptr(alpha_row), per_token, _ptr(bias), m, n, k, _stream()), "lq_gemm_int8_panels")
@@ -747,12 +750,11 @@ def fp8_linear_gated(a_q, w_rows32, a_scale, b_scale, bias, gate, residual, rows
     _chk(b_scale, "b_scale", (torch.float32,))
     _chk(residual, "residual", _FLOATS)
     _chk(gate, "gate", (residual.dtype,))
-    if bias is not None:
-        _chk(bias, "bias", (residual.dtype,))
     m, k = a_q.shape
     n = w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
+    _chk_bias(bias, residual.dtype, n, m)
     if residual.numel() != m * n or rows_per_gate <= 0 or gate.numel() != ((m + rows_per_gate - 1) // rows_per_gate) * n:
         raise ValueError("residual must be [M,N] and gate [ceil(M/rows_per_gate), N]")
     if out is None:
@@ -774,12 +776,11 @@ def fp8_linear_codes(a_q, w_rows32, a_scale, b_scale, bias, out_fp8_scale, gelu:
     _chk(a_scale, "a_scale", (torch.float32,))
     _chk(b_scale, "b_scale", (torch.float32,))
     _chk(out_fp8_scale, "out_fp8_scale", (torch.float32,))
-    if bias is not None:
-        _chk(bias, "bias", (round_dtype,))
     m, k = a_q.shape
     n = w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
+    _chk_bias(bias, round_dtype, n, m)
     if out is None:
         out = torch.empty(m, n, dtype=torch.uint8, device=a_q.device)
     _chk(out, "out", (torch.uint8,))
@@ -799,14 +800,13 @@ def fp8_linear_gated_panels(a_panels, w_rows32, a_scale, b_scale, bias, gate, re
     _chk(b_scale, "b_scale", (torch.float32,))
     _chk(residual, "residual", _FLOATS)
     _chk(gate, "gate", (residual.dtype,))
-    if bias is not None:
-        _chk(bias, "bias", (residual.dtype,))
     if a_panels.dim() != 3 or a_panels.shape[2] != 64:
         raise ValueError("a_panels must be [K/64, M, 64]")
     kp, m, _ = a_panels.shape
     k, n = kp * 64, w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
+    _chk_bias(bias, residual.dtype, n, m)
     if residual.numel() != m * n or rows_per_gate <= 0 or gate.numel() != ((m + rows_per_gate - 1) // rows_per_gate) * n:
         raise ValueError("residual must be [M,N] and gate [ceil(M/rows_per_gate), N]")
     if out is None:
@@ -828,14 +828,13 @@ def fp8_linear_codes_panels(a_panels, w_rows32, a_scale, b_scale, bias, out_fp8_
     _chk(a_scale, "a_scale", (torch.float32,))
     _chk(b_scale, "b_scale", (torch.float32,))
     _chk(out_fp8_scale, "out_fp8_scale", (torch.float32,))
-    if bias is not None:
-        _chk(bias, "bias", (round_dtype,))
     if a_panels.dim() != 3 or a_panels.shape[2] != 64:
         raise ValueError("a_panels must be [K/64, M, 64]")
     kp, m, _ = a_panels.shape
     k, n = kp * 64, w_rows32.shape[0]
     if w_rows32.shape[1] != k:
         raise ValueError("K mismatch between activation and weight")
+    _chk_bias(bias, round_dtype, n, m)
     if n % 64 != 0:
         raise ValueError("codes in k-panels need N % 64 == 0")
     if out is None:
@@ -1011,12 +1010,11 @@ def weight_only_linear(x, w_prepared, scales, bias=None, kind: str = "int8"):
     _chk(x, "x", (torch.float16, torch.bfloat16))
     _chk(w_prepared, "w_prepared", (torch.uint8,))
     _chk(scales, "scales", (x.dtype,))
-    if bias is not None:
-        _chk(bias, "bias", (x.dtype,))
     m, k = x.shape
     n = w_prepared.shape[0]
     if w_prepared.shape[1] != (k // 2 if kind == "int4" else k) or scales.numel() != n:
         raise ValueError("shape mismatch between x, w_prepared and scales")
+    _chk_bias(bias, x.dtype, n, m)
     c = torch.empty(m, n, dtype=x.dtype, device=x.device)
     _l.check(_l.load().lq_gemm_weight_only(_ptr(c), _ptr(x), _DT[x.dtype], _ptr(w_prepared), _KINDS[kind], _ptr(scales),
                                            _ptr(bias), m, n, k, _stream()), "lq_gemm_weight_only")
@@ -1107,8 +1105,7 @@ def _w4a4_gemm(launch, m, n, device, bias, out_dtype, lora_act, lora_up, gelu, a
                col_offset, want_output, out):
     """What the two operand forms share: checks of the low-rank branch and the epilogue options, the outputs, the call
     launch(output pointer, (lora_act, lora_up, their dtype, rank), epilogue pointer)."""
-    if bias is not None:
-        _chk(bias, "bias", (out_dtype,))
+    _chk_bias(bias, out_dtype, n, m)
     rank, lora_dt = 0, _l.LQ_BF16
     if (lora_act is None) != (lora_up is None):
         raise ValueError("the low-rank branch needs both lora_act and lora_up")

@@ -60,6 +60,39 @@ def test_fp8_linear_rows_refuses_short_scales_and_biases(ops, which, bad):
         ops.fp8_linear_rows(x, wrong)
 
 
+# every linear whose kernel reads N values of a bias; m rows, n outputs, k inputs
+_U8, _F = (lambda *s: torch.zeros(*s, dtype=torch.uint8)), torch.ones
+LINEARS = {
+    "int8_linear": lambda ops, b, m, n, k: ops.int8_linear(_U8(m, k), _U8(n, k), _F(n), _F(1), b, torch.float16),
+    "int8_linear_panels": lambda ops, b, m, n, k: ops.int8_linear_panels(_U8(k // 64, m, 64), _U8(n, k), _F(n), _F(1), b, torch.float16),
+    "sq_linear": lambda ops, b, m, n, k: ops.sq_linear(torch.zeros(m, k, dtype=torch.float16), _F(k), _F(1), _U8(n, k), _F(n), b),
+    "fp8_linear": lambda ops, b, m, n, k: ops.fp8_linear(_U8(m, k), _U8(n, k), _F(1), _F(1), b, out_dtype=torch.float16),
+    "fp8_linear_max": lambda ops, b, m, n, k: ops.fp8_linear_max(_U8(m, k), _U8(n, k), _F(1), _F(1), b, _F(1), torch.float16),
+    "fp8_linear_panels": lambda ops, b, m, n, k: ops.fp8_linear_panels(_U8(k // 64, m, 64), _U8(n, k), _F(1), _F(1), b, None, torch.float16),
+    "fp8_linear_gated": lambda ops, b, m, n, k: ops.fp8_linear_gated(_U8(m, k), _U8(n, k), _F(1), _F(1), b, _F(1, n), _F(m, n), max(m, 1)),
+    "fp8_linear_gated_panels": lambda ops, b, m, n, k: ops.fp8_linear_gated_panels(_U8(k // 64, m, 64), _U8(n, k), _F(1), _F(1), b, _F(1, n), _F(m, n), max(m, 1)),
+    "fp8_linear_codes": lambda ops, b, m, n, k: ops.fp8_linear_codes(_U8(m, k), _U8(n, k), _F(1), _F(1), b, _F(1)),
+    "fp8_linear_codes_panels": lambda ops, b, m, n, k: ops.fp8_linear_codes_panels(_U8(k // 64, m, 64), _U8(n, k), _F(1), _F(1), b, _F(1)),
+    "weight_only_linear": lambda ops, b, m, n, k: ops.weight_only_linear(torch.zeros(m, k, dtype=torch.float16), _U8(n, k), _F(n), b),
+    "w4a4_linear": lambda ops, b, m, n, k: ops.w4a4_linear(torch.zeros(m, k // 8, dtype=torch.int32), _U8(n, k // 2), _F(m, k // 64), _F(n, k // 64), b, torch.float16),
+    "w4a4_linear_codes": lambda ops, b, m, n, k: ops.w4a4_linear_codes(_U8(m, k), _U8(n, k), _F(k // 64, m), _F(k // 64, n), b, torch.float16),
+}
+
+
+@pytest.mark.parametrize("name", LINEARS)
+def test_linears_refuse_a_bias_that_ends_before_the_outputs(ops, monkeypatch, name):
+    monkeypatch.setattr(ops, "sq_quant", lambda x, pre, scale: torch.zeros(x.shape, dtype=torch.int8))
+    with pytest.raises(ValueError, match="bias must have N elements"):
+        LINEARS[name](ops, torch.zeros(63, dtype=torch.float16), 4, 64, 128)
+
+
+def test_no_bias_is_read_for_32_bit_sums_or_no_rows(ops, monkeypatch):
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    for m, bias, dt in ((4, torch.zeros(3, dtype=torch.int32), torch.int32), (0, torch.zeros(3, dtype=torch.float16), torch.float16), (4, torch.zeros(65).half(), torch.float16)):
+        with pytest.raises(pytest.fail.Exception, match="lq_gemm_int8 was called"):
+            ops.int8_linear(_U8(m, 128), _U8(64, 128), _F(64), _F(1), bias, dt)
+
+
 SIZES = [(m, n, k) for m in (1, 2, 4, 5, 8, 9) for n in (64, 9216, 32 * 1536) for k in (1024, 1280, 1344, 1536, 3072, 12288)]
 
 

@@ -79,6 +79,17 @@ def test_int8_linear_is_its_two_operations(dev, dt, dynamic):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dynamic", [False, True])
+def test_int8_linear_refuses_a_bias_that_ends_before_the_outputs(dev, dynamic):
+    from lyradiff_amd import weights as W
+
+    lin = W.Int8Linear(torch.zeros(96, 320, dtype=torch.int8, device=dev), torch.ones(96, device=dev), torch.ones(1, device=dev), torch.ones(320, device=dev),
+                       torch.zeros(95, dtype=torch.float16, device=dev))
+    with pytest.raises(ValueError, match="bias must have N elements"):
+        lin.forward(torch.zeros(4, 320, dtype=torch.float16, device=dev), dynamic=dynamic)
+
+
+@pytest.mark.gpu
 def test_fp8_linear_from_state_dict(dev):
     from lyradiff_amd import weights as W
 
