@@ -237,10 +237,10 @@ __device__ __forceinline__ int cvt_i32_sat(float x) {
 // these very values), so rint(t/s) cannot leave [LO, HI] and the clamp is skipped.
 template <int HI> __device__ __forceinline__ constexpr float tie_margin() { return 2.0f * 2.4e-7f * (float)(HI + 1); }
 // quant8_round: the quotients rounded, as floats; true when they come from the divisions.
-template <int HI> __device__ __forceinline__ bool quant8_round(const float* t, float s, float r, bool slow, float* rq) {
+template <int HI, int N = 8> __device__ __forceinline__ bool quant8_round(const float* t, float s, float r, bool slow, float* rq) {
     float dev = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < N; ++i) {
         float qa = t[i] * r;
         rq[i] = __builtin_rintf(qa);
         dev = fmaxf(dev, fabsf(qa - rq[i]));  // largest distance from an integer (NaN differences drop out)
@@ -248,7 +248,7 @@ template <int HI> __device__ __forceinline__ bool quant8_round(const float* t, f
     const bool risky = slow | !(dev <= 0.5f - tie_margin<HI>());
     if (__builtin_expect(risky, 0)) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) rq[i] = __builtin_rintf(t[i] / s);
+        for (int i = 0; i < N; ++i) rq[i] = __builtin_rintf(t[i] / s);
     }
     return risky;
 }
@@ -267,29 +267,22 @@ __device__ __forceinline__ void quant8(const float* t, float s, float r, bool sl
 // The dynamic per-token case: every |t[i]| <= amax and s = fl(amax / 127), so |t[i] / s| stays below 127.00002
 // and nothing needs clamping; the conversion writes its low byte straight into the packed result
 // (sub-dword destination select), which saves the clamp and the byte shuffles.  NaN -> 0 as above.
+template <int N> __device__ __forceinline__ void quant_pack_unclamped(const float* t, float s, float r, bool slow, u32* words) {
+    float rq[N];
+    quant8_round<127, N>(t, s, r, slow, rq);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        u32& w = words[i / 4];
+        if (i % 4 == 0) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD" : "=v"(w) : "v"(rq[i]));
+        if (i % 4 == 1) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(w) : "v"(rq[i]));
+        if (i % 4 == 2) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(w) : "v"(rq[i]));
+        if (i % 4 == 3) asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(w) : "v"(rq[i]));
+    }
+}
 __device__ __forceinline__ uint2 quant8_pack_unclamped(const float* t, float s, float r, bool slow) {
-    float rq[8], dev = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        float qa = t[i] * r;
-        rq[i] = __builtin_rintf(qa);
-        dev = fmaxf(dev, fabsf(qa - rq[i]));
-    }
-    const bool risky = slow | !(dev <= 0.5f - tie_margin<127>());
-    if (__builtin_expect(risky, 0)) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) rq[i] = __builtin_rintf(t[i] / s);
-    }
-    uint2 o;
-    asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD" : "=v"(o.x) : "v"(rq[0]));
-    asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(o.x) : "v"(rq[1]));
-    asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(o.x) : "v"(rq[2]));
-    asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(o.x) : "v"(rq[3]));
-    asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_0 dst_unused:UNUSED_PAD src0_sel:DWORD" : "=v"(o.y) : "v"(rq[4]));
-    asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_1 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(o.y) : "v"(rq[5]));
-    asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_2 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(o.y) : "v"(rq[6]));
-    asm("v_cvt_i32_f32_sdwa %0, %1 dst_sel:BYTE_3 dst_unused:UNUSED_PRESERVE src0_sel:DWORD" : "+v"(o.y) : "v"(rq[7]));
-    return o;
+    u32 w[2];
+    quant_pack_unclamped<8>(t, s, r, slow, w);
+    return make_uint2(w[0], w[1]);
 }
 // t[i] = fl(x[i] * f[i]) for the eight fp16 values of a 16-byte vector: the mixed-precision fma reads the
 // half operand directly (x*f + 0 rounds once, like convert-then-multiply; a zero product loses its sign,

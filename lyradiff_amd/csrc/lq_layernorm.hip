@@ -302,9 +302,10 @@ __global__ __launch_bounds__(SPLIT ? 384 : 256) void ln_quant_rows_kernel(uint8_
 // INT8, rows that a wavefront holds as a whole (lq_walk.h): it walks over rows with the vectors in registers, and requests the next row ahead of
 // this one's statistics.  What bounds it: vector instructions, beside the way of the first row (a sum of two tensors of 8192 x 640 takes
 // 4.0 us on this card, an empty launch 2.1).
-// us, the kernel above / this, f16, static scale: 8192 x 640 7.6 / 6.7, with residual and bias 11.5 / 8.4; 8192 x 768 7.8 / 7.5, 12.2 / 9.5; 4096 x 1152
-// 6.6 / 6.3, 9.7 / 8.0; 2048 x 1280 5.0 / 4.7, 6.5 / 5.8; 1024 x 1280 4.7 / 3.7, 5.9 / 4.3; 8192 x 1280 10.7 / 10.4, 18.1 / 14.1.  The sums in an order of
-// this layout's own, without the way through LDS: 8192 x 640 6.4, 8.1.  The residual's sums as packed f16: 9.1 -> 8.4.
+// us, the kernel above / this, f16, static scale: 8192 x 640 7.6 / 6.7, with residual and bias 11.4 / 8.4; 8192 x 768 7.9 / 7.5, 12.2 / 9.5; 4096 x 1152
+// 6.6 / 6.3, 9.8 / 8.1; 2048 x 1280 5.1 / 4.8, 6.7 / 5.9; 1024 x 1280 4.7 / 3.7, 5.9 / 4.2; 8192 x 1280 10.8 / 10.5, 18.0 / 14.1.  Per-token scales: 8192 x 640
+// 7.8 / 7.1, 11.7 / 8.8; 8192 x 1280 11.0 / 10.9, 18.2 / 14.5, bf16 without a residual 9.9 / 10.4, the one size of 1 to 65536 rows where it is behind.
+// The sums in an order of this layout's own, without the way through LDS: 8192 x 640 6.4, 8.1.  The residual's sums as packed f16: 9.1 -> 8.4.
 template <typename Tag, int NF, int TAIL, int QMODE, int RESID>
 __global__ __launch_bounds__(256) void ln_int8_walk_kernel(uint8_t* __restrict__ dst, void* __restrict__ dst2, float* __restrict__ scale_out,
                                                            const void* __restrict__ src, const void* __restrict__ residual,
@@ -421,7 +422,7 @@ __global__ __launch_bounds__(256) void ln_int8_walk_kernel(uint8_t* __restrict__
             if (amax <= 5.9604644775390625e-08f) s = 1.0f;
             if (lane == 0) scale_out[row] = s;
         }
-        Row::store_codes(dst, row, lane, h, s, fast_recip(s), scale_out_of_range(s));
+        Row::template store_codes<QMODE == 0>(dst, row, lane, h, s, fast_recip(s), scale_out_of_range(s));
         if (!more) break;
         row = next;
     }

@@ -145,8 +145,9 @@ __global__ __launch_bounds__(256) void sq_quant_rows_kernel(int8_t* __restrict__
 
 // Rows that a wavefront holds as a whole (lq_walk.h), 16-bit: the smoothing vector's share of a lane stays in registers, where staging it in LDS
 // puts a barrier and a second trip in front of every workgroup's first row; MODE as above.
-// us, f16 with a smoothing vector, per-token / static scales, the kernel above -> this: 1024 x 1280 3.7 -> 3.2, 3.4 -> 2.9; 4096 x 640 4.0 -> 3.6, 3.7 -> 3.2;
-// 8192 x 640 5.9 -> 5.0, 5.2 -> 4.3; 8192 x 1280 8.3 -> 7.7, 7.7 -> 6.8; an empty launch 2.1.  The same bits.
+// us, f16 with a smoothing vector, per-token / static scales, the kernel above -> this: 1024 x 1280 3.5 -> 3.1, 3.4 -> 2.9; 4096 x 640 4.0 -> 3.5, 3.8 -> 3.3;
+// 8192 x 640 5.7 -> 4.7, 5.3 -> 4.3; 8192 x 768 6.0 -> 5.2, 5.6 -> 4.9; 4096 x 1152 4.9 -> 4.4, 4.7 -> 4.2; 8192 x 1280 8.1 -> 7.2, 7.6 -> 6.9; an empty launch
+// 2.1.  Given per-row scales as static ones (8192 x 640 5.4 -> 4.4), bf16 within 0.2 of f16, without a vector no slower.  The same bits.
 template <typename Tag, int NF, int TAIL, int MODE>
 __global__ __launch_bounds__(256) void sq_quant_walk_kernel(int8_t* __restrict__ dst, float* __restrict__ scale_out, const void* __restrict__ src,
                                                             const float* __restrict__ pre, const float* __restrict__ in_scale, u32 rows) {
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(256) void sq_quant_walk_kernel(int8_t* __restrict__
         } else if constexpr (MODE == 1) {
             s = in_scale[row];
         }
-        Row::store_codes(dst, row, lane, t, s, fast_recip(s), scale_out_of_range(s));
+        Row::template store_codes<MODE != 2>(dst, row, lane, t, s, fast_recip(s), scale_out_of_range(s));
         if (!more) break;
         row = next;
     }

@@ -6,27 +6,21 @@
 
 namespace lq {
 
-// int8 codes of N values (see quant8_round), two or four to the last word
-template <int N> __device__ __forceinline__ void walk_quant_s8(const float* t, float s, float r, bool slow, u32* words) {
-    float rq[N], dev = 0.0f;
+// int8 codes of N values, two or four to the last word; CLAMP false: s is the values' own largest over 127 (quant_pack_unclamped)
+template <int N, bool CLAMP> __device__ __forceinline__ void walk_quant_s8(const float* t, float s, float r, bool slow, u32* words) {
+    if constexpr (!CLAMP) quant_pack_unclamped<N>(t, s, r, slow, words);
+    else {
+        float rq[N];
+        quant8_round<127, N>(t, s, r, slow, rq);
+        int q[(N + 3) / 4 * 4] = {};
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const float qa = t[i] * r;
-        rq[i] = __builtin_rintf(qa);
-        dev = fmaxf(dev, fabsf(qa - rq[i]));
+        for (int i = 0; i < N; ++i) {
+            const int v = cvt_i32_sat(rq[i]);
+            q[i] = v < -128 ? -128 : (v > 127 ? 127 : v);
+        }
+#pragma unroll
+        for (int i = 0; i < N; i += 4) words[i / 4] = pack4_s8(q[i], q[i + 1], q[i + 2], q[i + 3]);
     }
-    if (__builtin_expect(slow | !(dev <= 0.5f - tie_margin<127>()), 0)) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) rq[i] = __builtin_rintf(t[i] / s);
-    }
-    int q[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const int v = cvt_i32_sat(rq[i]);
-        q[i] = v < -128 ? -128 : (v > 127 ? 127 : v);
-    }
-#pragma unroll
-    for (int i = 0; i < N; i += 4) words[i / 4] = pack4_s8(q[i], q[i + 1], i + 2 < N ? q[i + 2 < N ? i + 2 : 0] : 0, i + 3 < N ? q[i + 3 < N ? i + 3 : 0] : 0);
 }
 
 template <typename Tag, int NF, int TAIL> struct WalkRow {
@@ -83,16 +77,16 @@ template <typename Tag, int NF, int TAIL> struct WalkRow {
             o[8 * NF + i] = f.x; o[8 * NF + i + 1] = f.y;
         }
     }
-    static __device__ __forceinline__ void store_codes(void* base, size_t row, int lane, const float* t, float s, float r, bool slow) {
+    template <bool CLAMP> static __device__ __forceinline__ void store_codes(void* base, size_t row, int lane, const float* t, float s, float r, bool slow) {
         uint8_t* o = static_cast<uint8_t*>(base) + row * DIM;
 #pragma unroll
         for (int i = 0; i < NF; ++i) {
             u32 w[2];
-            walk_quant_s8<8>(t + 8 * i, s, r, slow, w);
+            walk_quant_s8<8, CLAMP>(t + 8 * i, s, r, slow, w);
             *reinterpret_cast<uint2*>(o + i * 512 + lane * 8) = make_uint2(w[0], w[1]);
         }
         u32 w;
-        walk_quant_s8<TAIL>(t + 8 * NF, s, r, slow, &w);
+        walk_quant_s8<TAIL, CLAMP>(t + 8 * NF, s, r, slow, &w);
         if constexpr (TAIL == 2) *reinterpret_cast<unsigned short*>(o + NF * 512 + lane * 2) = (unsigned short)w;
         else *reinterpret_cast<u32*>(o + NF * 512 + lane * 4) = w;
     }
