@@ -1,12 +1,13 @@
-"""FP8 and INT8 GEMMs of few tiles, whose wavefront groups share k out: every form at the edges of its range (remainders of rows and
-columns, the smallest k, activations as rows and as k-panels) and the epilogues of the FLUX blocks, against 64-bit references."""
+"""FP8 and INT8 GEMMs of few tiles, whose wavefront groups share k out or whose eight wavefronts walk 128-byte k-tiles: every form at the edges of
+its range (remainders of rows and columns, the smallest k, activations as rows and as k-panels) and the epilogues of the FLUX blocks, against
+64-bit references."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
-# (m, n, k): 32x32, 32x64 (k a multiple of 256), 64x128, 128x128 (a multiple of 128), and k that no form can share; 128x128 shared from
-# k = 2048 up, in 224 tiles, 256 and 264
+# (m, n, k): 32x32, 32x64 (k a multiple of 256), 64x128, 128x128 (a multiple of 128), and k that no form takes; eight wavefronts on 224, 256 and
+# 264 tiles of 128x128, the last as 192x128
 SIZES = [(1, 32, 1280), (33, 3072, 1280), (77, 3040, 1536), (65, 9216, 1152), (190, 9248, 1152), (333, 9216, 1152), (100, 12320, 2176),
          (300, 1056, 1088), (1000, 3552, 2048), (1024, 4096, 2176), (1000, 4128, 2048)]
 
@@ -90,8 +91,10 @@ def test_a_cached_tactic_stands(dev):
 
 
 # tiles of 128x128 and 192x128 in 128-byte k-tiles: one round of either, one tile less and more than a round of the former, k from where INT8
-# takes them on, rows and columns that leave tiles partly filled
-@pytest.mark.parametrize("m,n,k", [(6000, 640, 640), (8191, 608, 768), (8192, 640, 1024), (2040, 2048, 1280), (2049, 2048, 1280), (1345, 3040, 1152)])
+# takes them on, rows and columns that leave tiles partly filled; two rounds, which k-panels and at short k more than scales and bias leave to
+# other tiles
+@pytest.mark.parametrize("m,n,k", [(6000, 640, 640), (8191, 608, 768), (8192, 640, 1024), (2040, 2048, 1280), (2049, 2048, 1280), (1345, 3040, 1152),
+                                   (900, 9184, 1152), (1000, 9216, 2560)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
 def test_forms_of_eight_wavefronts(dev, m, n, k, dt):
     from lyradiff_amd import ops

@@ -70,10 +70,10 @@ def test_fused_residual_bias_layernorm_int8(ops, dev, dt, with_bias):
     close_codes(q.cpu().numpy(), q_ref, "fused residual layernorm int8")
 
 
-# rows that share a wavefront: fewer than wavefronts, one more than they are, a last turn that only some have; the four widths that are walked
-# this way and, behind the last, one that is not
+# the four widths that 4096 wavefronts walk over, with fewer rows than these and with a second turn that one, some or all of them have (the
+# residual sum of the row requested ahead, a second store of everything), and one that is not walked
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
-@pytest.mark.parametrize("rows,dim", [(1, 640), (2049, 640), (4100, 768), (3, 1152), (2050, 1280), (5, 1024)])
+@pytest.mark.parametrize("rows,dim", [(1, 640), (2049, 640), (4097, 640), (8192, 640), (4100, 768), (3, 1152), (4099, 1152), (2050, 1280), (4101, 1280), (5, 1024)])
 @pytest.mark.parametrize("dynamic", [False, True])
 @pytest.mark.parametrize("residual", ["none", "residual", "bias"])
 def test_layernorm_int8_several_rows_a_wavefront(ops, dev, dt, rows, dim, dynamic, residual):
@@ -112,6 +112,30 @@ def test_layernorm_int8_has_the_modulated_layernorms_statistics(ops, dev, dt, ro
     assert torch.equal(q, ops.sq_quant(y, pre, s_in))
     want, scale = ops.sq_quant_dynamic(y, pre)
     assert torch.equal(qd, want) and torch.equal(sd, scale)
+
+
+# An infinity or a NaN in a row, among the columns of the full passes or behind them, leaves codes of 0 and a scale of 1 in that row, and nothing in the
+# rows that its wavefront walks over before and after it.
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("dim", [640, 768, 1152, 1280, 1024])
+@pytest.mark.parametrize("residual", [False, True])
+def test_layernorm_int8_nan_and_inf_rows(ops, dev, dt, dim, residual):
+    rows, t = 3 * 4096 + 1, TORCH_DT[dt]
+    g = torch.Generator(device=dev).manual_seed(dim)
+    x, res = (torch.randn(rows, dim, generator=g, device=dev).to(t) for _ in range(2))
+    gamma, beta, pre = torch.ones(dim, dtype=t, device=dev), torch.zeros(dim, dtype=t, device=dev), 0.5 + torch.rand(dim, generator=g, device=dev)
+    call = lambda x, s: ops.layernorm_int8(x, gamma, beta, pre, s, res if residual else None)
+    s_in = torch.full((1,), 0.02, device=dev)
+    (q0, _, _), (d0, s0, _) = call(x, s_in), call(x, None)
+    bad = {4096: (3, "nan"), 4097: (dim - 1, "nan"), 4098: (0, "inf"), 4099: (dim - 2, "-inf"), 8191: (dim // 2, "inf"), 12288: (dim - 1, "inf")}
+    for row, (col, v) in bad.items():
+        x[row, col] = float(v)
+    (q, _, _), (d, s, h) = call(x, s_in), call(x, None)
+    rest = torch.ones(rows, dtype=torch.bool, device=dev)
+    rest[list(bad)] = False
+    assert torch.equal(q[rest], q0[rest]) and torch.equal(d[rest], d0[rest]) and torch.equal(s[rest], s0[rest])
+    assert not q[~rest].any() and not d[~rest].any() and bool((s[~rest] == 1).all())
+    assert (h is None) if not residual else torch.equal(h.isfinite(), (x + res).isfinite())
 
 
 @pytest.mark.parametrize("dt", ["bf16", "f16"])

@@ -34,9 +34,9 @@ def test_sq_dynamic_quant(ops, dev, dt, m, k):
     assert np.array_equal(s2.cpu().numpy(), s2_ref) and np.array_equal(q2.cpu().numpy(), q2_ref)
 
 
-# widths that a wavefront holds as a whole: one row, as many as wavefronts and one more, a second turn that some of them have
+# widths that a wavefront holds as a whole: one row, as many as the 4096 wavefronts, a second turn that one or some of them have
 @pytest.mark.parametrize("dt", ["f16", "bf16"])
-@pytest.mark.parametrize("m,k", [(1, 640), (4097, 640), (5000, 768), (4096, 1152), (70, 1280)])
+@pytest.mark.parametrize("m,k", [(1, 640), (4097, 640), (5000, 768), (4096, 1152), (4097, 1152), (70, 1280), (4099, 1280)])
 def test_sq_quant_rows_of_whole_wavefronts(ops, dev, dt, m, k):
     x = make_outlier_acts(m, k, 8, 20.0, TORCH_DT[dt], 2000 + m + k)
     pre = (torch.rand(k, generator=rng_t(9)) * 1.5 + 0.25).float()
@@ -66,6 +66,27 @@ def test_sq_dynamic_nan_and_inf_rows(ops, dev, k):
         q_ref, s_ref = O.sq_dynamic_quant(x.numpy(), None if pre is None else pre.numpy())
         assert np.array_equal(s.cpu().numpy(), s_ref, equal_nan=True)
         assert np.array_equal(q.cpu().numpy(), q_ref)
+
+
+# the same in rows that 4096 wavefronts walk over, special values among the columns of the full passes and behind them, with given scales too
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("k", [640, 768, 1152, 1280])
+def test_sq_nan_and_inf_rows_of_whole_wavefronts(ops, dev, dt, k):
+    m = 4096 + 4097
+    x = (torch.randn(m, k, generator=rng_t(k)) * 3).to(TORCH_DT[dt])
+    for row, col, v in ((1, 5, "nan"), (4097, k - 1, "nan"), (4098, 7, "inf"), (4099, k - 3, "-inf"), (4100, 9, "-inf"), (4100, k - 1, "nan"), (8192, 0, "inf")):
+        x[row, col] = float(v)
+    x[4101, :] = float("nan")
+    one, each = torch.tensor([0.02]), 0.01 + 0.1 * torch.rand(m, generator=rng_t(10))
+    each[5], each[4102], each[4103] = float("inf"), float("nan"), 0.0
+    for pre in (None, (torch.rand(k, generator=rng_t(3)) + 0.5).float()):
+        on, p_np = (None if pre is None else pre.to(dev)), (None if pre is None else pre.numpy())
+        q, s = ops.sq_quant_dynamic(x.to(dev), on)
+        q_ref, s_ref = O.sq_dynamic_quant(to_np_f32(x), p_np)
+        assert np.array_equal(s.cpu().numpy(), s_ref, equal_nan=True) and np.array_equal(q.cpu().numpy(), q_ref)
+        for scale, per_token in ((one, False), (each, True)):
+            q = ops.sq_quant(x.to(dev), on, scale.to(dev), per_token)
+            assert np.array_equal(q.cpu().numpy(), O.sq_input_quant(to_np_f32(x), p_np, scale.numpy(), per_token))
 
 
 def test_sq_dynamic_zero_rows(ops, dev):

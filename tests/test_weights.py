@@ -76,6 +76,12 @@ def test_int8_linear_is_its_two_operations(dev, dt, dynamic):
                                  ("weight_rows32", w.t(), ValueError), ("bias", lin.weight_scale.double(), TypeError), ("weight_scale", None, TypeError)):
             with pytest.raises(error):
                 W.Int8Linear(**{**vars(lin), name: bad}).forward(x, dynamic=dynamic)
+        no_scale = W.Int8Linear(**{**vars(lin), "input_quant_scale": None})
+        if dynamic:
+            assert torch.equal(no_scale.forward(x, dynamic=True), want)
+        else:
+            with pytest.raises(TypeError):
+                no_scale.forward(x)
 
 
 @pytest.mark.gpu
