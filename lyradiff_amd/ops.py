@@ -34,10 +34,12 @@ def _chk(t: torch.Tensor, name: str, dtypes=None) -> torch.Tensor:
 
 def _chk_bias(bias, dtype, n: int, m: int) -> None:
     """bias of a linear of N outputs, or None; a longer one has its first N values used.  A kernel would read a shorter one past its end."""
-    if bias is not None:
+    if bias is None:
+        return
+    if not isinstance(bias, _Tensor) or not bias.is_cuda or not bias.is_contiguous() or bias.dtype is not dtype:
         _chk(bias, "bias", (dtype,))
-        if bias.numel() < n and m:
-            raise ValueError("bias must have N elements")
+    if bias.numel() < n and m:
+        raise ValueError("bias must have N elements")
 
 
 def _ptr(t):
