@@ -25,11 +25,10 @@
 // Measured (settled, random operands, bf16; in parentheses before the last paragraph's changes, same run, then the library attention):
 // 24 heads of 128, 4608 tokens 257 us = 1.0 PFLOP/s (264; 506), 6912 tokens 576 us (596; 908), 1600 tokens 44.7 us (45.9; 135), 1000 tokens
 // 23.7 us (24.2); 2 x 10 heads of 64, 4096 tokens 122.7 us (125.5; 190).  NW == 4 at 24 x 4608 tokens of 128: 299 us; NW == 8 at 64: 147 us.
-// What was measured and is not here (4608 tokens, beside 257 us): a rescaled output only where the maximum grew by more than 2^8, 239 us, but
-// the error against 64 bits goes from 1.93e-3 to 2.31e-3, since the largest probabilities are then rounded; the rescaling moved between the
-// matrix instructions, 252; softmax and matrix instructions mixed in one wavefront's stream, 286; tiles of 128 keys, 254.
-// The row sum of the fp32 probabilities takes as long as one of the rounded ones, and makes the error against 64 bits that of the library
-// attention (bf16, 4608 tokens, 2-norm: 2.264e-3 both).
+// Error against 64 bits, 2-norm, standard normal operands, 24 heads of 128: bf16 2.22e-3 at 1000 tokens, 2.27e-3 at 4608 (the library
+// attention too), 2.29e-3 at 6912; f16 2.7e-4 to 2.9e-4.  The row sum is that of the fp32 probabilities, which takes as long as one of the rounded ones.
+// What was measured and is not here (4608 tokens, beside 257 us): a rescaled output only where the maximum grew by more than 2^8, 239 us, but a
+// fifth more error, since the largest probabilities are then rounded; softmax and matrix instructions mixed in one wavefront's stream, 286.
 #include "lq_common.h"
 
 namespace lq {
@@ -444,7 +443,8 @@ template <typename Tag, int DH, int NW> static int launch_attention(AttnParams p
 template <typename Tag> static int attention_typed(const AttnParams& p, int head_dim, hipStream_t st) {
     if (head_dim == 64) return launch_attention<Tag, 64, 4>(p, st);
     // Blocks of 128 queries, one workgroup per CU or fewer: spread over the chip.  From there on the phased form with 256
-    // queries per workgroup (24 heads, us, NW == 4 / NW == 8: 1000 tokens 25 / 33, 1600 tokens 53 / 45, 4608 tokens 299 / 261).
+    // queries per workgroup (24 heads, us, NW == 4 / NW == 8: 1000 tokens 27.6 / 34.8, 1200 tokens 32.8 / 40.5, 1365 tokens 50.6 / 45.5, 1600 tokens
+    // 57.3 / 51.0, 4608 tokens 310 / 273, 6912 tokens 677 / 597).
     const long long small = (long long)p.batch * p.heads * ((p.sq + 127) / 128);
     return small <= device_cu_count() ? launch_attention<Tag, 128, 4>(p, st) : launch_attention<Tag, 128, 8>(p, st);
 }

@@ -41,7 +41,8 @@ template <typename OutTag> static int run_fp8_as(GemmParams p, hipStream_t st) {
         t = few_tiles_form(p.m, 0, p.n, p.k, p.a_panel == 0 && (plain_epilogue || p.k >= 2560));
         if (t >= SMALL_32x32_K4) return run_small(K_FP8, p, out_enum<OutTag>(), t, st);
     }
-    if (t == 1 && (p.kb % 128 != 0 || p.a_panel)) t = 0;  // the 128-byte k-tile needs k % 128 == 0 and a row-major activation
+    // The 128-byte k-tile needs k % 128 == 0.  On k-panels, whose cache lines are whole in any k-tile, tactic 0 has the same bits and leads (4608x12288x3072 151 / 170 us, 4608x3072x12288 131 / 145).
+    if (t == 1 && (p.kb % 128 != 0 || p.a_panel)) t = 0;
     // The per-shape cache is filled by timing the plain epilogue.  With one wavefront per SIMD nothing runs beside tactic 6's
     // epilogue: one that does more than scale and bias (activation, output maximum, codes, gate, residual) costs 13-18 us
     // per 256x256 tile there (transcendentals, or one exposed memory round trip per group of rows) and next to nothing with

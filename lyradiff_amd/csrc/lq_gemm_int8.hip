@@ -45,7 +45,8 @@ template <typename OutTag> static int run_int8(GemmParams p, hipStream_t st) {
         if (form >= SMALL_32x32_K4) return run_small(K_INT8, p, out_enum<OutTag>(), form, st);
         if (form >= 0) t = form;
     }
-    if (t == 1 && (p.kb % 128 != 0 || p.a_panel)) t = 0;  // the 128-byte k-tile needs k % 128 == 0 and a row-major activation
+    // The 128-byte k-tile needs k % 128 == 0.  On k-panels, whose cache lines are whole in any k-tile, tactic 0 has the same bits and leads (4608x12288x3072 174 / 179 us, 4608x3072x12288 147 / 153).
+    if (t == 1 && (p.kb % 128 != 0 || p.a_panel)) t = 0;
     if (t == 7) {  // the persistent form of tactic 6 where it applies, tactic 6 itself elsewhere
         const int rc = launch_persist_int8(p, out_enum<OutTag>(), st);
         if (rc != 1) return rc;

@@ -1,4 +1,4 @@
-// 8-bit GEMMs whose tiles leave most of the chip idle: the forms of GemmKernel whose wavefront groups share k out.
+// 8-bit GEMMs of few tiles: the forms of GemmKernel whose wavefront groups share k out, and those whose eight wavefronts walk 128-byte k-tiles.
 //
 // What bounds them: a workgroup alone on a CU takes 0.17 us (64x64) to 0.3 us (128x256) per 64-byte k-tile whatever it computes --
 // the barrier, the LDS round trip of the fragments, the transfers' issue and the matrix instructions follow each other -- and walks k by
@@ -12,6 +12,8 @@
 //     22.6 / 19.4, 4096x640x2560 13.7 / 12.4 / 11.4).  192x128, general / now: FP8 512x9216x3072 20.3 / 16.7, 700x12288x3072 34.5 / 30.4 (two
 //     rounds); INT8 8192x640x2560 21.2 / 17.1, 4096x1280x5120 33.4 / 29.6.  Three or four stages, four wavefronts of 64x64 in place of
 //     eight of 64x32, level; 256x128 tiles 20.7 where 192x128 take 17.1.
+// The second kind adds up k in one chain where k-shared groups add two or four: no other error against 64 bits in FP8 (2-norm, one chain and
+// two alike: 333x9216x3072 bf16 1.6624e-3, 1024x3072x12288 f16 2.0735e-4, most of it the output's own rounding).
 // More than one round of the second kind: for a row-major activation, with a residual, an activation function, gates or codes in the epilogue
 // from k = 2560 up.  Two workgroups of four wavefronts per CU overlap one's epilogue with the other's walk, and k-panels take the cache
 // lines' advantage away (us, four wavefronts / two rounds of these -- row-major, scales and bias: FP8 1024x9216x3072 37.9 / 32.7, x1152 18.4 /

@@ -629,7 +629,7 @@ def test_fp8_panel_ops_under_stream_capture_and_argument_checks(ops, dev):
     assert lib.lq_fp8_amax_cast_panels(buf.data_ptr(), sc.data_ptr(), x.data_ptr(), 2, 8, 96, 0) < 0  # k % 64 != 0
     assert lib.lq_fp8_gelu_cast_panels(buf.data_ptr(), sc.data_ptr(), x.data_ptr(), 2, 8, 96, sc.data_ptr(), None, 0) < 0
     assert lib.lq_fp8_amax_cast_panels(buf.data_ptr(), sc.data_ptr(), x.data_ptr(), 2, 0, 64, 0) == 0  # empty
-    with ops.gemm_thread_tactic(1):  # the 128-byte k-tile configuration reads row-major activations only: another one runs
+    with ops.gemm_thread_tactic(1):  # on k-panels another configuration runs in place of the 128-byte k-tiles
         w = ops.repack_weight(ops.fp8_quant((torch.randn(256, 192, generator=g) * 0.05).bfloat16().to(dev))[0])
         qp, sp = ops.fp8_quant_panels(x)
         assert torch.equal(ops.fp8_linear_panels(qp, w, sp, sp, None), ops.fp8_linear(qa, w, sa, sa, None, False, None, 0.0, torch.bfloat16))
