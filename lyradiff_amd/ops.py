@@ -534,8 +534,10 @@ def sq_linear(x, pre_quant_scale, input_quant_scale, w_rows32, weight_scale, bia
                                                and input_quant_scale.is_contiguous() and input_quant_scale.numel() == 1))):
         c = torch.empty(m, n, dtype=dt, device=x.device)
         work = torch.empty(m * k if input_quant_scale is not None else m * (k + 4), dtype=torch.int8, device=x.device)
-        _l.check(_l.load().lq_sq_linear(c.data_ptr(), x.data_ptr(), _DT[dt], pre_quant_scale.data_ptr(), _ptr(input_quant_scale), work.data_ptr(),
-                                        w_rows32.data_ptr(), weight_scale.data_ptr(), _ptr(bias), m, n, k, _stream()), "lq_sq_linear")
+        rc = _l.load().lq_sq_linear(c.data_ptr(), x.data_ptr(), _DT[dt], pre_quant_scale.data_ptr(), _ptr(input_quant_scale), work.data_ptr(),
+                                    w_rows32.data_ptr(), weight_scale.data_ptr(), _ptr(bias), m, n, k, _stream())
+        if rc:
+            _l.check(rc, "lq_sq_linear")
         return c
     if input_quant_scale is None:
         q, input_quant_scale = sq_quant_dynamic(x, pre_quant_scale)

@@ -104,10 +104,10 @@ class Int8Linear:
     bias: Optional[torch.Tensor] = None
 
     def forward(self, x: torch.Tensor, dynamic: bool = False) -> torch.Tensor:
-        # dynamic: per-token scales computed on the fly instead of the calibrated one, which the other mode does not do without
-        if not dynamic and self.input_quant_scale is None:
+        scale = None  # dynamic: per-token scales computed on the fly instead of the calibrated one, which the other mode does not do without
+        if not dynamic and (scale := self.input_quant_scale) is None:
             raise TypeError("input_quant_scale must be a torch.Tensor")
-        y = ops.sq_linear(_rows(x), self.pre_quant_scale, None if dynamic else self.input_quant_scale, self.weight_rows32, self.weight_scale, self.bias)
+        y = ops.sq_linear(_rows(x), self.pre_quant_scale, scale, self.weight_rows32, self.weight_scale, self.bias)
         return _shaped(y, x)
 
 
