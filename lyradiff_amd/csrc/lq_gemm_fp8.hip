@@ -170,6 +170,8 @@ static long pair_tiles(int m, int m2, int n, int rows, int cols) {
 // up to 256 128x256 tiles behind full rounds 18.
 static int launch_form(int m, int m2, int n, int k, bool plain, bool persist, float* cost) {
     const long t256 = pair_tiles(m, m2, n, 256, 256), last256 = t256 % 256;
+    // More than one round of eight wavefronts: the rule knows no layout here.  Pairs come as k-panels, where two rounds are level at long k with no
+    // more than scales and bias and behind otherwise (600 + 512 rows 9216x3072, us, four wavefronts / two rounds: 44.7 / 41.8).
     if (t256 < 192) return few_tiles_form(m, m2, n, k, plain && k >= 2560, cost);
     *cost = (float)((t256 + 255) / 256) * (persist && t256 > 256 ? 35.0f : 38.0f);
     const bool wide = (last256 != 0 && last256 < 128) || (!plain && t256 > 256);
